@@ -61,6 +61,8 @@ extern "C" emd_status emd_create(int device, emd_ctx **out) {
             hipMalloc(&ctx->d_dsmall, 64 * sizeof(double)) == hipSuccess &&
             hipHostMalloc(&ctx->h_small, 64 * sizeof(int), hipHostMallocDefault) == hipSuccess &&
             hipHostMalloc(&ctx->h_dsmall, 64 * sizeof(double), hipHostMallocDefault) == hipSuccess &&
+            hipHostMalloc(&ctx->h_mail, (EMD_MAIL_DATA + EMD_MAIL_MAX) * sizeof(int),
+                          hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess &&
             hipMalloc(&ctx->d_ljtab, EMD_LJ_TABLE_BYTES) == hipSuccess &&
             hipHostMalloc(&ctx->h_ljtab, EMD_LJ_TABLE_BYTES, hipHostMallocDefault) == hipSuccess &&
             hipEventCreateWithFlags(&ctx->ljtab_ev, hipEventDisableTiming) == hipSuccess;
@@ -69,6 +71,7 @@ extern "C" emd_status emd_create(int device, emd_ctx **out) {
     return EMD_ERR_ALLOC;
   }
   hipMemset(ctx->d_small, 0, 64 * sizeof(int));
+  memset(ctx->h_mail, 0, (EMD_MAIL_DATA + EMD_MAIL_MAX) * sizeof(int));
   // the allocation-free entry points' scratch: this device's copy
   if (emd_lj_scratch_setup(ctx) != EMD_OK) {
     emd_destroy(ctx);
@@ -88,8 +91,8 @@ extern "C" emd_status emd_create(int device, emd_ctx **out) {
   if (const char *e = getenv("EMD_FOLD_ONE")) ctx->fold_one = atoi(e) != 0;
   // host waits for counts: poll an event (1) or hipStreamSynchronize (0)
   if (const char *e = getenv("EMD_SPIN_WAIT")) ctx->spin_wait = atoi(e) != 0;
-  // exchange_halo of a small system (<= 16384 local + ghost atoms) in one
-  // launch (1) or as six scans with a host sync each (0)
+  // exchange_halo of a small system (<= HALO_ONE_MAX local atoms) in one
+  // launch (1) or as count, offset and emit kernels (0)
   if (const char *e = getenv("EMD_HALO_ONE")) ctx->halo_one = atoi(e) != 0;
   // binning of a small range (<= 7168 atoms, <= 4096 bins) in one launch
   if (const char *e = getenv("EMD_BIN_ONE")) ctx->bin_one = atoi(e) != 0;
@@ -111,6 +114,7 @@ extern "C" emd_status emd_destroy(emd_ctx *ctx) {
   if (ctx->d_dsmall) hipFree(ctx->d_dsmall);
   if (ctx->h_small) hipHostFree(ctx->h_small);
   if (ctx->h_dsmall) hipHostFree(ctx->h_dsmall);
+  if (ctx->h_mail) hipHostFree(ctx->h_mail);
   if (ctx->d_scan) hipFree(ctx->d_scan);
   if (ctx->d_tmp) hipFree(ctx->d_tmp);
   if (ctx->d_tmp2) hipFree(ctx->d_tmp2);
@@ -135,6 +139,21 @@ emd_status emd_wait(emd_ctx *ctx) {
   while ((e = hipEventQuery(ctx->wait_ev)) == hipErrorNotReady) {
   }
   EMD_HIP(ctx, e);
+  return EMD_OK;
+}
+
+emd_status emd_mail_wait(emd_ctx *ctx, const emd_mail &m, const int **payload) {
+  if (!ctx->spin_wait) EMD_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  // the stream is asked now and then, so that a failed kernel ends the wait
+  for (long spin = 1; __atomic_load_n(m.box, __ATOMIC_ACQUIRE) != m.seq; spin++) {
+    if (spin % 65536 != 0 && ctx->spin_wait) continue;
+    const hipError_t e = hipStreamQuery(ctx->stream);
+    if (e == hipErrorNotReady) continue;
+    EMD_HIP(ctx, e);
+    if (__atomic_load_n(m.box, __ATOMIC_ACQUIRE) != m.seq)
+      return emd_set_error(ctx, EMD_ERR_STATE, "a kernel ended without its counts");
+  }
+  *payload = m.box + EMD_MAIL_DATA;
   return EMD_OK;
 }
 

@@ -63,6 +63,11 @@ struct emd_ctx {
   // static scratch array (resolved once at emd_create)
   double *noalloc_scratch = nullptr;
 
+  // counts for the host: pinned, coherent memory that a kernel writes itself
+  // (emd_mail_post) and the host polls (emd_mail_wait)
+  int *h_mail = nullptr;       // [0] sequence number, [EMD_MAIL_DATA..] payload
+  int mail_seq = 0;
+
   // host waits: an event recorded on the stream and polled, so a wait for a
   // count ends as soon as the copy lands (no blocking-sync wake-up latency)
   hipEvent_t wait_ev = nullptr;
@@ -131,6 +136,27 @@ void emd_prof_end(emd_ctx *ctx, emd_prof_rec *rec);
 emd_status emd_ensure(emd_ctx *ctx, void **p, size_t *cap, size_t bytes);
 // wait until all work queued on the context's stream has completed
 emd_status emd_wait(emd_ctx *ctx);
+
+// A count that the host needs: the kernel that forms it writes it to the
+// context's mailbox (payload, then the sequence number) and the host polls
+// for that number, instead of a device-to-host copy (3 us on the GPU, plus
+// its submission) and an event behind it.  The host reads the count while
+// the kernel, or kernels queued after it, still run.  One message at a time:
+// each is waited for before the next is posted.
+constexpr int EMD_MAIL_DATA = 16;  // first payload int (the number has a line of its own)
+constexpr int EMD_MAIL_MAX = 48;
+struct emd_mail {
+  int *box;
+  int seq;
+};
+inline emd_mail emd_mail_next(emd_ctx *ctx) { return emd_mail{ctx->h_mail, ++ctx->mail_seq}; }
+// the payload of message m (valid until the next message is posted)
+emd_status emd_mail_wait(emd_ctx *ctx, const emd_mail &m, const int **payload);
+// device side, by one thread after it has written box[EMD_MAIL_DATA + ...]
+__device__ __forceinline__ void emd_mail_post(const emd_mail &m) {
+  __threadfence_system();
+  __hip_atomic_store(m.box, m.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 template <class T>
 inline emd_status emd_ensure_t(emd_ctx *ctx, T **p, size_t *cap, size_t count) {
   return emd_ensure(ctx, reinterpret_cast<void **>(p), cap, count * sizeof(T));
