@@ -17,8 +17,6 @@
 
 #include <type_traits>
 
-__global__ void k_max_int(const int *__restrict__ a, int n, int *__restrict__ out);
-
 // ------------------------------------------------------------------ binning
 // BinOp3D::bin (Kokkos_Sort.hpp) as used by binning_kksort.cpp:105-113: the
 // bin of an atom, clamped into the grid (an atom outside it raises the
@@ -94,6 +92,13 @@ struct bin_offsets_op {
   }
 };
 
+// sum and largest value only (no offsets kept)
+struct count_op {
+  const int *count;
+  __device__ int value(int i) const { return count[i]; }
+  __device__ void emit(int, int, int) const {}
+};
+
 __global__ void k_bin_scatter(const int *__restrict__ binid, int n, int *__restrict__ cursor,
                               int *__restrict__ permute) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -141,93 +146,79 @@ k_bin_order(const int *__restrict__ count, const int *__restrict__ offset, int n
 }
 
 // Small ranges (n <= BIN_ONE_MAX_N atoms, nbins <= BIN_ONE_MAX_BINS) in one
-// workgroup launch: bin ids, an LDS histogram, the exclusive scan of the
-// counts, an LDS scatter, then an insertion sort of each bin's slice of the
-// LDS permutation (ascending index: the radix path's order), the largest
-// count and the out-of-grid flag -- one launch instead of the key, sort,
-// bounds and max kernels.
+// workgroup launch: bin ids and an LDS histogram whose atomics also give each
+// atom a slot of its bin, the exclusive scan of the counts (after which the
+// largest count and the out-of-grid flag go to the host), the atoms put in
+// their slots in LDS, then each atom's place in its bin's slice as the number
+// of smaller indices there: one thread per atom, ~25 independent LDS reads
+// (mostly broadcasts) where one thread per bin sorting its slice by insertion
+// made a chain of ~170 dependent LDS reads and writes.  Bound: LDS latency
+// and the launch.  A call for the locals and ghosts of an LJ melt, host wait
+// included: 72 -> 13 us at 864 atoms (32 per bin), 75 -> 14 us at 2048; the
+// counting sort takes 16 us from 4000 atoms (8000 with ghosts) on.
 constexpr int BIN_ONE_THREADS = 1024;
 constexpr int BIN_ONE_MAX_BINS = 4096;
-constexpr int BIN_ONE_MAX_N = 7168;  // LDS: 2 x 16 KiB bin tables + 28 KiB permutation
+constexpr int BIN_ONE_MAX_N = 7168;  // LDS: 2 x 16 KiB bin tables, 8 B per atom
 
 __global__ void __launch_bounds__(BIN_ONE_THREADS)
 k_bin_one(const double *__restrict__ x, int r0, int n, double minx, double miny, double minz,
           double mulx, double muly, double mulz, int nbx, int nby, int nbz, int nbins,
           int *__restrict__ bincount, int *__restrict__ binoffsets, int *__restrict__ permute,
-          int *__restrict__ small) {
-  __shared__ int s_cnt[BIN_ONE_MAX_BINS];  // counts, then scatter cursors
+          emd_mail mail) {
+  __shared__ int s_cnt[BIN_ONE_MAX_BINS];
   __shared__ int s_off[BIN_ONE_MAX_BINS];
   __shared__ int s_perm[BIN_ONE_MAX_N];
-  __shared__ int s_w[BIN_ONE_THREADS / EMD_WAVE];
+  __shared__ unsigned short s_bin[BIN_ONE_MAX_N], s_slot[BIN_ONE_MAX_N];
+  __shared__ int s_w[2][BIN_ONE_THREADS / EMD_WAVE];
   __shared__ int s_err, s_max;
   const int tid = threadIdx.x, wid = tid / EMD_WAVE, lane = tid % EMD_WAVE;
   for (int b = tid; b < nbins; b += BIN_ONE_THREADS) s_cnt[b] = 0;
   if (tid == 0) { s_err = 0; s_max = 0; }
   __syncthreads();
-  // pass 1: histogram (the bin id is recomputed in pass 2, not stored)
-  auto bin_of = [&](int i, bool &bad) {
-    return bin_index(x + 3 * (size_t)(r0 + i), minx, miny, minz, mulx, muly, mulz, nbx, nby, nbz,
-                     bad);
-  };
   for (int i = tid; i < n; i += BIN_ONE_THREADS) {
     bool bad;
-    const int b = bin_of(i, bad);
+    const int b = bin_index(x + 3 * (size_t)(r0 + i), minx, miny, minz, mulx, muly, mulz, nbx,
+                            nby, nbz, bad);
     if (bad) s_err = 1;
-    atomicAdd(&s_cnt[b], 1);
+    s_bin[i] = (unsigned short)b;
+    s_slot[i] = (unsigned short)atomicAdd(&s_cnt[b], 1);
   }
   __syncthreads();
   // exclusive scan of the counts, 1024 bins per round
-  int carry = 0, mymax = 0;
-  for (int base = 0; base < nbins; base += BIN_ONE_THREADS) {
+  int carry = 0, mymax = 0, r = 0;
+  for (int base = 0; base < nbins; base += BIN_ONE_THREADS, r ^= 1) {
     const int b = base + tid;
     const int v = b < nbins ? s_cnt[b] : 0;
     mymax = v > mymax ? v : mymax;
     const int inc = emd_wave_incl_scan(v);
-    if (lane == EMD_WAVE - 1) s_w[wid] = inc;
+    if (lane == EMD_WAVE - 1) s_w[r][wid] = inc;
     __syncthreads();
-    int woff = 0, tot = 0;
+    int off = carry + inc - v;
 #pragma unroll
     for (int w = 0; w < BIN_ONE_THREADS / EMD_WAVE; w++) {
-      const int sw = s_w[w];
-      woff += (w < wid) ? sw : 0;
-      tot += sw;
+      const int sw = s_w[r][w];
+      off += (w < wid) ? sw : 0;
+      carry += sw;
     }
     if (b < nbins) {
-      const int off = carry + woff + inc - v;
       bincount[b] = v;
       binoffsets[b] = off;
       s_off[b] = off;
-      s_cnt[b] = off;  // scatter cursor
-    }
-    carry += tot;
-    __syncthreads();
-  }
-  atomicMax(&s_max, mymax);
-  // pass 2: scatter (any order), then sort each bin's slice
-  for (int i = tid; i < n; i += BIN_ONE_THREADS) {
-    bool bad;
-    const int b = bin_of(i, bad);
-    s_perm[atomicAdd(&s_cnt[b], 1)] = i;
-  }
-  __syncthreads();
-  for (int b = tid; b < nbins; b += BIN_ONE_THREADS) {
-    int *p = s_perm + s_off[b];
-    const int c = s_cnt[b] - s_off[b];
-    for (int k = 1; k < c; k++) {
-      const int v = p[k];
-      int m = k - 1;
-      while (m >= 0 && p[m] > v) {
-        p[m + 1] = p[m];
-        m--;
-      }
-      p[m + 1] = v;
     }
   }
+  mymax = emd_wave_max(mymax);
+  if (lane == 0) atomicMax(&s_max, mymax);
   __syncthreads();
-  for (int i = tid; i < n; i += BIN_ONE_THREADS) permute[i] = s_perm[i];
-  if (tid == 0) {
-    small[1] = s_max;
-    small[2] = s_err;
+  if (tid == 0) emd_scan_post(mail, n, s_max, &s_err);
+  for (int i = tid; i < n; i += BIN_ONE_THREADS) s_perm[s_off[s_bin[i]] + s_slot[i]] = i;
+  __syncthreads();
+  for (int k = tid; k < n; k += BIN_ONE_THREADS) {
+    const int v = s_perm[k];
+    const int b = s_bin[v], off = s_off[b], c = s_cnt[b];
+    int rank = 0;
+#pragma unroll 4
+    for (int m = 0; m < c; m++) rank += s_perm[off + m] < v;
+    permute[off + rank] = v;
   }
 }
 
@@ -251,6 +242,13 @@ __global__ void k_bin_gather(const int *__restrict__ perm, int r0, int n,
   tq[i] = q[s];
   ttype[i] = type[s];
   tid[i] = id[s];
+}
+
+// the counts and the lost-atom flag
+__global__ void k_bin_zero(int *__restrict__ count, int nbins, int *__restrict__ err) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < nbins) count[i] = 0;
+  if (i == 0) *err = 0;
 }
 
 __global__ void k_fill_int(int *p, int n, int v) {
@@ -280,14 +278,15 @@ __global__ void k_bin_copy_back(int r0, int n, const double *__restrict__ tx,
   id[r0 + i] = ti[i];
 }
 
-// common tail: largest count and out-of-grid flag to the host (the one sync
-// of a binning), then BinSort::sort of the range when asked
-static emd_status bin_finish(emd_ctx *ctx, emd_system *s, emd_bins *b, int r0, int n, int sort) {
-  EMD_HIP(ctx, hipMemcpyAsync(ctx->h_small + 1, ctx->d_small + 1, 2 * sizeof(int),
-                              hipMemcpyDeviceToHost, ctx->stream));
-  EMD_TRY(emd_wait(ctx));
-  b->max_count = ctx->h_small[1];
-  if (ctx->h_small[2])
+// common tail: largest count and out-of-grid flag from the message of the
+// counting pass (the one wait of a binning; the kernels behind that pass are
+// still running), then BinSort::sort of the range when asked
+static emd_status bin_finish(emd_ctx *ctx, emd_system *s, emd_bins *b, int r0, int n, int sort,
+                             const emd_mail &mail) {
+  const int *got = nullptr;
+  EMD_TRY(emd_mail_wait(ctx, mail, &got));
+  b->max_count = got[1];
+  if (got[2])
     return emd_set_error(ctx, EMD_ERR_OVERFLOW,
                          "emd_binning: an atom lies outside the bin grid (lost atom?)");
   if (sort && n > 0) {
@@ -347,35 +346,32 @@ extern "C" emd_status emd_binning(emd_ctx *ctx, emd_system *s, double dx_in, dou
   EMD_TRY(emd_ensure_int(ctx, &b->permute, &b->cap_range, n));
   EMD_TRY(emd_ensure_int(ctx, &b->binid, &cap_r2, n));
   b->cap_range = b->cap_range < cap_r2 ? b->cap_range : cap_r2;
+  const emd_mail mail = emd_mail_next(ctx);
   if (ctx->bin_one && n <= BIN_ONE_MAX_N && nbt <= BIN_ONE_MAX_BINS) {
     EMD_LAUNCH(ctx, "binning", k_bin_one, 1, BIN_ONE_THREADS, 0, s->x, r0, n, mn[0], mn[1], mn[2],
                mul[0], mul[1], mul[2], nb[0], nb[1], nb[2], (int)nbt, b->bincount,
-               b->binoffsets, b->permute, ctx->d_small);
-    return bin_finish(ctx, s, b, r0, n, sort);
+               b->binoffsets, b->permute, mail);
+    return bin_finish(ctx, s, b, r0, n, sort, mail);
   }
   // counting sort: counts, offsets (with cursors in scratch), scatter,
-  // per-bin ordering; the largest count and the lost-atom flag in d_small
+  // per-bin ordering; the scan posts the largest count and the lost-atom flag
   EMD_TRY(emd_ensure(ctx, &ctx->d_tmp2, &ctx->tmp2_cap, (size_t)nbt * sizeof(int)));
   int *cursor = static_cast<int *>(ctx->d_tmp2);
-  EMD_LAUNCH(ctx, "binning", k_fill_int, 1, 64, 0, ctx->d_small + 1, 2, 0);
-  EMD_LAUNCH(ctx, "binning", k_fill_int, emd_blocks(nbt, 256), 256, 0, b->bincount, (int)nbt, 0);
+  EMD_LAUNCH(ctx, "binning", k_bin_zero, emd_blocks(nbt, 256), 256, 0, b->bincount, (int)nbt,
+             ctx->d_small + 2);
   if (n > 0)
     EMD_LAUNCH(ctx, "binning", k_bin_count, emd_blocks(n, 256), 256, 0, s->x, r0, n, mn[0], mn[1],
                mn[2], mul[0], mul[1], mul[2], nb[0], nb[1], nb[2], b->binid, b->bincount,
                ctx->d_small + 2);
   EMD_TRY(emd_scan(ctx, bin_offsets_op{b->bincount, b->binoffsets, cursor}, (int)nbt,
-                   "binning_scan", nullptr));
+                   "binning_scan", ctx->d_small + 2, mail));
   if (n > 0)
     EMD_LAUNCH(ctx, "binning", k_bin_scatter, emd_blocks(n, 256), 256, 0, b->binid, n, cursor,
                b->permute);
   EMD_LAUNCH(ctx, "binning_order", k_bin_order,
              emd_blocks(nbt, BIN_ORDER_THREADS / EMD_WAVE), BIN_ORDER_THREADS, 0, b->bincount,
              b->binoffsets, (int)nbt, b->permute);
-  {
-    const int nbm = emd_blocks(nbt, 256) < 512 ? emd_blocks(nbt, 256) : 512;
-    EMD_LAUNCH(ctx, "binning", k_max_int, nbm, 256, 0, b->bincount, (int)nbt, ctx->d_small + 1);
-  }
-  return bin_finish(ctx, s, b, r0, n, sort);
+  return bin_finish(ctx, s, b, r0, n, sort, mail);
 }
 
 // bins of another binning (the reference's View<int***> bincount and
@@ -420,13 +416,11 @@ extern "C" emd_status emd_bins_import(emd_ctx *ctx, int nbinx, int nbiny, int nb
   if (n_range > 0)
     EMD_HIP(ctx, hipMemcpyAsync(b->permute, permute, (size_t)n_range * sizeof(int),
                                 hipMemcpyDeviceToDevice, ctx->stream));
-  EMD_LAUNCH(ctx, "bins_import", k_fill_int, 1, 64, 0, ctx->d_small + 1, 1, 0);
-  const int nbm = emd_blocks(nbt, 256) < 512 ? emd_blocks(nbt, 256) : 512;
-  EMD_LAUNCH(ctx, "bins_import", k_max_int, nbm, 256, 0, b->bincount, (int)nbt, ctx->d_small + 1);
-  EMD_HIP(ctx, hipMemcpyAsync(ctx->h_small + 1, ctx->d_small + 1, sizeof(int),
-                              hipMemcpyDeviceToHost, ctx->stream));
-  EMD_TRY(emd_wait(ctx));
-  b->max_count = ctx->h_small[1];
+  const emd_mail mail = emd_mail_next(ctx);
+  EMD_TRY(emd_scan(ctx, count_op{b->bincount}, (int)nbt, "bins_import", nullptr, mail, false));
+  const int *got = nullptr;
+  EMD_TRY(emd_mail_wait(ctx, mail, &got));
+  b->max_count = got[1];
   return EMD_OK;
 }
 
@@ -454,7 +448,7 @@ __global__ void __launch_bounds__(NB_THREADS)
 k_neigh(const double *__restrict__ x, const int *__restrict__ bincount,
         const int *__restrict__ binoffsets, const int *__restrict__ permute, neigh_geom g,
         int n_local, double cutsq, int newton, int *__restrict__ num, const int *__restrict__ row,
-        int pitch, int *__restrict__ entries, int *__restrict__ cursor, int *__restrict__ maxrow, int cap, int write_num) {
+        int pitch, int *__restrict__ entries, int *__restrict__ cursor, int cap, int write_num) {
 #pragma clang fp contract(off)
   __shared__ double s_x[NB_MAXC], s_y[NB_MAXC], s_z[NB_MAXC];
   __shared__ int s_j[NB_MAXC];
@@ -588,27 +582,6 @@ k_neigh(const double *__restrict__ x, const int *__restrict__ bincount,
   }
 }
 
-// longest row: block max, one atomic per block (atomics from every atom or
-// wavefront on one address serialise at the L2)
-__global__ void __launch_bounds__(256) k_max_int(const int *__restrict__ a, int n,
-                                                 int *__restrict__ out) {
-  __shared__ int s_m[4];
-  int m = 0;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-    m = a[i] > m ? a[i] : m;
-#pragma unroll
-  for (int o = EMD_WAVE / 2; o > 0; o >>= 1) {
-    const int t = __shfl_xor(m, o, EMD_WAVE);
-    m = t > m ? t : m;
-  }
-  if (__lane_id() == 0) s_m[threadIdx.x / EMD_WAVE] = m;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < 4; w++) m = s_m[w] > m ? s_m[w] : m;
-    if (m > 0) atomicMax(out, m);
-  }
-}
-
 // padded rows (pitch P) -> CSR rows, 16 lanes per row
 constexpr int COMPACT_LANES = 16;
 __global__ void __launch_bounds__(256)
@@ -657,7 +630,6 @@ extern "C" emd_status emd_neigh_build(emd_ctx *ctx, const emd_system *s, const e
   EMD_TRY(emd_ensure(ctx, &ctx->d_tmp2, &ctx->tmp2_cap, (size_t)(n + 1) * sizeof(int)));
   int *cursor = (int *)ctx->d_tmp2;
   if (n > 0) EMD_LAUNCH(ctx, "neigh_count", k_fill_int, emd_blocks(n, 256), 256, 0, nl->num, n, 0);
-  EMD_LAUNCH(ctx, "neigh_count", k_fill_int, 1, 64, 0, ctx->d_small + 4, 1, 0);
 
   // k_neigh launch: fill?, CSR row offsets (or null: rows at i * pitch),
   // pitch, entries, row capacity, record full row lengths in num?
@@ -667,11 +639,11 @@ extern "C" emd_status emd_neigh_build(emd_ctx *ctx, const emd_system *s, const e
       if (half)                                                                              \
         EMD_LAUNCH(ctx, name, (k_neigh<true, F>), nib, NB_THREADS, 0, s->x, b->bincount,     \
                    b->binoffsets, b->permute, g, n, cutsq, newton, nl->num, ROW, PITCH, ENT, \
-                   cursor, ctx->d_small + 4, CAP, WNUM);                                     \
+                   cursor, CAP, WNUM);                                                       \
       else                                                                                   \
         EMD_LAUNCH(ctx, name, (k_neigh<false, F>), nib, NB_THREADS, 0, s->x, b->bincount,    \
                    b->binoffsets, b->permute, g, n, cutsq, newton, nl->num, ROW, PITCH, ENT, \
-                   cursor, ctx->d_small + 4, CAP, WNUM);                                     \
+                   cursor, CAP, WNUM);                                                       \
     }                                                                                        \
   } while (0)
 
@@ -717,18 +689,20 @@ extern "C" emd_status emd_neigh_build(emd_ctx *ctx, const emd_system *s, const e
   }
   if (P == 0 || n == 0)
     NB_LAUNCH("neigh_count", false, nullptr, 0, nullptr, 0, 0);
-  // row offsets and the longest row
+  // the entries, the longest row and (CSR) the row offsets
+  int total = 0, maxrow = 0;
   if (n > 0) {
-    const int nbm = emd_blocks(n, 256) < 512 ? emd_blocks(n, 256) : 512;
-    EMD_LAUNCH(ctx, "neigh_offsets", k_max_int, nbm, 256, 0, nl->num, n, ctx->d_small + 4);
+    const emd_mail mail = emd_mail_next(ctx);
+    if (layout == EMD_NEIGH_2D)
+      EMD_TRY(emd_scan(ctx, count_op{nl->num}, n, "neigh_offsets", nullptr, mail, false));
+    else
+      EMD_TRY(emd_scan(ctx, row_offsets_op{nl->num, nl->row, n}, n, "neigh_offsets", nullptr,
+                       mail));
+    const int *got = nullptr;
+    EMD_TRY(emd_mail_wait(ctx, mail, &got));
+    total = got[0];
+    maxrow = got[1];
   }
-  int total = 0;
-  row_offsets_op op{nl->num, nl->row, n};
-  if (n > 0) EMD_TRY(emd_scan(ctx, op, n, "neigh_offsets", &total));
-  EMD_HIP(ctx, hipMemcpyAsync(ctx->h_small + 4, ctx->d_small + 4, sizeof(int),
-                              hipMemcpyDeviceToHost, ctx->stream));
-  EMD_TRY(emd_wait(ctx));
-  const int maxrow = ctx->h_small[4];
   nl->total = total;
   if (layout == EMD_NEIGH_2D) {
     const bool fits = P > 0 && maxrow <= P;

@@ -18,27 +18,35 @@ extern "C" const char *emd_last_error(const emd_ctx *ctx) { return ctx ? ctx->er
 extern "C" const char *emd_version(void) { return "examinimd-amd 0.1 (gfx950)"; }
 
 // ------------------------------------------------------------ scan helper
-__global__ void __launch_bounds__(1024) k_scan_blocks(int *bs, int nb, int *total) {
-  __shared__ int s_w[16];
-  __shared__ int s_carry;
-  if (threadIdx.x == 0) s_carry = 0;
-  __syncthreads();
+__global__ void __launch_bounds__(1024) k_scan_blocks(int *sums, int nb, const int *flag,
+                                                      emd_mail mail) {
+  __shared__ int s_w[2][16], s_m[16];
   const int wid = threadIdx.x / EMD_WAVE;
-  for (int base = 0; base < nb; base += 1024) {
-    int i = base + threadIdx.x;
-    int v = (i < nb) ? bs[i] : 0;
-    int inc = emd_wave_incl_scan(v);
-    if (__lane_id() == EMD_WAVE - 1) s_w[wid] = inc;
+  int carry = 0, most = 0, r = 0;
+  for (int base = 0; base < nb; base += 1024, r ^= 1) {
+    const int i = base + threadIdx.x;
+    const int v = (i < nb) ? sums[i] : 0;
+    const int m = (i < nb) ? sums[nb + i] : 0;
+    most = m > most ? m : most;
+    const int inc = emd_wave_incl_scan(v);
+    if (__lane_id() == EMD_WAVE - 1) s_w[r][wid] = inc;
     __syncthreads();
-    int woff = 0;
-    for (int w = 0; w < wid; w++) woff += s_w[w];
-    int carry = s_carry;
-    if (i < nb) bs[i] = carry + woff + inc - v;
-    __syncthreads();
-    if (threadIdx.x == 1023) s_carry = carry + woff + inc;
-    __syncthreads();
+    int off = carry + inc - v;
+#pragma unroll
+    for (int w = 0; w < 16; w++) {
+      const int sw = s_w[r][w];
+      off += w < wid ? sw : 0;
+      carry += sw;
+    }
+    if (i < nb) sums[i] = off;
   }
-  if (threadIdx.x == 0) total[0] = s_carry;
+  most = emd_wave_max(most);
+  if (__lane_id() == 0) s_m[wid] = most;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 16; w++) most = s_m[w] > most ? s_m[w] : most;
+    emd_scan_post(mail, carry, most, flag);
+  }
 }
 
 // ------------------------------------------------------------- context
