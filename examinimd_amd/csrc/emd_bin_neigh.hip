@@ -15,6 +15,7 @@
 // with an exclusive scan between them, as NeighborCSR does.
 #include "emd_internal.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 // ------------------------------------------------------------------ binning
@@ -441,6 +442,14 @@ constexpr int NB_WAVES = NB_THREADS / EMD_WAVE;
 constexpr int NB_MAXC = 640;  // candidates staged per LDS chunk (27 bins of an LJ melt: ~500);
                                // a multiple of 128 (two 64-candidate groups per step)
 static_assert(NB_MAXC % (2 * EMD_WAVE) == 0, "staging holds whole iterations");
+// A box of few bins leaves most CUs idle with one block per bin (27 bins of
+// an 864-atom melt: 27 blocks of 256 CUs), so up to NB_SPLIT_MAX blocks share
+// a bin's atoms, each staging the candidates for itself, while the grid stays
+// within NB_SPLIT_BLOCKS.  2D build, one block per bin -> this rule: 864
+// atoms 49 -> 21 us, 4000 (125 bins) 48 -> 24 us, 6912 (343 bins) 29 -> 25;
+// from 729 bins on a second block per bin only repeats the staging (256 000
+// atoms 132 us with one, 145 with two).
+constexpr int NB_SPLIT_MAX = 8, NB_SPLIT_BLOCKS = 1024;
 
 // NeighborCSR Tag{Count,Fill}Neigh{Full,Half}, src/neighbor_types/neighbor_csr.h:176-358
 template <bool HALF, bool FILL>
@@ -497,7 +506,7 @@ k_neigh(const double *__restrict__ x, const int *__restrict__ bincount,
     }
     __syncthreads();
     const bool last = (cs + NB_MAXC >= T);
-    for (int bi = wave; bi < c_cnt; bi += NB_WAVES) {
+    for (int bi = blockIdx.y * NB_WAVES + wave; bi < c_cnt; bi += NB_WAVES * gridDim.y) {
       // the centre bin is stencil bin 13: its atoms are staged too, so the
       // row atom's index and position come from LDS when in this round
       const int pc = s_pre[13] + bi - cs;
@@ -631,20 +640,19 @@ extern "C" emd_status emd_neigh_build(emd_ctx *ctx, const emd_system *s, const e
   int *cursor = (int *)ctx->d_tmp2;
   if (n > 0) EMD_LAUNCH(ctx, "neigh_count", k_fill_int, emd_blocks(n, 256), 256, 0, nl->num, n, 0);
 
+  const int split = (int)std::min<long>(NB_SPLIT_MAX, std::max<long>(1, NB_SPLIT_BLOCKS / std::max(1l, nib)));
   // k_neigh launch: fill?, CSR row offsets (or null: rows at i * pitch),
   // pitch, entries, row capacity, record full row lengths in num?
-#define NB_LAUNCH(name, F, ROW, PITCH, ENT, CAP, WNUM)                                        \
-  do {                                                                                       \
-    if (nib > 0) {                                                                           \
-      if (half)                                                                              \
-        EMD_LAUNCH(ctx, name, (k_neigh<true, F>), nib, NB_THREADS, 0, s->x, b->bincount,     \
-                   b->binoffsets, b->permute, g, n, cutsq, newton, nl->num, ROW, PITCH, ENT, \
-                   cursor, CAP, WNUM);                                                       \
-      else                                                                                   \
-        EMD_LAUNCH(ctx, name, (k_neigh<false, F>), nib, NB_THREADS, 0, s->x, b->bincount,    \
-                   b->binoffsets, b->permute, g, n, cutsq, newton, nl->num, ROW, PITCH, ENT, \
-                   cursor, CAP, WNUM);                                                       \
-    }                                                                                        \
+#define NB_LAUNCH_AS(name, H, F, ROW, PITCH, ENT, CAP, WNUM)                                 \
+  EMD_LAUNCH(ctx, name, (k_neigh<H, F>), dim3(nib, split), NB_THREADS, 0, s->x, b->bincount, \
+             b->binoffsets, b->permute, g, n, cutsq, newton, nl->num, ROW, PITCH, ENT, cursor, \
+             CAP, WNUM)
+#define NB_LAUNCH(name, F, ROW, PITCH, ENT, CAP, WNUM)                    \
+  do {                                                                    \
+    if (nib > 0) {                                                        \
+      if (half) NB_LAUNCH_AS(name, true, F, ROW, PITCH, ENT, CAP, WNUM);  \
+      else NB_LAUNCH_AS(name, false, F, ROW, PITCH, ENT, CAP, WNUM);      \
+    }                                                                     \
   } while (0)
 
   // One pass when a row capacity is known: the fill writes rows padded to
@@ -723,6 +731,7 @@ extern "C" emd_status emd_neigh_build(emd_ctx *ctx, const emd_system *s, const e
     nl->maxneighs = maxrow;
   }
 #undef NB_LAUNCH
+#undef NB_LAUNCH_AS
   return EMD_OK;
 }
 
