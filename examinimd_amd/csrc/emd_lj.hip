@@ -203,17 +203,45 @@ k_lj_full(const double *__restrict__ x, const int *__restrict__ type,
 }
 
 // ForceLJNeigh TagHalfNeigh, force_lj_neigh_impl.h:208-254: each pair's
-// force is added to i and subtracted from j (atomically: rows of other
-// atoms reach j too).  LJH_K lanes per atom take every LJH_K-th entry of the
-// row, issuing the index loads of LJH_U entries and then their gathers
-// before the arithmetic (a half row holds ~37 entries: one round); the
-// lanes' i sums are reduced across the group and added once.  Pair
-// arithmetic as the full-list kernel: FP64 as the reference writes it,
-// mixed with FP64 distances and emd_lj_fpair_mixed.  DIAL: ForceLJIDialNeigh
-// TagHalfNeigh, force_lj_idial_neigh_impl.h:169-219, which subtracts the
-// reaction only from local j (:208-212).  Atomic order varies from run to
-// run, so sums agree to rounding, not bitwise.
+// force is added to i and subtracted from j (which rows of other atoms reach
+// too).  LJH_K lanes per atom take every LJH_K-th entry of the row, issuing
+// the index loads of LJH_U entries and then their gathers before the
+// arithmetic (a half row holds ~37 entries: one round).  Pair arithmetic as
+// the full-list kernel: FP64 as the reference writes it, mixed with FP64
+// distances and emd_lj_fpair_mixed.  DIAL: ForceLJIDialNeigh TagHalfNeigh,
+// force_lj_idial_neigh_impl.h:169-219, which subtracts the reaction only
+// from local j (:208-212).
+//
+// What bounds it is the atomic traffic to L2: three scattered additions per
+// pair (7.2 M for 87 000 atoms) took 258 us at any occupancy.  Atoms are in
+// bin order, so the LJH_ATOMS atoms of a block share most of their
+// neighbours (~900 pairs, ~350 different j): their forces are added up in an
+// LDS table first (open addressing on j with LJH_PROBES steps; a j that finds
+// no slot goes to memory directly), and each slot is added to memory once,
+// by three neighbouring lanes, consecutive j in consecutive slots: 36 us at
+// 87 000 atoms (FP64); 1.50 ms FP64 and 1.41 mixed at 4 million (11.2 mixed
+// with the scattered additions).  The table is FP64 in both precisions: LDS
+// additions in FP32 measured slower (2.02 ms mixed).  Additions reach an
+// address in varying order, so sums agree from run to run to rounding, not
+// bitwise.
 constexpr int LJH_K = 8, LJH_U = 5;
+constexpr int LJH_ATOMS = LJ_THREADS / LJH_K;
+constexpr int LJH_SLOTS = 1024, LJH_PROBES = 4;
+
+// slot of atom j in the block's table (claimed if free), or -1
+__device__ __forceinline__ int ljh_slot(int *key, int j) {
+  int h = j & (LJH_SLOTS - 1);
+#pragma unroll 1
+  for (int p = 0; p < LJH_PROBES; p++, h = (h + 37) & (LJH_SLOTS - 1)) {
+    int k = key[h];
+    if (k == j) return h;
+    if (k < 0) {
+      k = atomicCAS(&key[h], -1, j);
+      if (k < 0 || k == j) return h;
+    }
+  }
+  return -1;
+}
 
 template <bool MIXED, bool DIAL>
 __global__ void __launch_bounds__(LJ_THREADS)
@@ -222,84 +250,89 @@ k_lj_half(const double *__restrict__ x, const int *__restrict__ type, const int 
           lj_tv tab, double *__restrict__ f, float *__restrict__ f32) {
 #pragma clang fp contract(off)
   typedef typename lj_acc<MIXED>::T T;
-  const int gid = blockIdx.x * LJ_THREADS + threadIdx.x;
-  const int i = gid / LJH_K, sub = gid % LJH_K;
-  if (i >= n) return;  // whole groups of LJH_K lanes leave together
-  const double x_i = x[3 * (size_t)i], y_i = x[3 * (size_t)i + 1], z_i = x[3 * (size_t)i + 2];
-  const int type_i = type[i];
-  const int *rowp = entries + (row ? (size_t)row[i] : (size_t)i * (size_t)pitch);
-  const int cnt = num[i];
-  T fxi = 0, fyi = 0, fzi = 0;
-  auto sub_j = [&](int j, T vx, T vy, T vz) {
-    if (MIXED) {
-      atomicAdd(&f32[3 * (size_t)j], -(float)vx);
-      atomicAdd(&f32[3 * (size_t)j + 1], -(float)vy);
-      atomicAdd(&f32[3 * (size_t)j + 2], -(float)vz);
+  __shared__ int s_key[LJH_SLOTS];
+  __shared__ double s_f[3 * LJH_SLOTS];
+  T *fout;
+  if constexpr (MIXED) fout = f32;
+  else fout = f;
+  for (int k = threadIdx.x; k < LJH_SLOTS; k += LJ_THREADS) s_key[k] = -1;
+  for (int k = threadIdx.x; k < 3 * LJH_SLOTS; k += LJ_THREADS) s_f[k] = 0;
+  __syncthreads();
+  auto add = [&](int j, T vx, T vy, T vz) {
+    const int h = ljh_slot(s_key, j);
+    if (h >= 0) {
+      atomicAdd(&s_f[3 * h], (double)vx);
+      atomicAdd(&s_f[3 * h + 1], (double)vy);
+      atomicAdd(&s_f[3 * h + 2], (double)vz);
     } else {
-      atomicAdd(&f[3 * (size_t)j], -(double)vx);
-      atomicAdd(&f[3 * (size_t)j + 1], -(double)vy);
-      atomicAdd(&f[3 * (size_t)j + 2], -(double)vz);
+      atomicAdd(&fout[3 * (size_t)j], vx);
+      atomicAdd(&fout[3 * (size_t)j + 1], vy);
+      atomicAdd(&fout[3 * (size_t)j + 2], vz);
     }
   };
-  for (int jj = sub; jj < cnt; jj += LJH_U * LJH_K) {
-    int j[LJH_U];
-    bool ok[LJH_U];
+  const int tile = emd_xcd_tile(blockIdx.x, gridDim.x);
+  const int i = tile * LJH_ATOMS + (int)threadIdx.x / LJH_K, sub = threadIdx.x % LJH_K;
+  if (i < n) {
+    const double x_i = x[3 * (size_t)i], y_i = x[3 * (size_t)i + 1], z_i = x[3 * (size_t)i + 2];
+    const int type_i = type[i];
+    const int *rowp = entries + (row ? (size_t)row[i] : (size_t)i * (size_t)pitch);
+    const int cnt = num[i];
+    T fxi = 0, fyi = 0, fzi = 0;
+    for (int jj = sub; jj < cnt; jj += LJH_U * LJH_K) {
+      int j[LJH_U];
+      bool ok[LJH_U];
 #pragma unroll
-    for (int u = 0; u < LJH_U; u++) {
-      ok[u] = jj + u * LJH_K < cnt;
-      j[u] = rowp[ok[u] ? jj + u * LJH_K : cnt - 1];
-    }
-    double xj[LJH_U], yj[LJH_U], zj[LJH_U];
+      for (int u = 0; u < LJH_U; u++) {
+        ok[u] = jj + u * LJH_K < cnt;
+        j[u] = rowp[ok[u] ? jj + u * LJH_K : cnt - 1];
+      }
+      double xj[LJH_U], yj[LJH_U], zj[LJH_U];
 #pragma unroll
-    for (int u = 0; u < LJH_U; u++) {
-      xj[u] = x[3 * (size_t)j[u]];
-      yj[u] = x[3 * (size_t)j[u] + 1];
-      zj[u] = x[3 * (size_t)j[u] + 2];
-    }
+      for (int u = 0; u < LJH_U; u++) {
+        xj[u] = x[3 * (size_t)j[u]];
+        yj[u] = x[3 * (size_t)j[u] + 1];
+        zj[u] = x[3 * (size_t)j[u] + 2];
+      }
 #pragma unroll
-    for (int u = 0; u < LJH_U; u++) {
-      const double dx = x_i - xj[u];
-      const double dy = y_i - yj[u];
-      const double dz = z_i - zj[u];
-      const double rsq = dx * dx + dy * dy + dz * dz;
-      const int t = type_i * tab.stride + type[j[u]];
-      if (ok[u] && rsq < tab.cutsq[t]) {
-        T vx, vy, vz;
-        if (MIXED) {
-          float fpair = emd_lj_fpair_mixed(rsq, (float)tab.lj1[t], (float)tab.lj2[t]);
-          if (DIAL) fpair = dial_sum(fpair / (float)tab.rep[t], dial_trips(tab.rep[t]));
-          vx = (float)dx * fpair;
-          vy = (float)dy * fpair;
-          vz = (float)dz * fpair;
-        } else {
-          const double r2inv = 1.0 / rsq;
-          const double r6inv = r2inv * r2inv * r2inv;
-          double fpair = (r6inv * (tab.lj1[t] * r6inv - tab.lj2[t])) * r2inv;
-          if (DIAL) fpair = dial_sum(fpair / tab.rep[t], dial_trips(tab.rep[t]));
-          vx = dx * fpair;
-          vy = dy * fpair;
-          vz = dz * fpair;
+      for (int u = 0; u < LJH_U; u++) {
+        const double dx = x_i - xj[u];
+        const double dy = y_i - yj[u];
+        const double dz = z_i - zj[u];
+        const double rsq = dx * dx + dy * dy + dz * dz;
+        const int t = type_i * tab.stride + type[j[u]];
+        if (ok[u] && rsq < tab.cutsq[t]) {
+          T vx, vy, vz;
+          if (MIXED) {
+            float fpair = emd_lj_fpair_mixed(rsq, (float)tab.lj1[t], (float)tab.lj2[t]);
+            if (DIAL) fpair = dial_sum(fpair / (float)tab.rep[t], dial_trips(tab.rep[t]));
+            vx = (float)dx * fpair;
+            vy = (float)dy * fpair;
+            vz = (float)dz * fpair;
+          } else {
+            const double r2inv = 1.0 / rsq;
+            const double r6inv = r2inv * r2inv * r2inv;
+            double fpair = (r6inv * (tab.lj1[t] * r6inv - tab.lj2[t])) * r2inv;
+            if (DIAL) fpair = dial_sum(fpair / tab.rep[t], dial_trips(tab.rep[t]));
+            vx = dx * fpair;
+            vy = dy * fpair;
+            vz = dz * fpair;
+          }
+          fxi += vx;
+          fyi += vy;
+          fzi += vz;
+          if (!DIAL || j[u] < n) add(j[u], -vx, -vy, -vz);
         }
-        fxi += vx;
-        fyi += vy;
-        fzi += vz;
-        if (!DIAL || j[u] < n) sub_j(j[u], vx, vy, vz);
       }
     }
+    fxi = group_sum<LJH_K>(fxi);
+    fyi = group_sum<LJH_K>(fyi);
+    fzi = group_sum<LJH_K>(fzi);
+    if (sub == 0) add(i, fxi, fyi, fzi);
   }
-  fxi = group_sum<LJH_K>(fxi);
-  fyi = group_sum<LJH_K>(fyi);
-  fzi = group_sum<LJH_K>(fzi);
-  if (sub == 0) {
-    if (MIXED) {
-      atomicAdd(&f32[3 * (size_t)i], (float)fxi);
-      atomicAdd(&f32[3 * (size_t)i + 1], (float)fyi);
-      atomicAdd(&f32[3 * (size_t)i + 2], (float)fzi);
-    } else {
-      atomicAdd(&f[3 * (size_t)i], (double)fxi);
-      atomicAdd(&f[3 * (size_t)i + 1], (double)fyi);
-      atomicAdd(&f[3 * (size_t)i + 2], (double)fzi);
-    }
+  __syncthreads();
+  for (int e = threadIdx.x; e < 3 * LJH_SLOTS; e += LJ_THREADS) {
+    const int j = s_key[e / 3];
+    if (j >= 0) atomicAdd(&fout[3 * (size_t)j + e % 3], (T)s_f[e]);
   }
 }
 
@@ -459,7 +492,7 @@ static emd_status lj_idial_force(emd_ctx *ctx, emd_system *s, const emd_neigh *n
   if (lj->ntypes > 1 || half) EMD_TRY(upload_tv(ctx, lj, p->intensity, &tab));
   const int *row = nl->layout == EMD_NEIGH_CSR ? nl->row : nullptr;
   if (half) {
-    const int nb = emd_blocks((long)s->n_local * LJH_K, LJ_THREADS);
+    const int nb = emd_blocks(s->n_local, LJH_ATOMS);
     if (precision == EMD_MIXED)
       EMD_LAUNCH(ctx, "lj_idial_half", (k_lj_half<true, true>), nb, LJ_THREADS, 0, s->x,
                  s->type, row, nl->num, nl->entries, nl->maxneighs, s->n_local, tab, s->f,
@@ -486,7 +519,7 @@ static emd_status lj_force(emd_ctx *ctx, emd_system *s, const emd_neigh *nl,
   if (p->ntypes > 1 || half || p->table) EMD_TRY(upload_tv(ctx, p, nullptr, &tab));
   const int *row = nl->layout == EMD_NEIGH_CSR ? nl->row : nullptr;
   if (half) {
-    const int nb = emd_blocks((long)s->n_local * LJH_K, LJ_THREADS);
+    const int nb = emd_blocks(s->n_local, LJH_ATOMS);
     if (precision == EMD_MIXED)
       EMD_LAUNCH(ctx, "lj_force_half", (k_lj_half<true, false>), nb, LJ_THREADS, 0, s->x,
                  s->type, row, nl->num, nl->entries, nl->maxneighs, s->n_local, tab, s->f,
