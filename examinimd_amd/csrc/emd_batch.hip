@@ -63,7 +63,7 @@ struct emd_batch {
   size_t entries_cap = 0;  // bytes
   int cap = 0;
   int *flags = nullptr;    // [0] largest row seen
-  double *part = nullptr;  // [2 * nrep]
+  double *part = nullptr;  // thermo sums (4 * BT_SLICES per replica), then the masses
   double *save = nullptr;  // autotune snapshot: x, v, f (FP64 or FP32 bits)
   long step = 0;
   bool ready = false;
@@ -141,22 +141,17 @@ __global__ void k_bfill(const int *__restrict__ binof, int *__restrict__ cursor,
   binatoms[atomicAdd(&cursor[binof[i]], 1)] = i;
 }
 
-// ascending atom order inside each bin (deterministic rows)
-__global__ void k_bsort(const int *__restrict__ start, const int *__restrict__ count,
-                        int *__restrict__ binatoms, int nbins) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nbins) return;
-  int *a = binatoms + start[b];
-  const int c = count[b];
-  for (int k = 1; k < c; k++) {
-    const int v = a[k];
-    int m = k - 1;
-    while (m >= 0 && a[m] > v) {
-      a[m + 1] = a[m];
-      m--;
-    }
-    a[m + 1] = v;
-  }
+// ascending atom order inside each bin (deterministic rows), one wavefront
+// per bin (one thread per bin sorting by insertion in memory took 400 us for
+// the bins of 256 replicas)
+constexpr int BS_THREADS = 256;
+__global__ void __launch_bounds__(BS_THREADS)
+k_bsort(const int *__restrict__ start, const int *__restrict__ count, int *__restrict__ binatoms,
+        int nbins) {
+  const int b = blockIdx.x * (BS_THREADS / EMD_WAVE) + threadIdx.x / EMD_WAVE;
+  if (b < nbins)
+    emd_wave_sort(binatoms + __builtin_amdgcn_readfirstlane(start[b]),
+                  __builtin_amdgcn_readfirstlane(count[b]));
 }
 
 // image position of an entry on one axis (the ghost copy's arithmetic)
@@ -165,15 +160,20 @@ __device__ __forceinline__ double b_image(double xj, unsigned c, double L) {
 }
 
 constexpr int BN_THREADS = 256;
-constexpr int BN_MAXC = 1024;  // candidates staged per LDS chunk
+constexpr int BN_MAXC = 640;  // candidates staged per LDS chunk (~520 in an LJ melt)
+static_assert(BN_MAXC % (2 * EMD_WAVE) == 0, "staging holds whole iterations");
 
 // one block per bin (the plain neighbour build's scheme): the 27 stencil
 // bins of the bin's replica, each with its periodic image code, are staged in
 // LDS as candidates (stencil order, each bin in ascending atom order, image
 // positions as the force kernel forms them); each wavefront takes atoms of
-// the bin and tests 64 candidates per step, compacting hits with ballot and
-// popcount, so rows come out in stencil-then-bin order.  Keeps
-// rsq <= cutneighsq except the atom itself (image code 0).
+// the bin and tests 128 candidates per step, compacting hits with ballot and
+// mbcnt, so rows come out in stencil-then-bin order.  Keeps
+// rsq <= cutneighsq except the atom itself (image code 0: its entry equals
+// its index).  Bound: VALU and LDS reads of the ~520 tests per atom (more in
+// boxes two or three bins wide); the row index as a scalar, row atoms from
+// LDS, two groups in flight and 18 instead of 28 KB of LDS (8 blocks per CU)
+// took 256 replicas (661 284 atoms) from 578 to 440 us.
 __global__ void __launch_bounds__(BN_THREADS)
 k_bneigh(const double *__restrict__ x, const rep_info *__restrict__ info,
          const int *__restrict__ binrep, const int *__restrict__ binstart,
@@ -216,7 +216,6 @@ k_bneigh(const double *__restrict__ x, const rep_info *__restrict__ info,
   __syncthreads();
   const int T = s_pre[27];
   const int c_start = binstart[g];
-  const unsigned long long lt = emd_lanemask_lt();
   int mymax = 0;
   for (int cs = 0; cs < T; cs += BN_MAXC) {
     const int cn = (T - cs) < BN_MAXC ? (T - cs) : BN_MAXC;
@@ -233,27 +232,58 @@ k_bneigh(const double *__restrict__ x, const rep_info *__restrict__ info,
     __syncthreads();
     const bool last = cs + BN_MAXC >= T;
     for (int bi = wave; bi < c_cnt; bi += BN_THREADS / EMD_WAVE) {
-      const int i = binatoms[c_start + bi];
-      const double xi = x[3 * (size_t)i], yi = x[3 * (size_t)i + 1], zi = x[3 * (size_t)i + 2];
-      unsigned *row = entries + (size_t)i * cap;
-      int run = cs > 0 ? num[i] : 0;
-      for (int c0 = 0; c0 < cn; c0 += EMD_WAVE) {
-        const int c = c0 + lane;
-        bool keep = false;
-        unsigned e = 0u;
-        if (c < cn) {
-          e = s_e[c];
-          const double dx = xi - s_x[c], dy = yi - s_y[c], dz = zi - s_z[c];
-          const double rsq = dx * dx + dy * dy + dz * dz;
-          keep = rsq <= cutneighsq && !((int)(e & B_JMASK) == i && (e >> B_CODE_SHIFT) == 0u);
-        }
-        const unsigned long long m = __ballot(keep);
-        if (keep) {
-          const int pos = run + __popcll(m & lt);
-          if (pos < cap) row[pos] = e;
-        }
-        run += __popcll(m);
+      // the bin itself is stencil slot 13 (image code 0): its atoms are staged
+      const int pc = s_pre[13] + bi - cs;
+      int i;
+      double xi, yi, zi;
+      if (pc >= 0 && pc < cn) {
+        i = (int)s_e[pc];
+        xi = s_x[pc];
+        yi = s_y[pc];
+        zi = s_z[pc];
+      } else {
+        i = binatoms[c_start + bi];
+        xi = x[3 * (size_t)i];
+        yi = x[3 * (size_t)i + 1];
+        zi = x[3 * (size_t)i + 2];
       }
+      i = __builtin_amdgcn_readfirstlane(i);  // the row is the wavefront's
+      unsigned *const row = entries + (size_t)i * cap;
+      int run = cs > 0 ? num[i] : 0;
+      // only the last iteration of a chunk (TAIL) reaches positions past the
+      // staged count; they hold stale candidates and are masked
+      auto test = [&](auto tail, int c, unsigned e, double xj, double yj, double zj) -> bool {
+        const double dx = xi - xj, dy = yi - yj, dz = zi - zj;
+        const double rsq = dx * dx + dy * dy + dz * dz;
+        const bool staged = !decltype(tail)::value || c < cn;
+        return staged & (rsq <= cutneighsq) & (e != (unsigned)i);
+      };
+      auto put = [&](bool keep, unsigned long long m, int at, unsigned e) {
+        if (keep) {
+          const unsigned pos = __builtin_amdgcn_mbcnt_hi(
+              (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, (unsigned)at));
+          if ((int)pos < cap) row[pos] = e;
+        }
+      };
+      // two 64-candidate groups per iteration: both groups' LDS reads are
+      // issued before either distance test
+      auto iteration = [&](auto tail, int c0) {
+        const int ca = c0 + lane, cb = c0 + EMD_WAVE + lane;
+        const unsigned ea = s_e[ca], eb = s_e[cb];
+        const double xa = s_x[ca], ya = s_y[ca], za = s_z[ca];
+        const double xb = s_x[cb], yb = s_y[cb], zb = s_z[cb];
+        const bool ka = test(tail, ca, ea, xa, ya, za);
+        const bool kb = test(tail, cb, eb, xb, yb, zb);
+        const unsigned long long ma = __builtin_amdgcn_ballot_w64(ka);
+        const unsigned long long mb = __builtin_amdgcn_ballot_w64(kb);
+        put(ka, ma, run, ea);
+        const int runb = run + __popcll(ma);
+        put(kb, mb, runb, eb);
+        run = runb + __popcll(mb);
+      };
+      int c0 = 0;
+      for (; c0 + 2 * EMD_WAVE <= cn; c0 += 2 * EMD_WAVE) iteration(std::false_type{}, c0);
+      if (c0 < cn) iteration(std::true_type{}, c0);
       if (lane == 0) num[i] = last ? (run < cap ? run : cap) : run;
       if (last) mymax = run > mymax ? run : mymax;
     }
@@ -316,17 +346,14 @@ k_bstep(const double *__restrict__ x, double *__restrict__ xn, double *__restric
       }
     }
   };
-  // U entries per lane per memory round (index loads, then gathers, then
-  // arithmetic); slots past the row end re-read its last entry, masked
-  for (int jj = sub; jj < cnt; jj += U * K) {
-    unsigned e[U];
-    bool ok[U];
+  // U entries per lane per memory round: index loads, then gathers, then
+  // arithmetic.  The first round's index loads do not wait for the row length
+  // (loaded beside them): its slots are clamped to the capacity, and a slot
+  // past the row end (left from an earlier build, or never written) is
+  // replaced by the atom itself before anything is gathered, and masked.
+  // While a round's loads issue the wavefront runs at a raised priority.
+  auto gather = [&](const unsigned (&e)[U], const bool (&ok)[U]) {
     double xj[U], yj[U], zj[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      ok[u] = jj + u * K < cnt;
-      e[u] = __builtin_nontemporal_load(rowp + (ok[u] ? jj + u * K : cnt - 1));
-    }
 #pragma unroll
     for (int u = 0; u < U; u++) {
       const size_t j = e[u] & B_JMASK;
@@ -334,8 +361,36 @@ k_bstep(const double *__restrict__ x, double *__restrict__ xn, double *__restric
       yj[u] = x[3 * j + 1];
       zj[u] = x[3 * j + 2];
     }
+    if (MIXED) __builtin_amdgcn_s_setprio(0);
 #pragma unroll
     for (int u = 0; u < U; u++) pair(ok[u], e[u], xj[u], yj[u], zj[u]);
+  };
+  {
+    unsigned e[U];
+    bool ok[U];
+    if (MIXED) __builtin_amdgcn_s_setprio(2);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int k = sub + u * K;
+      e[u] = __builtin_nontemporal_load(rowp + (k < cap ? k : cap - 1));
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      ok[u] = sub + u * K < cnt;
+      e[u] = ok[u] ? e[u] : (unsigned)i;
+    }
+    gather(e, ok);
+  }
+  for (int jj = sub + U * K; jj < cnt; jj += U * K) {
+    unsigned e[U];
+    bool ok[U];
+    if (MIXED) __builtin_amdgcn_s_setprio(2);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      ok[u] = jj + u * K < cnt;
+      e[u] = __builtin_nontemporal_load(rowp + (ok[u] ? jj + u * K : cnt - 1));
+    }
+    gather(e, ok);
   }
   if (K > 1) {
     fxi = group_sum<K>(fxi);
@@ -399,54 +454,62 @@ __global__ void k_binit(double *__restrict__ x, double *__restrict__ v,
   x[o + 2] += dtv * v2;
 }
 
-// one block per replica: sum m v^2 (Temperature/KinE summand,
+// per replica sum m v^2 (Temperature/KinE summand,
 // property_temperature.h:54-56) and the shifted pair energy
-// (force_lj_neigh_impl.h:256-300), both compensated
-__global__ void __launch_bounds__(256)
+// (force_lj_neigh_impl.h:256-300), both compensated: BT_SLICES blocks per
+// replica, BT_K lanes per atom (lane sub takes row entries sub, sub + BT_K,
+// ...), each block's double-double sums to part[(replica * BT_SLICES + slice)
+// * 4 + {0,1} kinetic, {2,3} potential}.  Bound: latency of the row and
+// gather loads; 281 us for both sums of 256 replicas (661 284 atoms), where
+// one block per replica with a thread per row took 611 us for each.
+constexpr int BT_THREADS = 256, BT_K = 16, BT_SLICES = 16;
+__global__ void __launch_bounds__(BT_THREADS)
 k_bthermo(const double *__restrict__ x, const double *__restrict__ v,
           const rep_info *__restrict__ info, const int *__restrict__ num,
           const unsigned *__restrict__ entries, int cap, const double *__restrict__ mass,
-          double lj1, double lj2, double cutsq, int what, double *__restrict__ part) {
+          double lj1, double lj2, double cutsq, double *__restrict__ part) {
 #pragma clang fp contract(off)
-  const rep_info R = info[blockIdx.x];
-  double hi = 0.0, lo = 0.0;
-  for (int k = threadIdx.x; k < R.n; k += blockDim.x) {
-    const int i = R.start + k;
-    const size_t o = 3 * (size_t)i;
-    double t = 0.0;
-    if (what == 0) {
-      t = (v[o] * v[o] + v[o + 1] * v[o + 1] + v[o + 2] * v[o + 2]) * mass[blockIdx.x];
-    } else {
-      const double r2invc = 1.0 / cutsq;
-      const double r6invc = r2invc * r2invc * r2invc;
-      const double eshift = 0.5 * r6invc * (0.5 * lj1 * r6invc - lj2) / 6.0;
-      for (int jj = 0; jj < num[i]; jj++) {
-        const unsigned e = entries[(size_t)i * cap + jj];
-        const size_t j = e & B_JMASK;
-        const unsigned c = e >> B_CODE_SHIFT;
-        const double dx = x[o] - b_image(x[3 * j], c & 3u, R.L[0]);
-        const double dy = x[o + 1] - b_image(x[3 * j + 1], (c >> 2) & 3u, R.L[1]);
-        const double dz = x[o + 2] - b_image(x[3 * j + 2], (c >> 4) & 3u, R.L[2]);
-        const double rsq = dx * dx + dy * dy + dz * dz;
-        if (rsq < cutsq) {
-          const double r2inv = 1.0 / rsq;
-          const double r6inv = r2inv * r2inv * r2inv;
-          double s, e2;
-          two_sum(t, 0.5 * r6inv * (0.5 * lj1 * r6inv - lj2) / 6.0, s, e2);
-          t = s;
-          lo += e2;
-          two_sum(t, -eshift, s, e2);
-          t = s;
-          lo += e2;
-        }
-      }
-    }
+  const int rep = blockIdx.x / BT_SLICES, slice = blockIdx.x % BT_SLICES;
+  const rep_info R = info[rep];
+  const int sub = threadIdx.x % BT_K;
+  const double r2invc = 1.0 / cutsq;
+  const double r6invc = r2invc * r2invc * r2invc;
+  const double eshift = 0.5 * r6invc * (0.5 * lj1 * r6invc - lj2) / 6.0;
+  double khi = 0.0, klo = 0.0, phi = 0.0, plo = 0.0;
+  auto add = [](double &hi, double &lo, double t) {
     double s, e;
     two_sum(hi, t, s, e);
     hi = s;
     lo += e;
+  };
+  constexpr int ATOMS = BT_THREADS / BT_K;
+  for (int k = slice * ATOMS + (int)threadIdx.x / BT_K; k < R.n; k += BT_SLICES * ATOMS) {
+    const int i = R.start + k;
+    const size_t o = 3 * (size_t)i;
+    const double x_i = x[o], y_i = x[o + 1], z_i = x[o + 2];
+    if (sub == 0)
+      add(khi, klo,
+          (v[o] * v[o] + v[o + 1] * v[o + 1] + v[o + 2] * v[o + 2]) * mass[rep]);
+    const int cnt = num[i];
+    for (int jj = sub; jj < cnt; jj += BT_K) {
+      const unsigned e = entries[(size_t)i * cap + jj];
+      const size_t j = e & B_JMASK;
+      const unsigned c = e >> B_CODE_SHIFT;
+      const double dx = x_i - b_image(x[3 * j], c & 3u, R.L[0]);
+      const double dy = y_i - b_image(x[3 * j + 1], (c >> 2) & 3u, R.L[1]);
+      const double dz = z_i - b_image(x[3 * j + 2], (c >> 4) & 3u, R.L[2]);
+      const double rsq = dx * dx + dy * dy + dz * dz;
+      if (rsq < cutsq) {
+        const double r2inv = 1.0 / rsq;
+        const double r6inv = r2inv * r2inv * r2inv;
+        add(phi, plo, 0.5 * r6inv * (0.5 * lj1 * r6inv - lj2) / 6.0);
+        add(phi, plo, -eshift);
+      }
+    }
   }
-  block_dd_sum(hi, lo, part);
+  block_dd_sum(khi, klo, part, 4);
+  __syncthreads();
+  block_dd_sum(phi, plo, part + 2, 4);
 }
 
 // -------------------------------------------------------------- host side
@@ -507,7 +570,7 @@ emd_status rebuild(emd_ctx *ctx, emd_batch *b) {
              b->bincur);
   EMD_LAUNCH(ctx, "batch_bin_fill", k_bfill, emd_blocks(n, 256), 256, 0, b->binof, b->bincur,
              b->binatoms, n);
-  EMD_LAUNCH(ctx, "batch_bin_sort", k_bsort, emd_blocks(nb, 256), 256, 0, b->binstart,
+  EMD_LAUNCH(ctx, "batch_bin_sort", k_bsort, emd_blocks(nb, BS_THREADS / EMD_WAVE), BS_THREADS, 0, b->binstart,
              b->bincount, b->binatoms, nb);
   EMD_LAUNCH(ctx, "batch_neigh", k_bneigh, nb, BN_THREADS, 0, x, b->info, b->binrep,
              b->binstart, b->bincount, b->binatoms, b->cutneighsq, b->cap, b->num, b->entries,
@@ -692,7 +755,7 @@ extern "C" emd_status emd_batch_create(emd_ctx *ctx, const emd_batch_desc *d, em
   if (st == EMD_OK) st = dalloc(ctx, &b->binrep, nbins);
   if (st == EMD_OK) st = dalloc(ctx, &b->num, total);
   if (st == EMD_OK) st = dalloc(ctx, &b->flags, 16);
-  if (st == EMD_OK) st = dalloc(ctx, &b->part, 2 * (size_t)d->nrep + d->nrep);
+  if (st == EMD_OK) st = dalloc(ctx, &b->part, (4 * (size_t)BT_SLICES + 1) * d->nrep);
   if (st == EMD_OK) st = dalloc(ctx, &b->save, 3 * n3);
   if (st != EMD_OK) {
     emd_batch_destroy(ctx, b);
@@ -708,8 +771,8 @@ extern "C" emd_status emd_batch_create(emd_ctx *ctx, const emd_batch_desc *d, em
     for (int k = 0; k < nbr; k++) binrep[R.binbase + k] = r;
   }
   EMD_HIP(ctx, hipMemcpy(b->binrep, binrep.data(), nbins * sizeof(int), hipMemcpyHostToDevice));
-  // masses live after the 2*nrep reduction partials
-  EMD_HIP(ctx, hipMemcpy(b->part + 2 * d->nrep, mass.data(), d->nrep * sizeof(double),
+  // masses live after the thermo sums
+  EMD_HIP(ctx, hipMemcpy(b->part + 4 * (size_t)BT_SLICES * d->nrep, mass.data(), d->nrep * sizeof(double),
                          hipMemcpyHostToDevice));
   EMD_HIP(ctx, hipMemset(b->f, 0, n3 * sizeof(double)));
   EMD_HIP(ctx, hipMemset(b->f32, 0, n3 * sizeof(float)));
@@ -830,19 +893,29 @@ extern "C" emd_status emd_batch_run(emd_ctx *ctx, emd_batch *b, int nsteps, int 
 extern "C" emd_status emd_batch_thermo(emd_ctx *ctx, emd_batch *b, double *ke, double *pe) {
   if (!ctx || !b) return EMD_ERR_ARG;
   if (!b->ready) return emd_set_error(ctx, EMD_ERR_STATE, "emd_batch_thermo before setup");
-  std::vector<double> h(2 * (size_t)b->nrep);
-  for (int what = 0; what < 2; what++) {
-    double *out = what == 0 ? ke : pe;
-    if (!out) continue;
-    EMD_LAUNCH(ctx, "batch_thermo", k_bthermo, b->nrep, 256, 0, b->x[b->cur], b->v, b->info,
-               b->num, b->entries, b->cap, b->part + 2 * b->nrep, b->lj1, b->lj2, b->cutsq,
-               what, b->part);
-    EMD_HIP(ctx, hipMemcpyAsync(h.data(), b->part, h.size() * sizeof(double),
-                                hipMemcpyDeviceToHost, ctx->stream));
-    EMD_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    for (int r = 0; r < b->nrep; r++)
-      out[r] = (what == 0 ? 0.5 : 1.0) * (h[2 * r] + h[2 * r + 1]);
-  }
+  if (!ke && !pe) return EMD_OK;
+  const size_t count = 4 * (size_t)b->nrep * BT_SLICES;
+  std::vector<double> h(count);
+  EMD_LAUNCH(ctx, "batch_thermo", k_bthermo, BT_SLICES * b->nrep, BT_THREADS, 0,
+             b->x[b->cur], b->v, b->info, b->num, b->entries, b->cap, b->part + count, b->lj1,
+             b->lj2, b->cutsq, b->part);
+  EMD_HIP(ctx, hipMemcpyAsync(h.data(), b->part, count * sizeof(double), hipMemcpyDeviceToHost,
+                              ctx->stream));
+  EMD_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  for (int r = 0; r < b->nrep; r++)
+    for (int what = 0; what < 2; what++) {
+      double *out = what == 0 ? ke : pe;
+      if (!out) continue;
+      // the slices' (hi, lo) pairs, compensated (Neumaier)
+      double sum = 0.0, c = 0.0;
+      for (int k = 0; k < BT_SLICES; k++)
+        for (int w = 0; w < 2; w++) {
+          const double v = h[4 * ((size_t)r * BT_SLICES + k) + 2 * what + w], t = sum + v;
+          c += fabs(sum) >= fabs(v) ? (sum - t) + v : (v - t) + sum;
+          sum = t;
+        }
+      out[r] = (what == 0 ? 0.5 : 1.0) * (sum + c);
+    }
   return EMD_OK;
 }
 

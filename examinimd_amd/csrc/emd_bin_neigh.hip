@@ -40,10 +40,8 @@ __device__ __forceinline__ int bin_index(const double *xi, double minx, double m
 // (1) each atom's bin id, counted into the bins with atomics;
 // (2) exclusive scan of the counts (wavefront scans, emd_scan) -> offsets;
 // (3) scatter through per-bin cursors;
-// (4) each bin's slice put in ascending atom order by one wavefront: a
-//     lane's rank is the number of smaller indices in the slice (64-wide
-//     shuffle sweep, registers only; slices over 64 atoms, which a dense
-//     cluster or a wide bin can give, take an insertion sort).
+// (4) each bin's slice put in ascending atom order by one wavefront
+//     (emd_wave_sort).
 // Atoms were sorted by bin at the previous rebuild and have moved little,
 // so consecutive atoms mostly share a bin: in (1) and (3) a wavefront's runs
 // of equal bin ids make one atomic per run (the run's first lane adds the
@@ -118,32 +116,9 @@ __global__ void __launch_bounds__(BIN_ORDER_THREADS)
 k_bin_order(const int *__restrict__ count, const int *__restrict__ offset, int nbins,
             int *__restrict__ permute) {
   const int b = blockIdx.x * (BIN_ORDER_THREADS / EMD_WAVE) + threadIdx.x / EMD_WAVE;
-  const int lane = threadIdx.x % EMD_WAVE;
-  int c = 0;
-  if (b < nbins) {
-    c = count[b];
-    int *p = permute + offset[b];
-    if (c <= EMD_WAVE) {
-      const int v = lane < c ? p[lane] : 0x7fffffff;
-      // slices already in order (one run of the previous order) stay
-      const int next = __shfl_down(v, 1, EMD_WAVE);
-      if (__ballot(lane + 1 < c && next < v) != 0ull) {
-        int rank = 0;
-        for (int k = 0; k < c; k++) rank += __shfl(v, k, EMD_WAVE) < v;
-        if (lane < c) p[rank] = v;
-      }
-    } else if (lane == 0) {
-      for (int k = 1; k < c; k++) {
-        const int v = p[k];
-        int m = k - 1;
-        while (m >= 0 && p[m] > v) {
-          p[m + 1] = p[m];
-          m--;
-        }
-        p[m + 1] = v;
-      }
-    }
-  }
+  if (b < nbins)
+    emd_wave_sort(permute + __builtin_amdgcn_readfirstlane(offset[b]),
+                  __builtin_amdgcn_readfirstlane(count[b]));
 }
 
 // Small ranges (n <= BIN_ONE_MAX_N atoms, nbins <= BIN_ONE_MAX_BINS) in one

@@ -192,6 +192,54 @@ __device__ __forceinline__ int emd_wave_sum(int v) {
   return v;
 }
 
+// the c ints at p put in ascending order by one wavefront (distinct values):
+// a value's place is the number of smaller ones, counted by broadcasting every
+// value in turn; slices already in order are left alone.  Up to 256 values in
+// registers (bins of an LJ melt hold ~20, of a box two bins wide up to ~70);
+// longer slices, which only a dense cluster or a very wide bin gives, by
+// insertion.
+__device__ __forceinline__ void emd_wave_sort(int *p, int c) {
+  const int lane = __lane_id();
+  if (c <= EMD_WAVE) {
+    const int v = lane < c ? p[lane] : 0x7fffffff;
+    const int next = __shfl_down(v, 1, EMD_WAVE);
+    if (__ballot(lane + 1 < c && next < v) == 0ull) return;
+    int rank = 0;
+    for (int k = 0; k < c; k++) rank += __builtin_amdgcn_readlane(v, k) < v;
+    if (lane < c) p[rank] = v;
+  } else if (c <= 4 * EMD_WAVE) {
+    int v[4], rank[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int k = q * EMD_WAVE + lane;
+      v[q] = k < c ? p[k] : 0x7fffffff;
+      rank[q] = 0;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int m = c - q * EMD_WAVE < EMD_WAVE ? c - q * EMD_WAVE : EMD_WAVE;
+      for (int k = 0; k < m; k++) {
+        const int w = __builtin_amdgcn_readlane(v[q], k);
+#pragma unroll
+        for (int t = 0; t < 4; t++) rank[t] += w < v[t];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      if (q * EMD_WAVE + lane < c) p[rank[q]] = v[q];
+  } else if (lane == 0) {
+    for (int k = 1; k < c; k++) {
+      const int v = p[k];
+      int m = k - 1;
+      while (m >= 0 && p[m] > v) {
+        p[m + 1] = p[m];
+        m--;
+      }
+      p[m + 1] = v;
+    }
+  }
+}
+
 // map a physical block onto a logical tile so that each of the 8 XCDs (which
 // receive blocks round-robin) works on one contiguous range of tiles and
 // shares its L2 with spatially neighbouring atoms
@@ -374,8 +422,8 @@ __device__ __forceinline__ void two_sum(double a, double b, double &s, double &e
 }
 
 // block reduction of (hi, lo) pairs (blockDim.x <= 1024); the block's
-// double-double total lands in out[2*blockIdx.x + {0,1}]
-__device__ inline void block_dd_sum(double hi, double lo, double *out) {
+// double-double total lands in out[stride*blockIdx.x + {0,1}]
+__device__ inline void block_dd_sum(double hi, double lo, double *out, int stride = 2) {
 #pragma clang fp contract(off)
   __shared__ double s_hi[16], s_lo[16];
 #pragma unroll
@@ -397,8 +445,8 @@ __device__ inline void block_dd_sum(double hi, double lo, double *out) {
       H = s;
       Lo += s_lo[k] + e;
     }
-    out[2 * blockIdx.x] = H;
-    out[2 * blockIdx.x + 1] = Lo;
+    out[stride * (size_t)blockIdx.x] = H;
+    out[stride * (size_t)blockIdx.x + 1] = Lo;
   }
 }
 

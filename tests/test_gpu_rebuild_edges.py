@@ -25,7 +25,8 @@ def bin_ids(x, b):
 
 @pytest.mark.parametrize("n,edge,cut,cluster", [
     (1, 9.0, 2.8, 0), (64, 9.0, 2.8, 0), (1025, 12.0, 2.8, 0), (1500, 12.0, 2.8, 1500),
-    (7168, 14.0, 1.0, 0), (7168, 14.1, 1.0, 200), (7169, 14.0, 1.0, 0), (9000, 20.0, 2.8, 300)])
+    (7168, 14.0, 1.0, 0), (7168, 14.1, 1.0, 200), (7169, 14.0, 1.0, 0), (9000, 20.0, 2.8, 300),
+    (9000, 60.0, 2.8, 64), (9000, 60.0, 2.8, 65), (9000, 60.0, 2.8, 256), (9000, 60.0, 2.8, 257)])
 def test_binning_permutation(n, edge, cut, cluster):
     print(f"case: binning {n} atoms, bins {cut} in {edge}, cluster {cluster}", flush=True)
     rng = np.random.default_rng(n + cluster)
