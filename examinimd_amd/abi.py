@@ -123,6 +123,8 @@ HIP_PROTOS = {
                                 P(C.c_double)]),
     "emd_lj_energy_atoms": (C.c_int, [vp, P(EmdSystem), P(EmdNeigh), P(EmdLJParams), C.c_int,
                                       dptr]),
+    "emd_lj_force_energy_store": (C.c_int, [vp, P(EmdSystem), P(EmdNeigh), P(EmdLJParams),
+                                            C.c_int, dptr]),
     "emd_lj_energy_noalloc": (C.c_int, [vp, P(EmdSystem), P(EmdNeigh), P(EmdLJParams),
                                         C.c_int, P(C.c_double)]),
     "emd_lj_set_lanes": (C.c_int, [vp, C.c_int, C.c_int]),
@@ -146,6 +148,9 @@ HIP_PROTOS = {
                                  C.c_double, dptr, C.c_double, C.c_int, dptr]),
     "emd_lj_adjoint_atoms": (C.c_int, [vp, P(EmdSystem), P(EmdNeigh), C.c_double, C.c_double,
                                        C.c_double, dptr, dptr, C.c_int, dptr]),
+    "emd_fit_residual": (C.c_int, [vp, P(EmdSystem), C.c_int, dptr, dptr, C.c_int, iptr, dptr,
+                                   dptr, dptr, dptr]),
+    "emd_fit_loss": (C.c_int, [vp, dptr]),
     "emd_batch_create": (C.c_int, [vp, P(EmdBatchDesc), P(vp)]),
     "emd_batch_destroy": (C.c_int, [vp, vp]),
     "emd_batch_upload": (C.c_int, [vp, vp, dptr, dptr]),

@@ -69,7 +69,7 @@ extern "C" emd_status emd_create(int device, emd_ctx **out) {
             hipMalloc(&ctx->d_dsmall, 64 * sizeof(double)) == hipSuccess &&
             hipHostMalloc(&ctx->h_small, 64 * sizeof(int), hipHostMallocDefault) == hipSuccess &&
             hipHostMalloc(&ctx->h_dsmall, 64 * sizeof(double), hipHostMallocDefault) == hipSuccess &&
-            hipHostMalloc(&ctx->h_mail, (EMD_MAIL_DATA + EMD_MAIL_MAX) * sizeof(int),
+            hipHostMalloc(&ctx->h_mail, 2 * EMD_MAIL_INTS * sizeof(int),
                           hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess &&
             hipMalloc(&ctx->d_ljtab, EMD_LJ_TABLE_BYTES) == hipSuccess &&
             hipHostMalloc(&ctx->h_ljtab, EMD_LJ_TABLE_BYTES, hipHostMallocDefault) == hipSuccess &&
@@ -79,7 +79,7 @@ extern "C" emd_status emd_create(int device, emd_ctx **out) {
     return EMD_ERR_ALLOC;
   }
   hipMemset(ctx->d_small, 0, 64 * sizeof(int));
-  memset(ctx->h_mail, 0, (EMD_MAIL_DATA + EMD_MAIL_MAX) * sizeof(int));
+  memset(ctx->h_mail, 0, 2 * EMD_MAIL_INTS * sizeof(int));
   // the allocation-free entry points' scratch: this device's copy
   if (emd_lj_scratch_setup(ctx) != EMD_OK) {
     emd_destroy(ctx);

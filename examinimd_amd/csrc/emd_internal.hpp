@@ -65,8 +65,11 @@ struct emd_ctx {
 
   // counts for the host: pinned, coherent memory that a kernel writes itself
   // (emd_mail_post) and the host polls (emd_mail_wait)
-  int *h_mail = nullptr;       // [0] sequence number, [EMD_MAIL_DATA..] payload
+  int *h_mail = nullptr;       // [0] sequence number, [EMD_MAIL_DATA..] payload; then a
+                               // second box of the same size for emd_fit_loss
   int mail_seq = 0;
+  bool fit_pending = false;    // a loss is in the second box or on its way there,
+  int fit_seq = 0;             // under this number
 
   // host waits: an event recorded on the stream and polled, so a wait for a
   // count ends as soon as the copy lands (no blocking-sync wake-up latency)
@@ -149,6 +152,7 @@ struct emd_mail {
   int *box;
   int seq;
 };
+constexpr int EMD_MAIL_INTS = EMD_MAIL_DATA + EMD_MAIL_MAX;
 inline emd_mail emd_mail_next(emd_ctx *ctx) { return emd_mail{ctx->h_mail, ++ctx->mail_seq}; }
 // the payload of message m (valid until the next message is posted)
 emd_status emd_mail_wait(emd_ctx *ctx, const emd_mail &m, const int **payload);

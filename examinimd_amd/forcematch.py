@@ -209,6 +209,17 @@ class MergedSystem:
             return f32.astype(np.float64)
         return self._dl(self.s.f, 3 * n).reshape(n, 3)
 
+    def write(self, ptr, a):
+        """host values into a device array of doubles"""
+        a = np.ascontiguousarray(a, dtype=np.float64)
+        self.chk(self.L.emd_memcpy_h2d(self.ctx.h, C.cast(ptr, C.c_void_p),
+                                       a.ctypes.data_as(C.c_void_p), a.nbytes), "h2d")
+
+    def fit_loss(self):
+        loss = C.c_double()
+        self.chk(self.L.emd_fit_loss(self.ctx.h, C.byref(loss)), "loss")
+        return loss.value
+
     def close(self):
         for p in self._bufs:
             self.L.emd_free(self.ctx.h, p)
@@ -270,8 +281,20 @@ class SnapForceMatchMerged:
         # the configurations never move: the compaction, neighbour parameters
         # and U_tot depend on them only, so force and adjoint calls reuse them
         m.chk(L.emd_snap_static_geometry(c, self.pl.snap, 1), "static geometry")
-        self.Ft = self._forces(EMD_FP64)
+        self._ft = m._put(np.zeros(3 * n))
+        self._forces(EMD_FP64)
+        self.Ft = m.forces(EMD_FP64)
         self.Et = self.energies(beta_true)
+
+    @property
+    def Ft(self):
+        """target forces of the merged locals, library order (kept on the
+        device; assign to change them)"""
+        return self.m._dl(self._ft, 3 * self.m.s.n_local).reshape(-1, 3)
+
+    @Ft.setter
+    def Ft(self, F):
+        self.m.write(self._ft, F)
 
     def energies(self, beta):
         """per-configuration energies, E_c = N_c beta_0 + S_c . beta_1.. + R_c"""
@@ -283,27 +306,26 @@ class SnapForceMatchMerged:
         s = C.byref(m.s)
         m.chk(L.emd_snap_force_zeroed(c, s, C.byref(m.nl), self.pl.snap, precision), "snap")
         m.chk(L.emd_comm_update_force(c, s, C.byref(m.h), precision), "fold")
-        return m.forces(precision)
 
     def evaluate(self, beta, precision, grad=True):
         beta = np.ascontiguousarray(beta, dtype=np.float64)
+        L, c, m = self.L, self.ctx.h, self.m
         self.pl.snap_set_coeff(beta)
-        dF = self._forces(precision) - self.Ft
-        n = self.m.n_atoms
+        self._forces(precision)
+        # the residuals, the cotangent and the force loss stay on the device
+        m.chk(L.emd_fit_residual(c, C.byref(m.s), precision, self._ft, self._g, 0, None, None,
+                                 None, None, None), "residual")
+        n = m.n_atoms
         dE = self.energies(beta) - self.Et
-        loss = float((dF * dF).sum()) + 100.0 * float(np.sum((dE / n) ** 2))
         g = np.zeros(len(beta))
         if grad:
-            L, c, m = self.L, self.ctx.h, self.m
-            gF = np.ascontiguousarray(2.0 * dF)
-            m.chk(L.emd_memcpy_h2d(c, self._g, gF.ctypes.data_as(C.c_void_p), gF.nbytes), "h2d")
             m.chk(L.emd_snap_adjoint_beta(c, C.byref(m.s), C.byref(m.nl), C.byref(m.h),
                                           self.pl.snap, self._g, 0.0, precision,
                                           g.ctypes.data_as(C.POINTER(C.c_double))), "adjoint")
             gE = 200.0 * dE / n ** 2
             g[0] += float(np.sum(gE * n))
             g[1:] += gE @ self.S
-        return loss, g
+        return m.fit_loss() + 100.0 * float(np.sum((dE / n) ** 2)), g
 
     def close(self):
         self.m.close()
@@ -312,10 +334,11 @@ class SnapForceMatchMerged:
 
 class LJForceMatchMerged:
     """loss(eps, sigma) and its gradient over LJ boxes merged into one system:
-    per evaluation one force launch (stored forces), one per-atom energy
-    launch and one adjoint launch for the whole set, the energy cotangent of
-    each box entering the adjoint as a weight on its atoms
-    (emd_lj_adjoint_atoms).  Same loss and gradient as LJForceMatch."""
+    per evaluation one launch for forces and per-atom energies, one for the
+    residuals (emd_fit_residual) and one adjoint for the whole set, the energy
+    cotangent of each box entering the adjoint as a weight on its atoms
+    (emd_lj_adjoint_atoms); only the loss and the gradient leave the device.
+    Same loss and gradient as LJForceMatch."""
 
     def __init__(self, configs, true=(1.0, 1.0), ctx=None, rc=2.5):
         self.rc = rc
@@ -335,7 +358,34 @@ class LJForceMatchMerged:
         self._eatom = self.m._put(np.zeros(n))
         self._g = self.m._put(np.zeros(3 * n))
         self._w = self.m._put(np.zeros(n))
-        self.Ft, self.Et = self._force_energy(EMD_FP64, *true)
+        self._start = self.m._put(np.append(self.m.starts, n).astype(np.int32))
+        self._ft = self.m._put(np.zeros(3 * n))
+        self._et = self.m._put(np.zeros(len(configs)))
+        self._force_energy(EMD_FP64, *true)
+        self.Ft = self.m.forces(EMD_FP64)
+        # the boxes' energies as the residual forms them (loss 0 at `true`)
+        self.m.chk(self.L.emd_fit_residual(
+            ctx.h, C.byref(self.m.s), EMD_FP64, self._ft, self._g, len(configs), self._start,
+            self._eatom, self.m._put(np.zeros(len(configs))), self._w, self._et), "targets")
+
+    @property
+    def Ft(self):
+        """target forces of the merged locals, library order (kept on the
+        device; assign to change them)"""
+        return self.m._dl(self._ft, 3 * self.m.s.n_local).reshape(-1, 3)
+
+    @Ft.setter
+    def Ft(self, F):
+        self.m.write(self._ft, F)
+
+    @property
+    def Et(self):
+        """target energy of each box (kept on the device; assign to change)"""
+        return self.m._dl(self._et, len(self.m.n_atoms))
+
+    @Et.setter
+    def Et(self, E):
+        self.m.write(self._et, E)
 
     def _params(self, eps, sig):
         from examinimd_amd.abi import EmdLJParams
@@ -349,30 +399,21 @@ class LJForceMatchMerged:
     def _force_energy(self, precision, eps, sig):
         L, c, m = self.L, self.ctx.h, self.m
         p = self._params(eps, sig)
-        m.chk(L.emd_lj_force_store(c, C.byref(m.s), C.byref(m.nl), C.byref(p), precision), "lj")
-        F = m.forces(precision)
-        m.chk(L.emd_lj_energy_atoms(c, C.byref(m.s), C.byref(m.nl), C.byref(p), 0, self._eatom),
-              "energy")
-        return F, np.add.reduceat(m._dl(self._eatom, m.s.n_local), m.starts)
+        m.chk(L.emd_lj_force_energy_store(c, C.byref(m.s), C.byref(m.nl), C.byref(p), precision,
+                                          self._eatom), "lj")
 
     def evaluate(self, theta, precision, grad=True):
         eps, sig = (float(t) for t in theta)
-        F, E = self._force_energy(precision, eps, sig)
-        dF = F - self.Ft
-        n = self.m.n_atoms
-        dE = E - self.Et
-        loss = float((dF * dF).sum()) + 100.0 * float(np.sum((dE / n) ** 2))
+        L, c, m = self.L, self.ctx.h, self.m
+        self._force_energy(precision, eps, sig)
+        m.chk(L.emd_fit_residual(c, C.byref(m.s), precision, self._ft, self._g, len(m.n_atoms),
+                                 self._start, self._eatom, self._et, self._w, None), "residual")
         g = np.zeros(2)
         if grad:
-            L, c, m = self.L, self.ctx.h, self.m
-            w = np.repeat(200.0 * dE / n ** 2, n)
-            gF = np.ascontiguousarray(2.0 * dF)
-            m.chk(L.emd_memcpy_h2d(c, self._g, gF.ctypes.data_as(C.c_void_p), gF.nbytes), "h2d")
-            m.chk(L.emd_memcpy_h2d(c, self._w, w.ctypes.data_as(C.c_void_p), w.nbytes), "h2d")
             m.chk(L.emd_lj_adjoint_atoms(c, C.byref(m.s), C.byref(m.nl), eps, sig, self.rc,
                                          self._g, self._w, precision,
                                          g.ctypes.data_as(C.POINTER(C.c_double))), "adjoint")
-        return loss, g
+        return m.fit_loss(), g
 
     def close(self):
         self.m.close()

@@ -260,6 +260,10 @@ emd_status emd_lj_energy(emd_ctx *ctx, const emd_system *s, const emd_neigh *nl,
  * wholly to the row atom and half to a ghost j's) */
 emd_status emd_lj_energy_atoms(emd_ctx *ctx, const emd_system *s, const emd_neigh *nl,
                                const emd_lj_params *p, int half, double *eatom);
+/* emd_lj_force_store and emd_lj_energy_atoms on a full list in one pass over
+ * the pairs (what a force-matching evaluation needs); the same values */
+emd_status emd_lj_force_energy_store(emd_ctx *ctx, emd_system *s, const emd_neigh *nl,
+                                     const emd_lj_params *p, int precision, double *eatom);
 /* No counterpart in the reference.  emd_lj_energy for callers that cannot
  * allocate (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): the same energy (to rounding: the block sums are added
@@ -376,6 +380,24 @@ emd_status emd_lj_adjoint(emd_ctx *ctx, const emd_system *s, const emd_neigh *nl
 emd_status emd_lj_adjoint_atoms(emd_ctx *ctx, const emd_system *s, const emd_neigh *nl,
                                 double eps, double sigma, double cut, const double *dLdF,
                                 const double *dLdE_atom, int precision, double *out);
+
+/* No counterpart in the reference.  Loss of a force-matching fit over
+ * configurations merged into one system, and the cotangents its adjoint
+ * needs, formed where the forces are:
+ *   g = 2 (F - f_target)          (DEVICE, double[n_local][3])
+ *   E_c = sum of eatom over the atoms start[c] .. start[c+1] - 1
+ *   w = 200 (E_c - e_target[c]) / N_c^2 for every atom of c (double[n_local])
+ *   loss = sum |F - f_target|^2 + 100 sum_c ((E_c - e_target[c]) / N_c)^2
+ * F is the force array of `precision`.  start is DEVICE int[nconf + 1],
+ * eatom and e_target DEVICE; nconf = 0 leaves the energies out (start,
+ * eatom, e_target and w may then be NULL).  econf (DEVICE double[nconf],
+ * not e_target, or NULL) receives the E_c.  Does not wait: emd_fit_loss
+ * returns the loss of the last call (EMD_ERR_STATE without one). */
+emd_status emd_fit_residual(emd_ctx *ctx, const emd_system *s, int precision,
+                            const double *f_target, double *g, int nconf, const int *start,
+                            const double *eatom, const double *e_target, double *w,
+                            double *econf);
+emd_status emd_fit_loss(emd_ctx *ctx, double *loss);
 
 /* -------------------------------------------------- batched replicas */
 /* No counterpart in the reference: many independent periodic LJ systems
