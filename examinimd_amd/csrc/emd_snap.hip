@@ -40,9 +40,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
-#include <functional>
 #include <map>
-#include <queue>
 #include <set>
 #include <tuple>
 #include <vector>
@@ -536,7 +534,7 @@ __device__ __forceinline__ void y_entry(const snap_dev_tables &t, int e, int &J,
 // are served like two b64 reads, and a 16-byte stride leaves only 16
 // residues.  So FP32 U_tot is stored as (re, im) pairs and FP64 U_tot as an
 // array of real parts and one of imaginary parts, each read with b64 loads
-// at word residue u mod 32.  For twojmax <= 8 U_tot is staged four times,
+// at word residue u mod 32.  U_tot is staged four times,
 // copy c at word offset c * stride + shift(c), and the host gives every
 // read of every term the copy whose residue no other address of its
 // 32-lane group takes (a matching per group; with the shifts 0, 5, 11, 19
@@ -558,12 +556,12 @@ struct alignas(2 * sizeof(T)) cpair {
 template <class T, int J>
 struct yf_layout {
   static constexpr bool SOA = sizeof(T) == 8;
-  static constexpr int NCOPY = J <= SNAP_MAXJ ? 4 : 1;
+  static constexpr int NCOPY = 4;
   static constexpr int MOD = 32;    // bank residues of an 8-byte word
   static constexpr int GROUP = 32;  // lanes served per cycle
   static constexpr int STRIDE = (snap_dim<J>::NU + MOD - 1) / MOD * MOD;
   __host__ __device__ static constexpr int shift(int c) {
-    return NCOPY == 1 ? 0 : (c == 0 ? 0 : c == 1 ? 5 : c == 2 ? 11 : 19);
+    return c == 0 ? 0 : c == 1 ? 5 : c == 2 ? 11 : 19;
   }
   __host__ __device__ static constexpr int base(int c) { return c * STRIDE + shift(c); }
   static constexpr int NUC = base(NCOPY - 1) + snap_dim<J>::NU;  // words the copies span
@@ -1361,54 +1359,64 @@ k_snap_fij_rev(snap_dev_tables t, const rg_rp<T> *__restrict__ rgp, const rg_map
   }
 }
 
-// per-atom energy: beta_0 + sum_k beta_k B_k + pair repulsion (FP64)
-__global__ void __launch_bounds__(256)
-k_snap_energy(snap_dev_tables t, const double *__restrict__ cg,
-              const etab_entry *__restrict__ etab, int ne, double beta0, int bzero,
+// per-atom energy: beta_0 + sum_k beta_k B_k + pair repulsion (FP64), one
+// wavefront per atom.  The energy is a cubic form of U_tot whose variation is
+// dE = sum' w Re(conj(dU) Y) (the identity the forces rest on), so by Euler's
+// theorem for homogeneous functions sum_k beta_k B_k = 1/3 sum' w Re(conj(U)
+// Y): one pass of the Y stream and a 155- (434- at twojmax 12) term dot
+// product instead of every component's Z double sum (164 us for 420 atoms at
+// twojmax 8, 713 us for 1024 at 12).
+struct snap_edot {
+  int u;      // U_tot index of half-plane entry e
+  float wgt;  // its half-plane weight (1, 1/2 or 0)
+};
+constexpr int ENERGY_WAVES = 4;
+
+__global__ void __launch_bounds__(64 * ENERGY_WAVES)
+k_snap_energy(int nu, int ny, const snap_edot *__restrict__ dot, double e0, double rcut,
               const int *__restrict__ nin, const double *__restrict__ nr, int maxn, int n,
               const double *__restrict__ utot_r, const double *__restrict__ utot_i,
+              const double *__restrict__ y_r, const double *__restrict__ y_i,
               double *__restrict__ eatom) {
-  __shared__ double su_r[SNAP_NU_BIG], su_i[SNAP_NU_BIG];
-  __shared__ double s_red[4];
-  const int i = blockIdx.x;
+  const int i = blockIdx.x * ENERGY_WAVES + threadIdx.x / 64, l = threadIdx.x % 64;
   if (i >= n) return;
-  for (int k = threadIdx.x; k < t.nu; k += blockDim.x) {
-    su_r[k] = utot_r[(size_t)i * t.nu + k];
-    su_i[k] = utot_i[(size_t)i * t.nu + k];
-  }
-  __syncthreads();
+  const double *ur = utot_r + (size_t)i * nu, *ui = utot_i + (size_t)i * nu;
+  const double *yr = y_r + (size_t)i * ny, *yi = y_i + (size_t)i * ny;
   double e = 0.0;
-  // work items: (k, half-plane entry of J = j_k)
-  for (int k = 0; k < ne; k++) {
-    const etab_entry te = etab[k];
-    const int J = te.j;
-    const int nyj = t.ystart[J + 1] - t.ystart[J];
-    for (int q = threadIdx.x; q < nyj; q += blockDim.x) {
-      const int mb = q / (J + 1), ma = q - mb * (J + 1);
-      double wgt = 1.0;
-      if (2 * mb == J) wgt = (ma < mb) ? 1.0 : ((ma == mb) ? 0.5 : 0.0);
-      if (wgt == 0.0) continue;
-      const cplx<double> z = z_entry<double>(t, cg, su_r, su_i, te.j1, te.j2, J, te.cgoff, ma, mb);
-      const int u = t.ustart[J] + ma * (J + 1) + mb;
-      e += te.beta * 2.0 * wgt * (su_r[u] * z.r + su_i[u] * z.i);
-    }
+  for (int k = l; k < ny; k += 64) {
+    const snap_edot d = dot[k];
+    e += (double)d.wgt * (ur[d.u] * yr[k] + ui[d.u] * yi[k]);
   }
-  // bzero and the repulsion (rc-shifted), done by thread 0
-  if (threadIdx.x == 0) {
-    if (bzero)
-      for (int k = 0; k < ne; k++) e -= etab[k].beta * t.wself * t.wself * t.wself * (etab[k].j + 1);
-    const double rc12 = 1.0 / pow(t.rcut * t.rcut, 6.0);
-    for (int jj = 0; jj < nin[i]; jj++) {
-      const size_t o = (size_t)i * maxn + jj;
-      const double rsq = nr[3 * o] * nr[3 * o] + nr[3 * o + 1] * nr[3 * o + 1] + nr[3 * o + 2] * nr[3 * o + 2];
-      e += 1.25e5 * (1.0 / pow(rsq, 6.0) - rc12);
-    }
+  e *= 1.0 / 3.0;
+  // the rc-shifted repulsion of the atom's neighbours
+  const double rc2 = rcut * rcut, rc12 = 1.0 / (rc2 * rc2 * rc2 * (rc2 * rc2 * rc2));
+  for (int k = l; k < nin[i]; k += 64) {
+    const double *r = nr + 3 * ((size_t)i * maxn + k);
+    const double r2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2], r6 = r2 * r2 * r2;
+    e += 1.25e5 * (1.0 / (r6 * r6) - rc12);
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off, 64);
-  if (threadIdx.x % 64 == 0) s_red[threadIdx.x / 64] = e;
-  __syncthreads();
-  if (threadIdx.x == 0) eatom[i] = beta0 + ((s_red[0] + s_red[1]) + (s_red[2] + s_red[3]));
+  if (l == 0) eatom[i] = e0 + e;
+}
+
+// sum of n values in double-double, to the host
+__global__ void __launch_bounds__(1024) k_snap_energy_sum(const double *__restrict__ v, int n,
+                                                          emd_mail mail) {
+#pragma clang fp contract(off)
+  __shared__ double s_out[2];
+  double hi = 0.0, lo = 0.0;
+  for (int k = threadIdx.x; k < n; k += blockDim.x) {
+    double s, e;
+    two_sum(hi, v[k], s, e);
+    hi = s;
+    lo += e;
+  }
+  block_dd_sum(hi, lo, s_out);
+  if (threadIdx.x == 0) {
+    *reinterpret_cast<double *>(mail.box + EMD_MAIL_DATA) = s_out[0] + s_out[1];
+    emd_mail_post(mail);
+  }
 }
 
 // ============================================================ host side
@@ -1449,6 +1457,7 @@ struct emd_snap {
   size_t cap_u = 0, cap_y = 0, cap_ui = 0, cap_yi = 0;
   double *eatom = nullptr;
   int cap_e = 0;
+  snap_edot *edot = nullptr;  // energy dot product: U index and weight of each entry
   // flat Y term stream (k_snap_yflat): codes (LDS byte offsets for FP32 and
   // FP64 U_tot), key per slot, cg products, weights for the current
   // coefficients, run slot per (chunk, thread), first run per entry
@@ -1479,9 +1488,15 @@ struct emd_snap {
 };
 
 static double host_factorial(int n) {
-  double r = 1.0;
-  for (int k = 2; k <= n; k++) r *= k;
-  return r;
+  struct table {
+    double v[2 * SNAP_JBIG + 2];
+    table() {
+      v[0] = 1.0;
+      for (int k = 1; k < 2 * SNAP_JBIG + 2; k++) v[k] = v[k - 1] * k;
+    }
+  };
+  static const table f;
+  return f.v[n];
 }
 
 // Clebsch-Gordan <j1/2 m1; j2/2 m2 | j/2 m1+m2> by the Racah formula
@@ -1518,56 +1533,63 @@ static double host_cg(int j1, int j2, int j, int k1, int k2) {
 // (augmenting paths); an entry left unmatched takes the least loaded
 // residue among its copies.  Lanes reading the same entry read the same copy.
 template <class L>
+struct yf_matching {
+  int na = 0;
+  int addr[L::GROUP], copy_of[L::GROUP], owner[L::MOD];
+  bool seen[L::MOD];
+  bool augment(int a) {
+    for (int c = 0; c < L::NCOPY; c++) {
+      const int b = (addr[a] + L::shift(c)) % L::MOD;
+      if (seen[b]) continue;
+      seen[b] = true;
+      if (owner[b] < 0 || augment(owner[b])) {
+        owner[b] = a;
+        copy_of[a] = c;
+        return true;
+      }
+    }
+    return false;
+  }
+  // copies of the group's entries u[0 .. GROUP)
+  void assign(const int *u, int *cp, std::vector<int> &index) {
+    na = 0;
+    for (int l = 0; l < L::GROUP; l++)
+      if (index[u[l]] < 0) {
+        index[u[l]] = na;
+        addr[na++] = u[l];
+      }
+    std::fill(owner, owner + L::MOD, -1);
+    std::fill(copy_of, copy_of + na, -1);
+    int load[L::MOD] = {0};
+    for (int a = 0; a < na; a++) {
+      std::fill(seen, seen + L::MOD, false);
+      augment(a);
+    }
+    for (int a = 0; a < na; a++)
+      if (copy_of[a] >= 0) load[(addr[a] + L::shift(copy_of[a])) % L::MOD]++;
+    for (int a = 0; a < na; a++)
+      if (copy_of[a] < 0) {
+        int best = 0;
+        for (int c = 1; c < L::NCOPY; c++)
+          if (load[(addr[a] + L::shift(c)) % L::MOD] < load[(addr[a] + L::shift(best)) % L::MOD])
+            best = c;
+        copy_of[a] = best;
+        load[(addr[a] + L::shift(best)) % L::MOD]++;
+      }
+    for (int l = 0; l < L::GROUP; l++) cp[l] = copy_of[index[u[l]]];
+    for (int a = 0; a < na; a++) index[addr[a]] = -1;
+  }
+};
+
+template <class L>
 static void yf_assign_copies(const std::vector<int> &u1, const std::vector<int> &u2, int steps,
-                             std::vector<uint32_t> &code) {
-  std::vector<int> cp1(u1.size(), 0), cp2(u2.size(), 0);
-  for (int st = 0; st < steps; st++)
-    for (int w0 = 0; w0 < YF_THREADS; w0 += 64)
-      for (int op = 0; op < 2; op++)
-        for (int g0 = w0; g0 < w0 + 64; g0 += L::GROUP) {
-          const std::vector<int> &u = op ? u2 : u1;
-          std::vector<int> &cp = op ? cp2 : cp1;
-          const size_t s0 = (size_t)st * YF_THREADS + g0;
-          std::vector<int> addr;  // distinct entries of the group
-          for (int l = 0; l < L::GROUP; l++)
-            if (std::find(addr.begin(), addr.end(), u[s0 + l]) == addr.end()) addr.push_back(u[s0 + l]);
-          const int na = (int)addr.size();
-          std::vector<int> owner(L::MOD, -1), copy_of(na, -1);
-          std::function<bool(int, std::vector<char> &)> augment = [&](int a,
-                                                                      std::vector<char> &seen) {
-            for (int c = 0; c < L::NCOPY; c++) {
-              const int b = (addr[a] + L::shift(c)) % L::MOD;
-              if (seen[b]) continue;
-              seen[b] = 1;
-              if (owner[b] < 0 || augment(owner[b], seen)) {
-                owner[b] = a;
-                copy_of[a] = c;
-                return true;
-              }
-            }
-            return false;
-          };
-          std::vector<int> load(L::MOD, 0);
-          for (int a = 0; a < na; a++) {
-            std::vector<char> seen(L::MOD, 0);
-            augment(a, seen);
-          }
-          for (int a = 0; a < na; a++)
-            if (copy_of[a] >= 0) load[(addr[a] + L::shift(copy_of[a])) % L::MOD]++;
-          for (int a = 0; a < na; a++)
-            if (copy_of[a] < 0) {
-              int best = 0;
-              for (int c = 1; c < L::NCOPY; c++)
-                if (load[(addr[a] + L::shift(c)) % L::MOD] < load[(addr[a] + L::shift(best)) % L::MOD])
-                  best = c;
-              copy_of[a] = best;
-              load[(addr[a] + L::shift(best)) % L::MOD]++;
-            }
-          for (int l = 0; l < L::GROUP; l++) {
-            const int a = (int)(std::find(addr.begin(), addr.end(), u[s0 + l]) - addr.begin());
-            cp[s0 + l] = copy_of[a];
-          }
-        }
+                             int nu, std::vector<uint32_t> &code) {
+  std::vector<int> cp1(u1.size(), 0), cp2(u2.size(), 0), index(nu, -1);
+  yf_matching<L> m;
+  for (size_t g0 = 0; g0 < (size_t)steps * YF_THREADS; g0 += L::GROUP) {
+    m.assign(&u1[g0], &cp1[g0], index);
+    m.assign(&u2[g0], &cp2[g0], index);
+  }
   for (size_t k = 0; k < u1.size(); k++)
     code[k] = (uint32_t)((L::base(cp1[k]) + u1[k]) * 8) |
               ((uint32_t)((L::base(cp2[k]) + u2[k]) * 8) << 16);
@@ -1589,6 +1611,7 @@ static emd_status snap_build_yflat(emd_ctx *ctx, emd_snap *sn) {
     double cgw;
   };
   std::vector<std::vector<term>> eterms(t.ny);
+  std::vector<int> seen;
   for (int J = 0; J <= t.twojmax; J++)
     for (int mb = 0; 2 * mb <= J; mb++)
       for (int ma = 0; ma <= J; ma++) {
@@ -1597,6 +1620,9 @@ static emd_status snap_build_yflat(emd_ctx *ctx, emd_snap *sn) {
           int a, b, JJ;
           std::tie(a, b, JJ) = sn->yf_keys[q];
           if (JJ != J) continue;
+          // a == b: (i1, i2) -> the term of this key and entry that holds it
+          const int key0 = (int)eterms[e].size();
+          if (a == b) seen.assign((size_t)(a + 1) * (a + 1) * (a + 1) * (a + 1), -1);
           const int cgoff = sn->cgoff.at(sn->yf_keys[q]);
           const int ma1lo = std::max(0, (2 * ma - J - b + a) / 2);
           const int ma1hi = std::min(a, (2 * ma - J + b + a) / 2);
@@ -1609,8 +1635,19 @@ static emd_status snap_build_yflat(emd_ctx *ctx, emd_snap *sn) {
               const int mb2 = (2 * mb - J - (2 * mb1 - a) + b) / 2;
               const double cw = cma * sn->cg_h[cgoff + mb1 * (b + 1) + mb2];
               if (cw == 0.0) continue;
-              eterms[e].push_back(term{t.ustart[a] + ma1 * (a + 1) + mb1,
-                                       t.ustart[b] + ma2 * (b + 1) + mb2, (int)q, cw});
+              int i1 = t.ustart[a] + ma1 * (a + 1) + mb1, i2 = t.ustart[b] + ma2 * (b + 1) + mb2;
+              // a == b: (i1, i2) and (i2, i1) are the same product (39 610 ->
+              // 32 687 terms at twojmax 8, 427 703 -> 373 959 at 12)
+              if (a == b) {
+                if (i1 < i2) std::swap(i1, i2);
+                int &at = seen[(size_t)(i1 - t.ustart[a]) * (a + 1) * (a + 1) + (i2 - t.ustart[a])];
+                if (at >= key0) {
+                  eterms[e][at].cgw += cw;
+                  continue;
+                }
+                at = (int)eterms[e].size();
+              }
+              eterms[e].push_back(term{i1, i2, (int)q, cw});
             }
           }
         }
@@ -1683,10 +1720,10 @@ static emd_status snap_build_yflat(emd_ctx *ctx, emd_snap *sn) {
       }
     }
   if (small) {
-    yf_assign_copies<yf_layout<float, SNAP_MAXJ>>(u1, u2, steps, code32);
+    yf_assign_copies<yf_layout<float, SNAP_MAXJ>>(u1, u2, steps, t.nu, code32);
     code64 = code32;  // the same word offsets (FP64: into the real array)
   } else {
-    yf_assign_copies<yf_layout<float, SNAP_JBIG>>(u1, u2, steps, code32);
+    yf_assign_copies<yf_layout<float, SNAP_JBIG>>(u1, u2, steps, t.nu, code32);
     code64 = code32;
   }
   sn->yf_steps = steps;
@@ -1930,6 +1967,18 @@ extern "C" emd_status emd_snap_create(emd_ctx *ctx, const emd_snap_params *p, em
   }
   EMD_HIP(ctx, hipMemcpy(sn->cg, sn->cg_h.data(), sn->cg_h.size() * sizeof(double),
                          hipMemcpyHostToDevice));
+  {
+    std::vector<snap_edot> dot(std::max(1, t.ny));
+    for (int j = 0; j <= twojmax; j++)
+      for (int mb = 0; 2 * mb <= j; mb++)
+        for (int ma = 0; ma <= j; ma++)
+          dot[t.ystart[j] + mb * (j + 1) + ma] =
+              snap_edot{t.ustart[j] + ma * (j + 1) + mb,
+                        2 * mb != j || ma < mb ? 1.0f : (ma == mb ? 0.5f : 0.0f)};
+    EMD_HIP(ctx, hipMalloc(&sn->edot, dot.size() * sizeof(snap_edot)));
+    EMD_HIP(ctx, hipMemcpy(sn->edot, dot.data(), dot.size() * sizeof(snap_edot),
+                           hipMemcpyHostToDevice));
+  }
   emd_status st = snap_build_yflat(ctx, sn);
   if (st == EMD_OK && twojmax <= SNAP_MAXJ) st = snap_build_rg(ctx, sn);
   if (st == EMD_OK) st = snap_upload_coeff(ctx, sn);
@@ -1946,7 +1995,7 @@ extern "C" emd_status emd_snap_destroy(emd_ctx *ctx, emd_snap *sn) {
   if (ctx) hipStreamSynchronize(ctx->stream);
   void *ptrs[] = {sn->cg, sn->ytab, sn->etab, sn->nin, sn->nj, sn->nr, sn->par, sn->fdv,
                   sn->rg_rp32, sn->rg_rp64, sn->rg_map_d,
-                  sn->stab, sn->w_r,
+                  sn->stab, sn->w_r, sn->edot,
                   sn->w_i, sn->sbuf,
                   sn->u_r, sn->u_i, sn->y_r, sn->y_i, sn->eatom,
                   sn->yf_code32, sn->yf_code64, sn->yf_key, sn->yf_meta, sn->yf_cgw,
@@ -2076,15 +2125,16 @@ static emd_status snap_y(emd_ctx *ctx, emd_snap *sn, int n) {
   T *ur = (T *)sn->u_r, *ui = (T *)sn->u_i, *yr = (T *)sn->y_r, *yi = (T *)sn->y_i;
   const T *w = std::is_same<T, float>::value ? (const T *)sn->yf_w32 : (const T *)sn->yf_w64;
   const uint32_t *code = std::is_same<T, float>::value ? sn->yf_code32 : sn->yf_code64;
-  // twojmax <= 8: two atoms per block share each term's code and weight
-  // load (SNAP-2k: 26.8 / 47.2 us mixed / FP64, against 31.5 / 60.9 with one
-  // atom and 28.2 / 55.9 with three)
+  // two atoms per block share each term's code and weight load (SNAP-2k:
+  // 26.8 / 47.2 us mixed / FP64, against 31.5 / 60.9 with one atom and 28.2 /
+  // 55.9 with three; 1024 atoms at twojmax 12: 109 / 218 us, against 199
+  // mixed with one atom and a single U_tot copy)
   if (sn->t.twojmax <= SNAP_MAXJ)
     EMD_LAUNCH(ctx, "snap_y", (k_snap_yflat<T, SNAP_MAXJ, 2>), (n + 1) / 2, YF_THREADS, 0, sn->t.nu,
                sn->t.ny, sn->yf_nch, code, w, sn->yf_meta, sn->yf_rstart, n, ur, ui, yr, yi);
   else
-    EMD_LAUNCH(ctx, "snap_y", (k_snap_yflat<T, SNAP_JBIG, 1>), n, YF_THREADS, 0, sn->t.nu, sn->t.ny,
-               sn->yf_nch, code, w, sn->yf_meta, sn->yf_rstart, n, ur, ui, yr, yi);
+    EMD_LAUNCH(ctx, "snap_y", (k_snap_yflat<T, SNAP_JBIG, 2>), (n + 1) / 2, YF_THREADS, 0, sn->t.nu,
+               sn->t.ny, sn->yf_nch, code, w, sn->yf_meta, sn->yf_rstart, n, ur, ui, yr, yi);
   return EMD_OK;
 }
 
@@ -2180,28 +2230,34 @@ extern "C" emd_status emd_snap_energy(emd_ctx *ctx, const emd_system *s, const e
   const int n = s->n_local;
   *energy = 0.0;
   if (n <= 0) return EMD_OK;
-  sn->geom_prec = -1;  // the compaction and U_tot are rewritten
-  EMD_TRY(snap_neigh(ctx, s, nl, sn, -1, EMD_FP64));
-  EMD_TRY(launch_ui<double>(ctx, sn, n, (double *)sn->u_r, (double *)sn->u_i));
+  if (sn->t.twojmax <= SNAP_MAXJ) {
+    if (!snap_geom_cached(sn, s, nl, EMD_FP64)) {
+      EMD_TRY(snap_neigh_ui(ctx, s, nl, sn, -1, EMD_FP64));
+      snap_geom_record(sn, s, nl, EMD_FP64);
+    }
+  } else {
+    EMD_TRY(snap_neigh(ctx, s, nl, sn, -1, EMD_FP64));
+    EMD_TRY(launch_ui<double>(ctx, sn, n, (double *)sn->u_r, (double *)sn->u_i));
+  }
+  EMD_TRY(snap_y<double>(ctx, sn, n));
   double *ea = eatom;
   if (!ea) {
     EMD_TRY(emd_ensure_int(ctx, (int **)&sn->eatom, &sn->cap_e, 2l * n));
     ea = sn->eatom;
   }
-  EMD_LAUNCH(ctx, "snap_energy", k_snap_energy, n, 256, 0, sn->t, sn->cg, sn->etab,
-             sn->ncoeff, sn->beta[0], sn->bzeroflag, sn->nin, sn->nr, sn->cap_maxn, n,
-             (const double *)sn->u_r, (const double *)sn->u_i, ea);
-  std::vector<double> h(n);
-  EMD_HIP(ctx, hipMemcpyAsync(h.data(), ea, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  EMD_TRY(emd_wait(ctx));
-  double sum = 0.0, c = 0.0;
-  for (int k = 0; k < n; k++) {
-    const double v = h[k], tt = sum + v;
-    if (std::fabs(sum) >= std::fabs(v)) c += (sum - tt) + v;
-    else c += (v - tt) + sum;
-    sum = tt;
-  }
-  *energy = sum + c;
+  double e0 = sn->beta[0];
+  if (sn->bzeroflag)
+    for (int k = 0; k < sn->ncoeff; k++)
+      e0 -= sn->beta[k + 1] * sn->t.wself * sn->t.wself * sn->t.wself * (sn->idxj[3 * k + 2] + 1);
+  EMD_LAUNCH(ctx, "snap_energy", k_snap_energy, emd_blocks(n, ENERGY_WAVES), 64 * ENERGY_WAVES, 0,
+             sn->t.nu, sn->t.ny, sn->edot, e0, sn->t.rcut, sn->nin, sn->nr, sn->cap_maxn, n,
+             (const double *)sn->u_r, (const double *)sn->u_i, (const double *)sn->y_r,
+             (const double *)sn->y_i, ea);
+  const emd_mail mail = emd_mail_next(ctx);
+  EMD_LAUNCH(ctx, "snap_energy", k_snap_energy_sum, 1, 1024, 0, ea, n, mail);
+  const int *got = nullptr;
+  EMD_TRY(emd_mail_wait(ctx, mail, &got));
+  memcpy(energy, got, sizeof(double));
   return EMD_OK;
 }
 
