@@ -641,21 +641,50 @@ k_lj_energy(const double *__restrict__ x, const int *__restrict__ type,
   }
 }
 
-static emd_status finish_dd(emd_ctx *ctx, double *part, int nb, double *out) {
-  std::vector<double> h(2 * (size_t)nb);
-  EMD_HIP(ctx, hipMemcpyAsync(h.data(), part, h.size() * sizeof(double), hipMemcpyDeviceToHost,
-                              ctx->stream));
-  EMD_TRY(emd_wait(ctx));
-  // Neumaier summation of the block (hi, lo) pairs
-  double sum = 0.0, c = 0.0;
-  for (size_t k = 0; k < h.size(); k++) {
-    const double v = h[k];
-    const double t = sum + v;
-    if (fabs(sum) >= fabs(v)) c += (sum - t) + v;
-    else c += (v - t) + sum;
-    sum = t;
+// sums of block pairs (hi, lo) in double-double: block b's share into
+// out[2 b], or with a mailbox (one block) the total to the host
+__global__ void __launch_bounds__(1024)
+k_dd_sum(const double *__restrict__ part, int nb, double *__restrict__ out, emd_mail mail) {
+#pragma clang fp contract(off)
+  __shared__ double s_out[2];
+  double hi = 0.0, lo = 0.0;
+  const int stride = gridDim.x * blockDim.x;
+#pragma unroll 4
+  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nb; k += stride) {
+    double s, e;
+    two_sum(hi, part[2 * (size_t)k], s, e);
+    hi = s;
+    lo += part[2 * (size_t)k + 1] + e;
   }
-  *out = sum + c;
+  if (!mail.box) {
+    block_dd_sum(hi, lo, out);
+    return;
+  }
+  block_dd_sum(hi, lo, s_out);
+  if (threadIdx.x == 0) {
+    *reinterpret_cast<double *>(mail.box + EMD_MAIL_DATA) = s_out[0] + s_out[1];
+    emd_mail_post(mail);
+  }
+}
+
+// the total of nb block pairs on the host: added on the device (in two stages
+// from DD_ONE_MAX pairs on) and posted, where the pairs used to be copied and
+// added by the host (4 MB for an energy of 4 million atoms).  An LJ energy
+// takes 0.93 ms at 4 million atoms (1.55), 73 us at 256 000 (131), 24 us at
+// 32 000 (57).  part has room for DD_STAGE more pairs.
+constexpr int DD_ONE_MAX = 8192, DD_STAGE = 256;
+static emd_status finish_dd(emd_ctx *ctx, double *part, int nb, double *out) {
+  if (nb > DD_ONE_MAX) {
+    EMD_LAUNCH(ctx, "dd_sum", k_dd_sum, DD_STAGE, 1024, 0, part, nb, part + 2 * (size_t)nb,
+               (emd_mail{nullptr, 0}));
+    part += 2 * (size_t)nb;
+    nb = DD_STAGE;
+  }
+  const emd_mail mail = emd_mail_next(ctx);
+  EMD_LAUNCH(ctx, "dd_sum", k_dd_sum, 1, 1024, 0, part, nb, nullptr, mail);
+  const int *got = nullptr;
+  EMD_TRY(emd_mail_wait(ctx, mail, &got));
+  memcpy(out, got, sizeof(double));
   return EMD_OK;
 }
 
@@ -668,7 +697,8 @@ extern "C" emd_status emd_lj_energy(emd_ctx *ctx, const emd_system *s, const emd
   lj_tv tab;
   EMD_TRY(upload_tv(ctx, p, nullptr, &tab));
   const int nb = emd_blocks((long)n * LJE_K, LJ_THREADS);
-  EMD_TRY(emd_ensure(ctx, &ctx->d_tmp2, &ctx->tmp2_cap, (size_t)nb * 2 * sizeof(double)));
+  EMD_TRY(emd_ensure(ctx, &ctx->d_tmp2, &ctx->tmp2_cap,
+                     ((size_t)nb + DD_STAGE) * 2 * sizeof(double)));
   double *part = (double *)ctx->d_tmp2;
   const int *row = nl->layout == EMD_NEIGH_CSR ? nl->row : nullptr;
   if (p->ntypes == 1)
@@ -1224,7 +1254,12 @@ k_step_boundary_one(double *__restrict__ x, double *__restrict__ v, double *__re
     emd_halo_update_at(g, x, root, image, n, lx, ly, lz);
 }
 
-constexpr int STEP_ONE_MAX = 16384;  // local atoms of a one-workgroup step boundary
+// locals + ghosts of a one-workgroup step boundary: one CU moves ~0.35 us per
+// hundred atoms, the separate launches take 6.5 us without a fold (5.5 at 3059
+// atoms in one workgroup, 8.0 at 4941) and 10-14 us with one (9.4 / 11.0
+// mixed / FP64 at 4941, 10.8 / 12.9 at 6083); at 26 000 atoms one workgroup
+// takes 37-47 us
+constexpr int STEP_ONE_MAX = 3500, STEP_ONE_MAX_FOLD = 5500;
 
 extern "C" emd_status emd_nve_step_boundary(emd_ctx *ctx, emd_system *s, const emd_halo *h,
                                             int fold, int update_halo, double dtf, double dtv,
@@ -1232,11 +1267,11 @@ extern "C" emd_status emd_nve_step_boundary(emd_ctx *ctx, emd_system *s, const e
   if (!ctx || !s || !h) return EMD_ERR_ARG;
   const int n = s->n_local;
   fold_phases ph;
-  long ghosts = emd_fold_phases_of(s, h, ph);
+  const long ghosts = emd_fold_phases_of(s, h, ph);
   if (!fold)
     for (int p = 0; p < 6; p++) ph.num[p] = 0;
   const int n_halo = update_halo ? h->n_ghost : 0;
-  if (!ctx->fold_one || n > STEP_ONE_MAX || ghosts > FOLD_ONE_MAX || n_halo > FOLD_ONE_MAX) {
+  if (!ctx->fold_one || (long)n + h->n_ghost > (fold ? STEP_ONE_MAX_FOLD : STEP_ONE_MAX)) {
     // larger systems: the separate launches (their grids fill the GPU)
     if (fold) EMD_TRY(emd_comm_update_force(ctx, s, h, precision));
     EMD_TRY(emd_nve_final_initial(ctx, s, dtf, dtv, precision));
@@ -1315,7 +1350,8 @@ extern "C" emd_status emd_reduce_mv2(emd_ctx *ctx, const emd_system *s, double *
   const int n = s->n_local;
   if (n <= 0) { *mv2 = 0.0; return EMD_OK; }
   const int nb = emd_blocks(n, 256);
-  EMD_TRY(emd_ensure(ctx, &ctx->d_tmp2, &ctx->tmp2_cap, (size_t)nb * 2 * sizeof(double)));
+  EMD_TRY(emd_ensure(ctx, &ctx->d_tmp2, &ctx->tmp2_cap,
+                     ((size_t)nb + DD_STAGE) * 2 * sizeof(double)));
   double *part = (double *)ctx->d_tmp2;
   EMD_LAUNCH(ctx, "reduce_mv2", k_mv2, nb, 256, 0, s->v, s->type, s->mass, n, part);
   return finish_dd(ctx, part, nb, mv2);

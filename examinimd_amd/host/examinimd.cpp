@@ -134,9 +134,12 @@ void ExaMiniMD::thermo(double out[3]) {
   Temperature temp(comm);
   PotE pote(comm);
   KinE kine(comm);
-  T_FLOAT T = temp.compute(system);
+  // temperature and kinetic energy are the same sum of m v^2
+  double mv2 = 0.0;
+  EMD_CALL(system->ctx, emd_reduce_mv2(system->ctx, system->view(), &mv2));
+  T_FLOAT T = temp.compute(system, mv2);
   T_FLOAT PE = pote.compute(system, binning, neighbor, force) / system->N;
-  T_FLOAT KE = kine.compute(system) / system->N;
+  T_FLOAT KE = kine.compute(system, mv2) / system->N;
   out[0] = T;
   out[1] = PE;
   out[2] = PE + KE;

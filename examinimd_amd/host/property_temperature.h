@@ -11,6 +11,8 @@ class Temperature {
 public:
   Temperature(Comm* comm_) : comm(comm_) {}
   T_V_FLOAT compute(System*);
+  // the same from a known sum of m v^2 (this process's share)
+  T_V_FLOAT compute(System*, double mv2);
 };
 
 class KinE {
@@ -18,6 +20,7 @@ class KinE {
 public:
   KinE(Comm* comm_) : comm(comm_) {}
   T_V_FLOAT compute(System*);
+  T_V_FLOAT compute(System*, double mv2);
 };
 
 class PotE {
