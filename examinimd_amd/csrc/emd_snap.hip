@@ -16,27 +16,21 @@
 // column ma <= J/2 with weight 1/2 on the diagonal).
 //
 // Kernels (T = double, or float for the mixed path):
-//   k_snap_neigh  one wavefront per atom: compacts the in-cutoff neighbours
-//                 (FP64 distance test, list order kept) with ballots and
-//                 writes each neighbour's Cayley-Klein parameters, switching
-//                 function and derivative factors (snap_par) once
-//   k_snap_neigh_ui (twojmax <= 8, force path) the compaction and U_tot of
-//                 k_snap_ui_rg in the same wavefront: one launch
-//   k_snap_ui_rg  (twojmax <= 8) one wavefront per atom, seven neighbours at
-//                 a time, nine lanes per neighbour: the layer recursion in
-//                 registers (lane ma holds column entries (ma, mb)), sums
-//                 sfac*U per lane, then over the groups; U_tot (285 complex
-//                 at twojmax 8) written with its mirror entries
+//   k_snap_neigh_ui  one wavefront per atom: compacts the in-cutoff neighbours
+//                 (FP64 distance test, list order kept) with ballots, writes
+//                 each neighbour's Cayley-Klein parameters, switching function
+//                 and derivative factors (snap_par) once, and sums sfac*U over
+//                 the neighbours with the layer recursion in registers (nine
+//                 lanes per neighbour, seven neighbours at a time at twojmax
+//                 <= 8); U_tot (285 complex at twojmax 8) written with its
+//                 mirror entries.  k_snap_ui_rg: U_tot alone
 //   k_snap_yflat  one block per atom: U_tot staged in LDS, Y (155 half-plane
 //                 entries at twojmax 8) from a host-built flat stream of
 //                 weighted U_a U_b products
-//   k_snap_fij_rev (twojmax <= 8) the force as the gradient of
-//                 sum Re(conj(U) sfac w Y): U forward in registers (same
-//                 layout), adjoints backward, two complex sums per lane,
-//                 seven neighbours per wavefront, atomic scatter to f_i / f_j
-//   k_snap_ui, k_snap_fij  the same for the size class twojmax <= 12: one
-//                 neighbour per wavefront, layers in LDS
-//   k_snap_energy one block per atom: B_k from U_tot and Z, energy
+//   k_snap_fij_rev  the force as the gradient of sum Re(conj(U) sfac w Y): U
+//                 forward in registers (same layout), adjoints backward, two
+//                 complex sums per lane, atomic scatter to f_i / f_j
+//   k_snap_energy a third of Re(conj(U_tot) Y) per atom, and the repulsion
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
@@ -50,18 +44,16 @@
 namespace {
 
 // Two size classes: twojmax <= 8 (the kernels tuned for SNAP-2k, whose
-// twojmax is 8) and twojmax <= 12 (the same kernels with larger LDS tables,
-// one neighbour per wavefront in the force kernel).  Per class J:
+// twojmax is 8) and twojmax <= 12 (the same kernels with larger tables and
+// more registers, four neighbours per wavefront).  Per class J:
 constexpr int SNAP_MAXJ = 8;                 // the first class
 constexpr int SNAP_JBIG = 12;                // the second class: the largest twojmax
-constexpr int SNAP_RPD = SNAP_JBIG + 2;      // row length of the rootpq table
 constexpr double SNAP_PI = 3.14159265358979323846;
 
 // U entries sum_j (j+1)^2, half-plane entries sum_j (j+1)(j/2+1), (a,b,J)
 // triples and bispectrum components (diagonalstyle 3) up to twojmax J
 constexpr int snap_nu(int J) { return J < 0 ? 0 : snap_nu(J - 1) + (J + 1) * (J + 1); }
 constexpr int snap_ny(int J) { return J < 0 ? 0 : snap_ny(J - 1) + (J + 1) * (J / 2 + 1); }
-constexpr int snap_hp(int j) { return (j + 1) * (j / 2 + 1); }  // half plane of layer j
 constexpr int snap_counts(int J, bool coeff) {
   int n = 0;
   for (int j1 = 0; j1 <= J; j1++)
@@ -72,12 +64,8 @@ constexpr int snap_counts(int J, bool coeff) {
 }
 template <int J>
 struct snap_dim {
-  static constexpr int JD = J + 1;
   static constexpr int NU = snap_nu(J);
   static constexpr int NY = snap_ny(J);
-  static constexpr int HPW = (snap_hp(J) + 63) / 64 * 64;  // lane-table width of a layer
-  static constexpr int HPPREV = snap_hp(J - 1);             // half plane of layer J-1
-  static constexpr int FULLPREV = J * J;                    // full layer J-1
 };
 constexpr int SNAP_MAXT = snap_counts(SNAP_JBIG, false);  // (a,b,J) triples: 343
 constexpr int SNAP_MAXC = snap_counts(SNAP_JBIG, true);   // components: 140
@@ -94,7 +82,6 @@ struct snap_dev_tables {
   int ystart[SNAP_JBIG + 2];       // half-plane offsets: ystart[J] + mb*(J+1) + ma
   int yjstart[SNAP_JBIG + 2];      // (a,b) list for each J in ytab
   int ny_terms;
-  double rootpq[SNAP_RPD * SNAP_RPD];  // sqrt(p/q) at p * SNAP_RPD + q
   double rfac0, rmin0, rcut, wj, wself;
   int switchflag;
 };
@@ -122,6 +109,9 @@ struct cplx {
   T r, i;
 };
 
+__device__ __forceinline__ void snap_sincos(float a, float &s, float &c) { sincosf(a, &s, &c); }
+__device__ __forceinline__ void snap_sincos(double a, double &s, double &c) { sincos(a, &s, &c); }
+
 // ------------------------------------------------------------- switching
 template <class T>
 __device__ __forceinline__ void sfac_dsfac(const snap_dev_tables &t, T r, T &sfac, T &dsfac) {
@@ -136,8 +126,10 @@ __device__ __forceinline__ void sfac_dsfac(const snap_dev_tables &t, T r, T &sfa
     dsfac = 0;
   } else {
     const T rcutfac = (T)(SNAP_PI / (t.rcut - t.rmin0));
-    sfac = (T)0.5 * (cos((r - (T)t.rmin0) * rcutfac) + (T)1);
-    dsfac = (T)-0.5 * sin((r - (T)t.rmin0) * rcutfac) * rcutfac;
+    T cs, sn;
+    snap_sincos((r - (T)t.rmin0) * rcutfac, sn, cs);
+    sfac = (T)0.5 * (cs + (T)1);
+    dsfac = (T)-0.5 * sn * rcutfac;
   }
 }
 
@@ -166,7 +158,8 @@ __device__ __forceinline__ void snap_par_of(const snap_dev_tables &t, double dx,
   const T r = sqrt(rsq);
   const T rscale0 = (T)t.rfac0 * (T)SNAP_PI / ((T)t.rcut - (T)t.rmin0);
   const T theta0 = (r - (T)t.rmin0) * rscale0;
-  const T cs = cos(theta0), sn = sin(theta0);
+  T cs, sn;
+  snap_sincos(theta0, sn, cs);
   const T z0 = r * cs / sn;
   const T dz0dr = z0 / r - (r * rscale0) * (rsq + z0 * z0) / rsq;
   const T rinv = (T)1 / r;
@@ -193,8 +186,8 @@ __device__ __forceinline__ void snap_par_of(const snap_dev_tables &t, double dx,
 
 // the reference's ad-hoc pair repulsion as F/r, force_snap_neigh_impl.h:705-711
 __device__ __forceinline__ double snap_fdivr(double dx, double dy, double dz) {
-  const double rsq = dx * dx + dy * dy + dz * dz;
-  return -1.5e6 / pow(rsq, 7.0);
+  const double r2 = dx * dx + dy * dy + dz * dz, r4 = r2 * r2;
+  return -1.5e6 / (r4 * r4 * r4 * r2);
 }
 
 }  // namespace
@@ -209,14 +202,14 @@ __device__ __forceinline__ double snap_fdivr(double dx, double dy, double dz) {
 // parameters (snap_par, FP32 or FP64) and the repulsion F/r (fdv) are
 // written as well.
 // (the body of k_snap_neigh for atom i and one wavefront; returns the count)
+template <class T>
 __device__ __forceinline__ int snap_compact(const snap_dev_tables &t, int i, const double *__restrict__ x,
                                             const int *__restrict__ row, const int *__restrict__ num,
                                             const int *__restrict__ entries, int pitch, int n,
                                             double cutsq, int maxn, int *__restrict__ nin,
                                             int *__restrict__ nj, double *__restrict__ nr,
                                             double *__restrict__ f64, float *__restrict__ f32,
-                                            int ntot, snap_par<float> *__restrict__ p32,
-                                            snap_par<double> *__restrict__ p64,
+                                            int ntot, snap_par<T> *__restrict__ par,
                                             double *__restrict__ fdv) {
 #pragma clang fp contract(off)  // the distance test as the reference (the parameters are
                                 // computed in functions of their own)
@@ -256,28 +249,14 @@ __device__ __forceinline__ int snap_compact(const snap_dev_tables &t, int i, con
         nr[3 * o] = dx;
         nr[3 * o + 1] = dy;
         nr[3 * o + 2] = dz;
-        if (p64) snap_par_of<double>(t, dx, dy, dz, p64[o]);
-        if (p32) snap_par_of<float>(t, dx, dy, dz, p32[o]);
-        if (fdv) fdv[o] = snap_fdivr(dx, dy, dz);
+        snap_par_of<T>(t, dx, dy, dz, par[o]);
+        fdv[o] = snap_fdivr(dx, dy, dz);
       }
     }
     run += __popcll(m);
   }
   if (lane == 0) nin[i] = run < maxn ? run : maxn;
   return run < maxn ? run : maxn;
-}
-
-__global__ void __launch_bounds__(64)
-k_snap_neigh(snap_dev_tables t, const double *__restrict__ x, const int *__restrict__ row,
-             const int *__restrict__ num, const int *__restrict__ entries, int pitch, int n,
-             double cutsq, int maxn, int *__restrict__ nin, int *__restrict__ nj,
-             double *__restrict__ nr, double *__restrict__ f64, float *__restrict__ f32,
-             int ntot, snap_par<float> *__restrict__ p32, snap_par<double> *__restrict__ p64,
-             double *__restrict__ fdv) {
-  const int i = blockIdx.x;
-  if (i >= n) return;
-  snap_compact(t, i, x, row, num, entries, pitch, n, cutsq, maxn, nin, nj, nr, f64, f32, ntot, p32,
-               p64, fdv);
 }
 
 // the neighbour parameters of one precision (and the repulsion F/r) from the
@@ -296,178 +275,11 @@ k_snap_par(snap_dev_tables t, const int *__restrict__ nin, const double *__restr
   }
 }
 
-// layer entry owned by lane l in layer j: (ma, mb) with mb <= j/2
-__device__ __forceinline__ bool lane_entry(int l, int j, int &ma, int &mb) {
-  mb = l / (j + 1);
-  ma = l - mb * (j + 1);
-  return 2 * mb <= j;
-}
-
-// per-layer lane table, built once per block in LDS: for layer j and
-// half-plane entry e (e = mb*(j+1) + ma, mb <= j/2) the indices (ma, mb), and
-// the rootpq table; the per-neighbour layer loop then does no integer
-// division and reads the recursion factors rootpq(j-ma, j-mb) and
-// rootpq(ma, j-mb) from LDS
-template <class T, int J>
-struct layer_tab {
-  static constexpr int JD = snap_dim<J>::JD, W = snap_dim<J>::HPW;
-  int mm[JD][W];                // ma | mb << 8 | (entry exists) << 16
-  T rp[JD * JD];                // rootpq(p, q) at p * JD + q
-  __device__ T rpa(int j, int ma, int mb) const { return rp[(j - ma) * JD + (j - mb)]; }
-  __device__ T rpb(int j, int ma, int mb) const { return rp[ma * JD + (j - mb)]; }
-};
-
-template <class T, int J>
-__device__ __forceinline__ void layer_tab_fill(const snap_dev_tables &t, layer_tab<T, J> &L) {
-  constexpr int JD = layer_tab<T, J>::JD, W = layer_tab<T, J>::W;
-  for (int k = threadIdx.x; k < JD * W; k += blockDim.x) {
-    const int j = k / W, e = k % W;
-    const int mb = e / (j + 1), ma = e - mb * (j + 1);
-    const bool own = j <= t.twojmax && e < snap_hp(j);
-    L.mm[j][e] = ma | (mb << 8) | (own ? 1 << 16 : 0);
-  }
-  for (int k = threadIdx.x; k < JD * JD; k += blockDim.x)
-    L.rp[k] = (T)t.rootpq[(k / JD) * SNAP_RPD + (k % JD)];
-}
-
-// one entry of layer j from the full layer j-1 (row-major ma*j+mb), with the
-// recursion factors from the layer table:
-// U(j,ma,mb) = [ma<j] rp(j-ma,j-mb) conj(a) U(j-1,ma,mb)
-//            - [ma>0] rp(ma,j-mb)  conj(b) U(j-1,ma-1,mb)
-// (SNA::compute_uarray, sna_impl.hpp:663-695)
-template <class T>
-__device__ __forceinline__ cplx<T> u_step_tab(const T *pr, const T *pi, int j, int ma, int mb,
-                                              T rpa, T rpb, T a_r, T a_i, T b_r, T b_i) {
-  cplx<T> u{0, 0};
-  if (ma < j) {
-    const T ur = pr[ma * j + mb], ui = pi[ma * j + mb];
-    u.r += rpa * (a_r * ur + a_i * ui);
-    u.i += rpa * (a_r * ui - a_i * ur);
-  }
-  if (ma > 0) {
-    const T ur = pr[(ma - 1) * j + mb], ui = pi[(ma - 1) * j + mb];
-    u.r += -rpb * (b_r * ur + b_i * ui);
-    u.i += -rpb * (b_r * ui - b_i * ur);
-  }
-  return u;
-}
-
-// Cayley-Klein parameters a = (z0 - i z)/r0, b = (y - i x)/r0
-template <class T>
-__device__ __forceinline__ void ck_params(T x, T y, T z, T z0, T r, T &a_r, T &a_i, T &b_r,
-                                          T &b_i) {
-  const T r0inv = (T)1 / sqrt(r * r + z0 * z0);
-  a_r = r0inv * z0;
-  a_i = -r0inv * z;
-  b_r = r0inv * y;
-  b_i = -r0inv * x;
-}
-
 // ordering of LDS traffic among the lanes of one wavefront (no block barrier)
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// U_tot of every atom for the size class twojmax <= 12 (SNA::compute_ui,
-// sna_impl.hpp:152-190): one block of
-// UI_WAVES wavefronts per atom, wavefront w takes neighbours w, w+UI_WAVES, ...
-// (lanes over the half-plane entries of a layer, 64 at a time, the previous
-// layer in the wavefront's own LDS buffer), then the partial sums of the
-// wavefronts are added in wavefront order (deterministic)
-constexpr int UI_WAVES = 4;
-
-template <class T, int J>
-__global__ void __launch_bounds__(64 * UI_WAVES)
-k_snap_ui(snap_dev_tables t, const int *__restrict__ nin, const double *__restrict__ nr,
-          int maxn, int n, T *__restrict__ utot_r, T *__restrict__ utot_i) {
-  constexpr int JD = snap_dim<J>::JD, W = snap_dim<J>::HPW;
-  __shared__ T s_r[UI_WAVES][2][JD * JD], s_i[UI_WAVES][2][JD * JD];
-  __shared__ T s_pr[UI_WAVES][snap_dim<J>::NY], s_pi[UI_WAVES][snap_dim<J>::NY];
-  __shared__ layer_tab<T, J> LT;
-  const int i = blockIdx.x;
-  if (i >= n) return;
-  layer_tab_fill(t, LT);
-  __syncthreads();
-  const int w = threadIdx.x / 64, l = threadIdx.x % 64;
-  const int twojmax = t.twojmax;
-  // this wavefront's sums over its neighbours, half-plane index
-  // ystart[j] + e (only the lane of entry e ever touches it)
-  T *acc_r = s_pr[w], *acc_i = s_pi[w];
-  for (int k = l; k < t.ny; k += 64) acc_r[k] = acc_i[k] = 0;
-  wave_sync();
-  const int cnt = nin[i];
-  T (*br)[JD * JD] = s_r[w];
-  T (*bi)[JD * JD] = s_i[w];
-  for (int jj = w; jj < cnt; jj += UI_WAVES) {
-    const size_t o = (size_t)i * maxn + jj;
-    const T x = (T)nr[3 * o], y = (T)nr[3 * o + 1], z = (T)nr[3 * o + 2];
-    const T r = sqrt(x * x + y * y + z * z);
-    const T theta0 = (r - (T)t.rmin0) * (T)t.rfac0 * (T)SNAP_PI / ((T)t.rcut - (T)t.rmin0);
-    const T z0 = r / tan(theta0);
-    T a_r, a_i, b_r, b_i;
-    ck_params(x, y, z, z0, r, a_r, a_i, b_r, b_i);
-    T sfac, dsfac;
-    sfac_dsfac(t, r, sfac, dsfac);
-    sfac *= (T)t.wj;
-    // layer 0
-    if (l == 0) {
-      br[0][0] = 1;
-      bi[0][0] = 0;
-      acc_r[0] += sfac;
-    }
-    wave_sync();
-    for (int j = 1; j <= twojmax; j++) {
-      const int p = (j - 1) & 1, c = j & 1;
-      for (int e = l; e < W; e += 64) {
-        const int info = LT.mm[j][e];
-        const bool own = info >> 16;
-        const int ma = info & 255, mb = (info >> 8) & 255;
-        if (own) {
-          const cplx<T> u = u_step_tab<T>(br[p], bi[p], j, ma, mb, LT.rpa(j, ma, mb),
-                                          LT.rpb(j, ma, mb), a_r, a_i, b_r, b_i);
-          // full layer j: own entry and, off the middle column, its mirror
-          br[c][ma * (j + 1) + mb] = u.r;
-          bi[c][ma * (j + 1) + mb] = u.i;
-          if (2 * mb != j) {
-            const T sg = ((ma + mb) & 1) ? (T)-1 : (T)1;
-            br[c][(j - ma) * (j + 1) + (j - mb)] = sg * u.r;
-            bi[c][(j - ma) * (j + 1) + (j - mb)] = -sg * u.i;
-          }
-          acc_r[t.ystart[j] + e] += sfac * u.r;
-          acc_i[t.ystart[j] + e] += sfac * u.i;
-        }
-      }
-      wave_sync();
-    }
-  }
-  __syncthreads();
-  if (w != 0) return;
-  // U_tot = wself * I + sum over wavefronts; own entries and mirrors
-  T *ur = utot_r + (size_t)i * t.nu, *ui = utot_i + (size_t)i * t.nu;
-  for (int j = 0; j <= twojmax; j++) {
-    for (int e = l; e < W; e += 64) {
-      const int info = LT.mm[j][e];
-      const int ma = info & 255, mb = (info >> 8) & 255;
-      if (info >> 16) {
-        T vr = 0, vi = 0;
-#pragma unroll
-        for (int q = 0; q < UI_WAVES; q++) {
-          vr += s_pr[q][t.ystart[j] + e];
-          vi += s_pi[q][t.ystart[j] + e];
-        }
-        if (ma == mb) vr += (T)t.wself;
-        ur[t.ustart[j] + ma * (j + 1) + mb] = vr;
-        ui[t.ustart[j] + ma * (j + 1) + mb] = vi;
-        if (2 * mb != j) {
-          const T sg = ((ma + mb) & 1) ? (T)-1 : (T)1;
-          ur[t.ustart[j] + (j - ma) * (j + 1) + (j - mb)] = sg * vr;
-          ui[t.ustart[j] + (j - ma) * (j + 1) + (j - mb)] = -sg * vi;
-        }
-      }
-    }
-  }
 }
 
 // Z_{abJ}(ma,mb) = sum_ma1 cg(ma1,ma2) sum_mb1 cg(mb1,mb2) U_a(ma1,mb1) U_b(ma2,mb2)
@@ -699,238 +511,48 @@ __global__ void k_yf_weights(int nslots, const unsigned short *__restrict__ key,
   w32[s] = (float)v;
 }
 
-// F_ij of the size class J = 12, one (atom, neighbour) pair per wavefront
-// (SNA::compute_duidrj + compute_duarray, sna_impl.hpp:290-321 / 728-893,
-// then the Y contraction): the lanes take the half-plane entries of a layer
-// 64 at a time (layers below the top have up to 72 entries, two steps), the
-// previous layer of U and dU in LDS.  (For twojmax <= 8 the register-resident
-// k_snap_fij_rev replaces it.)
-constexpr int FIJ_WAVES = 2;  // wavefronts per block
-
-template <class T, class TF, int J>
-__global__ void __launch_bounds__(64 * FIJ_WAVES)
-k_snap_fij(snap_dev_tables t, const int *__restrict__ nin, const int *__restrict__ nj,
-           const double *__restrict__ nr, int maxn, int n, const T *__restrict__ y_r,
-           const T *__restrict__ y_i, TF *__restrict__ f) {
-  constexpr int LG = 64;                      // lanes per neighbour
-  constexpr int NBW = 64 / LG;                // neighbours per wavefront
-  constexpr int FIJ_NB = FIJ_WAVES * NBW;     // neighbours per block
-  constexpr int FIJ_HP = snap_dim<J>::HPPREV;  // half-plane entries of layer J-1
-  // a layer below the top takes at most two steps (kept in registers below)
-  static_assert((FIJ_HP + LG - 1) / LG <= 2, "two steps per layer below the top");
-  static_assert(((snap_hp(J) + LG - 1) / LG) * LG <= snap_dim<J>::HPW, "lane table width");
-  // previous layer (j-1 <= 7) of each neighbour: U and dU (3 components) of
-  // its half plane (mb <= (j-1)/2, at mb*j + ma: at most 32 entries); the
-  // middle column of an even layer reads its mirror image
-  // U(j-1-ma, j-1-mb) = (-1)^(ma+mb) conj U(ma, mb) (the same symmetry holds
-  // for dU), so no lane writes a mirror entry.  One buffer: a layer's
-  // entries are kept in registers until every lane has read the previous
-  // layer (a layer below the top has at most 32 entries, two steps of 16
-  // lanes), then written over it.
-  __shared__ T s_u[FIJ_NB][8][FIJ_HP];
-  __shared__ T s_y[2][snap_dim<J>::NY];
-  __shared__ layer_tab<T, J> LT;
-  const int w = threadIdx.x / 64, l = threadIdx.x % 64;
-  const int hs = l / LG, hl = l % LG;  // neighbour slot of the wavefront, lane in it
-  const int i = blockIdx.x;
-  if (i >= n) return;
-  const int cnt_i = nin[i];
-  if (blockIdx.y * FIJ_NB >= cnt_i) return;  // no neighbour for this block
-  // Y of atom i, read by every layer of every neighbour of the block
-  for (int k = threadIdx.x; k < t.ny; k += blockDim.x) {
-    s_y[0][k] = y_r[(size_t)i * t.ny + k];
-    s_y[1][k] = y_i[(size_t)i * t.ny + k];
-  }
-  layer_tab_fill(t, LT);
-  __syncthreads();
-  const int jj0 = blockIdx.y * FIJ_NB + NBW * w;  // the wavefront's first neighbour
-  if (jj0 >= cnt_i) return;                       // uniform over the wavefront
-  const int jj = jj0 + hs;
-  const bool act = jj < cnt_i;
-  const size_t o = (size_t)i * maxn + (act ? jj : jj0);
-  const double xd = nr[3 * o], yd = nr[3 * o + 1], zd = nr[3 * o + 2];
-  const T x = (T)xd, y = (T)yd, z = (T)zd;
-  const T rsq = x * x + y * y + z * z;
-  const T r = sqrt(rsq);
-  const T rscale0 = (T)t.rfac0 * (T)SNAP_PI / ((T)t.rcut - (T)t.rmin0);
-  const T theta0 = (r - (T)t.rmin0) * rscale0;
-  const T cs = cos(theta0), sn = sin(theta0);
-  const T z0 = r * cs / sn;
-  const T dz0dr = z0 / r - (r * rscale0) * (rsq + z0 * z0) / rsq;
-  const T rinv = (T)1 / r;
-  const T u3[3] = {x * rinv, y * rinv, z * rinv};
-  const T r0inv = (T)1 / sqrt(r * r + z0 * z0);
-  const T a_r = z0 * r0inv, a_i = -z * r0inv, b_r = y * r0inv, b_i = -x * r0inv;
-  const T dr0invdr = -(r0inv * r0inv * r0inv) * (r + z0 * dz0dr);
-  T da_r[3], da_i[3], db_r[3], db_i[3];
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-    const T dr0 = dr0invdr * u3[k], dz = dz0dr * u3[k];
-    da_r[k] = dz * r0inv + z0 * dr0;
-    da_i[k] = -z * dr0;
-    db_r[k] = y * dr0;
-    db_i[k] = -x * dr0;
-  }
-  da_i[2] += -r0inv;
-  db_i[0] += -r0inv;
-  db_r[1] += r0inv;
-  T sfac, dsfac;
-  sfac_dsfac(t, r, sfac, dsfac);
-  sfac *= (T)t.wj;
-  dsfac *= (T)t.wj;
-
-  T (*buf)[FIJ_HP] = s_u[NBW * w + hs];
-  const T *yr = s_y[0], *yi = s_y[1];
-  T fx = 0, fy = 0, fz = 0;
-  // layer 0: U = 1, dU = 0; its dU_tot = dsfac * u; contraction with Y_0
-  if (hl == 0) {
-    buf[0][0] = 1; buf[1][0] = 0;
-    for (int k = 0; k < 3; k++) { buf[2 + 2 * k][0] = 0; buf[3 + 2 * k][0] = 0; }
-    const T w0 = (T)0.5;  // J = 0: the single entry is the middle-column diagonal
-    const T c = dsfac * w0 * yr[0];
-    fx += c * u3[0];
-    fy += c * u3[1];
-    fz += c * u3[2];
-  }
-  wave_sync();
-  constexpr int FIJ_STEPS = (snap_hp(J) + LG - 1) / LG;  // steps of the top layer
-  for (int j = 1; j <= t.twojmax; j++) {
-    const int ne = (j + 1) * (j / 2 + 1);
-    T keep[2][8];  // this layer's own entries of steps 0 and 1
-#pragma unroll
-    for (int st = 0; st < FIJ_STEPS; st++) {
-      const int s0 = st * LG;
-      if (s0 >= ne) break;
-      const int e = s0 + hl;
-      const int info = LT.mm[j][e];
-      const int ma = info & 255, mb = (info >> 8) & 255;
-      const bool own = info >> 16;
-      T ur = 0, ui = 0, dr[3] = {0, 0, 0}, di[3] = {0, 0, 0};
-      if (own) {
-        const T *P = &buf[0][0];
-        // P[q*FIJ_HP + idx]: q = 0 U_r, 1 U_i, 2+2k dU_r[k], 3+2k dU_i[k].
-        // Layer j-1 entries (ma, mb) and (ma-1, mb); on the middle column of
-        // an even layer (mb = j/2 > (j-1)/2) they are read as mirrors.
-        const bool mir = 2 * mb == j;
-        const T sgn = ((ma + mb) & 1) ? (T)-1 : (T)1;
-        const T s_r = mir ? sgn : (T)1, s_i = mir ? -sgn : (T)1;  // (ma, mb); (ma-1, mb) flips sgn
-        if (ma < j) {
-          const T rp = LT.rpa(j, ma, mb);
-          const int sidx = mir ? (j - 1 - mb) * j + (j - 1 - ma) : mb * j + ma;
-          const T pr = s_r * P[sidx], pi = s_i * P[FIJ_HP + sidx];
-          ur += rp * (a_r * pr + a_i * pi);
-          ui += rp * (a_r * pi - a_i * pr);
-#pragma unroll
-          for (int k = 0; k < 3; k++) {
-            const T dpr = s_r * P[(2 + 2 * k) * FIJ_HP + sidx];
-            const T dpi = s_i * P[(3 + 2 * k) * FIJ_HP + sidx];
-            dr[k] += rp * (da_r[k] * pr + da_i[k] * pi + a_r * dpr + a_i * dpi);
-            di[k] += rp * (da_r[k] * pi - da_i[k] * pr + a_r * dpi - a_i * dpr);
-          }
-        }
-        if (ma > 0) {
-          const T rp = LT.rpb(j, ma, mb);
-          const int sidx = mir ? (j - 1 - mb) * j + (j - ma) : mb * j + ma - 1;
-          const T tr = mir ? -s_r : (T)1, ti = mir ? -s_i : (T)1;
-          const T pr = tr * P[sidx], pi = ti * P[FIJ_HP + sidx];
-          ur += -rp * (b_r * pr + b_i * pi);
-          ui += -rp * (b_r * pi - b_i * pr);
-#pragma unroll
-          for (int k = 0; k < 3; k++) {
-            const T dpr = tr * P[(2 + 2 * k) * FIJ_HP + sidx];
-            const T dpi = ti * P[(3 + 2 * k) * FIJ_HP + sidx];
-            dr[k] += -rp * (db_r[k] * pr + db_i[k] * pi + b_r * dpr + b_i * dpi);
-            di[k] += -rp * (db_r[k] * pi - db_i[k] * pr + b_r * dpi - b_i * dpr);
-          }
-        }
-      }
-      if (st < 2) {
-        keep[st][0] = ur; keep[st][1] = ui;
-#pragma unroll
-        for (int k = 0; k < 3; k++) { keep[st][2 + 2 * k] = dr[k]; keep[st][3 + 2 * k] = di[k]; }
-      }
-      if (own) {
-        // half-plane weight of (ma, mb) in layer j
-        T wgt = 1;
-        if (2 * mb == j) wgt = (ma < mb) ? (T)1 : ((ma == mb) ? (T)0.5 : (T)0);
-        if (wgt != (T)0) {
-          const int ey = t.ystart[j] + mb * (j + 1) + ma;
-          const T Yr = wgt * yr[ey], Yi = wgt * yi[ey];
-          const T uy = ur * Yr + ui * Yi;   // Re(conj(U) Y) (switching-derivative term)
-          const T g[3] = {dr[0] * Yr + di[0] * Yi, dr[1] * Yr + di[1] * Yi, dr[2] * Yr + di[2] * Yi};
-          fx += dsfac * uy * u3[0] + sfac * g[0];
-          fy += dsfac * uy * u3[1] + sfac * g[1];
-          fz += dsfac * uy * u3[2] + sfac * g[2];
-        }
-      }
-    }
-    wave_sync();  // every lane has read layer j-1
-    if (j < t.twojmax) {
-      // own half-plane entries only (ne <= 32 below the top layer)
-#pragma unroll
-      for (int st = 0; st < 2; st++) {
-        const int e = st * LG + hl;
-        if (st * LG < ne && (LT.mm[j][e] >> 16)) {
-#pragma unroll
-          for (int q = 0; q < 8; q++) buf[q][e] = keep[st][q];
-        }
-      }
-    }
-    wave_sync();
-  }
-  // sum of the force components over the neighbour's lanes
-#pragma unroll
-  for (int off = LG / 2; off > 0; off >>= 1) {
-    fx += __shfl_xor(fx, off, LG);
-    fy += __shfl_xor(fy, off, LG);
-    fz += __shfl_xor(fz, off, LG);
-  }
-  if (hl == 0 && act) {
-    // ad-hoc repulsion of the reference, force_snap_neigh_impl.h:705-711
-    const double rsqd = xd * xd + yd * yd + zd * zd;
-    const double fdivr = -1.5e6 / pow(rsqd, 7.0);
-    const TF Fx = (TF)fx + (TF)(xd * fdivr);
-    const TF Fy = (TF)fy + (TF)(yd * fdivr);
-    const TF Fz = (TF)fz + (TF)(zd * fdivr);
-    const int j = nj[o];
-    atomicAdd(&f[3 * (size_t)i], Fx);
-    atomicAdd(&f[3 * (size_t)i + 1], Fy);
-    atomicAdd(&f[3 * (size_t)i + 2], Fz);
-    atomicAdd(&f[3 * (size_t)j], -Fx);
-    atomicAdd(&f[3 * (size_t)j + 1], -Fy);
-    atomicAdd(&f[3 * (size_t)j + 2], -Fz);
-  }
-}
-
 // ------------------------------------------- register-resident recursion
-// For twojmax <= 8 a neighbour's layer fits nine lanes: lane ma (0..8) of
-// the neighbour's group holds the entries (ma, mb) of every half-plane
-// column mb (0..4) of the current layer in registers.  The recursion
-//   U_j(ma,mb) = rpa conj(a) U_{j-1}(ma,mb) - rpb conj(b) U_{j-1}(ma-1,mb)
-// reads U_{j-1}(ma,mb) from the lane's own register and U_{j-1}(ma-1,mb)
-// from the lane below (a DPP shift of the whole wavefront by one lane; at
-// ma = 0 rpb is 0 and the value from the group below is not used).  The
-// middle column mb = j/2 of an even layer needs U_{j-1}(ma, j/2), outside
-// the previous half plane: it is the mirror (-1)^(ma+j/2) conj
-// U_{j-1}(j-1-ma, j/2-1), fetched from lane j-1-ma of the group by one
-// permute per value.  Seven neighbours per wavefront (lane 63 idle); no LDS
-// traffic for the layers and no barriers between them.  The recursion
-// factors and the half-plane-weighted Y of each (column, ma) come from one
-// LDS record, zero where the entry does not exist (ma > j), so lanes past
-// the layer compute exact zeros.
-constexpr int RG_W = SNAP_MAXJ + 1;  // lanes per neighbour (ma = 0..8)
-constexpr int RG_NB = 64 / RG_W;     // neighbours per wavefront: 7
-constexpr int RG_COLS = SNAP_MAXJ / 2 + 1;
-// first column slot of layer j: sum over layers j' < j of (j'/2 + 1) columns
+// A neighbour's layer j fits the J + 1 lanes of its group: lane ma holds the
+// entries (ma, mb) of every half-plane column mb = 0..j/2 in registers.
+// The kernels carry V rather than U,
+//   U_j(ma,mb) = norm_j(ma,mb) V_j(ma,mb),
+//   norm_j(ma,mb) = sqrt(ma! (j-ma)! / (mb! (j-mb)!)),
+// because the factors sqrt((j-ma)/(j-mb)) and sqrt(ma/(j-mb)) of the
+// recursion of SNA::compute_uarray (sna_impl.hpp:663-695) cancel in V:
+//   V_j(ma,mb)  = conj(a) V_{j-1}(ma,mb)   - conj(b) V_{j-1}(ma-1,mb)
+// and, its mirror image (the norm is the same at (j-ma, j-mb)),
+//   V_j(ma,j/2) = b V_{j-1}(ma,j/2-1) + a V_{j-1}(ma-1,j/2-1)
+// for the middle column of an even layer, whose first form would need
+// columns outside the half plane.  So an entry takes 8 multiply-adds (12 and
+// a table record with the factors), V(ma-1) comes from the lane below by a
+// DPP shift and nothing is permuted.  V is exactly 0 where the entry does
+// not exist (ma > j): the borders need no test, and what the lane shifts
+// carry over a group's edge meets only such zeros.  The norm is applied once
+// per atom, to the sums over the neighbours or to Y.
+// FP64 (FP32) arithmetic bounds all three kernels (70 % of its issue rate in
+// the force kernel).  Against U with its factors, FP64, 16 000 atoms of 26
+// neighbours, twojmax 8: U_tot 174 -> 81 us, force 232 -> 148 us; W of 64 BCC
+// configurations of 128 to 1024 atoms 820 -> 275 us; mixed, 2000 atoms: 24.4 -> 15.9 and 28.6 -> 15.7 us.  Twojmax 12,
+// 1024 atoms, against one neighbour per wavefront with the layers in LDS:
+// U_tot 140 -> 27 us (FP64), force 141 -> 29 us (mixed).
+// Groups of 9 lanes, seven per wavefront (one lane idle), for twojmax <= 8;
+// of 13 lanes, four per wavefront, up to 12.
 __host__ __device__ constexpr int rg_slot0(int j) { return j <= 0 ? 0 : j + (j - 1) * (j - 1) / 4; }
-constexpr int RG_SLOTS = rg_slot0(SNAP_MAXJ + 1);  // (layer, column) pairs of layers 0..8: 25
+template <int J>
+struct rg {
+  static constexpr int W = J + 1;                // lanes per neighbour (ma = 0..J)
+  static constexpr int NB = 64 / W;              // neighbours per wavefront
+  static constexpr int COLS = J / 2 + 1;         // columns of the top layer
+  static constexpr int SLOTS = rg_slot0(J + 1);  // (layer, column) pairs of layers 0..J
+};
+// first column slot of layer j: sum over layers j' < j of (j'/2 + 1) columns
 static_assert(rg_slot0(1) == 1 && rg_slot0(2) == 2 && rg_slot0(3) == 4 && rg_slot0(8) == 20 &&
-                  RG_SLOTS == 25,
+                  rg<8>::SLOTS == 25 && rg<12>::SLOTS == 49,
               "column slots");
 
 template <class T>
-struct alignas(4 * sizeof(T)) rg_rec {
-  T rpa, rpb, yr, yi;  // recursion factors and weighted Y of (j, ma, mb)
+struct alignas(2 * sizeof(T)) rg_rec {
+  T yr, yi;  // weighted Y of (j, ma, mb), in V's norm
 };
 
 // value of lane l - 1 (0 in lane 0): DPP wavefront shift right by one
@@ -945,220 +567,6 @@ __device__ __forceinline__ double lane_below(double v) {
   const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), 0x138, 0xf, 0xf, true);
   return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
-
-// Per (column slot s, lane ma), k = s * RG_W + ma, built on the host once:
-// the recursion factors (zero where the entry does not exist), and
-//   ey   the half-plane index of Y (or -1), wgt its half-plane weight
-//   uo   the U_tot index of (ma, mb) (or -1), um that of the mirror
-//        (j-ma, j-mb) off the middle column (or -1), neg its sign (-1)^(ma+mb)
-//        and diag for ma == mb (wself)
-template <class T>
-struct rg_rp {
-  T rpa, rpb;
-};
-struct rg_map {
-  int ey, uo, um;
-  unsigned char wq, neg, diag, pad;  // wgt = wq / 2
-};
-
-// the records of one atom: column slot s = rg_slot0(j) + mb, lane ma
-template <class T, int NT>
-__device__ __forceinline__ void rg_fill(const rg_rp<T> *__restrict__ rp,
-                                        const rg_map *__restrict__ map, int ny,
-                                        const T *__restrict__ y_r, const T *__restrict__ y_i,
-                                        int i, rg_rec<T> *rec) {
-#pragma unroll
-  for (int q = 0; q < (RG_SLOTS * RG_W + NT - 1) / NT; q++) {
-    const int k = q * NT + (int)threadIdx.x;
-    if (k < RG_SLOTS * RG_W) {
-      const rg_rp<T> r = rp[k];
-      T yr = 0, yi = 0;
-      if (y_r) {
-        const rg_map m = map[k];
-        if (m.ey >= 0) {
-          const T wgt = (T)0.5 * (T)m.wq;
-          yr = wgt * y_r[(size_t)i * ny + m.ey];
-          yi = wgt * y_i[(size_t)i * ny + m.ey];
-        }
-      }
-      rec[k] = rg_rec<T>{r.rpa, r.rpb, yr, yi};
-    }
-  }
-}
-
-// Sums over the neighbours base0, base0 + stride, ... (seven at a time) of
-// atom i of sfac * U for the lane's entries (ma, mb) of every column of every
-// layer (SNA::compute_ui, sna_impl.hpp:152-190, with the register layout
-// above), added to acc[column slot]
-template <class T>
-__device__ __forceinline__ void rg_u_sums(const snap_dev_tables &t, const rg_rec<T> *s_rec,
-                                          const snap_par<T> *__restrict__ par, int i, int maxn,
-                                          int cnt, int base0, int stride, int g, int ma,
-                                          T (&acc)[RG_SLOTS][2]) {
-  for (int base = base0; base < cnt; base += stride) {
-    const int jj = base + g;
-    const bool act = g < RG_NB && jj < cnt;
-    const size_t o = (size_t)i * maxn + (act ? jj : base);
-    const T a_r = par[o].a_r, a_i = par[o].a_i, b_r = par[o].b_r, b_i = par[o].b_i;
-    const T sfac = act ? par[o].sfac : (T)0;  // an idle group adds nothing
-    T c[RG_COLS][2];
-#pragma unroll
-    for (int mb = 0; mb < RG_COLS; mb++) c[mb][0] = c[mb][1] = 0;
-    c[0][0] = ma == 0 ? (T)1 : (T)0;  // layer 0: U = 1
-    acc[0][0] += sfac * c[0][0];
-#pragma unroll
-    for (int j = 1; j <= SNAP_MAXJ; j++) {
-      if (j > t.twojmax) break;
-      T mir[2], mirb[2];  // even j: U_{j-1}(ma, j/2) and U_{j-1}(ma-1, j/2)
-      if ((j & 1) == 0) {
-        const int src = g * RG_W + (j - 1 - ma > 0 ? j - 1 - ma : 0);
-        const T sg = ((ma + j / 2) & 1) ? (T)-1 : (T)1;
-        mir[0] = sg * __shfl(c[j / 2 - 1][0], src, 64);
-        mir[1] = -sg * __shfl(c[j / 2 - 1][1], src, 64);
-        mirb[0] = lane_below(mir[0]);
-        mirb[1] = lane_below(mir[1]);
-      }
-#pragma unroll
-      for (int mb = 0; mb <= j / 2; mb++) {
-        const int slot = rg_slot0(j) + mb;
-        const rg_rec<T> q = s_rec[slot * RG_W + ma];
-        const bool mid = (j & 1) == 0 && mb == j / 2;
-        const T p0 = mid ? mir[0] : c[mb][0], p1 = mid ? mir[1] : c[mb][1];
-        const T q0 = mid ? mirb[0] : lane_below(c[mb][0]);
-        const T q1 = mid ? mirb[1] : lane_below(c[mb][1]);
-        const T ur = q.rpa * (a_r * p0 + a_i * p1) - q.rpb * (b_r * q0 + b_i * q1);
-        const T ui = q.rpa * (a_r * p1 - a_i * p0) - q.rpb * (b_r * q1 - b_i * q0);
-        c[mb][0] = ur;
-        c[mb][1] = ui;
-        acc[slot][0] += sfac * ur;
-        acc[slot][1] += sfac * ui;
-      }
-    }
-  }
-}
-
-// acc summed over the seven groups of the wavefront (in TA) by a fixed tree
-// of lane shifts (groups 4-6 onto 0-2, then 2-3 onto 0-1, then 1 onto 0);
-// lanes 0..8 store the sums at out[column slot * RG_W + lane]
-template <class T, class TA>
-__device__ __forceinline__ void rg_group_sum(T (&acc)[RG_SLOTS][2], int l, TA *out_r, TA *out_i) {
-#pragma unroll
-  for (int s = 0; s < RG_SLOTS; s++) {
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      TA v = (TA)acc[s][q];
-      TA u = __shfl_down(v, 4 * RG_W, 64);
-      if (l < 3 * RG_W) v += u;
-      u = __shfl_down(v, 2 * RG_W, 64);
-      if (l < 2 * RG_W) v += u;
-      u = __shfl_down(v, RG_W, 64);
-      if (l < RG_W) {
-        v += u;
-        (q ? out_i : out_r)[s * RG_W + l] = v;
-      }
-    }
-  }
-}
-
-// U_tot with the register-resident recursion (twojmax <= 8): a block of
-// UR_WAVES wavefronts per atom, wavefront w over the neighbours 7w, 7w +
-// 7 UR_WAVES, ...; the lane sums added over the groups and then over the
-// wavefronts in order: deterministic.
-template <class T, int UR_WAVES>
-__global__ void __launch_bounds__(64 * UR_WAVES)
-k_snap_ui_rg(snap_dev_tables t, const rg_rp<T> *__restrict__ rgp, const rg_map *__restrict__ rgm,
-             const int *__restrict__ nin, const snap_par<T> *__restrict__ par, int maxn, int n,
-             T *__restrict__ utot_r, T *__restrict__ utot_i) {
-  __shared__ rg_rec<T> s_rec[RG_SLOTS * RG_W];
-  __shared__ T s_acc[UR_WAVES][2][RG_SLOTS * RG_W];
-  const int i = blockIdx.x;
-  if (i >= n) return;
-  rg_fill<T, 64 * UR_WAVES>(rgp, rgm, 0, nullptr, nullptr, i, s_rec);
-  __syncthreads();
-  const int w = threadIdx.x / 64, l = threadIdx.x % 64;
-  const int g = l / RG_W, ma = l - g * RG_W;  // g = 7 only for the idle lane 63
-  T acc[RG_SLOTS][2];
-#pragma unroll
-  for (int s = 0; s < RG_SLOTS; s++) acc[s][0] = acc[s][1] = 0;
-  rg_u_sums<T>(t, s_rec, par, i, maxn, nin[i], w * RG_NB, UR_WAVES * RG_NB, g, ma, acc);
-  rg_group_sum<T, T>(acc, l, s_acc[w][0], s_acc[w][1]);
-  __syncthreads();
-  // U_tot = wself * I + the wavefront sums in order; own entries and mirrors
-  T *ur = utot_r + (size_t)i * t.nu, *ui = utot_i + (size_t)i * t.nu;
-  for (int k = threadIdx.x; k < RG_SLOTS * RG_W; k += blockDim.x) {
-    const rg_map m = rgm[k];
-    if (m.uo < 0) continue;
-    T vr = 0, vi = 0;
-#pragma unroll
-    for (int q = 0; q < UR_WAVES; q++) {
-      vr += s_acc[q][0][k];
-      vi += s_acc[q][1][k];
-    }
-    if (m.diag) vr += (T)t.wself;
-    ur[m.uo] = vr;
-    ui[m.uo] = vi;
-    if (m.um >= 0) {
-      const T sg = m.neg ? (T)-1 : (T)1;
-      ur[m.um] = sg * vr;
-      ui[m.um] = -sg * vi;
-    }
-  }
-}
-
-// The compaction of k_snap_neigh (with the neighbour parameters in T's
-// precision) followed by U_tot in the same wavefront (twojmax <= 8, one
-// wavefront per atom as k_snap_ui_rg<T, 1>): one launch less per force
-// evaluation, and the parameters just written are read back from the cache.
-template <class T>
-__global__ void __launch_bounds__(64)
-k_snap_neigh_ui(snap_dev_tables t, const rg_rp<T> *__restrict__ rgp, const rg_map *__restrict__ rgm,
-                const double *__restrict__ x, const int *__restrict__ row,
-                const int *__restrict__ num, const int *__restrict__ entries, int pitch, int n,
-                double cutsq, int maxn, int *__restrict__ nin, int *__restrict__ nj,
-                double *__restrict__ nr, double *__restrict__ f64, float *__restrict__ f32,
-                int ntot, snap_par<T> *__restrict__ par, double *__restrict__ fdv,
-                T *__restrict__ utot_r, T *__restrict__ utot_i) {
-  __shared__ rg_rec<T> s_rec[RG_SLOTS * RG_W];
-  __shared__ T s_acc[2][RG_SLOTS * RG_W];
-  const int i = blockIdx.x;
-  if (i >= n) return;
-  rg_fill<T, 64>(rgp, rgm, 0, nullptr, nullptr, i, s_rec);
-  snap_par<float> *p32 = nullptr;
-  snap_par<double> *p64 = nullptr;
-  if (sizeof(T) == 4) p32 = reinterpret_cast<snap_par<float> *>(par);
-  else p64 = reinterpret_cast<snap_par<double> *>(par);
-  const int cnt = snap_compact(t, i, x, row, num, entries, pitch, n, cutsq, maxn, nin, nj, nr, f64,
-                               f32, ntot, p32, p64, fdv);
-  __syncthreads();  // the wavefront's parameter writes, and the records, are visible
-  const int l = threadIdx.x;
-  const int g = l / RG_W, ma = l - g * RG_W;
-  T acc[RG_SLOTS][2];
-#pragma unroll
-  for (int q = 0; q < RG_SLOTS; q++) acc[q][0] = acc[q][1] = 0;
-  rg_u_sums<T>(t, s_rec, par, i, maxn, cnt, 0, RG_NB, g, ma, acc);
-  rg_group_sum<T, T>(acc, l, s_acc[0], s_acc[1]);
-  __syncthreads();
-  T *ur = utot_r + (size_t)i * t.nu, *ui = utot_i + (size_t)i * t.nu;
-  for (int k = l; k < RG_SLOTS * RG_W; k += 64) {
-    const rg_map m = rgm[k];
-    if (m.uo < 0) continue;
-    T vr = s_acc[0][k];
-    const T vi = s_acc[1][k];
-    if (m.diag) vr += (T)t.wself;
-    ur[m.uo] = vr;
-    ui[m.uo] = vi;
-    if (m.um >= 0) {
-      const T sg = m.neg ? (T)-1 : (T)1;
-      ur[m.um] = sg * vr;
-      ui[m.um] = -sg * vi;
-    }
-  }
-}
-
-// Blocks of RG_WAVES wavefronts take 7 * RG_WAVES neighbours of one atom in
-// the force kernel (grid.y over the neighbour slots).
-constexpr int RG_WAVES = 4;
-
 // value of lane l + 1 (0 in lane 63): DPP wavefront shift left by one
 __device__ __forceinline__ float lane_above(float v) {
   return __builtin_bit_cast(float,
@@ -1171,191 +579,353 @@ __device__ __forceinline__ double lane_above(double v) {
   return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
-// F_ij in reverse mode.  With G_j(e) = sfac * w(e) Y_j(e) (w the half-plane
-// weight) the force on the pair is the gradient of
-//   L = sum_j sum_e Re(conj(U_j(e)) G_j(e))
-// with respect to r_ij.  U_j(e) = alpha_e P_e + beta_e Q_e with
-// alpha = rpa conj(a), beta = -rpb conj(b), P_e = U_{j-1}(ma, mb) and
-// Q_e = U_{j-1}(ma-1, mb) (mirrors on the middle column of an even layer),
-// and r enters only through a, b and sfac.  So, with the adjoints
-// Ubar_j(e) = dL/dRe U + i dL/dIm U propagated from the top layer down,
-//   Ubar_{j-1}(P_e) += conj(alpha) Ubar_j(e),  Ubar_{j-1}(Q_e) += conj(beta) Ubar_j(e)
-// (through a mirror M = s conj(U'): Ubar(U') += s conj(conj(alpha) Ubar_j(e))),
-//   dL/dr_k = dsfac u_k sum Re(conj(U) w Y) + Re(conj(da_k) Sa) - Re(conj(db_k) Sb),
-//   Sa = sum_e rpa conj(Ubar_j(e)) P_e,  Sb = sum_e rpb conj(Ubar_j(e)) Q_e.
-// The forward pass keeps U of layers 0..7 in registers (lane ma holds
-// (ma, mb) of every column, as in k_snap_ui_rg); the backward pass moves
-// adjoints to the lane below with a DPP shift and back through the mirror
-// permutation.  About half the arithmetic of carrying dU/dr forward.
-template <class T, class TF>
-__global__ void __launch_bounds__(64 * RG_WAVES) __attribute__((amdgpu_waves_per_eu(3)))
-k_snap_fij_rev(snap_dev_tables t, const rg_rp<T> *__restrict__ rgp, const rg_map *__restrict__ rgm,
-               const int *__restrict__ nin, const int *__restrict__ nj,
-               const double *__restrict__ nr, const snap_par<T> *__restrict__ par,
-               const double *__restrict__ fdv, int maxn, int n, const T *__restrict__ y_r,
-               const T *__restrict__ y_i, TF *__restrict__ f) {
-  constexpr int TJ = SNAP_MAXJ;
-  __shared__ rg_rec<T> s_rec[RG_SLOTS * RG_W];
-  __shared__ T s_red[RG_WAVES][3][64];
+// Per (column slot s, lane ma), k = s * W + ma, built on the host once:
+//   norm norm_j(ma, mb)
+//   ey   the half-plane index of Y (or -1: the entry does not exist), wgt its
+//        half-plane weight
+//   uo   the U_tot index of (ma, mb), um that of the mirror (j-ma, j-mb) off
+//        the middle column (or -1), neg its sign (-1)^(ma+mb) and diag for
+//        ma == mb (wself)
+struct rg_map {
+  double norm;
+  int ey, uo, um;
+  unsigned char wq, neg, diag, pad;  // wgt = wq / 2
+};
+
+// body(j) for j = FIRST .. LAST (up or down), each j a constant of its own:
+// the register arrays are indexed by it, and the unroller gives up on a loop
+// over the layers at twojmax 12
+template <int FIRST, int LAST, class F>
+__device__ __forceinline__ void rg_layers(const F &body) {
+  body(std::integral_constant<int, FIRST>{});
+  if constexpr (FIRST < LAST) rg_layers<FIRST + 1, LAST>(body);
+  else if constexpr (FIRST > LAST) rg_layers<FIRST - 1, LAST>(body);
+}
+
+// layer j from layer j-1, in place
+template <int j, class T, int COLS>
+__device__ __forceinline__ void rg_layer(T a_r, T a_i, T b_r, T b_i, T (&c)[COLS][2]) {
+  T q[COLS][2];
+#pragma unroll
+  for (int mb = 0; mb <= (j - 1) / 2; mb++) {
+    q[mb][0] = lane_below(c[mb][0]);
+    q[mb][1] = lane_below(c[mb][1]);
+  }
+  if constexpr ((j & 1) == 0) {
+    constexpr int m = j / 2 - 1;
+    c[m + 1][0] = b_r * c[m][0] - b_i * c[m][1] + a_r * q[m][0] - a_i * q[m][1];
+    c[m + 1][1] = b_r * c[m][1] + b_i * c[m][0] + a_r * q[m][1] + a_i * q[m][0];
+  }
+#pragma unroll
+  for (int mb = 0; 2 * mb < j; mb++) {
+    const T p0 = c[mb][0], p1 = c[mb][1];
+    c[mb][0] = a_r * p0 + a_i * p1 - b_r * q[mb][0] - b_i * q[mb][1];
+    c[mb][1] = a_r * p1 - a_i * p0 - b_r * q[mb][1] + b_i * q[mb][0];
+  }
+}
+
+// Sums over the neighbours (NB at a time) of atom i of sfac * V for the
+// lane's entries (ma, mb) of every column of every layer (SNA::compute_ui,
+// sna_impl.hpp:152-190), added to acc[column slot].  The recursion is linear:
+// it starts from sfac.
+template <class T, int J>
+__device__ __forceinline__ void rg_u_sums(const snap_dev_tables &t,
+                                          const snap_par<T> *__restrict__ par, int i, int maxn,
+                                          int cnt, int g, int ma, T (&acc)[rg<J>::SLOTS][2]) {
+  using R = rg<J>;
+  for (int base = 0; base < cnt; base += R::NB) {
+    const int jj = base + g;
+    const bool act = g < R::NB && jj < cnt;
+    const size_t o = (size_t)i * maxn + (act ? jj : base);
+    const T a_r = par[o].a_r, a_i = par[o].a_i, b_r = par[o].b_r, b_i = par[o].b_i;
+    T c[R::COLS][2];
+#pragma unroll
+    for (int mb = 0; mb < R::COLS; mb++) c[mb][0] = c[mb][1] = 0;
+    c[0][0] = act && ma == 0 ? par[o].sfac : (T)0;  // an idle group adds nothing
+    acc[0][0] += c[0][0];
+    rg_layers<1, J>([&](auto jc) {
+      constexpr int j = jc;
+      if (j > t.twojmax) return;
+      rg_layer<j>(a_r, a_i, b_r, b_i, c);
+#pragma unroll
+      for (int mb = 0; mb <= j / 2; mb++) {
+        acc[rg_slot0(j) + mb][0] += c[mb][0];
+        acc[rg_slot0(j) + mb][1] += c[mb][1];
+      }
+    });
+  }
+}
+
+// acc summed over the groups of the wavefront in group order (in TA) and
+// handed to out(column slot * W + ma, sum_r, sum_i), one entry per lane at a
+// time.  Through LDS, RG_CHUNK slots at a time: a row of the buffer holds one
+// value of every lane, and the pitch of 64 + W keeps the W-wide pieces that
+// one read takes from successive rows in successive banks.
+template <int J>
+struct rg_sum {
+  static constexpr int CH = 63 / rg<J>::W;      // column slots at a time
+  static constexpr int PITCH = 64 + rg<J>::W;   // of a row of the buffer
+  static constexpr int BUF = 2 * CH * PITCH;    // values of T
+};
+template <class TA, int J, class T, class F>
+__device__ __forceinline__ void rg_group_sum(const T (&acc)[rg<J>::SLOTS][2], int l, T *buf,
+                                             const F &out) {
+  using R = rg<J>;
+  using S = rg_sum<J>;
+#pragma unroll
+  for (int s0 = 0; s0 < R::SLOTS; s0 += S::CH) {
+    const int ns = R::SLOTS - s0 < S::CH ? R::SLOTS - s0 : S::CH;
+    wave_sync();  // the previous slots have been read
+#pragma unroll
+    for (int s = 0; s < ns; s++) {
+      buf[s * S::PITCH + l] = acc[s0 + s][0];
+      buf[(S::CH + s) * S::PITCH + l] = acc[s0 + s][1];
+    }
+    wave_sync();
+    if (l < ns * R::W) {
+      const T *b = buf + (l / R::W) * S::PITCH + l % R::W;
+      TA vr = 0, vi = 0;
+#pragma unroll
+      for (int g = 0; g < R::NB; g++) {
+        vr += (TA)b[g * R::W];
+        vi += (TA)b[S::CH * S::PITCH + g * R::W];
+      }
+      out(s0 * R::W + l, vr, vi);
+    }
+  }
+}
+
+// U_tot of atom i from the lanes' sums: wself * I + norm * sum, own entries
+// and mirrors
+template <class T, int J>
+__device__ __forceinline__ void rg_store_u(const snap_dev_tables &t,
+                                           const rg_map *__restrict__ rgm,
+                                           const T (&acc)[rg<J>::SLOTS][2], int l, T *buf,
+                                           T *__restrict__ ur, T *__restrict__ ui) {
+  rg_group_sum<T, J>(acc, l, buf, [&](int k, T vr, T vi) {
+    const rg_map m = rgm[k];
+    if (m.ey < 0) return;
+    vr *= (T)m.norm;
+    vi *= (T)m.norm;
+    if (m.diag) vr += (T)t.wself;
+    ur[m.uo] = vr;
+    ui[m.uo] = vi;
+    if (m.um >= 0) {
+      ur[m.um] = m.neg ? -vr : vr;
+      ui[m.um] = m.neg ? vi : -vi;
+    }
+  });
+}
+
+// U_tot from the neighbour parameters of the last compaction, one wavefront
+// per atom; every sum in a fixed order: deterministic.
+template <class T, int J>
+__global__ void __launch_bounds__(64)
+k_snap_ui_rg(snap_dev_tables t, const rg_map *__restrict__ rgm, const int *__restrict__ nin,
+             const snap_par<T> *__restrict__ par, int maxn, int n, T *__restrict__ utot_r,
+             T *__restrict__ utot_i) {
+  __shared__ T s_buf[rg_sum<J>::BUF];
+  const int i = blockIdx.x;
+  if (i >= n) return;
+  const int l = threadIdx.x;
+  const int g = l / rg<J>::W, ma = l - g * rg<J>::W;  // g = NB only for idle lanes
+  T acc[rg<J>::SLOTS][2];
+#pragma unroll
+  for (int s = 0; s < rg<J>::SLOTS; s++) acc[s][0] = acc[s][1] = 0;
+  rg_u_sums<T, J>(t, par, i, maxn, nin[i], g, ma, acc);
+  rg_store_u<T, J>(t, rgm, acc, l, s_buf, utot_r + (size_t)i * t.nu, utot_i + (size_t)i * t.nu);
+}
+
+// The compaction (with the neighbour parameters in T's precision) followed by
+// U_tot in the same wavefront, one wavefront per atom as k_snap_ui_rg: one
+// launch less per force evaluation, and the parameters just written are read
+// back from the cache.
+template <class T, int J>
+__global__ void __launch_bounds__(64)
+k_snap_neigh_ui(snap_dev_tables t, const rg_map *__restrict__ rgm,
+                const double *__restrict__ x, const int *__restrict__ row,
+                const int *__restrict__ num, const int *__restrict__ entries, int pitch, int n,
+                double cutsq, int maxn, int *__restrict__ nin, int *__restrict__ nj,
+                double *__restrict__ nr, double *__restrict__ f64, float *__restrict__ f32,
+                int ntot, snap_par<T> *__restrict__ par, double *__restrict__ fdv,
+                T *__restrict__ utot_r, T *__restrict__ utot_i) {
+  __shared__ T s_buf[rg_sum<J>::BUF];
+  const int i = blockIdx.x;
+  if (i >= n) return;
+  const int cnt = snap_compact<T>(t, i, x, row, num, entries, pitch, n, cutsq, maxn, nin, nj, nr,
+                                  f64, f32, ntot, par, fdv);
+  __syncthreads();  // the wavefront's parameter writes are visible
+  const int l = threadIdx.x;
+  const int g = l / rg<J>::W, ma = l - g * rg<J>::W;
+  T acc[rg<J>::SLOTS][2];
+#pragma unroll
+  for (int q = 0; q < rg<J>::SLOTS; q++) acc[q][0] = acc[q][1] = 0;
+  rg_u_sums<T, J>(t, par, i, maxn, cnt, g, ma, acc);
+  rg_store_u<T, J>(t, rgm, acc, l, s_buf, utot_r + (size_t)i * t.nu, utot_i + (size_t)i * t.nu);
+}
+
+// Blocks of RG_WAVES wavefronts take NB * RG_WAVES neighbours of one atom in
+// the force kernel (grid.y over the neighbour slots).
+constexpr int RG_WAVES = 4;
+
+// F_ij in reverse mode.  With G_j(e) = w(e) norm_j(e) Y_j(e) (w the
+// half-plane weight) the force on the pair is the gradient with respect to
+// r_ij of sfac * L,
+//   L = sum_j sum_e Re(conj(V_j(e)) G_j(e)).
+// V is linear in V_{j-1} and r enters only through a, b and sfac.  So, with
+// the adjoints A_j(e) = dL/dRe V + i dL/dIm V propagated from the top layer
+// down and A'_j(ma) = A_j(ma+1) from the lane above,
+//   A_{j-1}(ma,mb) = G_{j-1} + a A_j - b A'_j               (2 mb < j)
+//                  + conj(b) A_j(m) + conj(a) A'_j(m)       (mb = j/2-1, m = j/2)
+//   dL/dr_k = Re(conj(da_k) Sa) - Re(conj(db_k) Sb),
+//   Sa = sum conj(A_j) V_{j-1} + sum_m A'_j conj(V_{j-1}(j/2-1)),
+//   Sb = sum conj(A'_j) V_{j-1} - sum_m A_j conj(V_{j-1}(j/2-1)),
+// and L itself is A_0 (V_0 = 1), so the forward pass does not read Y.  It
+// keeps V of layers 0..J-1 in registers; what the lane shifts carry past a
+// group's edge stays in entries with ma > j, where V is 0.  24 multiply-adds,
+// 4 lane shifts of a value and one LDS read of Y per entry (about 44, 6 and
+// three records with the factors in U).  The
+// force on i is added up over the wavefront before its atomics, and a
+// component takes a lane: 2 atomic instructions per seven neighbours (6 each).
+template <class T, class TF, int J>
+__global__ void __launch_bounds__(64 * RG_WAVES, J <= SNAP_MAXJ ? 3 : 1)
+k_snap_fij_rev(snap_dev_tables t, const rg_map *__restrict__ rgm, const int *__restrict__ nin,
+               const int *__restrict__ nj, const double *__restrict__ nr,
+               const snap_par<T> *__restrict__ par, const double *__restrict__ fdv, int maxn, int n,
+               const T *__restrict__ y_r, const T *__restrict__ y_i, TF *__restrict__ f) {
+  using R = rg<J>;
+  constexpr int NT = 64 * RG_WAVES, RP = 64 + 3;  // RP: the components' rows in different banks
+  __shared__ rg_rec<T> s_rec[R::SLOTS * R::W];
+  __shared__ T s_red[RG_WAVES][3][RP];
+  __shared__ TF s_f[RG_WAVES][3][R::NB];
   const int i = blockIdx.x;
   if (i >= n) return;
   const int cnt_i = nin[i];
-  const int row0 = blockIdx.y * (RG_WAVES * RG_NB);
+  const int row0 = blockIdx.y * (RG_WAVES * R::NB);
   if (row0 >= cnt_i) return;  // no neighbour for this block
-  rg_fill<T, 64 * RG_WAVES>(rgp, rgm, t.ny, y_r, y_i, i, s_rec);
+#pragma unroll
+  for (int q = 0; q < (R::SLOTS * R::W + NT - 1) / NT; q++) {
+    const int k = q * NT + (int)threadIdx.x;
+    if (k < R::SLOTS * R::W) {
+      const rg_map m = rgm[k];
+      rg_rec<T> r{0, 0};
+      if (m.ey >= 0) {
+        const T wgt = (T)(0.5 * m.wq * m.norm);
+        r.yr = wgt * y_r[(size_t)i * t.ny + m.ey];
+        r.yi = wgt * y_i[(size_t)i * t.ny + m.ey];
+      }
+      s_rec[k] = r;
+    }
+  }
   __syncthreads();
   const int w = threadIdx.x / 64, l = threadIdx.x % 64;
-  const int g = l / RG_W, ma = l - g * RG_W;  // g = 7 only for the idle lane 63
-  const int jj0 = row0 + w * RG_NB;
+  const int g = l / R::W, ma = l - g * R::W;  // g = NB only for idle lanes
+  const int jj0 = row0 + w * R::NB;
   if (jj0 >= cnt_i) return;  // uniform over the wavefront; no block barrier follows
   const int jj = jj0 + g;
-  const bool act = g < RG_NB && jj < cnt_i;
+  const bool act = g < R::NB && jj < cnt_i;
   const size_t o = (size_t)i * maxn + (act ? jj : jj0);
   const T a_r = par[o].a_r, a_i = par[o].a_i, b_r = par[o].b_r, b_i = par[o].b_i;
-  const T sfac = par[o].sfac;
   const int tj = t.twojmax;
 
-  // forward: U of layers 0..TJ-1 (column slot rg_slot0(j) + mb), and
-  // sum Re(conj(U) w Y) over the lane's entries of every layer
-  T us[RG_SLOTS][2];
+  // forward: V of layers 0..J-1 (column slot rg_slot0(j) + mb)
+  T vs[rg_slot0(J)][2];
 #pragma unroll
-  for (int s = 0; s < RG_SLOTS; s++) us[s][0] = us[s][1] = 0;
-  us[0][0] = ma == 0 ? (T)1 : (T)0;
-  T auy = us[0][0] * s_rec[ma].yr;
+  for (int s = 0; s < rg_slot0(J); s++) vs[s][0] = vs[s][1] = 0;
+  {
+    T c[R::COLS][2];
 #pragma unroll
-  for (int j = 1; j <= TJ; j++) {
-    if (j > tj) break;
-    T mir[2], mirb[2];
-    if ((j & 1) == 0) {
-      const int src = g * RG_W + (j - 1 - ma > 0 ? j - 1 - ma : 0);
-      const T sg = ((ma + j / 2) & 1) ? (T)-1 : (T)1;
-      const int sp = rg_slot0(j - 1) + j / 2 - 1;
-      mir[0] = sg * __shfl(us[sp][0], src, 64);
-      mir[1] = -sg * __shfl(us[sp][1], src, 64);
-      mirb[0] = lane_below(mir[0]);
-      mirb[1] = lane_below(mir[1]);
-    }
+    for (int mb = 0; mb < R::COLS; mb++) c[mb][0] = c[mb][1] = 0;
+    c[0][0] = ma == 0 ? (T)1 : (T)0;
+    vs[0][0] = c[0][0];
+    rg_layers<1, J - 1>([&](auto jc) {
+      constexpr int j = jc;
+      if (j >= tj) return;
+      rg_layer<j>(a_r, a_i, b_r, b_i, c);
 #pragma unroll
-    for (int mb = 0; mb <= j / 2; mb++) {
-      const int slot = rg_slot0(j) + mb;
-      const rg_rec<T> q = s_rec[slot * RG_W + ma];
-      const bool mid = (j & 1) == 0 && mb == j / 2;
-      const int sp = rg_slot0(j - 1) + mb;  // (unused on the middle column)
-      const T p0 = mid ? mir[0] : us[sp][0], p1 = mid ? mir[1] : us[sp][1];
-      const T q0 = mid ? mirb[0] : lane_below(us[sp][0]);
-      const T q1 = mid ? mirb[1] : lane_below(us[sp][1]);
-      const T ur = q.rpa * (a_r * p0 + a_i * p1) - q.rpb * (b_r * q0 + b_i * q1);
-      const T ui = q.rpa * (a_r * p1 - a_i * p0) - q.rpb * (b_r * q1 - b_i * q0);
-      auy += ur * q.yr + ui * q.yi;
-      if (j < TJ) {
-        us[slot][0] = ur;
-        us[slot][1] = ui;
+      for (int mb = 0; mb <= j / 2; mb++) {
+        vs[rg_slot0(j) + mb][0] = c[mb][0];
+        vs[rg_slot0(j) + mb][1] = c[mb][1];
       }
-    }
+    });
   }
 
   // backward: adjoints of layer j (columns 0..j/2), from the top layer down
-  T ub[RG_COLS][2];
+  T ad[R::COLS][2];
 #pragma unroll
-  for (int mb = 0; mb < RG_COLS; mb++) ub[mb][0] = ub[mb][1] = 0;
+  for (int mb = 0; mb < R::COLS; mb++) ad[mb][0] = ad[mb][1] = 0;
   T sa_r = 0, sa_i = 0, sb_r = 0, sb_i = 0;
-#pragma unroll
-  for (int j = TJ; j >= 1; j--) {
-    if (j > tj) continue;
+  if (tj == 0) ad[0][0] = s_rec[ma].yr;  // no layer below the top one
+  rg_layers<J, 1>([&](auto jc) {
+    constexpr int j = jc;
+    if (j > tj) return;
     if (j == tj) {  // the top layer's adjoint is its own term
 #pragma unroll
       for (int mb = 0; mb <= j / 2; mb++) {
-        const rg_rec<T> q = s_rec[(rg_slot0(j) + mb) * RG_W + ma];
-        ub[mb][0] = sfac * q.yr;
-        ub[mb][1] = sfac * q.yi;
+        const rg_rec<T> q = s_rec[(rg_slot0(j) + mb) * R::W + ma];
+        ad[mb][0] = q.yr;
+        ad[mb][1] = q.yi;
       }
     }
-    T mir[2], mirb[2];
-    if ((j & 1) == 0) {
-      const int src = g * RG_W + (j - 1 - ma > 0 ? j - 1 - ma : 0);
-      const T sg = ((ma + j / 2) & 1) ? (T)-1 : (T)1;
-      const int sp = rg_slot0(j - 1) + j / 2 - 1;
-      mir[0] = sg * __shfl(us[sp][0], src, 64);
-      mir[1] = -sg * __shfl(us[sp][1], src, 64);
-      mirb[0] = lane_below(mir[0]);
-      mirb[1] = lane_below(mir[1]);
-    }
-    T ubp[RG_COLS][2];  // adjoints of layer j-1
-#pragma unroll
-    for (int mb = 0; mb < RG_COLS; mb++) ubp[mb][0] = ubp[mb][1] = 0;
+    T up[R::COLS][2];
 #pragma unroll
     for (int mb = 0; mb <= j / 2; mb++) {
-      const rg_rec<T> q = s_rec[(rg_slot0(j) + mb) * RG_W + ma];
-      const bool mid = (j & 1) == 0 && mb == j / 2;
-      const int sp = rg_slot0(j - 1) + mb;
-      const T p0 = mid ? mir[0] : us[sp][0], p1 = mid ? mir[1] : us[sp][1];
-      const T q0 = mid ? mirb[0] : lane_below(us[sp][0]);
-      const T q1 = mid ? mirb[1] : lane_below(us[sp][1]);
-      const T u0 = ub[mb][0], u1 = ub[mb][1];
-      // Sa += rpa conj(Ubar) P, Sb += rpb conj(Ubar) Q
-      sa_r += q.rpa * (u0 * p0 + u1 * p1);
-      sa_i += q.rpa * (u0 * p1 - u1 * p0);
-      sb_r += q.rpb * (u0 * q0 + u1 * q1);
-      sb_i += q.rpb * (u0 * q1 - u1 * q0);
-      // conj(alpha) Ubar = rpa a Ubar, conj(beta) Ubar = -rpb b Ubar
-      const T za0 = q.rpa * (a_r * u0 - a_i * u1), za1 = q.rpa * (a_r * u1 + a_i * u0);
-      const T zb0 = -q.rpb * (b_r * u0 - b_i * u1), zb1 = -q.rpb * (b_r * u1 + b_i * u0);
-      if (!mid) {
-        ubp[mb][0] += za0 + lane_above(zb0);
-        ubp[mb][1] += za1 + lane_above(zb1);
-      } else {
-        // P = s conj(U'(j-1-ma, j/2-1)), Q = -s conj(U'(j-ma, j/2-1)):
-        // lane m' of column j/2-1 collects s conj(za) of lane j-1-m' and
-        // -s conj(zb) of lane j-m'
-        const T sg = ((ma + j / 2) & 1) ? (T)-1 : (T)1;
-        const T v0 = sg * za0 + lane_above(-sg * zb0);
-        const T v1 = -sg * za1 + lane_above(sg * zb1);
-        const int src = g * RG_W + (j - 1 - ma > 0 ? j - 1 - ma : 0);
-        const T g0 = __shfl(v0, src, 64), g1 = __shfl(v1, src, 64);
-        const bool own = ma <= j - 1;
-        ubp[j / 2 - 1][0] += own ? g0 : (T)0;
-        ubp[j / 2 - 1][1] += own ? g1 : (T)0;
-      }
+      up[mb][0] = lane_above(ad[mb][0]);
+      up[mb][1] = lane_above(ad[mb][1]);
     }
-    // layer j-1's own term
+    constexpr int m = j / 2;
 #pragma unroll
-    for (int mb = 0; mb <= (j - 1) / 2; mb++) {
-      const rg_rec<T> q = s_rec[(rg_slot0(j - 1) + mb) * RG_W + ma];
-      ub[mb][0] = ubp[mb][0] + sfac * q.yr;
-      ub[mb][1] = ubp[mb][1] + sfac * q.yi;
+    for (int mb = 0; 2 * mb < j; mb++) {
+      const rg_rec<T> q = s_rec[(rg_slot0(j - 1) + mb) * R::W + ma];
+      const T p0 = vs[rg_slot0(j - 1) + mb][0], p1 = vs[rg_slot0(j - 1) + mb][1];
+      const T u0 = ad[mb][0], u1 = ad[mb][1], w0 = up[mb][0], w1 = up[mb][1];
+      sa_r += u0 * p0 + u1 * p1;
+      sa_i += u0 * p1 - u1 * p0;
+      sb_r += w0 * p0 + w1 * p1;
+      sb_i += w0 * p1 - w1 * p0;
+      T z0 = q.yr + a_r * u0 - a_i * u1 - b_r * w0 + b_i * w1;
+      T z1 = q.yi + a_r * u1 + a_i * u0 - b_r * w1 - b_i * w0;
+      if (2 * mb + 2 == j) {  // this column also feeds the middle one
+        const T c0 = ad[m][0], c1 = ad[m][1], d0 = up[m][0], d1 = up[m][1];
+        sa_r += d0 * p0 + d1 * p1;
+        sa_i += d1 * p0 - d0 * p1;
+        sb_r -= c0 * p0 + c1 * p1;
+        sb_i -= c1 * p0 - c0 * p1;
+        z0 += b_r * c0 + b_i * c1 + a_r * d0 + a_i * d1;
+        z1 += b_r * c1 - b_i * c0 + a_r * d1 - a_i * d0;
+      }
+      ad[mb][0] = z0;
+      ad[mb][1] = z1;
     }
-  }
-  // the lane's share of F_ij, summed over the nine lanes of the group in order
+  });
+  const T auy = ma == 0 ? ad[0][0] : (T)0;
+  // the lane's share of F_ij
   const T u3[3] = {par[o].u[0], par[o].u[1], par[o].u[2]};
   const T c1 = par[o].c1, c2 = par[o].c2, c3 = par[o].c3, c4 = par[o].c4, r0i = par[o].r0inv;
-  const T dsfac = par[o].dsfac;
+  const T sfac = par[o].sfac, dsfac = par[o].dsfac;
 #pragma unroll
   for (int k = 0; k < 3; k++) {
     const T da_r = c1 * u3[k], da_i = c2 * u3[k] - (k == 2 ? r0i : (T)0);
     const T db_r = c3 * u3[k] + (k == 1 ? r0i : (T)0), db_i = c4 * u3[k] - (k == 0 ? r0i : (T)0);
-    s_red[w][k][l] = dsfac * auy * u3[k] + (da_r * sa_r + da_i * sa_i) - (db_r * sb_r + db_i * sb_i);
+    s_red[w][k][l] = dsfac * auy * u3[k] +
+                     sfac * ((da_r * sa_r + da_i * sa_i) - (db_r * sb_r + db_i * sb_i));
   }
   wave_sync();
-  if (ma == 0 && act) {
-    T fx = 0, fy = 0, fz = 0;
+  if (ma < 3 && g < R::NB) {  // lane ma adds up component ma over its group
+    T s = 0;
 #pragma unroll
-    for (int m = 0; m < RG_W; m++) {
-      fx += s_red[w][0][l + m];
-      fy += s_red[w][1][l + m];
-      fz += s_red[w][2][l + m];
-    }
+    for (int m = 0; m < R::W; m++) s += s_red[w][ma][g * R::W + m];
     // ad-hoc repulsion of the reference, force_snap_neigh_impl.h:705-711
-    const double fdivr = fdv[o];
-    const TF Fx = (TF)fx + (TF)(nr[3 * o] * fdivr);
-    const TF Fy = (TF)fy + (TF)(nr[3 * o + 1] * fdivr);
-    const TF Fz = (TF)fz + (TF)(nr[3 * o + 2] * fdivr);
-    const int jn = nj[o];
-    atomicAdd(&f[3 * (size_t)i], Fx);
-    atomicAdd(&f[3 * (size_t)i + 1], Fy);
-    atomicAdd(&f[3 * (size_t)i + 2], Fz);
-    atomicAdd(&f[3 * (size_t)jn], -Fx);
-    atomicAdd(&f[3 * (size_t)jn + 1], -Fy);
-    atomicAdd(&f[3 * (size_t)jn + 2], -Fz);
+    const TF F = act ? (TF)s + (TF)(nr[3 * o + ma] * fdv[o]) : (TF)0;
+    if (act) atomicAdd(&f[3 * (size_t)nj[o] + ma], -F);
+    s_f[w][ma][g] = F;
+  }
+  wave_sync();
+  if (l < 3) {
+    TF s = 0;
+#pragma unroll
+    for (int q = 0; q < R::NB; q++) s += s_f[w][l][q];
+    atomicAdd(&f[3 * (size_t)i + l], s);
   }
 }
 
@@ -1446,11 +1016,7 @@ struct emd_snap {
   // repulsion F/r, with the precision the parameters were last written in
   void *par = nullptr;
   double *fdv = nullptr;
-  // register-layout tables (twojmax <= 8): recursion factors in both
-  // precisions and the index map, per (column slot, lane)
-  rg_rp<float> *rg_rp32 = nullptr;
-  rg_rp<double> *rg_rp64 = nullptr;
-  rg_map *rg_map_d = nullptr;
+  rg_map *rg_map_d = nullptr;  // the register layout's index map, per (column slot, lane)
   size_t cap_par = 0, cap_fdv = 0;
   int par_prec = -1;
   void *u_r = nullptr, *u_i = nullptr, *y_r = nullptr, *y_i = nullptr;
@@ -1763,23 +1329,23 @@ static emd_status snap_build_yflat(emd_ctx *ctx, emd_snap *sn) {
   return EMD_OK;
 }
 
-// the register-layout tables for twojmax <= 8 (see rg_map)
+// the index map of the register layout (see rg_map)
+template <int J>
 static emd_status snap_build_rg(emd_ctx *ctx, emd_snap *sn) {
+  using R = rg<J>;
   const snap_dev_tables &t = sn->t;
-  std::vector<rg_rp<float>> r32(RG_SLOTS * RG_W);
-  std::vector<rg_rp<double>> r64(RG_SLOTS * RG_W);
-  std::vector<rg_map> mp(RG_SLOTS * RG_W);
-  for (int sl = 0; sl < RG_SLOTS; sl++)
-    for (int ma = 0; ma < RG_W; ma++) {
-      const int k = sl * RG_W + ma;
+  double fact[J + 1];
+  fact[0] = 1.0;
+  for (int k = 1; k <= J; k++) fact[k] = fact[k - 1] * k;
+  std::vector<rg_map> mp(R::SLOTS * R::W);
+  for (int sl = 0; sl < R::SLOTS; sl++)
+    for (int ma = 0; ma < R::W; ma++) {
       int j = 0;
-      while (j < SNAP_MAXJ && rg_slot0(j + 1) <= sl) j++;
+      while (j < J && rg_slot0(j + 1) <= sl) j++;
       const int mb = sl - rg_slot0(j);
-      double rpa = 0, rpb = 0;
-      rg_map m{-1, -1, -1, 0, 0, 0, 0};
+      rg_map m{0.0, -1, -1, -1, 0, 0, 0, 0};
       if (j <= t.twojmax && ma <= j) {
-        if (ma < j) rpa = t.rootpq[(j - ma) * SNAP_RPD + (j - mb)];
-        if (ma > 0) rpb = t.rootpq[ma * SNAP_RPD + (j - mb)];
+        m.norm = std::sqrt(fact[ma] * fact[j - ma] / (fact[mb] * fact[j - mb]));
         // the reference's half plane: middle column ma < mb, diagonal 1/2
         m.wq = 2 * mb == j ? (ma < mb ? 2 : (ma == mb ? 1 : 0)) : 2;
         m.ey = t.ystart[j] + mb * (j + 1) + ma;
@@ -1788,25 +1354,12 @@ static emd_status snap_build_rg(emd_ctx *ctx, emd_snap *sn) {
         m.neg = (ma + mb) & 1;
         m.diag = ma == mb;
       }
-      r32[k] = rg_rp<float>{(float)rpa, (float)rpb};
-      r64[k] = rg_rp<double>{rpa, rpb};
-      mp[k] = m;
+      mp[sl * R::W + ma] = m;
     }
-  EMD_HIP(ctx, hipMalloc(&sn->rg_rp32, r32.size() * sizeof(r32[0])));
-  EMD_HIP(ctx, hipMalloc(&sn->rg_rp64, r64.size() * sizeof(r64[0])));
   EMD_HIP(ctx, hipMalloc(&sn->rg_map_d, mp.size() * sizeof(mp[0])));
-  EMD_HIP(ctx, hipMemcpy(sn->rg_rp32, r32.data(), r32.size() * sizeof(r32[0]), hipMemcpyHostToDevice));
-  EMD_HIP(ctx, hipMemcpy(sn->rg_rp64, r64.data(), r64.size() * sizeof(r64[0]), hipMemcpyHostToDevice));
   EMD_HIP(ctx, hipMemcpy(sn->rg_map_d, mp.data(), mp.size() * sizeof(mp[0]), hipMemcpyHostToDevice));
   return EMD_OK;
 }
-
-template <class T>
-static const rg_rp<T> *rg_rp_of(const emd_snap *sn);
-template <>
-const rg_rp<float> *rg_rp_of<float>(const emd_snap *sn) { return sn->rg_rp32; }
-template <>
-const rg_rp<double> *rg_rp_of<double>(const emd_snap *sn) { return sn->rg_rp64; }
 
 static emd_status snap_upload_coeff(emd_ctx *ctx, emd_snap *sn) {
   const int twojmax = sn->t.twojmax;
@@ -1907,8 +1460,6 @@ extern "C" emd_status emd_snap_create(emd_ctx *ctx, const emd_snap_params *p, em
   t.ystart[twojmax + 1] = ny;
   t.nu = nu;
   t.ny = ny;
-  for (int a = 1; a <= twojmax; a++)
-    for (int b = 1; b <= twojmax; b++) t.rootpq[a * SNAP_RPD + b] = std::sqrt((double)a / b);
   t.rfac0 = p->rfac0;
   t.rmin0 = p->rmin0;
   t.rcut = (p->radelem + p->radelem) * p->rcutfac;
@@ -1980,7 +1531,8 @@ extern "C" emd_status emd_snap_create(emd_ctx *ctx, const emd_snap_params *p, em
                            hipMemcpyHostToDevice));
   }
   emd_status st = snap_build_yflat(ctx, sn);
-  if (st == EMD_OK && twojmax <= SNAP_MAXJ) st = snap_build_rg(ctx, sn);
+  if (st == EMD_OK)
+    st = twojmax <= SNAP_MAXJ ? snap_build_rg<SNAP_MAXJ>(ctx, sn) : snap_build_rg<SNAP_JBIG>(ctx, sn);
   if (st == EMD_OK) st = snap_upload_coeff(ctx, sn);
   if (st != EMD_OK) {
     emd_snap_destroy(ctx, sn);
@@ -1994,7 +1546,7 @@ extern "C" emd_status emd_snap_destroy(emd_ctx *ctx, emd_snap *sn) {
   if (!sn) return EMD_OK;
   if (ctx) hipStreamSynchronize(ctx->stream);
   void *ptrs[] = {sn->cg, sn->ytab, sn->etab, sn->nin, sn->nj, sn->nr, sn->par, sn->fdv,
-                  sn->rg_rp32, sn->rg_rp64, sn->rg_map_d,
+                  sn->rg_map_d,
                   sn->stab, sn->w_r, sn->edot,
                   sn->w_i, sn->sbuf,
                   sn->u_r, sn->u_i, sn->y_r, sn->y_i, sn->eatom,
@@ -2044,28 +1596,6 @@ static emd_status snap_scratch(emd_ctx *ctx, emd_snap *sn, int n, int maxn) {
   return EMD_OK;
 }
 
-// zero_prec: EMD_FP64 or EMD_MIXED to zero that precision's force array
-// (all n_local + n_ghost rows) in the same launch, or -1.  par_prec:
-// EMD_FP64 or EMD_MIXED to write the neighbour parameters in that precision
-// (for the U and force kernels that follow), or -1
-static emd_status snap_neigh(emd_ctx *ctx, const emd_system *s, const emd_neigh *nl, emd_snap *sn,
-                             int zero_prec, int par_prec) {
-  const int n = s->n_local;
-  const int maxn = nl->maxneighs > 0 ? nl->maxneighs : 1;
-  EMD_TRY(snap_scratch(ctx, sn, n, maxn));
-  const double rcutmax = 2.0 * sn->radelem * sn->rcutfac;
-  const int *row = nl->layout == EMD_NEIGH_CSR ? nl->row : nullptr;
-  double *f64 = zero_prec == EMD_FP64 ? s->f : nullptr;
-  float *f32 = zero_prec == EMD_MIXED ? s->f32 : nullptr;
-  snap_par<float> *p32 = par_prec == EMD_MIXED ? (snap_par<float> *)sn->par : nullptr;
-  snap_par<double> *p64 = par_prec == EMD_FP64 ? (snap_par<double> *)sn->par : nullptr;
-  EMD_LAUNCH(ctx, "snap_neigh", k_snap_neigh, n, 64, 0, sn->t, s->x, row, nl->num, nl->entries,
-             nl->maxneighs, n, rcutmax * rcutmax, sn->cap_maxn, sn->nin, sn->nj, sn->nr, f64,
-             f32, s->n_local + s->n_ghost, p32, p64, (p32 || p64) ? sn->fdv : nullptr);
-  sn->par_prec = (p32 || p64) ? par_prec : -1;
-  return EMD_OK;
-}
-
 // the neighbour parameters in T's precision (written by the compaction, or
 // here when it wrote the other precision)
 template <class T>
@@ -2078,45 +1608,49 @@ static emd_status snap_par_ready(emd_ctx *ctx, emd_snap *sn, int n) {
   return EMD_OK;
 }
 
-// twojmax <= 8: the compaction with the neighbour parameters in precision
-// prec and U_tot of every atom, in one launch (k_snap_neigh_ui)
-static emd_status snap_neigh_ui(emd_ctx *ctx, const emd_system *s, const emd_neigh *nl,
-                                emd_snap *sn, int zero_prec, int prec) {
+// The compaction with the neighbour parameters in precision prec and U_tot of
+// every atom, in one launch.  zero_prec: EMD_FP64 or EMD_MIXED to zero that
+// precision's force array (all n_local + n_ghost rows) in the same launch, or -1.
+template <class T>
+static emd_status snap_neigh_ui_as(emd_ctx *ctx, const emd_system *s, const emd_neigh *nl,
+                                   emd_snap *sn, int zero_prec) {
   const int n = s->n_local;
-  const int maxn = nl->maxneighs > 0 ? nl->maxneighs : 1;
-  EMD_TRY(snap_scratch(ctx, sn, n, maxn));
   const double rcutmax = 2.0 * sn->radelem * sn->rcutfac;
   const int *row = nl->layout == EMD_NEIGH_CSR ? nl->row : nullptr;
   double *f64 = zero_prec == EMD_FP64 ? s->f : nullptr;
   float *f32 = zero_prec == EMD_MIXED ? s->f32 : nullptr;
-  if (prec == EMD_MIXED)
-    EMD_LAUNCH(ctx, "snap_ui", k_snap_neigh_ui<float>, n, 64, 0, sn->t, sn->rg_rp32, sn->rg_map_d,
+  if (sn->t.twojmax <= SNAP_MAXJ)
+    EMD_LAUNCH(ctx, "snap_ui", (k_snap_neigh_ui<T, SNAP_MAXJ>), n, 64, 0, sn->t, sn->rg_map_d,
                s->x, row, nl->num, nl->entries, nl->maxneighs, n, rcutmax * rcutmax, sn->cap_maxn,
-               sn->nin, sn->nj, sn->nr, f64, f32, s->n_local + s->n_ghost,
-               (snap_par<float> *)sn->par, sn->fdv, (float *)sn->u_r, (float *)sn->u_i);
+               sn->nin, sn->nj, sn->nr, f64, f32, s->n_local + s->n_ghost, (snap_par<T> *)sn->par,
+               sn->fdv, (T *)sn->u_r, (T *)sn->u_i);
   else
-    EMD_LAUNCH(ctx, "snap_ui", k_snap_neigh_ui<double>, n, 64, 0, sn->t, sn->rg_rp64, sn->rg_map_d,
+    EMD_LAUNCH(ctx, "snap_ui", (k_snap_neigh_ui<T, SNAP_JBIG>), n, 64, 0, sn->t, sn->rg_map_d,
                s->x, row, nl->num, nl->entries, nl->maxneighs, n, rcutmax * rcutmax, sn->cap_maxn,
-               sn->nin, sn->nj, sn->nr, f64, f32, s->n_local + s->n_ghost,
-               (snap_par<double> *)sn->par, sn->fdv, (double *)sn->u_r, (double *)sn->u_i);
+               sn->nin, sn->nj, sn->nr, f64, f32, s->n_local + s->n_ghost, (snap_par<T> *)sn->par,
+               sn->fdv, (T *)sn->u_r, (T *)sn->u_i);
+  return EMD_OK;
+}
+
+static emd_status snap_neigh_ui(emd_ctx *ctx, const emd_system *s, const emd_neigh *nl,
+                                emd_snap *sn, int zero_prec, int prec) {
+  EMD_TRY(snap_scratch(ctx, sn, s->n_local, nl->maxneighs > 0 ? nl->maxneighs : 1));
+  if (prec == EMD_MIXED) EMD_TRY(snap_neigh_ui_as<float>(ctx, s, nl, sn, zero_prec));
+  else EMD_TRY(snap_neigh_ui_as<double>(ctx, s, nl, sn, zero_prec));
   sn->par_prec = prec;
   return EMD_OK;
 }
 
-// U_tot of every atom: the register-resident kernel for twojmax <= 8 (one
-// wavefront per atom: SNAP-2k 18.6 us mixed / 23.5 us FP64, against 18.8 /
-// 32.8 with two and 26.8 / 47.9 with four wavefronts per atom), else one
-// neighbour per wavefront
-template <class T>
-static emd_status launch_ui(emd_ctx *ctx, emd_snap *sn, int n, T *ur, T *ui) {
-  if (sn->t.twojmax <= SNAP_MAXJ) {
-    EMD_TRY(snap_par_ready<T>(ctx, sn, n));
-    EMD_LAUNCH(ctx, "snap_ui", (k_snap_ui_rg<T, 1>), n, 64, 0, sn->t, rg_rp_of<T>(sn), sn->rg_map_d,
-               sn->nin, (const snap_par<T> *)sn->par, sn->cap_maxn, n, ur, ui);
-  } else {
-    EMD_LAUNCH(ctx, "snap_ui", (k_snap_ui<T, SNAP_JBIG>), n, 64 * UI_WAVES, 0, sn->t, sn->nin,
-               sn->nr, sn->cap_maxn, n, ur, ui);
-  }
+// U_tot of every atom in FP64 from the last compaction
+static emd_status launch_ui(emd_ctx *ctx, emd_snap *sn, int n) {
+  EMD_TRY(snap_par_ready<double>(ctx, sn, n));
+  const snap_par<double> *par = (const snap_par<double> *)sn->par;
+  if (sn->t.twojmax <= SNAP_MAXJ)
+    EMD_LAUNCH(ctx, "snap_ui", (k_snap_ui_rg<double, SNAP_MAXJ>), n, 64, 0, sn->t, sn->rg_map_d,
+               sn->nin, par, sn->cap_maxn, n, (double *)sn->u_r, (double *)sn->u_i);
+  else
+    EMD_LAUNCH(ctx, "snap_ui", (k_snap_ui_rg<double, SNAP_JBIG>), n, 64, 0, sn->t, sn->rg_map_d,
+               sn->nin, par, sn->cap_maxn, n, (double *)sn->u_r, (double *)sn->u_i);
   return EMD_OK;
 }
 
@@ -2138,30 +1672,20 @@ static emd_status snap_y(emd_ctx *ctx, emd_snap *sn, int n) {
   return EMD_OK;
 }
 
-template <class T>
-static emd_status snap_ui_y(emd_ctx *ctx, emd_snap *sn, int n) {
-  EMD_TRY(launch_ui<T>(ctx, sn, n, (T *)sn->u_r, (T *)sn->u_i));
-  return snap_y<T>(ctx, sn, n);
-}
-
-// F_ij for every (atom, neighbour): the register-resident reverse-mode
-// kernel (seven neighbours per wavefront) for twojmax <= 8 (SNAP-2k: 29.6 /
-// 36.8 us mixed / FP64, against 40.6 / 50.6 us carrying dU/dr forward in the
-// same layout), one neighbour per wavefront above
+// F_ij for every (atom, neighbour)
 template <class T, class TF>
 static emd_status launch_fij(emd_ctx *ctx, emd_snap *sn, int n, const T *yr, const T *yi,
                              TF *f) {
-  if (sn->t.twojmax <= SNAP_MAXJ) {
-    EMD_TRY(snap_par_ready<T>(ctx, sn, n));
-    const dim3 grid(n, (sn->cap_maxn + RG_WAVES * RG_NB - 1) / (RG_WAVES * RG_NB));
-    EMD_LAUNCH(ctx, "snap_fij", (k_snap_fij_rev<T, TF>), grid, 64 * RG_WAVES, 0, sn->t,
-               rg_rp_of<T>(sn), sn->rg_map_d, sn->nin, sn->nj, sn->nr,
-               (const snap_par<T> *)sn->par, sn->fdv, sn->cap_maxn, n, yr, yi, f);
-  } else {
-    const dim3 grid(n, (sn->cap_maxn + FIJ_WAVES - 1) / FIJ_WAVES);
-    EMD_LAUNCH(ctx, "snap_fij", (k_snap_fij<T, TF, SNAP_JBIG>), grid, 64 * FIJ_WAVES, 0, sn->t,
-               sn->nin, sn->nj, sn->nr, sn->cap_maxn, n, yr, yi, f);
-  }
+  EMD_TRY(snap_par_ready<T>(ctx, sn, n));
+  const snap_par<T> *par = (const snap_par<T> *)sn->par;
+  const int nb = RG_WAVES * (sn->t.twojmax <= SNAP_MAXJ ? rg<SNAP_MAXJ>::NB : rg<SNAP_JBIG>::NB);
+  const dim3 grid(n, (sn->cap_maxn + nb - 1) / nb);
+  if (sn->t.twojmax <= SNAP_MAXJ)
+    EMD_LAUNCH(ctx, "snap_fij", (k_snap_fij_rev<T, TF, SNAP_MAXJ>), grid, 64 * RG_WAVES, 0, sn->t,
+               sn->rg_map_d, sn->nin, sn->nj, sn->nr, par, sn->fdv, sn->cap_maxn, n, yr, yi, f);
+  else
+    EMD_LAUNCH(ctx, "snap_fij", (k_snap_fij_rev<T, TF, SNAP_JBIG>), grid, 64 * RG_WAVES, 0, sn->t,
+               sn->rg_map_d, sn->nin, sn->nj, sn->nr, par, sn->fdv, sn->cap_maxn, n, yr, yi, f);
   return EMD_OK;
 }
 
@@ -2188,22 +1712,16 @@ static emd_status snap_force(emd_ctx *ctx, emd_system *s, const emd_neigh *nl, e
   const int n = s->n_local;
   if (n <= 0) return zero ? emd_force_zero(ctx, s, precision) : EMD_OK;
   const int prec = precision == EMD_MIXED ? EMD_MIXED : EMD_FP64;
-  if (sn->t.twojmax <= SNAP_MAXJ) {
-    // compaction, neighbour parameters and U_tot in one launch (or, with
-    // static geometry, those of the previous call), then Y
-    if (snap_geom_cached(sn, s, nl, prec)) {
-      if (zero) EMD_TRY(emd_force_zero(ctx, s, prec));
-    } else {
-      EMD_TRY(snap_neigh_ui(ctx, s, nl, sn, zero ? prec : -1, prec));
-      snap_geom_record(sn, s, nl, prec);
-    }
-    if (precision == EMD_MIXED) EMD_TRY(snap_y<float>(ctx, sn, n));
-    else EMD_TRY(snap_y<double>(ctx, sn, n));
+  // compaction, neighbour parameters and U_tot in one launch (or, with
+  // static geometry, those of the previous call), then Y
+  if (snap_geom_cached(sn, s, nl, prec)) {
+    if (zero) EMD_TRY(emd_force_zero(ctx, s, prec));
   } else {
-    EMD_TRY(snap_neigh(ctx, s, nl, sn, zero ? prec : -1, prec));
-    if (precision == EMD_MIXED) EMD_TRY(snap_ui_y<float>(ctx, sn, n));
-    else EMD_TRY(snap_ui_y<double>(ctx, sn, n));
+    EMD_TRY(snap_neigh_ui(ctx, s, nl, sn, zero ? prec : -1, prec));
+    snap_geom_record(sn, s, nl, prec);
   }
+  if (precision == EMD_MIXED) EMD_TRY(snap_y<float>(ctx, sn, n));
+  else EMD_TRY(snap_y<double>(ctx, sn, n));
   if (precision == EMD_MIXED) {
     EMD_TRY((launch_fij<float, float>(ctx, sn, n, (const float *)sn->y_r,
                                       (const float *)sn->y_i, s->f32)));
@@ -2230,14 +1748,9 @@ extern "C" emd_status emd_snap_energy(emd_ctx *ctx, const emd_system *s, const e
   const int n = s->n_local;
   *energy = 0.0;
   if (n <= 0) return EMD_OK;
-  if (sn->t.twojmax <= SNAP_MAXJ) {
-    if (!snap_geom_cached(sn, s, nl, EMD_FP64)) {
-      EMD_TRY(snap_neigh_ui(ctx, s, nl, sn, -1, EMD_FP64));
-      snap_geom_record(sn, s, nl, EMD_FP64);
-    }
-  } else {
-    EMD_TRY(snap_neigh(ctx, s, nl, sn, -1, EMD_FP64));
-    EMD_TRY(launch_ui<double>(ctx, sn, n, (double *)sn->u_r, (double *)sn->u_i));
+  if (!snap_geom_cached(sn, s, nl, EMD_FP64)) {
+    EMD_TRY(snap_neigh_ui(ctx, s, nl, sn, -1, EMD_FP64));
+    snap_geom_record(sn, s, nl, EMD_FP64);
   }
   EMD_TRY(snap_y<double>(ctx, sn, n));
   double *ea = eatom;
@@ -2270,270 +1783,93 @@ extern "C" emd_status emd_snap_energy(emd_ctx *ctx, const emd_system *s, const e
 // three-role combination of Z_{abJ}; so per triple (a,b,J) only
 // S_{abJ} = sum_i sum' Re(conj(W^i_J) Z^i_{abJ}) is needed.
 
-// one U/dU layer step for the lane's entry (same recursion as k_snap_fij);
-// P holds the previous layer in full, component q at P[q * FULL + ma * j + mb]
-template <class T, int FULL>
-__device__ __forceinline__ void du_step(const snap_dev_tables &t, const T *P, int j, int ma, int mb,
-                                        T a_r, T a_i, T b_r, T b_i, const T *da_r, const T *da_i,
-                                        const T *db_r, const T *db_i, T &ur, T &ui, T *dr, T *di) {
-  ur = ui = 0;
-#pragma unroll
-  for (int k = 0; k < 3; k++) dr[k] = di[k] = 0;
-  if (ma < j) {
-    const T rp = (T)t.rootpq[(j - ma) * SNAP_RPD + (j - mb)];
-    const int s = ma * j + mb;
-    const T pr = P[s], pi = P[FULL + s];
-    ur += rp * (a_r * pr + a_i * pi);
-    ui += rp * (a_r * pi - a_i * pr);
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-      const T dpr = P[(2 + 2 * k) * FULL + s], dpi = P[(3 + 2 * k) * FULL + s];
-      dr[k] += rp * (da_r[k] * pr + da_i[k] * pi + a_r * dpr + a_i * dpi);
-      di[k] += rp * (da_r[k] * pi - da_i[k] * pr + a_r * dpi - a_i * dpr);
-    }
-  }
-  if (ma > 0) {
-    const T rp = (T)t.rootpq[ma * SNAP_RPD + (j - mb)];
-    const int s = (ma - 1) * j + mb;
-    const T pr = P[s], pi = P[FULL + s];
-    ur += -rp * (b_r * pr + b_i * pi);
-    ui += -rp * (b_r * pi - b_i * pr);
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-      const T dpr = P[(2 + 2 * k) * FULL + s], dpi = P[(3 + 2 * k) * FULL + s];
-      dr[k] += -rp * (db_r[k] * pr + db_i[k] * pi + b_r * dpr + b_i * dpi);
-      di[k] += -rp * (db_r[k] * pi - db_i[k] * pr + b_r * dpi - b_i * dpr);
-    }
-  }
-}
-
-// W^i for every atom: one wavefront per atom, neighbours in list order, the
-// half-plane entries of a layer 64 at a time (NST steps), FP64 accumulators
-// (T is the arithmetic of the recursion)
-template <class T, int J>
-__global__ void __launch_bounds__(64)
-k_snap_w(snap_dev_tables t, const int *__restrict__ nin, const int *__restrict__ nj,
-         const double *__restrict__ nr, int maxn, int n, const int *__restrict__ root,
-         const double *__restrict__ g, double *__restrict__ w_r, double *__restrict__ w_i) {
-  constexpr int JD = snap_dim<J>::JD, FULL = snap_dim<J>::FULLPREV;
-  constexpr int NST = (snap_hp(J) + 63) / 64;
-  __shared__ T s_u[2][8][FULL];
-  const int i = blockIdx.x;
-  if (i >= n) return;
-  const int l = threadIdx.x;
-  double acc_r[JD][NST], acc_i[JD][NST];
-#pragma unroll
-  for (int j = 0; j < JD; j++)
-#pragma unroll
-    for (int st = 0; st < NST; st++) acc_r[j][st] = acc_i[j][st] = 0.0;
-  const double gi0 = g[3 * (size_t)i], gi1 = g[3 * (size_t)i + 1], gi2 = g[3 * (size_t)i + 2];
-  const int cnt = nin[i];
-  for (int jj = 0; jj < cnt; jj++) {
-    const size_t o = (size_t)i * maxn + jj;
-    const int jn = nj[o];
-    const int own_j = jn < n ? jn : root[jn - n];
-    const T gd[3] = {(T)(gi0 - g[3 * (size_t)own_j]), (T)(gi1 - g[3 * (size_t)own_j + 1]),
-                     (T)(gi2 - g[3 * (size_t)own_j + 2])};
-    const T x = (T)nr[3 * o], y = (T)nr[3 * o + 1], z = (T)nr[3 * o + 2];
-    const T rsq = x * x + y * y + z * z;
-    const T r = sqrt(rsq);
-    const T rscale0 = (T)t.rfac0 * (T)SNAP_PI / ((T)t.rcut - (T)t.rmin0);
-    const T theta0 = (r - (T)t.rmin0) * rscale0;
-    const T z0 = r * cos(theta0) / sin(theta0);
-    const T dz0dr = z0 / r - (r * rscale0) * (rsq + z0 * z0) / rsq;
-    const T rinv = (T)1 / r;
-    const T u3[3] = {x * rinv, y * rinv, z * rinv};
-    const T r0inv = (T)1 / sqrt(r * r + z0 * z0);
-    const T a_r = z0 * r0inv, a_i = -z * r0inv, b_r = y * r0inv, b_i = -x * r0inv;
-    const T dr0invdr = -(r0inv * r0inv * r0inv) * (r + z0 * dz0dr);
-    T da_r[3], da_i[3], db_r[3], db_i[3];
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-      const T dr0 = dr0invdr * u3[k], dz = dz0dr * u3[k];
-      da_r[k] = dz * r0inv + z0 * dr0;
-      da_i[k] = -z * dr0;
-      db_r[k] = y * dr0;
-      db_i[k] = -x * dr0;
-    }
-    da_i[2] += -r0inv;
-    db_i[0] += -r0inv;
-    db_r[1] += r0inv;
-    T sfac, dsfac;
-    sfac_dsfac(t, r, sfac, dsfac);
-    sfac *= (T)t.wj;
-    dsfac *= (T)t.wj;
-    const T gu = gd[0] * u3[0] + gd[1] * u3[1] + gd[2] * u3[2];
-    if (l == 0) {
-      s_u[0][0][0] = 1;
-      s_u[0][1][0] = 0;
-      for (int k = 0; k < 3; k++) { s_u[0][2 + 2 * k][0] = 0; s_u[0][3 + 2 * k][0] = 0; }
-      acc_r[0][0] += 0.5 * (double)(dsfac * gu);
-    }
-    __syncthreads();
-    for (int j = 1; j <= t.twojmax; j++) {
-      const int p = (j - 1) & 1, c = j & 1;
-      T ur[NST], ui[NST], dr[NST][3], di[NST][3];
-      int ma[NST], mb[NST];
-      bool own[NST];
-#pragma unroll
-      for (int st = 0; st < NST; st++) {
-        const int e = st * 64 + l;
-        own[st] = e < snap_hp(j) && lane_entry(e, j, ma[st], mb[st]);
-        ur[st] = ui[st] = 0;
-#pragma unroll
-        for (int k = 0; k < 3; k++) dr[st][k] = di[st][k] = 0;
-        if (own[st])
-          du_step<T, FULL>(t, &s_u[p][0][0], j, ma[st], mb[st], a_r, a_i, b_r, b_i, da_r, da_i,
-                           db_r, db_i, ur[st], ui[st], dr[st], di[st]);
-      }
-      __syncthreads();
-#pragma unroll
-      for (int st = 0; st < NST; st++) {
-        if (own[st] && j < t.twojmax) {
-          T *C = &s_u[c][0][0];
-          const int s = ma[st] * (j + 1) + mb[st];
-          C[s] = ur[st]; C[FULL + s] = ui[st];
-#pragma unroll
-          for (int k = 0; k < 3; k++) { C[(2 + 2 * k) * FULL + s] = dr[st][k]; C[(3 + 2 * k) * FULL + s] = di[st][k]; }
-          if (2 * mb[st] != j) {
-            const T sg = ((ma[st] + mb[st]) & 1) ? (T)-1 : (T)1;
-            const int m = (j - ma[st]) * (j + 1) + (j - mb[st]);
-            C[m] = sg * ur[st]; C[FULL + m] = -sg * ui[st];
-#pragma unroll
-            for (int k = 0; k < 3; k++) { C[(2 + 2 * k) * FULL + m] = sg * dr[st][k]; C[(3 + 2 * k) * FULL + m] = -sg * di[st][k]; }
-          }
-        }
-        if (own[st]) {
-          double wgt = 1.0;
-          if (2 * mb[st] == j) wgt = (ma[st] < mb[st]) ? 1.0 : ((ma[st] == mb[st]) ? 0.5 : 0.0);
-          const T wr = dsfac * ur[st] * gu +
-                       sfac * (gd[0] * dr[st][0] + gd[1] * dr[st][1] + gd[2] * dr[st][2]);
-          const T wi = dsfac * ui[st] * gu +
-                       sfac * (gd[0] * di[st][0] + gd[1] * di[st][1] + gd[2] * di[st][2]);
-          acc_r[j][st] += wgt * (double)wr;
-          acc_i[j][st] += wgt * (double)wi;
-        }
-      }
-      __syncthreads();
-    }
-  }
-  for (int j = 0; j <= t.twojmax; j++) {
-#pragma unroll
-    for (int st = 0; st < NST; st++) {
-      int ma, mb;
-      const int e = st * 64 + l;
-      if (e < snap_hp(j) && lane_entry(e, j, ma, mb)) {
-        const int ey = t.ystart[j] + mb * (j + 1) + ma;
-        w_r[(size_t)i * t.ny + ey] = acc_r[j][st];
-        w_i[(size_t)i * t.ny + ey] = acc_i[j][st];
-      }
-    }
-  }
-}
-
-// W^i for every atom with the register-resident recursion (twojmax <= 8):
+// W^i for every atom with the register-resident recursion:
 //   W^i_J(e) = sum_{j in N(i)} w(e) [dsfac (g . u) U_J(e) + sfac dU_J(e)/dr . g],
-// g = g_i - g_j (a ghost j carries its owner's cotangent).  Only the
-// derivative along g is needed, so each lane carries U and dU_g = g . dU/dr
-// (4 values per entry): its recursion is that of U with da_g = g . da/dr and
-// db_g = g . db/dr, both rank one in u plus constants:
+// g = g_i - g_j (a ghost j carries its owner's cotangent): the derivative
+// of sfac U along g.  Each lane carries sfac V and its derivative X (4 values
+// per entry), whose recursions are linear: they start from sfac and dsfac (g.u),
+//   X_j = conj(a) X_{j-1}(ma) - conj(b) X_{j-1}(ma-1)
+//       + conj(da_g) sfac V_{j-1}(ma) - conj(db_g) sfac V_{j-1}(ma-1)
+// with da_g = g . da/dr and db_g = g . db/dr, both rank one in u plus constants:
 //   da_g = c1 (g.u) + i (c2 (g.u) - r0inv g_z),  db_g = c3 (g.u) + r0inv g_y
 //                                                   + i (c4 (g.u) - r0inv g_x).
-// One wavefront per atom, seven neighbours at a time; each lane sums its
-// group's neighbours in T, the groups are added in FP64 (fixed tree):
+// One wavefront per atom, a group of lanes per neighbour; each lane sums its
+// group's neighbours (in TS), the groups are added in FP64 in order:
 // deterministic.
-template <class T>
+template <class T, class TS, int J>
 __global__ void __launch_bounds__(64)
-k_snap_w_rg(snap_dev_tables t, const rg_rp<T> *__restrict__ rgp, const rg_map *__restrict__ rgm,
-            const int *__restrict__ nin, const int *__restrict__ nj,
-            const snap_par<T> *__restrict__ par, int maxn, int n, const int *__restrict__ root,
-            const double *__restrict__ g, double *__restrict__ w_r, double *__restrict__ w_i) {
-  __shared__ rg_rec<T> s_rec[RG_SLOTS * RG_W];
-  __shared__ double s_acc[2][RG_SLOTS * RG_W];
+k_snap_w_rg(snap_dev_tables t, const rg_map *__restrict__ rgm, const int *__restrict__ nin,
+            const int *__restrict__ nj, const snap_par<T> *__restrict__ par, int maxn, int n,
+            const int *__restrict__ root, const double *__restrict__ g, double *__restrict__ w_r,
+            double *__restrict__ w_i) {
+  using R = rg<J>;
+  __shared__ TS s_buf[rg_sum<J>::BUF];
   const int i = blockIdx.x;
   if (i >= n) return;
-  rg_fill<T, 64>(rgp, rgm, 0, nullptr, nullptr, i, s_rec);
-  __syncthreads();
-  for (int k = threadIdx.x; k < RG_SLOTS * RG_W; k += 64)
-    s_rec[k].yr = (T)0.5 * (T)rgm[k].wq;  // the half-plane weight of the entry
-  __syncthreads();
   const int l = threadIdx.x;
-  const int gr = l / RG_W, ma = l - gr * RG_W;  // gr = 7 only for the idle lane 63
-  T acc[RG_SLOTS][2];
+  const int gr = l / R::W, ma = l - gr * R::W;  // gr = NB only for idle lanes
+  TS acc[R::SLOTS][2];
 #pragma unroll
-  for (int s = 0; s < RG_SLOTS; s++) acc[s][0] = acc[s][1] = 0;
+  for (int s = 0; s < R::SLOTS; s++) acc[s][0] = acc[s][1] = 0;
   const double gi0 = g[3 * (size_t)i], gi1 = g[3 * (size_t)i + 1], gi2 = g[3 * (size_t)i + 2];
   const int cnt = nin[i];
-  for (int base = 0; base < cnt; base += RG_NB) {
+  for (int base = 0; base < cnt; base += R::NB) {
     const int jj = base + gr;
-    const bool act = gr < RG_NB && jj < cnt;
+    const bool act = gr < R::NB && jj < cnt;
     const size_t o = (size_t)i * maxn + (act ? jj : base);
     const snap_par<T> pp = par[o];
     const int jn = nj[o];
     const int own_j = jn < n ? jn : root[jn - n];
-    const T g0 = act ? (T)(gi0 - g[3 * (size_t)own_j]) : (T)0;
-    const T g1 = act ? (T)(gi1 - g[3 * (size_t)own_j + 1]) : (T)0;
-    const T g2 = act ? (T)(gi2 - g[3 * (size_t)own_j + 2]) : (T)0;
+    const T g0 = (T)(gi0 - g[3 * (size_t)own_j]);
+    const T g1 = (T)(gi1 - g[3 * (size_t)own_j + 1]);
+    const T g2 = (T)(gi2 - g[3 * (size_t)own_j + 2]);
     const T gu = g0 * pp.u[0] + g1 * pp.u[1] + g2 * pp.u[2];
     const T a_r = pp.a_r, a_i = pp.a_i, b_r = pp.b_r, b_i = pp.b_i;
     const T da_r = pp.c1 * gu, da_i = pp.c2 * gu - pp.r0inv * g2;
     const T db_r = pp.c3 * gu + pp.r0inv * g1, db_i = pp.c4 * gu - pp.r0inv * g0;
-    const T sfac = pp.sfac, dsg = pp.dsfac * gu;  // dsg = 0 for an idle group
-    // c[mb]: U_r, U_i, dU_g r, dU_g i of (ma, mb)
-    T c[RG_COLS][4];
+    const bool first = act && ma == 0;  // an idle group adds nothing
+    T c[R::COLS][2], d[R::COLS][2];     // sfac V and X of (ma, mb)
 #pragma unroll
-    for (int mb = 0; mb < RG_COLS; mb++) c[mb][0] = c[mb][1] = c[mb][2] = c[mb][3] = 0;
-    c[0][0] = ma == 0 ? (T)1 : (T)0;  // layer 0: U = 1, dU = 0
-    acc[0][0] += (T)0.5 * dsg * c[0][0];
+    for (int mb = 0; mb < R::COLS; mb++) c[mb][0] = c[mb][1] = d[mb][0] = d[mb][1] = 0;
+    c[0][0] = first ? pp.sfac : (T)0;
+    d[0][0] = first ? pp.dsfac * gu : (T)0;
+    acc[0][0] += (TS)d[0][0];
+    rg_layers<1, J>([&](auto jc) {
+      constexpr int j = jc;
+      if (j > t.twojmax) return;
+      // the terms of V_{j-1}, then X_{j-1}'s own recursion
+      T e[R::COLS][2];
+      T q[2];
 #pragma unroll
-    for (int j = 1; j <= SNAP_MAXJ; j++) {
-      if (j > t.twojmax) break;
-      T mir[4], mirb[4];  // even j: (U, dU_g) of (ma, j/2) and (ma-1, j/2) in layer j-1
-      if ((j & 1) == 0) {
-        const int src = gr * RG_W + (j - 1 - ma > 0 ? j - 1 - ma : 0);
-        const T sg = ((ma + j / 2) & 1) ? (T)-1 : (T)1;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-          const T v = __shfl(c[j / 2 - 1][q], src, 64);
-          mir[q] = (q & 1) ? -sg * v : sg * v;
+      for (int mb = 0; 2 * mb < j; mb++) {
+        const T p0 = c[mb][0], p1 = c[mb][1];
+        q[0] = lane_below(p0);
+        q[1] = lane_below(p1);
+        e[mb][0] = da_r * p0 + da_i * p1 - db_r * q[0] - db_i * q[1];
+        e[mb][1] = da_r * p1 - da_i * p0 - db_r * q[1] + db_i * q[0];
+        if (2 * mb + 2 == j) {
+          e[mb + 1][0] = db_r * p0 - db_i * p1 + da_r * q[0] - da_i * q[1];
+          e[mb + 1][1] = db_r * p1 + db_i * p0 + da_r * q[1] + da_i * q[0];
         }
-#pragma unroll
-        for (int q = 0; q < 4; q++) mirb[q] = lane_below(mir[q]);
       }
+      rg_layer<j>(a_r, a_i, b_r, b_i, d);
+      rg_layer<j>(a_r, a_i, b_r, b_i, c);
 #pragma unroll
       for (int mb = 0; mb <= j / 2; mb++) {
-        const int slot = rg_slot0(j) + mb;
-        const rg_rec<T> q = s_rec[slot * RG_W + ma];
-        const bool mid = (j & 1) == 0 && mb == j / 2;
-        T P[4], Q[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-          P[k] = mid ? mir[k] : c[mb][k];
-          Q[k] = mid ? mirb[k] : lane_below(c[mb][k]);
-        }
-        const T ur = q.rpa * (a_r * P[0] + a_i * P[1]) - q.rpb * (b_r * Q[0] + b_i * Q[1]);
-        const T ui = q.rpa * (a_r * P[1] - a_i * P[0]) - q.rpb * (b_r * Q[1] - b_i * Q[0]);
-        const T dr = q.rpa * (da_r * P[0] + da_i * P[1] + a_r * P[2] + a_i * P[3]) -
-                     q.rpb * (db_r * Q[0] + db_i * Q[1] + b_r * Q[2] + b_i * Q[3]);
-        const T di = q.rpa * (da_r * P[1] - da_i * P[0] + a_r * P[3] - a_i * P[2]) -
-                     q.rpb * (db_r * Q[1] - db_i * Q[0] + b_r * Q[3] - b_i * Q[2]);
-        c[mb][0] = ur;
-        c[mb][1] = ui;
-        c[mb][2] = dr;
-        c[mb][3] = di;
-        acc[slot][0] += q.yr * (dsg * ur + sfac * dr);
-        acc[slot][1] += q.yr * (dsg * ui + sfac * di);
+        d[mb][0] += e[mb][0];
+        d[mb][1] += e[mb][1];
+        acc[rg_slot0(j) + mb][0] += (TS)d[mb][0];
+        acc[rg_slot0(j) + mb][1] += (TS)d[mb][1];
       }
-    }
+    });
   }
-  rg_group_sum<T, double>(acc, l, s_acc[0], s_acc[1]);
-  __syncthreads();
-  for (int k = l; k < RG_SLOTS * RG_W; k += 64) {
+  rg_group_sum<double, J>(acc, l, s_buf, [&](int k, double vr, double vi) {
     const rg_map m = rgm[k];
-    if (m.ey < 0) continue;
-    w_r[(size_t)i * t.ny + m.ey] = s_acc[0][k];
-    w_i[(size_t)i * t.ny + m.ey] = s_acc[1][k];
-  }
+    if (m.ey < 0) return;
+    const double wgt = 0.5 * m.wq * m.norm;
+    w_r[(size_t)i * t.ny + m.ey] = wgt * vr;
+    w_i[(size_t)i * t.ny + m.ey] = wgt * vi;
+  });
 }
 
 // S_{abJ} += sum' Re(conj(W^i_J) Z^i_{abJ}) over atoms (FP64 accumulation)
@@ -2735,17 +2071,16 @@ template <class T>
 static emd_status snap_adjoint_impl(emd_ctx *ctx, const emd_system *s, const emd_halo *h,
                                     emd_snap *sn, const double *g, double *S) {
   const int n = s->n_local;
-  // twojmax <= 8: U_tot came with the compaction (k_snap_neigh_ui)
-  if (sn->t.twojmax > SNAP_MAXJ) EMD_TRY(launch_ui<T>(ctx, sn, n, (T *)sn->u_r, (T *)sn->u_i));
-  if (sn->t.twojmax <= SNAP_MAXJ) {
-    EMD_TRY(snap_par_ready<T>(ctx, sn, n));
-    EMD_LAUNCH(ctx, "snap_adjoint_w", k_snap_w_rg<T>, n, 64, 0, sn->t, rg_rp_of<T>(sn),
-               sn->rg_map_d, sn->nin, sn->nj, (const snap_par<T> *)sn->par, sn->cap_maxn, n,
-               h ? h->root : nullptr, g, sn->w_r, sn->w_i);
-  }
+  // U_tot came with the compaction
+  EMD_TRY(snap_par_ready<T>(ctx, sn, n));
+  const snap_par<T> *par = (const snap_par<T> *)sn->par;
+  if (sn->t.twojmax <= SNAP_MAXJ)
+    EMD_LAUNCH(ctx, "snap_adjoint_w", (k_snap_w_rg<T, T, SNAP_MAXJ>), n, 64, 0, sn->t, sn->rg_map_d,
+               sn->nin, sn->nj, par, sn->cap_maxn, n, h ? h->root : nullptr, g, sn->w_r, sn->w_i);
   else
-    EMD_LAUNCH(ctx, "snap_adjoint_w", (k_snap_w<T, SNAP_JBIG>), n, 64, 0, sn->t, sn->nin, sn->nj,
-               sn->nr, sn->cap_maxn, n, h ? h->root : nullptr, g, sn->w_r, sn->w_i);
+    EMD_LAUNCH(ctx, "snap_adjoint_w", (k_snap_w_rg<T, double, SNAP_JBIG>), n, 64, 0, sn->t,
+               sn->rg_map_d, sn->nin, sn->nj, par, sn->cap_maxn, n, h ? h->root : nullptr, g,
+               sn->w_r, sn->w_i);
   const int ntrip = (int)sn->tid.size();
   if (sn->t.twojmax <= SNAP_MAXJ) {
     const uint32_t *code = std::is_same<T, float>::value ? sn->yf_code32 : sn->yf_code64;
@@ -2777,13 +2112,9 @@ extern "C" emd_status emd_snap_adjoint_beta(emd_ctx *ctx, const emd_system *s, c
   EMD_ARG(ctx, s->n_ghost == 0 || (h && h->root && h->n_ghost == s->n_ghost),
           "ghost atoms need the halo (owner of each ghost)");
   const int aprec = precision == EMD_MIXED ? EMD_MIXED : EMD_FP64;
-  if (sn->t.twojmax <= SNAP_MAXJ) {
-    if (!snap_geom_cached(sn, s, nl, aprec)) {
-      EMD_TRY(snap_neigh_ui(ctx, s, nl, sn, -1, aprec));
-      snap_geom_record(sn, s, nl, aprec);
-    }
-  } else {
-    EMD_TRY(snap_neigh(ctx, s, nl, sn, -1, aprec));
+  if (!snap_geom_cached(sn, s, nl, aprec)) {
+    EMD_TRY(snap_neigh_ui(ctx, s, nl, sn, -1, aprec));
+    snap_geom_record(sn, s, nl, aprec);
   }
   EMD_TRY(emd_ensure(ctx, (void **)&sn->w_r, &sn->cap_w, (size_t)n * sn->t.ny * sizeof(double)));
   EMD_TRY(emd_ensure(ctx, (void **)&sn->w_i, &sn->cap_wi, (size_t)n * sn->t.ny * sizeof(double)));
@@ -2799,7 +2130,7 @@ extern "C" emd_status emd_snap_adjoint_beta(emd_ctx *ctx, const emd_system *s, c
   // dE/dbeta_k = sum_i B_k^i in FP64
   if (dLdE != 0.0) {
     sn->geom_prec = -1;  // U_tot is rewritten in FP64
-    EMD_TRY(launch_ui<double>(ctx, sn, n, (double *)sn->u_r, (double *)sn->u_i));
+    EMD_TRY(launch_ui(ctx, sn, n));
     EMD_LAUNCH(ctx, "snap_adjoint_bsum", k_snap_bsum, n, 256, 0, sn->t, sn->cg, sn->etab,
                sn->ncoeff, sn->bzeroflag, n, (const double *)sn->u_r, (const double *)sn->u_i, B,
                nullptr);
@@ -2826,8 +2157,7 @@ extern "C" emd_status emd_snap_descriptors(emd_ctx *ctx, const emd_system *s, co
   const int n = s->n_local;
   if (n <= 0) return EMD_OK;
   sn->geom_prec = -1;  // the compaction and U_tot are rewritten
-  EMD_TRY(snap_neigh(ctx, s, nl, sn, -1, EMD_FP64));
-  EMD_TRY(launch_ui<double>(ctx, sn, n, (double *)sn->u_r, (double *)sn->u_i));
+  EMD_TRY(snap_neigh_ui(ctx, s, nl, sn, -1, EMD_FP64));
   EMD_LAUNCH(ctx, "snap_descriptors", k_snap_bsum, n, 256, 0, sn->t, sn->cg, sn->etab,
              sn->ncoeff, sn->bzeroflag, n, (const double *)sn->u_r, (const double *)sn->u_i,
              nullptr, B);

@@ -326,7 +326,7 @@ emd_status emd_snap_set_coeff(emd_ctx *ctx, emd_snap *sn, const double *coeff);
 /* No counterpart in the reference (it serves repeated force and beta-adjoint
  * evaluations of fixed configurations, e.g. force matching): with on != 0
  * the caller promises that positions, atom count and neighbour list stay as
- * they are; for twojmax <= 8 the compaction, neighbour parameters and U_tot
+ * they are; the compaction, neighbour parameters and U_tot
  * of the last force or adjoint call of a precision are then reused by later
  * calls of that precision (they depend on the geometry only, not on beta).
  * Calling it again (on or off) discards what was kept. */
