@@ -320,22 +320,31 @@ __device__ __forceinline__ void y_entry(const snap_dev_tables &t, int e, int &J,
   ma = k - mb * (J + 1);
 }
 
-// Y of AT atoms per block from a flat term stream.  Every half-plane entry
-// e = (J, ma, mb) is the sum over its (a, b) keys and (ma1, mb1) of
+// Y of AT atoms per block from a flat stream of products.  Every half-plane
+// entry e = (J, ma, mb) is the sum over its (a, b) keys and (ma1, mb1) of
 //   w * U_a(ma1, mb1) * U_b(ma2, mb2),  w = coef(a,b,J) cg(ma1,ma2) cg(mb1,mb2)
 // (the double sum of SNA::compute_zi, sna_impl.hpp:221-274, weighted as in
-// compute_dbidrj's three roles).  The host lists these products (zero
-// Clebsch-Gordan weights dropped) entry by entry, pads each entry's list with
-// zero-weight terms to whole chunks of YF_CHUNK, and gives thread t the
+// compute_dbidrj's three roles).  The host pairs an entry's products that
+// share a U entry (yf_pairs): a slot of the stream is
+//   U_c (w_x U_x + w_y U_y),
+// three LDS byte offsets (its code), two weights, eight multiply-adds and
+// three LDS reads for two products, where one product at a time takes twelve
+// and four.  Entries of half-plane weight 0 (the middle columns' ma > mb)
+// have no products.  The slots come entry by entry, each entry's list
+// padded with zero-weight slots to whole chunks of YF_CHUNK, and thread t gets the
 // chunks [t P, (t+1) P) of that sequence, interleaved so that step s of every
 // thread is one coalesced load.  Chunk boundaries are the same for every
-// lane, so the term loop carries no per-term branch: a term is two LDS byte
-// offsets (its code), a weight and six multiply-adds.  Once per chunk a
+// lane, so the slot loop carries no branch.  Once per chunk a
 // thread whose run of one entry's chunks ends stores the run's sum in LDS;
 // each entry adds its runs in thread order (fixed order: deterministic).
 // With AT atoms per block (U_tot of each in LDS) every code and weight load
-// serves AT atoms: with the LDS reads free of bank conflicts (below) the
-// stream of codes and weights from L2 is what bounds the kernel.
+// serves AT atoms.
+// Arithmetic (47 % of its issue rate at 16 000 atoms in FP64), LDS reads (40
+// %) and the stream from L2 (54 % of the address units, 14 TB/s) bound it
+// about equally, so all three had to shrink: one product at a time with the
+// middle columns in full took 303 us for 16 000 atoms (FP64, twojmax 8), 24.4
+// for 2000 (mixed), 222 / 109 for 1024 atoms at twojmax 12 (FP64 / mixed); this
+// takes 222, 18, 137 and 69.
 //
 // LDS banks: the LDS serves 256 bytes per cycle, so a wavefront's
 // ds_read_b64 is served 32 lanes per cycle, and two lanes of one cycle that
@@ -351,11 +360,13 @@ __device__ __forceinline__ void y_entry(const snap_dev_tables &t, int e, int &J,
 // read of every term the copy whose residue no other address of its
 // 32-lane group takes (a matching per group; with the shifts 0, 5, 11, 19
 // about 4 % of the groups keep one conflict).
-// threads per Y block (the stream is split this many ways): SNAP-2k 25.3 /
-// 43.7 us (mixed / FP64) against 27.0 / 47.3 with 256 and 28.7 / 47.2 with
-// 1024 (more padding, fewer blocks per CU)
-constexpr int YF_THREADS = 512;
-constexpr int YF_CHUNK = 16;
+// threads per Y block (the stream is split this many ways): 512, at twojmax
+// above 8, where one block's LDS fills a CU, 1024
+template <int J>
+constexpr int yf_threads() { return J <= SNAP_MAXJ ? 512 : 1024; }
+constexpr int SF_THREADS = 512;
+constexpr int YF_CHUNK = 8;   // slots
+constexpr int SF_CHUNK = 16;  // products (the beta adjoint's stream)
 
 template <class T>
 struct alignas(2 * sizeof(T)) cpair {
@@ -377,138 +388,185 @@ struct yf_layout {
   }
   __host__ __device__ static constexpr int base(int c) { return c * STRIDE + shift(c); }
   static constexpr int NUC = base(NCOPY - 1) + snap_dim<J>::NU;  // words the copies span
-  static constexpr int NUC_PAD = (NUC + MOD - 1) / MOD * MOD;
+  // an odd number of 256-byte rows: at a multiple of 512 bytes the compiler
+  // joins the real and imaginary (or two atoms') reads into ds_read2st64_b64,
+  // which takes twice as long as the two
+  static constexpr int NUC_PAD = ((NUC + MOD - 1) / MOD | 1) * MOD;
   static constexpr int IMB = SOA ? NUC_PAD * 8 : 0;            // imaginary array (FP64)
   static constexpr int UBYTES = SOA ? 2 * NUC_PAD * 8 : NUC_PAD * 8;
 };
 
-// code: byte offsets of the two U_tot entries in LDS, 16 bits each (the
-// host writes offsets for sizeof(cpair<T>)); meta[c][t]: the LDS slot of the
+// the byte offsets of a slot's U_tot entries in LDS
+struct alignas(8) yf_code {
+  unsigned short c, x, y, pad;
+};
+template <class T, int J>
+__device__ __forceinline__ cpair<T> yf_u(const unsigned char *ub, unsigned off) {
+  using L = yf_layout<T, J>;
+  if constexpr (L::SOA)
+    return cpair<T>{*reinterpret_cast<const T *>(ub + off),
+                    *reinterpret_cast<const T *>(ub + L::IMB + off)};
+  else
+    return *reinterpret_cast<const cpair<T> *>(ub + off);
+}
+
+// meta[c][t]: the LDS slot of the
 // run that ends with thread t's chunk c, or YF_NO_RUN.  A thread's runs are
 // the entries its chunk range touches, so there are at most ny + threads - 1.
 constexpr unsigned short YF_NO_RUN = 0xFFFFu;
 template <int J>
-constexpr int yf_maxruns() { return snap_dim<J>::NY + YF_THREADS; }
+constexpr int yf_maxruns() { return snap_dim<J>::NY + yf_threads<J>(); }
 static_assert(yf_layout<double, SNAP_JBIG>::NUC * 8 < 65536 &&
                   yf_layout<float, SNAP_JBIG>::NUC * 8 < 65536,
               "U_tot byte offsets fit 16 bits");
 
-// The term stream of AT atoms whose U_tot copies are in LDS at sb (a copy
-// set of yf_layout<T,J>::UBYTES per atom), run sums in part: Y of atoms
-// i0 .. i0 + AT - 1 (those below n)
-template <class T, int J, int AT>
-__device__ __forceinline__ void yf_stream(const unsigned char *sb, cpair<T> *part, int i0, int n,
-                                          int ny, int nch, const uint32_t *__restrict__ code,
-                                          const T *__restrict__ w,
-                                          const unsigned short *__restrict__ meta,
-                                          const int *__restrict__ rstart, T *__restrict__ y_r,
-                                          T *__restrict__ y_i) {
-  using L = yf_layout<T, J>;
-  T ar[AT], ai[AT];
-#pragma unroll
-  for (int a = 0; a < AT; a++) ar[a] = ai[a] = 0;
-  for (int c = 0; c < nch; c++) {
-    const unsigned short m = meta[(size_t)c * YF_THREADS + threadIdx.x];
-    // the chunk's loads are issued before its arithmetic
-    uint32_t cc[YF_CHUNK];
-    T ww[YF_CHUNK];
-#pragma unroll
-    for (int k = 0; k < YF_CHUNK; k++) {
-      const size_t slot = ((size_t)c * YF_CHUNK + k) * YF_THREADS + threadIdx.x;
-      cc[k] = code[slot];
-      ww[k] = w[slot];
-    }
-#pragma unroll
-    for (int k = 0; k < YF_CHUNK; k++) {
-#pragma unroll
-      for (int a = 0; a < AT; a++) {
-        const unsigned char *ub = sb + a * L::UBYTES;
-        cpair<T> u1, u2;
-        if (L::SOA) {
-          u1.r = *reinterpret_cast<const T *>(ub + (cc[k] & 0xFFFFu));
-          u1.i = *reinterpret_cast<const T *>(ub + L::IMB + (cc[k] & 0xFFFFu));
-          u2.r = *reinterpret_cast<const T *>(ub + (cc[k] >> 16));
-          u2.i = *reinterpret_cast<const T *>(ub + L::IMB + (cc[k] >> 16));
-        } else {
-          u1 = *reinterpret_cast<const cpair<T> *>(ub + (cc[k] & 0xFFFFu));
-          u2 = *reinterpret_cast<const cpair<T> *>(ub + (cc[k] >> 16));
-        }
-        const T pr = u1.r * u2.r - u1.i * u2.i;
-        const T pi = u1.r * u2.i + u1.i * u2.r;
-        ar[a] += ww[k] * pr;
-        ai[a] += ww[k] * pi;
-      }
-    }
-    if (m != YF_NO_RUN) {
-#pragma unroll
-      for (int a = 0; a < AT; a++) {
-        part[a * yf_maxruns<J>() + m] = cpair<T>{ar[a], ai[a]};
-        ar[a] = 0;
-        ai[a] = 0;
-      }
-    }
-  }
-  __syncthreads();
-  for (int a = 0; a < AT; a++) {
-    const int i = i0 + a;
-    if (i >= n) break;
-    for (int e = threadIdx.x; e < ny; e += YF_THREADS) {
-      T yr = 0, yi = 0;
-      for (int r = rstart[e]; r < rstart[e + 1]; r++) {
-        yr += part[a * yf_maxruns<J>() + r].r;
-        yi += part[a * yf_maxruns<J>() + r].i;
-      }
-      y_r[(size_t)i * ny + e] = yr;
-      y_i[(size_t)i * ny + e] = yi;
-    }
-  }
+// Place of slot k of (chunk c, thread t) in the stream: a wavefront's slots lie
+// together, one step of its lanes in a row, so all loads of a chunk have one
+// address and constant offsets.  Codes and FP32 weights take two slots
+// per 16-byte load.
+__host__ __device__ constexpr size_t yf_place(int P, int c, int k, int t) {
+  return ((size_t)(t / 64 * P + c) * YF_CHUNK + k) * 64 + t % 64;
+}
+__host__ __device__ constexpr size_t yf_place2(size_t place) {  // two slots of a lane together
+  return (place / 128 * 64 + place % 64) * 2 + place / 64 % 2;
 }
 
+// four slots of the stream in registers
+template <class T>
+struct yf_regs {
+  yf_code c[4];
+  cpair<T> w[4];
+  __device__ __forceinline__ void load(const yf_code *__restrict__ code,
+                                       const cpair<T> *__restrict__ wt, int step, int l) {
+    typedef unsigned v4 __attribute__((ext_vector_type(4)));
+    const v4 *cp = reinterpret_cast<const v4 *>(code) + ((size_t)step * 2 * 64 + l);
+    reinterpret_cast<v4 *>(c)[0] = cp[0];
+    reinterpret_cast<v4 *>(c)[1] = cp[64];
+    if constexpr (sizeof(T) == 4) {
+      const v4 *wp = reinterpret_cast<const v4 *>(wt) + ((size_t)step * 2 * 64 + l);
+      reinterpret_cast<v4 *>(w)[0] = wp[0];
+      reinterpret_cast<v4 *>(w)[1] = wp[64];
+    } else {
+      const cpair<T> *wp = wt + ((size_t)step * 4 * 64 + l);
+#pragma unroll
+      for (int k = 0; k < 4; k++) w[k] = wp[64 * k];
+    }
+  }
+};
+
 template <class T, int J, int AT>
-__global__ void __launch_bounds__(YF_THREADS)
-k_snap_yflat(int nu, int ny, int nch, const uint32_t *__restrict__ code,
-             const T *__restrict__ w, const unsigned short *__restrict__ meta,
+__global__ void __launch_bounds__(yf_threads<J>())
+k_snap_yflat(int nu, int ny, int nch, const yf_code *__restrict__ code,
+             const cpair<T> *__restrict__ w, const unsigned short *__restrict__ meta,
              const int *__restrict__ rstart, int n, const T *__restrict__ utot_r,
              const T *__restrict__ utot_i, T *__restrict__ y_r, T *__restrict__ y_i) {
   // the copies of U_tot from byte 0 (a static array: its LDS address is
   // known when the kernel is compiled, so a code's offset is the whole LDS
   // address), then the run sums
   using L = yf_layout<T, J>;
+  constexpr int NT = yf_threads<J>();
   static_assert(L::UBYTES % sizeof(cpair<T>) == 0, "run sums aligned");
   constexpr int UP = L::UBYTES / sizeof(cpair<T>);  // pairs per atom's U_tot copies
-  __shared__ cpair<T> s_yf[AT * (UP + yf_maxruns<J>())];
+  constexpr int MR = yf_maxruns<J>();
+  __shared__ cpair<T> s_yf[AT * (UP + MR)];
   unsigned char *sb = reinterpret_cast<unsigned char *>(s_yf);
+  cpair<T> *part = s_yf + AT * UP;
   const int i0 = blockIdx.x * AT;
   if (i0 >= n) return;
-  for (int a = 0; a < AT; a++) {
-    const int i = i0 + a < n ? i0 + a : i0;
-    unsigned char *ub = sb + a * L::UBYTES;
-    for (int k = threadIdx.x; k < nu; k += YF_THREADS) {
-      const T vr = utot_r[(size_t)i * nu + k], vi = utot_i[(size_t)i * nu + k];
+  const int l = threadIdx.x % 64;
+  const size_t wv = (size_t)(threadIdx.x / 64) * nch * YF_CHUNK * 64;  // the wavefront's slots
+  code += wv;
+  w += wv;
+  yf_regs<T> b0, b1;
+  b0.load(code, w, 0, l);  // under way while U_tot is staged
 #pragma unroll
-      for (int c = 0; c < L::NCOPY; c++) {
-        if (L::SOA) {
-          reinterpret_cast<T *>(ub)[L::base(c) + k] = vr;
-          reinterpret_cast<T *>(ub + L::IMB)[L::base(c) + k] = vi;
-        } else {
-          reinterpret_cast<cpair<T> *>(ub)[L::base(c) + k] = cpair<T>{vr, vi};
+  for (int k0 = 0; k0 < snap_dim<J>::NU; k0 += NT) {
+    const int k = k0 + (int)threadIdx.x;
+    if (k < nu) {
+      T vr[AT], vi[AT];
+#pragma unroll
+      for (int a = 0; a < AT; a++) {
+        const size_t i = i0 + a < n ? i0 + a : i0;
+        vr[a] = utot_r[i * nu + k];
+        vi[a] = utot_i[i * nu + k];
+      }
+#pragma unroll
+      for (int a = 0; a < AT; a++) {
+        unsigned char *ub = sb + a * L::UBYTES;
+#pragma unroll
+        for (int c = 0; c < L::NCOPY; c++) {
+          if (L::SOA) {
+            reinterpret_cast<T *>(ub)[L::base(c) + k] = vr[a];
+            reinterpret_cast<T *>(ub + L::IMB)[L::base(c) + k] = vi[a];
+          } else {
+            reinterpret_cast<cpair<T> *>(ub)[L::base(c) + k] = cpair<T>{vr[a], vi[a]};
+          }
         }
       }
     }
   }
   __syncthreads();
-  yf_stream<T, J, AT>(sb, s_yf + AT * UP, i0, n, ny, nch, code, w, meta, rstart, y_r, y_i);
+  T ar[AT], ai[AT];
+#pragma unroll
+  for (int a = 0; a < AT; a++) ar[a] = ai[a] = 0;
+  auto add = [&](const yf_regs<T> &b) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+#pragma unroll
+      for (int a = 0; a < AT; a++) {
+        const unsigned char *ub = sb + a * L::UBYTES;
+        const cpair<T> uc = yf_u<T, J>(ub, b.c[k].c), ux = yf_u<T, J>(ub, b.c[k].x),
+                       uy = yf_u<T, J>(ub, b.c[k].y);
+        const T vr = b.w[k].r * ux.r + b.w[k].i * uy.r;
+        const T vi = b.w[k].r * ux.i + b.w[k].i * uy.i;
+        ar[a] += uc.r * vr;  // two multiply-adds each, not a sum of products
+        ar[a] -= uc.i * vi;
+        ai[a] += uc.r * vi;
+        ai[a] += uc.i * vr;
+      }
+    }
+  };
+  static_assert(YF_CHUNK == 8, "two halves");
+#pragma unroll 1
+  for (int c = 0; c < nch; c++) {
+    // the next half's loads are under way while one half is added up
+    b1.load(code, w, 2 * c + 1, l);
+    const unsigned short m = meta[(size_t)c * NT + threadIdx.x];
+    add(b0);
+    b0.load(code, w, c + 1 < nch ? 2 * c + 2 : 0, l);
+    add(b1);
+    if (m != YF_NO_RUN) {
+#pragma unroll
+      for (int a = 0; a < AT; a++) {
+        part[a * MR + m] = cpair<T>{ar[a], ai[a]};
+        ar[a] = 0;
+        ai[a] = 0;
+      }
+    }
+  }
+  __syncthreads();
+  for (int q = threadIdx.x; q < AT * ny; q += NT) {
+    const int a = q / ny, e = q - a * ny;
+    if (i0 + a >= n) break;
+    T yr = 0, yi = 0;
+    for (int r = rstart[e]; r < rstart[e + 1]; r++) {
+      yr += part[a * MR + r].r;
+      yi += part[a * MR + r].i;
+    }
+    y_r[(size_t)(i0 + a) * ny + e] = yr;
+    y_i[(size_t)(i0 + a) * ny + e] = yi;
+  }
 }
 
-// term weights for the current coefficients: w = coef(key) * cg product
+// the slots' weights for the current coefficients (two products per slot)
 __global__ void k_yf_weights(int nslots, const unsigned short *__restrict__ key,
                              const double *__restrict__ cgw, const double *__restrict__ kcoef,
                              double *__restrict__ w64, float *__restrict__ w32) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= nslots) return;
+  if (s >= 2 * nslots) return;
   const double v = kcoef[key[s]] * cgw[s];
   w64[s] = v;
-  w32[s] = (float)v;
+  w32[2 * yf_place2(s / 2) + s % 2] = (float)v;
 }
 
 // ------------------------------------------- register-resident recursion
@@ -879,20 +937,29 @@ k_snap_fij_rev(snap_dev_tables t, const rg_map *__restrict__ rgm, const int *__r
       const rg_rec<T> q = s_rec[(rg_slot0(j - 1) + mb) * R::W + ma];
       const T p0 = vs[rg_slot0(j - 1) + mb][0], p1 = vs[rg_slot0(j - 1) + mb][1];
       const T u0 = ad[mb][0], u1 = ad[mb][1], w0 = up[mb][0], w1 = up[mb][1];
-      sa_r += u0 * p0 + u1 * p1;
-      sa_i += u0 * p1 - u1 * p0;
-      sb_r += w0 * p0 + w1 * p1;
-      sb_i += w0 * p1 - w1 * p0;
+      // (one multiply-add per product: a sum of products would round twice)
+      sa_r += u0 * p0;
+      sa_r += u1 * p1;
+      sa_i += u0 * p1;
+      sa_i -= u1 * p0;
+      sb_r += w0 * p0;
+      sb_r += w1 * p1;
+      sb_i += w0 * p1;
+      sb_i -= w1 * p0;
       T z0 = q.yr + a_r * u0 - a_i * u1 - b_r * w0 + b_i * w1;
       T z1 = q.yi + a_r * u1 + a_i * u0 - b_r * w1 - b_i * w0;
       if (2 * mb + 2 == j) {  // this column also feeds the middle one
         const T c0 = ad[m][0], c1 = ad[m][1], d0 = up[m][0], d1 = up[m][1];
-        sa_r += d0 * p0 + d1 * p1;
-        sa_i += d1 * p0 - d0 * p1;
-        sb_r -= c0 * p0 + c1 * p1;
-        sb_i -= c1 * p0 - c0 * p1;
-        z0 += b_r * c0 + b_i * c1 + a_r * d0 + a_i * d1;
-        z1 += b_r * c1 - b_i * c0 + a_r * d1 - a_i * d0;
+        sa_r += d0 * p0;
+        sa_r += d1 * p1;
+        sa_i += d1 * p0;
+        sa_i -= d0 * p1;
+        sb_r -= c0 * p0;
+        sb_r -= c1 * p1;
+        sb_i -= c1 * p0;
+        sb_i += c0 * p1;
+        z0 = z0 + b_r * c0 + b_i * c1 + a_r * d0 + a_i * d1;
+        z1 = z1 + b_r * c1 - b_i * c0 + a_r * d1 - a_i * d0;
       }
       ad[mb][0] = z0;
       ad[mb][1] = z1;
@@ -1024,17 +1091,22 @@ struct emd_snap {
   double *eatom = nullptr;
   int cap_e = 0;
   snap_edot *edot = nullptr;  // energy dot product: U index and weight of each entry
-  // flat Y term stream (k_snap_yflat): codes (LDS byte offsets for FP32 and
-  // FP64 U_tot), key per slot, cg products, weights for the current
-  // coefficients, run slot per (chunk, thread), first run per entry
-  uint32_t *yf_code32 = nullptr, *yf_code64 = nullptr;
+  // slot stream of k_snap_yflat: LDS byte offsets, keys and cg products of
+  // its two products per slot, their weights for the current coefficients,
+  // run slot per (chunk, thread), first run per entry
+  yf_code *yf_codes = nullptr;
   unsigned short *yf_key = nullptr, *yf_meta = nullptr;
-  unsigned short *yf_centry = nullptr;  // entry of each (chunk, thread), 0 if none
+  // product stream of k_snap_s_flat (twojmax <= 8): LDS byte offsets, key and
+  // cg product of each, entry of each (chunk, thread) (0 if none)
+  uint32_t *sf_code = nullptr;
+  unsigned short *sf_key = nullptr, *sf_centry = nullptr;
+  double *sf_cgw = nullptr;
+  int sf_nch = 0;
   unsigned short *yf_keytid = nullptr;  // adjoint triple id of each key
   double *s_part = nullptr;  // the beta adjoint's per-block key sums (k_snap_s_flat)
   size_t cap_spart = 0;
   // emd_snap_static_geometry: the compaction, neighbour parameters and U_tot
-  // of the last force or adjoint call (twojmax <= 8) are reused while the
+  // of the last force or adjoint call are reused while the
   // caller keeps positions and list fixed: their precision (-1: none), atom
   // count, and the position and list arrays they came from
   int geom_static = 0, geom_prec = -1, geom_n = -1;
@@ -1043,7 +1115,7 @@ struct emd_snap {
   double *yf_cgw = nullptr, *yf_w64 = nullptr, *yf_kcoef = nullptr;
   float *yf_w32 = nullptr;
   int *yf_rstart = nullptr;
-  int yf_steps = 0, yf_nch = 0, yf_nruns = 0;
+  int yf_nslots = 0, yf_nch = 0;
   std::vector<std::tuple<int, int, int>> yf_keys;  // (a, b, J), sorted
   // adjoint: every (a,b,J) triple grouped by J, with its id
   std::map<std::tuple<int, int, int>, int> tid;
@@ -1148,17 +1220,146 @@ struct yf_matching {
 };
 
 template <class L>
-static void yf_assign_copies(const std::vector<int> &u1, const std::vector<int> &u2, int steps,
-                             int nu, std::vector<uint32_t> &code) {
-  std::vector<int> cp1(u1.size(), 0), cp2(u2.size(), 0), index(nu, -1);
+static std::vector<unsigned short> yf_offsets(const std::vector<int> &u, int nu) {
+  std::vector<int> cp(u.size(), 0), index(nu, -1);
+  std::vector<unsigned short> off(u.size());
   yf_matching<L> m;
-  for (size_t g0 = 0; g0 < (size_t)steps * YF_THREADS; g0 += L::GROUP) {
-    m.assign(&u1[g0], &cp1[g0], index);
-    m.assign(&u2[g0], &cp2[g0], index);
+  for (size_t g0 = 0; g0 < u.size(); g0 += L::GROUP) m.assign(&u[g0], &cp[g0], index);
+  for (size_t k = 0; k < u.size(); k++) off[k] = (unsigned short)((L::base(cp[k]) + u[k]) * 8);
+  return off;
+}
+static std::vector<unsigned short> yf_offsets(const std::vector<int> &u, const snap_dev_tables &t) {
+  // (the same word offsets serve FP32 and FP64, there into the real array)
+  return t.twojmax <= SNAP_MAXJ ? yf_offsets<yf_layout<float, SNAP_MAXJ>>(u, t.nu)
+                                : yf_offsets<yf_layout<float, SNAP_JBIG>>(u, t.nu);
+}
+
+struct yf_term {
+  int i1, i2, key;
+  double cgw;
+};
+struct yf_slot {
+  int c, x, y;        // U_c (w_x U_x + w_y U_y)
+  int kx, ky;
+  double cx, cy;
+};
+
+// The products of one entry as slots of two that share a U entry: the
+// products are the edges of a graph over the U entries, and a connected graph
+// splits into pairs of adjacent edges but for one edge when their number is
+// odd (depth first: a vertex pairs the edges its subtree left to it, and takes
+// the edge to its parent for an odd one).
+struct yf_pairs {
+  const std::vector<yf_term> &t;
+  std::vector<yf_slot> &out;
+  std::vector<std::vector<int>> adj;
+  std::vector<char> used, seen;
+  yf_pairs(const std::vector<yf_term> &terms, int nu, std::vector<yf_slot> &slots)
+      : t(terms), out(slots), adj(nu), used(terms.size(), 0), seen(nu, 0) {
+    for (size_t e = 0; e < t.size(); e++) {
+      adj[t[e].i1].push_back((int)e);
+      if (t[e].i2 != t[e].i1) adj[t[e].i2].push_back((int)e);
+    }
+    for (const yf_term &q : t)
+      if (!seen[q.i1]) visit(q.i1, -1);
   }
-  for (size_t k = 0; k < u1.size(); k++)
-    code[k] = (uint32_t)((L::base(cp1[k]) + u1[k]) * 8) |
-              ((uint32_t)((L::base(cp2[k]) + u2[k]) * 8) << 16);
+  int other(int e, int v) const { return t[e].i1 == v ? t[e].i2 : t[e].i1; }
+  void emit(int v, int e1, int e2) {
+    yf_slot s{v, other(e1, v), 0, t[e1].key, 0, t[e1].cgw, 0.0};
+    if (e2 >= 0) {
+      s.y = other(e2, v);
+      s.ky = t[e2].key;
+      s.cy = t[e2].cgw;
+    } else {
+      s.y = s.x;  // weight 0
+      s.ky = s.kx;
+    }
+    out.push_back(s);
+  }
+  // true if v took the edge to its parent
+  bool visit(int v, int parent) {
+    seen[v] = 1;
+    int left = -1;
+    for (int e : adj[v]) {
+      if (used[e]) continue;
+      used[e] = 1;
+      const int w = other(e, v);
+      if (w != v && !seen[w] && visit(w, e)) continue;
+      if (left < 0) {
+        left = e;
+      } else {
+        emit(v, left, e);
+        left = -1;
+      }
+    }
+    if (left < 0) return false;
+    emit(v, left, parent);
+    return parent >= 0;
+  }
+};
+
+// Entries' lists of the given lengths in chunks of `chunk`, in entry order:
+// (entry, first element) of each, `threads` threads taking P each
+struct yf_chunks {
+  std::vector<std::pair<int, int>> at;
+  int P = 0;
+  yf_chunks(const std::vector<int> &len, int chunk, int threads) {
+    for (int e = 0; e < (int)len.size(); e++)
+      for (int f = 0; f < len[e]; f += chunk) at.push_back(std::make_pair(e, f));
+    P = ((int)at.size() + threads - 1) / threads;
+  }
+};
+
+template <class V>
+static emd_status yf_upload(emd_ctx *ctx, V **dst, const std::vector<V> &v) {
+  EMD_HIP(ctx, hipMalloc(dst, std::max<size_t>(1, v.size()) * sizeof(V)));
+  if (!v.empty()) EMD_HIP(ctx, hipMemcpy(*dst, v.data(), v.size() * sizeof(V), hipMemcpyHostToDevice));
+  return EMD_OK;
+}
+
+// the stream of k_snap_s_flat (see there)
+static emd_status snap_build_sflat(emd_ctx *ctx, emd_snap *sn,
+                                   const std::vector<std::vector<yf_term>> &eterms) {
+  const snap_dev_tables &t = sn->t;
+  std::vector<int> len(t.ny);
+  for (int e = 0; e < t.ny; e++) len[e] = (int)eterms[e].size();
+  const yf_chunks ch(len, SF_CHUNK, SF_THREADS);
+  const int nchunks = (int)ch.at.size(), P = ch.P;
+  const size_t nslots = (size_t)P * SF_CHUNK * SF_THREADS;
+  std::vector<int> u1(nslots, 0), u2(nslots, 0);
+  std::vector<unsigned short> key(nslots, 0), centry((size_t)P * SF_THREADS, 0);
+  std::vector<double> cgw(nslots, 0.0);
+  // A chunk's terms all belong to one entry, so their order within the
+  // chunk is free (it changes rounding only): by key, padding last, so that
+  // runs of one key are summed before the atomic add (1.8 runs per chunk at
+  // twojmax 8).  LDS bank conflicts are left to the copy assignment (offline:
+  // 1.08 cycles per read against 1.04 with a bank-greedy order).
+  for (int g = 0; g < nchunks; g++) {
+    const int e = ch.at[g].first, th = g / P, c = g % P;
+    const int f = ch.at[g].second, m = std::min(SF_CHUNK, len[e] - f);
+    std::vector<yf_term> pool(eterms[e].begin() + f, eterms[e].begin() + f + m);
+    std::stable_sort(pool.begin(), pool.end(), [](const yf_term &x, const yf_term &y) {
+      if (x.key != y.key) return x.key < y.key;
+      return x.i1 != y.i1 ? x.i1 < y.i1 : x.i2 < y.i2;
+    });
+    for (int k = 0; k < m; k++) {
+      const size_t slot = ((size_t)c * SF_CHUNK + k) * SF_THREADS + th;
+      u1[slot] = pool[k].i1;
+      u2[slot] = pool[k].i2;
+      key[slot] = (unsigned short)pool[k].key;
+      cgw[slot] = pool[k].cgw;
+    }
+    centry[(size_t)c * SF_THREADS + th] = (unsigned short)e;
+  }
+  const std::vector<unsigned short> o1 = yf_offsets(u1, t), o2 = yf_offsets(u2, t);
+  std::vector<uint32_t> code(nslots);
+  for (size_t k = 0; k < nslots; k++) code[k] = o1[k] | (uint32_t)o2[k] << 16;
+  sn->sf_nch = P;
+  EMD_TRY(yf_upload(ctx, &sn->sf_code, code));
+  EMD_TRY(yf_upload(ctx, &sn->sf_key, key));
+  EMD_TRY(yf_upload(ctx, &sn->sf_cgw, cgw));
+  EMD_TRY(yf_upload(ctx, &sn->sf_centry, centry));
+  return EMD_OK;
 }
 
 static emd_status snap_build_yflat(emd_ctx *ctx, emd_snap *sn) {
@@ -1172,15 +1373,12 @@ static emd_status snap_build_yflat(emd_ctx *ctx, emd_snap *sn) {
     keyset.insert(std::make_tuple(std::max(j1, j), std::min(j1, j), j2));
   }
   sn->yf_keys.assign(keyset.begin(), keyset.end());
-  struct term {
-    int i1, i2, key;
-    double cgw;
-  };
-  std::vector<std::vector<term>> eterms(t.ny);
+  std::vector<std::vector<yf_term>> eterms(t.ny);
   std::vector<int> seen;
   for (int J = 0; J <= t.twojmax; J++)
     for (int mb = 0; 2 * mb <= J; mb++)
       for (int ma = 0; ma <= J; ma++) {
+        if (2 * mb == J && ma > mb) continue;  // half-plane weight 0
         const int e = t.ystart[J] + mb * (J + 1) + ma;
         for (size_t q = 0; q < sn->yf_keys.size(); q++) {
           int a, b, JJ;
@@ -1202,8 +1400,7 @@ static emd_status snap_build_yflat(emd_ctx *ctx, emd_snap *sn) {
               const double cw = cma * sn->cg_h[cgoff + mb1 * (b + 1) + mb2];
               if (cw == 0.0) continue;
               int i1 = t.ustart[a] + ma1 * (a + 1) + mb1, i2 = t.ustart[b] + ma2 * (b + 1) + mb2;
-              // a == b: (i1, i2) and (i2, i1) are the same product (39 610 ->
-              // 32 687 terms at twojmax 8, 427 703 -> 373 959 at 12)
+              // a == b: (i1, i2) and (i2, i1) are the same product
               if (a == b) {
                 if (i1 < i2) std::swap(i1, i2);
                 int &at = seen[(size_t)(i1 - t.ustart[a]) * (a + 1) * (a + 1) + (i2 - t.ustart[a])];
@@ -1213,120 +1410,75 @@ static emd_status snap_build_yflat(emd_ctx *ctx, emd_snap *sn) {
                 }
                 at = (int)eterms[e].size();
               }
-              eterms[e].push_back(term{i1, i2, (int)q, cw});
+              eterms[e].push_back(yf_term{i1, i2, (int)q, cw});
             }
           }
         }
       }
-  // chunks of YF_CHUNK terms in entry order, an entry's last chunk padded
-  // with zero-weight terms (U offsets 0, weight 0); thread th takes chunks
-  // [th P, (th+1) P)
-  std::vector<std::pair<int, int>> crange;  // (entry, first term)
-  for (int e = 0; e < t.ny; e++)
-    for (int f = 0; f < (int)eterms[e].size(); f += YF_CHUNK) crange.push_back(std::make_pair(e, f));
-  const int nchunks = (int)crange.size();
-  const int P = (nchunks + YF_THREADS - 1) / YF_THREADS;
-  // runs: a thread's consecutive chunks of one entry; run slots numbered
-  // entry by entry, in thread order within an entry (= term order)
-  std::vector<std::vector<std::pair<int, int>>> eruns(t.ny);  // (thread, local chunk)
-  for (int th = 0; th < YF_THREADS; th++)
-    for (int c = 0; c < P; c++) {
-      const int g = th * P + c;
-      if (g >= nchunks) break;
-      const int e = crange[g].first;
-      const bool ends = c == P - 1 || g + 1 >= nchunks || crange[g + 1].first != e;
-      if (ends) eruns[e].push_back(std::make_pair(th, c));
-    }
-  std::vector<unsigned short> meta((size_t)P * YF_THREADS, YF_NO_RUN);
-  std::vector<int> rstart(t.ny + 1, 0);
-  int nruns = 0;
+  // ---- the slot stream of k_snap_yflat
+  std::vector<std::vector<yf_slot>> eslots(t.ny);
+  std::vector<int> len(t.ny);
   for (int e = 0; e < t.ny; e++) {
-    rstart[e] = nruns;
-    for (const auto &r : eruns[e]) meta[(size_t)r.second * YF_THREADS + r.first] = (unsigned short)nruns++;
+    yf_pairs(eterms[e], t.nu, eslots[e]);
+    len[e] = (int)eslots[e].size();
   }
-  rstart[t.ny] = nruns;
   const bool small = t.twojmax <= SNAP_MAXJ;
+  const int nt = small ? yf_threads<SNAP_MAXJ>() : yf_threads<SNAP_JBIG>();
+  const yf_chunks ch(len, YF_CHUNK, nt);
+  const int nchunks = (int)ch.at.size(), P = ch.P;
+  // runs: a thread's consecutive chunks of one entry; run slots numbered
+  // entry by entry, in thread order within an entry (= slot order)
+  std::vector<unsigned short> meta((size_t)P * nt, YF_NO_RUN);
+  std::vector<int> rstart(t.ny + 1, 0);
+  int nruns = 0, done = 0;
+  for (int g = 0; g < nchunks; g++) {
+    const int e = ch.at[g].first;
+    while (done <= e) rstart[done++] = nruns;
+    if (g % P == P - 1 || g + 1 == nchunks || ch.at[g + 1].first != e)
+      meta[(size_t)(g % P) * nt + g / P] = (unsigned short)nruns++;
+  }
+  while (done <= t.ny) rstart[done++] = nruns;
   if (nruns > (small ? yf_maxruns<SNAP_MAXJ>() : yf_maxruns<SNAP_JBIG>()) ||
       t.nu > (small ? snap_nu(SNAP_MAXJ) : snap_nu(SNAP_JBIG)))
     return emd_set_error(ctx, EMD_ERR_ARG, "emd_snap_create: Y stream too large");
-  const int steps = P * YF_CHUNK;
-  const size_t nslots = (size_t)steps * YF_THREADS;
-  std::vector<uint32_t> code32(nslots, 0u), code64(nslots, 0u);
-  std::vector<int> u1(nslots, 0), u2(nslots, 0);
-  std::vector<unsigned short> key(nslots, 0);
-  std::vector<double> cgw(nslots, 0.0);
-  // A chunk's terms all belong to one entry, so their order within the
-  // chunk is free (it changes rounding only): by key, padding last, so that
-  // the adjoint's S kernel sums runs of one key before its atomic add (1.8
-  // runs per chunk at twojmax 8).  LDS bank conflicts are left to the copy
-  // assignment below (offline: 1.08 cycles per read against 1.04 with a
-  // bank-greedy order).
-  const term zero_term{0, 0, 0, 0.0};
-  for (int th = 0; th < YF_THREADS; th++)
-    for (int c = 0; c < P; c++) {
-      const int g = th * P + c;
-      std::vector<term> pool;
-      for (int k = 0; k < YF_CHUNK; k++) {
-        if (g < nchunks && crange[g].second + k < (int)eterms[crange[g].first].size())
-          pool.push_back(eterms[crange[g].first][crange[g].second + k]);
-        else
-          pool.push_back(zero_term);
-      }
-      std::stable_sort(pool.begin(), pool.end(), [](const term &x, const term &y) {
-        if ((x.cgw == 0.0) != (y.cgw == 0.0)) return y.cgw == 0.0;
-        if (x.key != y.key) return x.key < y.key;
-        return x.i1 != y.i1 ? x.i1 < y.i1 : x.i2 < y.i2;
-      });
-      for (int k = 0; k < YF_CHUNK; k++) {
-        const size_t slot = ((size_t)c * YF_CHUNK + k) * YF_THREADS + th;
-        u1[slot] = pool[k].i1;
-        u2[slot] = pool[k].i2;
-        key[slot] = (unsigned short)pool[k].key;
-        cgw[slot] = pool[k].cgw;
-      }
+  const size_t nslots = (size_t)P * YF_CHUNK * nt;
+  std::vector<int> uc(nslots, 0), ux(nslots, 0), uy(nslots, 0);
+  std::vector<unsigned short> key(2 * nslots, 0);
+  std::vector<double> cgw(2 * nslots, 0.0);
+  for (int g = 0; g < nchunks; g++) {
+    const std::vector<yf_slot> &es = eslots[ch.at[g].first];
+    for (int k = 0; k < YF_CHUNK && ch.at[g].second + k < (int)es.size(); k++) {
+      const yf_slot &q = es[ch.at[g].second + k];
+      const size_t slot = yf_place(P, g % P, k, g / P);
+      uc[slot] = q.c;
+      ux[slot] = q.x;
+      uy[slot] = q.y;
+      key[2 * slot] = (unsigned short)q.kx;
+      key[2 * slot + 1] = (unsigned short)q.ky;
+      cgw[2 * slot] = q.cx;
+      cgw[2 * slot + 1] = q.cy;
     }
-  if (small) {
-    yf_assign_copies<yf_layout<float, SNAP_MAXJ>>(u1, u2, steps, t.nu, code32);
-    code64 = code32;  // the same word offsets (FP64: into the real array)
-  } else {
-    yf_assign_copies<yf_layout<float, SNAP_JBIG>>(u1, u2, steps, t.nu, code32);
-    code64 = code32;
   }
-  sn->yf_steps = steps;
-  sn->yf_nch = P;
-  sn->yf_nruns = nruns;
-  EMD_HIP(ctx, hipMalloc(&sn->yf_code32, nslots * sizeof(uint32_t)));
-  EMD_HIP(ctx, hipMalloc(&sn->yf_code64, nslots * sizeof(uint32_t)));
   {
-    std::vector<unsigned short> centry((size_t)P * YF_THREADS, 0);
-    for (int th = 0; th < YF_THREADS; th++)
-      for (int c = 0; c < P; c++) {
-        const int g = th * P + c;
-        if (g < nchunks) centry[(size_t)c * YF_THREADS + th] = (unsigned short)crange[g].first;
-      }
-    std::vector<unsigned short> keytid(std::max<size_t>(1, sn->yf_keys.size()), 0);
-    for (size_t q = 0; q < sn->yf_keys.size(); q++) keytid[q] = (unsigned short)sn->tid.at(sn->yf_keys[q]);
-    EMD_HIP(ctx, hipMalloc(&sn->yf_centry, centry.size() * sizeof(unsigned short)));
-    EMD_HIP(ctx, hipMalloc(&sn->yf_keytid, keytid.size() * sizeof(unsigned short)));
-    EMD_HIP(ctx, hipMemcpy(sn->yf_centry, centry.data(), centry.size() * sizeof(unsigned short),
-                           hipMemcpyHostToDevice));
-    EMD_HIP(ctx, hipMemcpy(sn->yf_keytid, keytid.data(), keytid.size() * sizeof(unsigned short),
-                           hipMemcpyHostToDevice));
+    const std::vector<unsigned short> oc = yf_offsets(uc, t), ox = yf_offsets(ux, t),
+                                      oy = yf_offsets(uy, t);
+    std::vector<yf_code> code(nslots);
+    for (size_t k = 0; k < nslots; k++) code[yf_place2(k)] = yf_code{oc[k], ox[k], oy[k], 0};
+    EMD_TRY(yf_upload(ctx, &sn->yf_codes, code));
   }
-  EMD_HIP(ctx, hipMalloc(&sn->yf_key, nslots * sizeof(unsigned short)));
-  EMD_HIP(ctx, hipMalloc(&sn->yf_meta, meta.size() * sizeof(unsigned short)));
-  EMD_HIP(ctx, hipMalloc(&sn->yf_cgw, nslots * sizeof(double)));
-  EMD_HIP(ctx, hipMalloc(&sn->yf_w64, nslots * sizeof(double)));
-  EMD_HIP(ctx, hipMalloc(&sn->yf_w32, nslots * sizeof(float)));
-  EMD_HIP(ctx, hipMalloc(&sn->yf_rstart, (t.ny + 1) * sizeof(int)));
+  sn->yf_nslots = (int)nslots;
+  sn->yf_nch = P;
+  std::vector<unsigned short> keytid(sn->yf_keys.size(), 0);
+  for (size_t q = 0; q < sn->yf_keys.size(); q++) keytid[q] = (unsigned short)sn->tid.at(sn->yf_keys[q]);
+  EMD_TRY(yf_upload(ctx, &sn->yf_keytid, keytid));
+  EMD_TRY(yf_upload(ctx, &sn->yf_key, key));
+  EMD_TRY(yf_upload(ctx, &sn->yf_meta, meta));
+  EMD_TRY(yf_upload(ctx, &sn->yf_cgw, cgw));
+  EMD_TRY(yf_upload(ctx, &sn->yf_rstart, rstart));
+  EMD_HIP(ctx, hipMalloc(&sn->yf_w64, std::max<size_t>(1, 2 * nslots) * sizeof(double)));
+  EMD_HIP(ctx, hipMalloc(&sn->yf_w32, std::max<size_t>(1, 2 * nslots) * sizeof(float)));
   EMD_HIP(ctx, hipMalloc(&sn->yf_kcoef, std::max<size_t>(1, sn->yf_keys.size()) * sizeof(double)));
-  EMD_HIP(ctx, hipMemcpy(sn->yf_code32, code32.data(), nslots * sizeof(uint32_t), hipMemcpyHostToDevice));
-  EMD_HIP(ctx, hipMemcpy(sn->yf_code64, code64.data(), nslots * sizeof(uint32_t), hipMemcpyHostToDevice));
-  EMD_HIP(ctx, hipMemcpy(sn->yf_key, key.data(), nslots * sizeof(unsigned short), hipMemcpyHostToDevice));
-  EMD_HIP(ctx, hipMemcpy(sn->yf_meta, meta.data(), meta.size() * sizeof(unsigned short), hipMemcpyHostToDevice));
-  EMD_HIP(ctx, hipMemcpy(sn->yf_cgw, cgw.data(), nslots * sizeof(double), hipMemcpyHostToDevice));
-  EMD_HIP(ctx, hipMemcpy(sn->yf_rstart, rstart.data(), (t.ny + 1) * sizeof(int), hipMemcpyHostToDevice));
-  return EMD_OK;
+  return small ? snap_build_sflat(ctx, sn, eterms) : EMD_OK;
 }
 
 // the index map of the register layout (see rg_map)
@@ -1420,7 +1572,7 @@ static emd_status snap_upload_coeff(emd_ctx *ctx, emd_snap *sn) {
   if (!et.empty())
     EMD_HIP(ctx, hipMemcpyAsync(sn->etab, et.data(), et.size() * sizeof(etab_entry),
                                 hipMemcpyHostToDevice, ctx->stream));
-  if (sn->yf_code32) {
+  if (sn->yf_codes) {
     std::vector<double> &kc = sn->h_kcoef;
     kc.assign(sn->yf_keys.size(), 0.0);
     for (size_t q = 0; q < kc.size(); q++) {
@@ -1430,9 +1582,9 @@ static emd_status snap_upload_coeff(emd_ctx *ctx, emd_snap *sn) {
     if (!kc.empty())
       EMD_HIP(ctx, hipMemcpyAsync(sn->yf_kcoef, kc.data(), kc.size() * sizeof(double),
                                   hipMemcpyHostToDevice, ctx->stream));
-    const int nslots = sn->yf_steps * YF_THREADS;
+    const int nslots = sn->yf_nslots;
     if (nslots > 0)
-      EMD_LAUNCH(ctx, "snap_coeff", k_yf_weights, emd_blocks(nslots, 256), 256, 0, nslots,
+      EMD_LAUNCH(ctx, "snap_coeff", k_yf_weights, emd_blocks(2 * nslots, 256), 256, 0, nslots,
                  sn->yf_key, sn->yf_cgw, sn->yf_kcoef, sn->yf_w64, sn->yf_w32);
   }
   return EMD_OK;
@@ -1550,8 +1702,8 @@ extern "C" emd_status emd_snap_destroy(emd_ctx *ctx, emd_snap *sn) {
                   sn->stab, sn->w_r, sn->edot,
                   sn->w_i, sn->sbuf,
                   sn->u_r, sn->u_i, sn->y_r, sn->y_i, sn->eatom,
-                  sn->yf_code32, sn->yf_code64, sn->yf_key, sn->yf_meta, sn->yf_cgw,
-                  sn->yf_centry, sn->yf_keytid, sn->s_part,
+                  sn->yf_codes, sn->yf_key, sn->yf_meta, sn->yf_cgw, sn->sf_code, sn->sf_key,
+                  sn->sf_cgw, sn->sf_centry, sn->yf_keytid, sn->s_part,
                   sn->yf_w64, sn->yf_w32, sn->yf_rstart, sn->yf_kcoef};
   for (void *q : ptrs)
     if (q) hipFree(q);
@@ -1657,19 +1809,36 @@ static emd_status launch_ui(emd_ctx *ctx, emd_snap *sn, int n) {
 template <class T>
 static emd_status snap_y(emd_ctx *ctx, emd_snap *sn, int n) {
   T *ur = (T *)sn->u_r, *ui = (T *)sn->u_i, *yr = (T *)sn->y_r, *yi = (T *)sn->y_i;
-  const T *w = std::is_same<T, float>::value ? (const T *)sn->yf_w32 : (const T *)sn->yf_w64;
-  const uint32_t *code = std::is_same<T, float>::value ? sn->yf_code32 : sn->yf_code64;
-  // two atoms per block share each term's code and weight load (SNAP-2k:
-  // 26.8 / 47.2 us mixed / FP64, against 31.5 / 60.9 with one atom and 28.2 /
-  // 55.9 with three; 1024 atoms at twojmax 12: 109 / 218 us, against 199
-  // mixed with one atom and a single U_tot copy)
-  if (sn->t.twojmax <= SNAP_MAXJ)
-    EMD_LAUNCH(ctx, "snap_y", (k_snap_yflat<T, SNAP_MAXJ, 2>), (n + 1) / 2, YF_THREADS, 0, sn->t.nu,
-               sn->t.ny, sn->yf_nch, code, w, sn->yf_meta, sn->yf_rstart, n, ur, ui, yr, yi);
-  else
-    EMD_LAUNCH(ctx, "snap_y", (k_snap_yflat<T, SNAP_JBIG, 2>), (n + 1) / 2, YF_THREADS, 0, sn->t.nu,
-               sn->t.ny, sn->yf_nch, code, w, sn->yf_meta, sn->yf_rstart, n, ur, ui, yr, yi);
-  return EMD_OK;
+  const cpair<T> *w = std::is_same<T, float>::value ? (const cpair<T> *)sn->yf_w32
+                                                    : (const cpair<T> *)sn->yf_w64;
+  // Atoms per block: more of them share each code and weight load, but take
+  // LDS from other blocks, and leave CUs without a block in small systems.
+  // us at twojmax 8 with 1 / 2 / 3 atoms: FP64 250 atoms 10.7 / 12.4 / 14.8,
+  // 432: 15.9 / 13.5 / 15.7, 16 000: 348 / 223 / 272; mixed 128 atoms 8.0 / 9.2 /
+  // 10.5, 1024: 20.3 / 14.5 / 15.3, 2000: 34 / 22.6 / 20.6, 16 000: 214 / 128 /
+  // 107: one while every atom can have a CU, in FP32 three once there are
+  // six per CU.  Twojmax 12 mixed, 2 (512 threads) / 4: 54 atoms 37 / 54, 1024:
+  // 79 / 71; FP64 with 512 / 1024 threads, two atoms, 1024: 162 / 151.
+  auto launch = [&](auto jc, auto ac) -> emd_status {
+    constexpr int J = jc, AT = ac;
+    EMD_LAUNCH(ctx, "snap_y", (k_snap_yflat<T, J, AT>), (n + AT - 1) / AT, yf_threads<J>(), 0,
+               sn->t.nu, sn->t.ny, sn->yf_nch, sn->yf_codes, w, sn->yf_meta, sn->yf_rstart, n, ur,
+               ui, yr, yi);
+    return EMD_OK;
+  };
+  using J8 = std::integral_constant<int, SNAP_MAXJ>;
+  using J12 = std::integral_constant<int, SNAP_JBIG>;
+  using A1 = std::integral_constant<int, 1>;
+  using A2 = std::integral_constant<int, 2>;
+  constexpr bool f32 = std::is_same<T, float>::value;
+  if (sn->t.twojmax > SNAP_MAXJ) {
+    if (n <= 256) return launch(J12{}, A1{});
+    if (f32 && n > 512) return launch(J12{}, std::integral_constant<int, f32 ? 4 : 2>{});
+    return launch(J12{}, A2{});
+  }
+  if (n <= 256) return launch(J8{}, A1{});
+  if (f32 && n > 1536) return launch(J8{}, std::integral_constant<int, f32 ? 3 : 2>{});
+  return launch(J8{}, A2{});
 }
 
 // F_ij for every (atom, neighbour)
@@ -1837,27 +2006,39 @@ k_snap_w_rg(snap_dev_tables t, const rg_map *__restrict__ rgm, const int *__rest
     rg_layers<1, J>([&](auto jc) {
       constexpr int j = jc;
       if (j > t.twojmax) return;
-      // the terms of V_{j-1}, then X_{j-1}'s own recursion
-      T e[R::COLS][2];
-      T q[2];
+      // X first: it needs V_{j-1}
+      T q[R::COLS][4];
 #pragma unroll
       for (int mb = 0; 2 * mb < j; mb++) {
-        const T p0 = c[mb][0], p1 = c[mb][1];
-        q[0] = lane_below(p0);
-        q[1] = lane_below(p1);
-        e[mb][0] = da_r * p0 + da_i * p1 - db_r * q[0] - db_i * q[1];
-        e[mb][1] = da_r * p1 - da_i * p0 - db_r * q[1] + db_i * q[0];
-        if (2 * mb + 2 == j) {
-          e[mb + 1][0] = db_r * p0 - db_i * p1 + da_r * q[0] - da_i * q[1];
-          e[mb + 1][1] = db_r * p1 + db_i * p0 + da_r * q[1] + da_i * q[0];
+        q[mb][0] = lane_below(c[mb][0]);
+        q[mb][1] = lane_below(c[mb][1]);
+        q[mb][2] = lane_below(d[mb][0]);
+        q[mb][3] = lane_below(d[mb][1]);
+      }
+#pragma unroll
+      for (int mb = j / 2; mb >= 0; mb--) {
+        const bool mid = 2 * mb == j;
+        const int k = mid ? mb - 1 : mb;  // the middle column comes from the one beside it
+        const T p0 = c[k][0], p1 = c[k][1], x0 = d[k][0], x1 = d[k][1];
+        const T q0 = q[k][0], q1 = q[k][1], y0 = q[k][2], y1 = q[k][3];
+        if (mid) {
+          d[mb][0] = db_r * p0 - db_i * p1 + da_r * q0 - da_i * q1 + b_r * x0 - b_i * x1 +
+                     a_r * y0 - a_i * y1;
+          d[mb][1] = db_r * p1 + db_i * p0 + da_r * q1 + da_i * q0 + b_r * x1 + b_i * x0 +
+                     a_r * y1 + a_i * y0;
+          c[mb][0] = b_r * p0 - b_i * p1 + a_r * q0 - a_i * q1;
+          c[mb][1] = b_r * p1 + b_i * p0 + a_r * q1 + a_i * q0;
+        } else {
+          d[mb][0] = da_r * p0 + da_i * p1 - db_r * q0 - db_i * q1 + a_r * x0 + a_i * x1 -
+                     b_r * y0 - b_i * y1;
+          d[mb][1] = da_r * p1 - da_i * p0 - db_r * q1 + db_i * q0 + a_r * x1 - a_i * x0 -
+                     b_r * y1 + b_i * y0;
+          c[mb][0] = a_r * p0 + a_i * p1 - b_r * q0 - b_i * q1;
+          c[mb][1] = a_r * p1 - a_i * p0 - b_r * q1 + b_i * q0;
         }
       }
-      rg_layer<j>(a_r, a_i, b_r, b_i, d);
-      rg_layer<j>(a_r, a_i, b_r, b_i, c);
 #pragma unroll
       for (int mb = 0; mb <= j / 2; mb++) {
-        d[mb][0] += e[mb][0];
-        d[mb][1] += e[mb][1];
         acc[rg_slot0(j) + mb][0] += (TS)d[mb][0];
         acc[rg_slot0(j) + mb][1] += (TS)d[mb][1];
       }
@@ -1905,9 +2086,9 @@ k_snap_s(snap_dev_tables t, const double *__restrict__ cg, const stab_entry *__r
   for (int k = threadIdx.x; k < ntrip; k += blockDim.x) atomicAdd(&S[k], sS[k]);
 }
 
-// S_{abJ} from the Y kernel's term stream (twojmax <= 8): a term of entry
+// S_{abJ} from a stream of single products (twojmax <= 8): a term of entry
 // e and key (a, b, J) adds cgw * Re(conj(W_e) U_a U_b) to S of its key (the
-// double sum of k_snap_s, term by term).  The stream's codes address the
+// double sum of k_snap_s, term by term).  Its codes address the
 // same bank-shifted U_tot copies as k_snap_yflat; AT atoms per block share
 // each term's loads, W of the chunk's entry is read once per chunk, a run of
 // one key within a chunk is summed in a register and added to the block's
@@ -1915,7 +2096,7 @@ k_snap_s(snap_dev_tables t, const double *__restrict__ cg, const stab_entry *__r
 // part (k_snap_s_reduce adds the rows up: no global atomics on the few key
 // addresses, and a fixed order).
 template <class T, int J, int AT>
-__global__ void __launch_bounds__(YF_THREADS)
+__global__ void __launch_bounds__(SF_THREADS)
 k_snap_s_flat(int nu, int ny, int nch, const uint32_t *__restrict__ code,
               const unsigned short *__restrict__ key, const double *__restrict__ cgw,
               const unsigned short *__restrict__ centry, const unsigned short *__restrict__ keytid,
@@ -1935,7 +2116,7 @@ k_snap_s_flat(int nu, int ny, int nch, const uint32_t *__restrict__ code,
   for (int a = 0; a < AT; a++) {
     const int i = i0 + a < n ? i0 + a : i0;
     unsigned char *ub = sb + a * L::UBYTES;
-    for (int k = threadIdx.x; k < nu; k += YF_THREADS) {
+    for (int k = threadIdx.x; k < nu; k += SF_THREADS) {
       const T vr = utot_r[(size_t)i * nu + k], vi = utot_i[(size_t)i * nu + k];
 #pragma unroll
       for (int c = 0; c < L::NCOPY; c++) {
@@ -1948,15 +2129,15 @@ k_snap_s_flat(int nu, int ny, int nch, const uint32_t *__restrict__ code,
       }
     }
     // the second atom of an odd-sized last block adds nothing
-    for (int e = threadIdx.x; e < ny; e += YF_THREADS) {
+    for (int e = threadIdx.x; e < ny; e += SF_THREADS) {
       s_w[a][0][e] = i0 + a < n ? w_r[(size_t)i * ny + e] : 0.0;
       s_w[a][1][e] = i0 + a < n ? w_i[(size_t)i * ny + e] : 0.0;
     }
   }
-  for (int k = threadIdx.x; k < nkeys; k += YF_THREADS) s_S[k] = 0.0;
+  for (int k = threadIdx.x; k < nkeys; k += SF_THREADS) s_S[k] = 0.0;
   __syncthreads();
   for (int c = 0; c < nch; c++) {
-    const int e = centry[(size_t)c * YF_THREADS + threadIdx.x];  // 0 for padding chunks
+    const int e = centry[(size_t)c * SF_THREADS + threadIdx.x];  // 0 for padding chunks
     double wr[AT], wi[AT];
 #pragma unroll
     for (int a = 0; a < AT; a++) {
@@ -1965,11 +2146,11 @@ k_snap_s_flat(int nu, int ny, int nch, const uint32_t *__restrict__ code,
     }
     // a chunk's terms come in runs of one key (padding, weight 0, last):
     // each run is summed here and added to S once
-    int run_key = key[(size_t)c * YF_CHUNK * YF_THREADS + threadIdx.x];
+    int run_key = key[(size_t)c * SF_CHUNK * SF_THREADS + threadIdx.x];
     double run = 0.0;
 #pragma unroll 4
-    for (int k = 0; k < YF_CHUNK; k++) {
-      const size_t slot = ((size_t)c * YF_CHUNK + k) * YF_THREADS + threadIdx.x;
+    for (int k = 0; k < SF_CHUNK; k++) {
+      const size_t slot = ((size_t)c * SF_CHUNK + k) * SF_THREADS + threadIdx.x;
       const uint32_t cc = code[slot];
       const double cw = cgw[slot];
       const int kk = key[slot];
@@ -1982,16 +2163,7 @@ k_snap_s_flat(int nu, int ny, int nch, const uint32_t *__restrict__ code,
 #pragma unroll
       for (int a = 0; a < AT; a++) {
         const unsigned char *ub = sb + a * L::UBYTES;
-        cpair<T> u1, u2;
-        if (L::SOA) {
-          u1.r = *reinterpret_cast<const T *>(ub + (cc & 0xFFFFu));
-          u1.i = *reinterpret_cast<const T *>(ub + L::IMB + (cc & 0xFFFFu));
-          u2.r = *reinterpret_cast<const T *>(ub + (cc >> 16));
-          u2.i = *reinterpret_cast<const T *>(ub + L::IMB + (cc >> 16));
-        } else {
-          u1 = *reinterpret_cast<const cpair<T> *>(ub + (cc & 0xFFFFu));
-          u2 = *reinterpret_cast<const cpair<T> *>(ub + (cc >> 16));
-        }
+        const cpair<T> u1 = yf_u<T, J>(ub, cc & 0xFFFFu), u2 = yf_u<T, J>(ub, cc >> 16);
         const T pr = u1.r * u2.r - u1.i * u2.i;
         const T pi = u1.r * u2.i + u1.i * u2.r;
         v += wr[a] * (double)pr + wi[a] * (double)pi;
@@ -2001,7 +2173,7 @@ k_snap_s_flat(int nu, int ny, int nch, const uint32_t *__restrict__ code,
     atomicAdd(&s_S[run_key], run);
   }
   __syncthreads();
-  for (int k = threadIdx.x; k < nkeys; k += YF_THREADS) part[(size_t)blockIdx.x * nkeys + k] = s_S[k];
+  for (int k = threadIdx.x; k < nkeys; k += SF_THREADS) part[(size_t)blockIdx.x * nkeys + k] = s_S[k];
 }
 
 // S of each key: its column of the per-block sums, added by one block in a
@@ -2083,12 +2255,11 @@ static emd_status snap_adjoint_impl(emd_ctx *ctx, const emd_system *s, const emd
                sn->w_r, sn->w_i);
   const int ntrip = (int)sn->tid.size();
   if (sn->t.twojmax <= SNAP_MAXJ) {
-    const uint32_t *code = std::is_same<T, float>::value ? sn->yf_code32 : sn->yf_code64;
     const int nb = (n + 1) / 2, nkeys = (int)sn->yf_keys.size();
     EMD_TRY(emd_ensure(ctx, (void **)&sn->s_part, &sn->cap_spart,
                        (size_t)nb * nkeys * sizeof(double)));
-    EMD_LAUNCH(ctx, "snap_adjoint_s", (k_snap_s_flat<T, SNAP_MAXJ, 2>), nb, YF_THREADS, 0,
-               sn->t.nu, sn->t.ny, sn->yf_nch, code, sn->yf_key, sn->yf_cgw, sn->yf_centry,
+    EMD_LAUNCH(ctx, "snap_adjoint_s", (k_snap_s_flat<T, SNAP_MAXJ, 2>), nb, SF_THREADS, 0,
+               sn->t.nu, sn->t.ny, sn->sf_nch, sn->sf_code, sn->sf_key, sn->sf_cgw, sn->sf_centry,
                sn->yf_keytid, nkeys, n, (const T *)sn->u_r, (const T *)sn->u_i, sn->w_r, sn->w_i,
                sn->s_part);
     if (nkeys > 0)
