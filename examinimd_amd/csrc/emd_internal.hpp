@@ -580,7 +580,10 @@ __device__ __forceinline__ void emd_halo_update_at(int g, double *__restrict__ x
 // fold_phases of a halo (emd_comm.hip); returns the number of ghosts
 long emd_fold_phases_of(const emd_system *s, const emd_halo *h, fold_phases &ph);
 constexpr int FOLD_ONE_THREADS = 1024;
-constexpr int FOLD_ONE_MAX = 16384;  // ghosts; above this the per-phase launches are faster
+// ghosts up to which one workgroup folds faster than a launch per dimension (8.3
+// us whatever the size): FP64 6667 ghosts 8.1 us, 9991 10.8; FP32 9991 5.9,
+// 16 237 8.5
+constexpr int FOLD_ONE_MAX_F64 = 7000, FOLD_ONE_MAX_F32 = 16000;
 
 // bin grid of a neighbour build: interior bins are the non-halo ones, one
 // block per interior bin; the 27-bin stencil order is dx, dy, dz = -1..1
