@@ -94,8 +94,8 @@ extern "C" emd_status emd_create(int device, emd_ctx **out) {
     const int k = ctx->lj_lanes[p];
     if (!(k == 0 || k == 1 || k == 2 || k == 4 || k == 8 || k == 16)) ctx->lj_lanes[p] = 0;
   }
-  // ghost force fold of a small halo (<= 16384 ghosts) in one launch (1) or
-  // one launch per phase (0)
+  // ghost force fold of a small halo (FOLD_ONE_MAX_*) in one launch (1) or
+  // one launch per dimension (0)
   if (const char *e = getenv("EMD_FOLD_ONE")) ctx->fold_one = atoi(e) != 0;
   // host waits for counts: poll an event (1) or hipStreamSynchronize (0)
   if (const char *e = getenv("EMD_SPIN_WAIT")) ctx->spin_wait = atoi(e) != 0;

@@ -26,7 +26,7 @@
 //                 mirror entries.  k_snap_ui_rg: U_tot alone
 //   k_snap_yflat  one block per atom: U_tot staged in LDS, Y (155 half-plane
 //                 entries at twojmax 8) from a host-built flat stream of
-//                 weighted U_a U_b products
+//                 weighted U_a U_b products, two to a slot
 //   k_snap_fij_rev  the force as the gradient of sum Re(conj(U) sfac w Y): U
 //                 forward in registers (same layout), adjoints backward, two
 //                 complex sums per lane, atomic scatter to f_i / f_j
@@ -80,15 +80,8 @@ struct snap_dev_tables {
   int nu, ny;                      // number of U entries / half-plane entries
   int ustart[SNAP_JBIG + 2];       // full layer offsets: ustart[j] + ma*(j+1) + mb
   int ystart[SNAP_JBIG + 2];       // half-plane offsets: ystart[J] + mb*(J+1) + ma
-  int yjstart[SNAP_JBIG + 2];      // (a,b) list for each J in ytab
-  int ny_terms;
   double rfac0, rmin0, rcut, wj, wself;
   int switchflag;
-};
-
-struct ytab_entry {
-  int a, b, cgoff, pad;
-  double coef;
 };
 
 struct etab_entry {
@@ -360,6 +353,7 @@ __device__ __forceinline__ void y_entry(const snap_dev_tables &t, int e, int &J,
 // read of every term the copy whose residue no other address of its
 // 32-lane group takes (a matching per group; with the shifts 0, 5, 11, 19
 // about 4 % of the groups keep one conflict).
+
 // threads per Y block (the stream is split this many ways): 512, at twojmax
 // above 8, where one block's LDS fills a CU, 1024
 template <int J>
@@ -589,10 +583,11 @@ __global__ void k_yf_weights(int nslots, const unsigned short *__restrict__ key,
 // per atom, to the sums over the neighbours or to Y.
 // FP64 (FP32) arithmetic bounds all three kernels (70 % of its issue rate in
 // the force kernel).  Against U with its factors, FP64, 16 000 atoms of 26
-// neighbours, twojmax 8: U_tot 174 -> 81 us, force 232 -> 148 us; W of 64 BCC
-// configurations of 128 to 1024 atoms 820 -> 275 us; mixed, 2000 atoms: 24.4 -> 15.9 and 28.6 -> 15.7 us.  Twojmax 12,
+// neighbours, twojmax 8: U_tot 174 -> 82 us, force 232 -> 144 us; W of 64 BCC
+// configurations of 128 to 1024 atoms 820 -> 262 us; mixed, 2000 atoms:
+// 24.4 -> 15.9 and 28.6 -> 14.9 us.  Twojmax 12,
 // 1024 atoms, against one neighbour per wavefront with the layers in LDS:
-// U_tot 140 -> 27 us (FP64), force 141 -> 29 us (mixed).
+// U_tot 140 -> 27 us (FP64), force 141 -> 28 us (mixed).
 // Groups of 9 lanes, seven per wavefront (one lane idle), for twojmax <= 8;
 // of 13 lanes, four per wavefront, up to 12.
 __host__ __device__ constexpr int rg_slot0(int j) { return j <= 0 ? 0 : j + (j - 1) * (j - 1) / 4; }
@@ -1065,12 +1060,10 @@ struct emd_snap {
   std::map<std::tuple<int, int, int>, int> cgoff;
   std::vector<double> cg_h;
   double *cg = nullptr;
-  ytab_entry *ytab = nullptr;
   etab_entry *etab = nullptr;
-  size_t ytab_cap = 0, etab_cap = 0;  // entries allocated (kept across coefficient updates)
+  size_t etab_cap = 0;  // entries allocated (kept across coefficient updates)
   // host sources of the last coefficient upload's stream-ordered copies
   // (kept until the next upload, which first waits for the stream)
-  std::vector<ytab_entry> h_ytab;
   std::vector<etab_entry> h_etab;
   std::vector<double> h_kcoef;
   int bzeroflag = 0;
@@ -1106,7 +1099,7 @@ struct emd_snap {
   double *s_part = nullptr;  // the beta adjoint's per-block key sums (k_snap_s_flat)
   size_t cap_spart = 0;
   // emd_snap_static_geometry: the compaction, neighbour parameters and U_tot
-  // of the last force or adjoint call are reused while the
+  // of the last force or adjoint call (twojmax <= 8) are reused while the
   // caller keeps positions and list fixed: their precision (-1: none), atom
   // count, and the position and list arrays they came from
   int geom_static = 0, geom_prec = -1, geom_n = -1;
@@ -1526,21 +1519,6 @@ static emd_status snap_upload_coeff(emd_ctx *ctx, emd_snap *sn) {
     coef[std::make_tuple(std::max(j1, j), std::min(j1, j), j2)] += 2.0 * b * (j + 1) / (j2 + 1.0);
   }
   EMD_HIP(ctx, hipStreamSynchronize(ctx->stream));  // the previous upload's copies are done
-  std::vector<ytab_entry> &yt = sn->h_ytab;
-  yt.clear();
-  for (int J = 0; J <= twojmax; J++) {
-    sn->t.yjstart[J] = (int)yt.size();
-    for (auto &kv : coef) {
-      int a, b, JJ;
-      std::tie(a, b, JJ) = kv.first;
-      if (JJ != J || kv.second == 0.0) continue;
-      ytab_entry e;
-      e.a = a; e.b = b; e.cgoff = sn->cgoff.at(kv.first); e.pad = 0; e.coef = kv.second;
-      yt.push_back(e);
-    }
-  }
-  sn->t.yjstart[twojmax + 1] = (int)yt.size();
-  sn->t.ny_terms = (int)yt.size();
   std::vector<etab_entry> &et = sn->h_etab;
   et.clear();
   for (int k = 0; k < nk; k++) {
@@ -1552,13 +1530,6 @@ static emd_status snap_upload_coeff(emd_ctx *ctx, emd_snap *sn) {
   }
   // the tables keep their allocation while they fit (coefficient updates
   // in a force-matching loop do not reallocate); copies are stream-ordered
-  if (yt.size() > sn->ytab_cap || !sn->ytab) {
-    EMD_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    if (sn->ytab) EMD_HIP(ctx, hipFree(sn->ytab));
-    sn->ytab = nullptr;
-    sn->ytab_cap = std::max<size_t>(1, yt.size());
-    EMD_HIP(ctx, hipMalloc(&sn->ytab, sn->ytab_cap * sizeof(ytab_entry)));
-  }
   if (et.size() > sn->etab_cap || !sn->etab) {
     EMD_HIP(ctx, hipStreamSynchronize(ctx->stream));
     if (sn->etab) EMD_HIP(ctx, hipFree(sn->etab));
@@ -1566,9 +1537,6 @@ static emd_status snap_upload_coeff(emd_ctx *ctx, emd_snap *sn) {
     sn->etab_cap = std::max<size_t>(1, et.size());
     EMD_HIP(ctx, hipMalloc(&sn->etab, sn->etab_cap * sizeof(etab_entry)));
   }
-  if (!yt.empty())
-    EMD_HIP(ctx, hipMemcpyAsync(sn->ytab, yt.data(), yt.size() * sizeof(ytab_entry),
-                                hipMemcpyHostToDevice, ctx->stream));
   if (!et.empty())
     EMD_HIP(ctx, hipMemcpyAsync(sn->etab, et.data(), et.size() * sizeof(etab_entry),
                                 hipMemcpyHostToDevice, ctx->stream));
@@ -1697,7 +1665,7 @@ extern "C" emd_status emd_snap_create(emd_ctx *ctx, const emd_snap_params *p, em
 extern "C" emd_status emd_snap_destroy(emd_ctx *ctx, emd_snap *sn) {
   if (!sn) return EMD_OK;
   if (ctx) hipStreamSynchronize(ctx->stream);
-  void *ptrs[] = {sn->cg, sn->ytab, sn->etab, sn->nin, sn->nj, sn->nr, sn->par, sn->fdv,
+  void *ptrs[] = {sn->cg, sn->etab, sn->nin, sn->nj, sn->nr, sn->par, sn->fdv,
                   sn->rg_map_d,
                   sn->stab, sn->w_r, sn->edot,
                   sn->w_i, sn->sbuf,
@@ -1862,7 +1830,7 @@ static emd_status launch_fij(emd_ctx *ctx, emd_snap *sn, int n, const T *yr, con
 // in precision prec those of this system and list?
 static bool snap_geom_cached(const emd_snap *sn, const emd_system *s, const emd_neigh *nl,
                              int prec) {
-  return sn->geom_static && sn->geom_prec == prec && sn->par_prec == prec &&
+  return sn->geom_static && sn->t.twojmax <= SNAP_MAXJ && sn->geom_prec == prec && sn->par_prec == prec &&
          sn->geom_n == s->n_local && sn->geom_x == s->x && sn->geom_ent == nl->entries;
 }
 

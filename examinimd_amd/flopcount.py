@@ -1,15 +1,18 @@
-"""Loop-bound FLOP count of this build's SNAP force (Y / adjoint form), per
-atom and step, for the algorithmic side of the SNAP roofline.
+"""FLOP count of the SNAP force in Y / adjoint form, per atom and step, for the
+algorithmic side of the SNAP roofline: a fixed measure of the work, counted
+with U and its square-root factors and one product per Y term.  The
+kernels of emd_snap.hip need fewer operations: they carry V = U / norm, in which
+the factors cancel, and add Y's products two at a time (about a third fewer
+in all), so rates from this count are rates of useful work, not of issue.
 
-Counts the floating-point adds and multiplies (an FMA counts 2; sqrt,
-division and transcendentals 1 each) executed by the four kernels of
-emd_snap.hip (twojmax <= 8) for an atom with n_in neighbours inside the
-cutoff:
+Counts floating-point adds and multiplies (an FMA counts 2; sqrt,
+division and transcendentals 1 each) for an atom with n_in neighbours inside
+the cutoff (twojmax <= 8):
 
-  P   k_snap_neigh : per in-cutoff neighbour the Cayley-Klein parameters,
+  P   parameters   : per in-cutoff neighbour the Cayley-Klein parameters,
                      their derivative factors, the switching function and
                      the r^-14 repulsion, once;
-  U   k_snap_ui_rg : per neighbour, for every half-plane entry of every layer
+  U   k_snap_neigh_ui: per neighbour, for every half-plane entry of every layer
                      j, the two recursion terms (SNA::compute_uarray,
                      sna_impl.hpp:663-695) and the sfac accumulation
                      (add_uarraytot, sna_impl.hpp:578-604);

@@ -295,11 +295,12 @@ emd_status emd_nve_final_initial(emd_ctx *ctx, emd_system *s, double dtf, double
  * comm->update_force() of step s if `fold` (src/examinimd.cpp:243,
  * comm_serial.h:200-213), final_integrate of s and initial_integrate of s+1
  * (src/examinimd.cpp:249 then 196), and comm->update_halo() of s+1 if
- * `update_halo` (src/examinimd.cpp:226, comm_serial.h:184-197).  Up to 16384
- * local atoms and 16384 ghosts the three run in one workgroup launch
- * separated by barriers; larger systems get the three separate launches.
+ * `update_halo` (src/examinimd.cpp:226, comm_serial.h:184-197).  Up to 3500
+ * local atoms and ghosts (5500 with the fold) the three run in one workgroup
+ * launch separated by barriers; larger systems get the separate launches.
  * Results are bitwise those of emd_comm_update_force, emd_nve_final_initial
- * and emd_comm_update_halo called in turn. */
+ * and emd_comm_update_halo called in turn (where the halo is deeper than half
+ * the box, the order of two of the fold's additions is free). */
 emd_status emd_nve_step_boundary(emd_ctx *ctx, emd_system *s, const emd_halo *h, int fold,
                                  int update_halo, double dtf, double dtv, int precision);
 
@@ -326,7 +327,7 @@ emd_status emd_snap_set_coeff(emd_ctx *ctx, emd_snap *sn, const double *coeff);
 /* No counterpart in the reference (it serves repeated force and beta-adjoint
  * evaluations of fixed configurations, e.g. force matching): with on != 0
  * the caller promises that positions, atom count and neighbour list stay as
- * they are; the compaction, neighbour parameters and U_tot
+ * they are; for twojmax <= 8 the compaction, neighbour parameters and U_tot
  * of the last force or adjoint call of a precision are then reused by later
  * calls of that precision (they depend on the geometry only, not on beta).
  * Calling it again (on or off) discards what was kept. */
