@@ -1885,10 +1885,10 @@ extern "C" emd_status emd_snap_energy(emd_ctx *ctx, const emd_system *s, const e
   const int n = s->n_local;
   *energy = 0.0;
   if (n <= 0) return EMD_OK;
-  if (!snap_geom_cached(sn, s, nl, EMD_FP64)) {
-    EMD_TRY(snap_neigh_ui(ctx, s, nl, sn, -1, EMD_FP64));
-    snap_geom_record(sn, s, nl, EMD_FP64);
-  }
+  // the static geometry serves force and adjoint calls: an energy is that of
+  // the positions as they are, and the compaction and U_tot are rewritten
+  sn->geom_prec = -1;
+  EMD_TRY(snap_neigh_ui(ctx, s, nl, sn, -1, EMD_FP64));
   EMD_TRY(snap_y<double>(ctx, sn, n));
   double *ea = eatom;
   if (!ea) {

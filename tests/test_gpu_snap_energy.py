@@ -62,3 +62,45 @@ def test_energy_equals_descriptor_sum(n, twojmax, bzero):
     assert (np.abs(e - want) <= 1e-11 * scale).all()
     assert abs(total.value - e.sum()) <= 1e-12 * np.abs(e).sum()
     pl.close()
+
+
+@pytest.mark.parametrize("twojmax", [4, 8])
+def test_energy_is_of_the_present_positions_with_static_geometry(twojmax):
+    """emd_snap_static_geometry keeps geometry for force and adjoint calls
+    only: an energy after the atoms have moved is bit for bit that of a SNAP
+    object that kept nothing, and it drops what was kept, so the force after it
+    is that object's too (atomic additions in another order: 1e-12 of the largest)"""
+    print(f"case: SNAP energy, static geometry, moved atoms, twojmax {twojmax}", flush=True)
+    n, a = 128, 3.1803
+    rng = np.random.default_rng(twojmax)
+    x = lattice("bcc", 4, a) + rng.normal(0, 0.05, (n, 3))
+    beta = list(decks.snap_beta(seed=7, sigma=0.05, ncoeff=len(flopcount.components(twojmax))))
+    pl, fresh = Pipeline(), None
+    try:
+        pl.load(x, (4 * a,) * 3, mass=183.84)
+        pl.build(5.73442, newton=1)
+        pl.snap_setup(beta, twojmax=twojmax)
+        L, c = pl.L, pl.ctx.h
+        pl.chk(L.emd_snap_static_geometry(c, pl.snap, 1), "static")
+        fresh = Pipeline(pl.ctx)
+        fresh.snap_setup(beta, twojmax=twojmax)
+        kept, new = pl.snap, fresh.snap
+        first = [pl.snap_energy(), pl.snap_force(emd.EMD_FP64)]
+        xs = np.zeros(3 * n)
+        pl.chk(L.emd_memcpy_d2h(c, xs.ctypes.data_as(C.c_void_p), C.cast(pl.s.x, C.c_void_p),
+                                xs.nbytes), "d2h")
+        xs += rng.normal(0, 0.05, 3 * n)
+        pl.chk(L.emd_memcpy_h2d(c, C.cast(pl.s.x, C.c_void_p), xs.ctypes.data_as(C.c_void_p),
+                                xs.nbytes), "h2d")
+        pl.chk(L.emd_comm_update_halo(c, C.byref(pl.s), C.byref(pl.h)), "halo")
+        got = [pl.snap_energy(), pl.snap_force(emd.EMD_FP64)]
+        pl.snap = new
+        want = [pl.snap_energy(), pl.snap_force(emd.EMD_FP64)]
+        pl.snap = kept
+    finally:
+        if fresh is not None:
+            fresh.close()
+        pl.close()
+    assert got[0] == want[0] != first[0]
+    scale = np.abs(want[1]).max()
+    assert np.abs(got[1] - want[1]).max() <= 1e-12 * scale < np.abs(first[1] - want[1]).max()
