@@ -209,12 +209,6 @@ class MergedSystem:
             return f32.astype(np.float64)
         return self._dl(self.s.f, 3 * n).reshape(n, 3)
 
-    def write(self, ptr, a):
-        """host values into a device array of doubles"""
-        a = np.ascontiguousarray(a, dtype=np.float64)
-        self.chk(self.L.emd_memcpy_h2d(self.ctx.h, C.cast(ptr, C.c_void_p),
-                                       a.ctypes.data_as(C.c_void_p), a.nbytes), "h2d")
-
     def fit_loss(self):
         loss = C.c_double()
         self.chk(self.L.emd_fit_loss(self.ctx.h, C.byref(loss)), "loss")
@@ -225,6 +219,41 @@ class MergedSystem:
             self.L.emd_free(self.ctx.h, p)
         self._bufs = []
         self.L.emd_system_free(self.ctx.h, C.byref(self.s))
+
+
+class _Target:
+    """Target values of a fit: an array of the host and its copy on the device.
+    Once the program has read or assigned the array, every evaluation uploads
+    it (broadcast to the target's shape, ValueError if it does not fit), so
+    changes made in it count as they do for any attribute."""
+
+    def __init__(self, m, dev, host):
+        self.m, self.dev, self.host, self.shape = m, dev, host, host.shape
+        self.shared = False
+
+    def ptr(self):
+        """the device copy, up to date"""
+        if self.shared:
+            a = np.asarray(self.host, dtype=np.float64)
+            a = np.ascontiguousarray(np.broadcast_to(a, self.shape))
+            m = self.m
+            m.chk(m.L.emd_memcpy_h2d(m.ctx.h, C.cast(self.dev, C.c_void_p),
+                                     a.ctypes.data_as(C.c_void_p), a.nbytes), "h2d")
+        return self.dev
+
+
+def _target(name, doc):
+    """property over the _Target in attribute `name`"""
+    def get(self):
+        target = getattr(self, name)
+        target.shared = True
+        return target.host
+
+    def put(self, a):
+        target = getattr(self, name)
+        target.host, target.shared = a, True
+
+    return property(get, put, doc=doc)
 
 
 def _dp(a):
@@ -281,20 +310,12 @@ class SnapForceMatchMerged:
         # the configurations never move: the compaction, neighbour parameters
         # and U_tot depend on them only, so force and adjoint calls reuse them
         m.chk(L.emd_snap_static_geometry(c, self.pl.snap, 1), "static geometry")
-        self._ft = m._put(np.zeros(3 * n))
         self._forces(EMD_FP64)
-        self.Ft = m.forces(EMD_FP64)
+        F = m.forces(EMD_FP64)
+        self._ft = _Target(m, m._put(F), F)
         self.Et = self.energies(beta_true)
 
-    @property
-    def Ft(self):
-        """target forces of the merged locals, library order (kept on the
-        device; assign to change them)"""
-        return self.m._dl(self._ft, 3 * self.m.s.n_local).reshape(-1, 3)
-
-    @Ft.setter
-    def Ft(self, F):
-        self.m.write(self._ft, F)
+    Ft = _target("_ft", "target forces of the merged locals, library order")
 
     def energies(self, beta):
         """per-configuration energies, E_c = N_c beta_0 + S_c . beta_1.. + R_c"""
@@ -313,7 +334,7 @@ class SnapForceMatchMerged:
         self.pl.snap_set_coeff(beta)
         self._forces(precision)
         # the residuals, the cotangent and the force loss stay on the device
-        m.chk(L.emd_fit_residual(c, C.byref(m.s), precision, self._ft, self._g, 0, None, None,
+        m.chk(L.emd_fit_residual(c, C.byref(m.s), precision, self._ft.ptr(), self._g, 0, None, None,
                                  None, None, None), "residual")
         n = m.n_atoms
         dE = self.energies(beta) - self.Et
@@ -359,33 +380,19 @@ class LJForceMatchMerged:
         self._g = self.m._put(np.zeros(3 * n))
         self._w = self.m._put(np.zeros(n))
         self._start = self.m._put(np.append(self.m.starts, n).astype(np.int32))
-        self._ft = self.m._put(np.zeros(3 * n))
-        self._et = self.m._put(np.zeros(len(configs)))
         self._force_energy(EMD_FP64, *true)
-        self.Ft = self.m.forces(EMD_FP64)
+        F = self.m.forces(EMD_FP64)
+        self._ft = _Target(self.m, self.m._put(F), F)
         # the boxes' energies as the residual forms them (loss 0 at `true`)
+        et = self.m._put(np.zeros(len(configs)))
         self.m.chk(self.L.emd_fit_residual(
-            ctx.h, C.byref(self.m.s), EMD_FP64, self._ft, self._g, len(configs), self._start,
-            self._eatom, self.m._put(np.zeros(len(configs))), self._w, self._et), "targets")
+            ctx.h, C.byref(self.m.s), EMD_FP64, self._ft.dev, self._g, len(configs),
+            self._start, self._eatom, self.m._put(np.zeros(len(configs))), self._w, et),
+            "targets")
+        self._et = _Target(self.m, et, self.m._dl(et, len(configs)))
 
-    @property
-    def Ft(self):
-        """target forces of the merged locals, library order (kept on the
-        device; assign to change them)"""
-        return self.m._dl(self._ft, 3 * self.m.s.n_local).reshape(-1, 3)
-
-    @Ft.setter
-    def Ft(self, F):
-        self.m.write(self._ft, F)
-
-    @property
-    def Et(self):
-        """target energy of each box (kept on the device; assign to change)"""
-        return self.m._dl(self._et, len(self.m.n_atoms))
-
-    @Et.setter
-    def Et(self, E):
-        self.m.write(self._et, E)
+    Ft = _target("_ft", "target forces of the merged locals, library order")
+    Et = _target("_et", "target energy of each box")
 
     def _params(self, eps, sig):
         from examinimd_amd.abi import EmdLJParams
@@ -406,8 +413,9 @@ class LJForceMatchMerged:
         eps, sig = (float(t) for t in theta)
         L, c, m = self.L, self.ctx.h, self.m
         self._force_energy(precision, eps, sig)
-        m.chk(L.emd_fit_residual(c, C.byref(m.s), precision, self._ft, self._g, len(m.n_atoms),
-                                 self._start, self._eatom, self._et, self._w, None), "residual")
+        m.chk(L.emd_fit_residual(c, C.byref(m.s), precision, self._ft.ptr(), self._g,
+                                 len(m.n_atoms), self._start, self._eatom, self._et.ptr(),
+                                 self._w, None), "residual")
         g = np.zeros(2)
         if grad:
             m.chk(L.emd_lj_adjoint_atoms(c, C.byref(m.s), C.byref(m.nl), eps, sig, self.rc,

@@ -93,3 +93,63 @@ def test_targets_can_be_replaced():
     want = 3.0 * n.sum() + 100.0 * ((2.0 / n) ** 2).sum()
     assert abs(l1 - want) <= 1e-9 * want
     s.close()
+
+
+def _loss(s, theta):
+    return s.evaluate(theta, emd.EMD_FP64, grad=False)[0]
+
+
+@pytest.mark.parametrize("kind", ["lj", "snap"])
+def test_targets_changed_in_place(kind):
+    """changes of elements of the target arrays count in the next evaluation,
+    before the first read and after it, as do later changes in an array that
+    was assigned; the arrays outlive close()"""
+    print(f"case: targets changed in place, {kind}", flush=True)
+    if kind == "lj":
+        s, theta = fm.LJForceMatchMerged(fm.lj_set(count=2)), (1.0, 1.0)
+    else:
+        theta = fm.snap_beta_true(seed=5)
+        s = fm.SnapForceMatchMerged(fm.snap_set(count=2, seed=3, sizes=(4,)), theta)
+    n = s.m.n_atoms
+    base = _loss(s, theta)  # 0, or (the fold's atomic order) rounding
+    assert base <= 1e-15
+    s.Ft[3] += (1.0, 2.0, 0.0)
+    s.Ft[-1, 2] -= 1.5
+    want = 1.0 + 4.0 + 2.25
+    assert abs(_loss(s, theta) - want) <= 1e-9 * want
+    s.Et[1] += 3.0
+    want += 100.0 * (3.0 / n[1]) ** 2
+    assert abs(_loss(s, theta) - want) <= 1e-9 * want
+    F = s.Ft.copy()
+    s.Ft = F
+    F[0, 0] += 0.5
+    want += 0.25
+    assert abs(_loss(s, theta) - want) <= 1e-9 * want
+    s.close()
+    assert np.array_equal(s.Ft, F)
+
+
+def test_targets_of_other_shapes():
+    """a target broadcasts to its shape, a wrong one raises before anything is
+    copied to the device"""
+    print("case: targets of other shapes", flush=True)
+    s = fm.LJForceMatchMerged(fm.lj_set(count=3))
+    n, F, E = s.m.n_atoms, s.Ft.copy(), s.Et.copy()
+    s.Et = 0.0
+    want = 100.0 * ((E / n) ** 2).sum()
+    assert abs(_loss(s, (1.0, 1.0)) - want) <= 1e-9 * want
+    s.Et, s.Ft = E, [0.0, 0.0, 0.0]
+    want = (F ** 2).sum()
+    assert abs(_loss(s, (1.0, 1.0)) - want) <= 1e-9 * want
+    for wrong in (np.zeros((len(F) + 1, 3)), np.zeros((len(F) - 1, 3)), np.zeros(3 * len(F))):
+        s.Ft = wrong
+        with pytest.raises(ValueError):
+            _loss(s, (1.0, 1.0))
+    s.Ft = F
+    for wrong in (np.zeros(2), np.zeros(4)):
+        s.Et = wrong
+        with pytest.raises(ValueError):
+            _loss(s, (1.0, 1.0))
+    s.Et = list(E)
+    assert _loss(s, (1.0, 1.0)) == 0.0
+    s.close()
