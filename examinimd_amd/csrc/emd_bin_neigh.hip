@@ -255,12 +255,12 @@ __global__ void k_bin_copy_back(int r0, int n, const double *__restrict__ tx,
 }
 
 // common tail: largest count and out-of-grid flag from the message of the
-// counting pass (the one wait of a binning; the kernels behind that pass are
-// still running), then BinSort::sort of the range when asked
+// counting pass (the one wait of a binning; with early counts the kernels
+// behind that pass are still running), then BinSort::sort of the range when asked
 static emd_status bin_finish(emd_ctx *ctx, emd_system *s, emd_bins *b, int r0, int n, int sort,
                              const emd_mail &mail) {
   const int *got = nullptr;
-  EMD_TRY(emd_mail_wait(ctx, mail, &got));
+  EMD_TRY(emd_count_wait(ctx, mail, &got));
   b->max_count = got[1];
   if (got[2])
     return emd_set_error(ctx, EMD_ERR_OVERFLOW,
@@ -682,7 +682,7 @@ extern "C" emd_status emd_neigh_build(emd_ctx *ctx, const emd_system *s, const e
       EMD_TRY(emd_scan(ctx, row_offsets_op{nl->num, nl->row, n}, n, "neigh_offsets", nullptr,
                        mail));
     const int *got = nullptr;
-    EMD_TRY(emd_mail_wait(ctx, mail, &got));
+    EMD_TRY(emd_count_wait(ctx, mail, &got));
     total = got[0];
     maxrow = got[1];
   }

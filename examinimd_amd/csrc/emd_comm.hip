@@ -371,7 +371,7 @@ extern "C" emd_status emd_comm_exchange_halo(emd_ctx *ctx, emd_system *s, double
       EMD_LAUNCH(ctx, "comm_exchange_halo", k_halo_emit, nb, HALO_THREADS, 0, a, nb, cnt, out);
     }
     const int *got = nullptr;
-    EMD_TRY(emd_mail_wait(ctx, a.mail, &got));
+    EMD_TRY(emd_count_wait(ctx, a.mail, &got));
     int num[6], total = 0;
     for (int p = 0; p < 6; p++) total += num[p] = got[p];
     if (got[6]) {

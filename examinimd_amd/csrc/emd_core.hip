@@ -97,7 +97,7 @@ extern "C" emd_status emd_create(int device, emd_ctx **out) {
   // ghost force fold of a small halo (FOLD_ONE_MAX_*) in one launch (1) or
   // one launch per dimension (0)
   if (const char *e = getenv("EMD_FOLD_ONE")) ctx->fold_one = atoi(e) != 0;
-  // host waits for counts: poll an event (1) or hipStreamSynchronize (0)
+  // host waits for counts: poll the mailbox or an event (1) or hipStreamSynchronize (0)
   if (const char *e = getenv("EMD_SPIN_WAIT")) ctx->spin_wait = atoi(e) != 0;
   // exchange_halo of a small system (<= HALO_ONE_MAX local atoms) in one
   // launch (1) or as count, offset and emit kernels (0)
@@ -162,6 +162,12 @@ emd_status emd_mail_wait(emd_ctx *ctx, const emd_mail &m, const int **payload) {
       return emd_set_error(ctx, EMD_ERR_STATE, "a kernel ended without its counts");
   }
   *payload = m.box + EMD_MAIL_DATA;
+  return EMD_OK;
+}
+
+extern "C" emd_status emd_set_early_counts(emd_ctx *ctx, int on) {
+  if (!ctx) return EMD_ERR_ARG;
+  ctx->early_counts = on != 0;
   return EMD_OK;
 }
 

@@ -16,7 +16,13 @@
  *    library (allocated through the *_grow / *_free calls) unless stated.
  *  - Work is ordered on the context's single HIP stream.  Only calls that
  *    must return a count or a scalar to the host synchronise (the same points
- *    at which the reference synchronises).  A context is not thread-safe.
+ *    at which the reference synchronises): the arrays that go with the count
+ *    (bins and permutation, ghosts, row lengths and offsets) are complete when
+ *    the call returns, unless emd_set_early_counts is on.  What such a call
+ *    queues after its count (emd_binning's sort of the atoms, the compaction
+ *    of CSR entries) and the work of all other calls may still run: other
+ *    streams order on emd_get_stream, or emd_synchronize first.  A context is
+ *    not thread-safe.
  *  - Layouts in HBM: x, v, f are AoS double[n_max][3] (the reference's t_x
  *    layout, src/types.h:88); f32 is AoS float[n_max][3] used by the
  *    mixed-precision path; type, id are int32[n_max]; q double[n_max];
@@ -53,6 +59,13 @@ emd_status  emd_destroy(emd_ctx *ctx);
 const char *emd_last_error(const emd_ctx *ctx);
 emd_status  emd_synchronize(emd_ctx *ctx);
 void       *emd_get_stream(emd_ctx *ctx);   /* the hipStream_t all work runs on */
+/* No counterpart in the reference.  on != 0: emd_binning,
+ * emd_comm_exchange_halo and emd_neigh_build return as soon as their counts
+ * are known, while kernels that fill their arrays may still run.  For callers
+ * that use those arrays only through this library or on the context's stream.
+ * Default: off (emd_app_run turns it on for its context while it runs, and
+ * off). */
+emd_status  emd_set_early_counts(emd_ctx *ctx, int on);
 const char *emd_version(void);
 
 /* device memory for callers (fixtures, tests, host modules) */

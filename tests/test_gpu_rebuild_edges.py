@@ -60,3 +60,50 @@ def test_csr_offsets_and_total(n):
         assert np.array_equal(row, np.concatenate([[0], np.cumsum(num)]))
         assert pl.nl.total == num.sum() and pl.nl.maxneighs == num.max()
     pl.close()
+
+
+@pytest.mark.parametrize("n", [864, 6000, 40000])
+def test_arrays_are_complete_with_their_counts(n):
+    """a call that returns a count has waited for the arrays that go with it
+    (the stream is idle where nothing is queued behind the count: binning
+    without sort, exchange_halo, a padded list of known width); with
+    emd_set_early_counts it need not have, and the arrays are the same"""
+    import torch
+    print(f"case: arrays complete with their counts, {n} atoms", flush=True)
+    edge, cut = (n / 0.8) ** (1.0 / 3.0), 1.5
+    pl = Pipeline()
+    pl.load(np.random.default_rng(n).uniform(0.0, edge, (n, 3)), (edge,) * 3)
+    L, c, s, h, b = pl.L, pl.ctx.h, C.byref(pl.s), pl.h, pl.b
+    for again in range(2):
+        pl.build(cut, layout=emd.EMD_NEIGH_2D)  # capacities
+    stream = torch.cuda.ExternalStream(L.emd_get_stream(c))
+    got = []
+    for early in (0, 1):
+        if early:
+            pl.chk(L.emd_set_early_counts(c, 1), "early counts")
+        idle, out = [], []
+
+        def took(*arrays):
+            idle.append(stream.query())
+            out.extend(emd.download_ints(c, ptr, k) for ptr, k in arrays)
+
+        pl.chk(L.emd_binning(c, s, cut, cut, cut, 1, 1, 0, 0, C.byref(b)), "bin")
+        took((b.permute, n), (b.bincount, b.nbins), (b.binoffsets, b.nbins))
+        pl.chk(L.emd_comm_exchange_halo(c, s, cut, C.byref(h)), "halo")
+        ng = pl.s.n_ghost
+        took((h.root, ng), (h.image, ng), (pl.s.id, n + ng),
+             *[(h.pack[p], h.num_ghost[p]) for p in range(6)])
+        pl.chk(L.emd_binning(c, s, cut, cut, cut, 1, 1, 1, 0, C.byref(b)), "bin all")
+        took((b.permute, n + ng), (b.bincount, b.nbins), (b.binoffsets, b.nbins))
+        pl.chk(L.emd_neigh_build(c, s, C.byref(b), cut, 0, 0, emd.EMD_NEIGH_2D,
+                                 C.byref(pl.nl)), "neigh")
+        took((pl.nl.num, n))
+        num = out[-1]
+        ent = emd.download_ints(c, pl.nl.entries, n * pl.nl.maxneighs).reshape(n, -1)
+        out.append(ent[np.arange(ent.shape[1]) < num[:, None]])
+        print("early", early, "idle after each call", idle)
+        if not early:
+            assert all(idle)
+        got.append(out)
+    pl.close()
+    assert all(np.array_equal(p, q) for p, q in zip(*got)) and len(got[0]) == len(got[1])
