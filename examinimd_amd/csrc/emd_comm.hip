@@ -413,13 +413,14 @@ extern "C" emd_status emd_comm_update_halo(emd_ctx *ctx, emd_system *s, const em
   return EMD_OK;
 }
 
-// CommSerial::TagHaloForceSelf, comm_serial.h:200-213, for both phases of a
-// dimension: the ghosts off .. off + n0 + n1 - 1, the first n0 owned by pack0.
-// Neither phase's owners are among the other's ghosts.  An atom can own a ghost
-// in each only where the halo is deeper than half the box, so the two additions
-// to it are atomic; elsewhere an address gets one addition per launch,
-// the sequential fold's result.  Bound by the launch, so three of them where
-// one per phase took six (86 000 atoms: 20 us a step).
+// CommSerial::TagHaloForceSelf, comm_serial.h:200-213, for the ghosts off ..
+// off + n0 + n1 - 1 of both phases of a dimension, the first n0 owned by pack0
+// (or, n1 = 0, of one phase).  Neither phase's owners are among the other's
+// ghosts, and where no atom owns a ghost in each (emd_comm_update_force's rule)
+// an address gets one addition per launch: the sequential fold's result.
+// (Atomic for a halo put together by the caller that has such atoms all the
+// same.)  Bound by the launch, so three of them where one per phase took six
+// (86 000 atoms: 20 us a step).
 template <class T>
 __global__ void k_halo_fold(T *__restrict__ f, const int *__restrict__ pack0, int n0,
                             const int *__restrict__ pack1, int n1, int off) {
@@ -464,16 +465,30 @@ extern "C" emd_status emd_comm_update_force(emd_ctx *ctx, emd_system *s, const e
                  ph);
     return EMD_OK;
   }
-  for (int p = 4; p >= 0; p -= 2) {
-    const int n0 = ph.num[p], n1 = ph.num[p + 1];
-    if (n0 + n1 <= 0) continue;
+  auto fold = [&](int p, int n0, int n1) -> emd_status {
+    if (n0 + n1 <= 0) return EMD_OK;
     const int blocks = emd_blocks(3l * (n0 + n1), 256);
     if (precision == EMD_MIXED)
       EMD_LAUNCH(ctx, "comm_update_force", k_halo_fold<float>, blocks, 256, 0, s->f32, ph.pack[p],
-                 n0, ph.pack[p + 1], n1, ph.off[p]);
+                 n0, n1 ? ph.pack[p + 1] : nullptr, n1, ph.off[p]);
     else
       EMD_LAUNCH(ctx, "comm_update_force", k_halo_fold<double>, blocks, 256, 0, s->f, ph.pack[p],
-                 n0, ph.pack[p + 1], n1, ph.off[p]);
+                 n0, n1 ? ph.pack[p + 1] : nullptr, n1, ph.off[p]);
+    return EMD_OK;
+  };
+  // An atom owns a ghost in both phases of a dimension only where the halo is
+  // deeper than half the box, hi - depth <= lo + depth; every source then passes
+  // at least one of the two face tests, so the phases have at least as many
+  // ghosts as there are sources.  Fewer: one launch; else one per phase, in the
+  // sequential fold's order.
+  for (int p = 4; p >= 0; p -= 2) {
+    const int n0 = ph.num[p], n1 = ph.num[p + 1];
+    if ((long)n0 + n1 < ph.off[p]) {
+      EMD_TRY(fold(p, n0, n1));
+    } else {
+      EMD_TRY(fold(p + 1, n1, 0));
+      EMD_TRY(fold(p, n0, 0));
+    }
   }
   return EMD_OK;
 }

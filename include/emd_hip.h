@@ -162,7 +162,8 @@ emd_status emd_comm_exchange_halo(emd_ctx *ctx, emd_system *s, double comm_depth
 /* CommSerial::update_halo, comm_serial.cpp:99-110 (positions only) */
 emd_status emd_comm_update_halo(emd_ctx *ctx, emd_system *s, const emd_halo *h);
 /* CommSerial::update_force, comm_serial.cpp:112-127 (folds f, or f32 when
- * precision == EMD_MIXED) */
+ * precision == EMD_MIXED; for a halo of emd_comm_exchange_halo every atom's
+ * additions are in the order of the phases 5..0) */
 emd_status emd_comm_update_force(emd_ctx *ctx, emd_system *s, const emd_halo *h,
                                  int precision);
 emd_status emd_halo_free(emd_ctx *ctx, emd_halo *h);
@@ -312,8 +313,7 @@ emd_status emd_nve_final_initial(emd_ctx *ctx, emd_system *s, double dtf, double
  * local atoms and ghosts (5500 with the fold) the three run in one workgroup
  * launch separated by barriers; larger systems get the separate launches.
  * Results are bitwise those of emd_comm_update_force, emd_nve_final_initial
- * and emd_comm_update_halo called in turn (where the halo is deeper than half
- * the box, the order of two of the fold's additions is free). */
+ * and emd_comm_update_halo called in turn. */
 emd_status emd_nve_step_boundary(emd_ctx *ctx, emd_system *s, const emd_halo *h, int fold,
                                  int update_halo, double dtf, double dtv, int precision);
 

@@ -1,9 +1,7 @@
 """emd_comm_update_force with one launch per dimension (both faces' ghosts at
-once) against the sequential fold f[pack_p] += f[ghosts_p], p = 5..0.  In boxes
-thinner than twice the halo an atom owns a ghost on either face, and the
-order of those two additions is free: 64 additions of values up to 8 leave 1e-13
-(1e-4 in FP32) of room; in wide boxes the result is the sequential one bit for
-bit."""
+once; per phase where an atom owns a ghost on either face, in boxes thinner
+than twice the halo) against the sequential fold f[pack_p] += f[ghosts_p],
+p = 5..0, bit for bit."""
 import ctypes as C
 
 import numpy as np
@@ -17,14 +15,18 @@ A_W = 3.1803
 
 
 @pytest.mark.parametrize("prec", [emd.EMD_FP64, emd.EMD_MIXED])
-@pytest.mark.parametrize("nc,cut", [(2, 5.73442), (3, 5.73442), (4, 5.73442), (7, 5.73442)])
-def test_fold_per_dimension(monkeypatch, nc, cut, prec):
-    print(f"case: fold per dimension, BCC {nc}^3, cut {cut}, precision {prec}", flush=True)
+@pytest.mark.parametrize("nc,cut,wide", [(2, 5.73442, 1), (3, 5.73442, 1), (4, 5.73442, 1),
+                                         (7, 5.73442, 1), (3, 5.73442, 16)])
+def test_fold_per_dimension(monkeypatch, nc, cut, wide, prec):
+    print(f"case: fold per dimension, BCC {nc}^3 x {wide}, cut {cut}, precision {prec}",
+          flush=True)
     monkeypatch.setenv("EMD_FOLD_ONE", "0")
-    x = lattice("bcc", nc, A_W) + np.random.default_rng(nc).normal(0, 0.05, (2 * nc ** 3, 3))
+    x = lattice("bcc", nc, A_W)
+    x = np.concatenate([x + (0, k * nc * A_W, 0) for k in range(wide)])  # thin in x and z only
+    x += np.random.default_rng(nc).normal(0, 0.05, x.shape)
     dt = np.float32 if prec == emd.EMD_MIXED else np.float64
     pl = Pipeline()
-    pl.load(x, (nc * A_W,) * 3, mass=183.84)
+    pl.load(x, (nc * A_W, wide * nc * A_W, nc * A_W), mass=183.84)
     pl.build(cut, newton=1)
     L, c = pl.L, pl.ctx.h
     n, counts = pl.s.n_local, [pl.h.num_ghost[p] for p in range(6)]
@@ -47,11 +49,7 @@ def test_fold_per_dimension(monkeypatch, nc, cut, prec):
     for p in range(5, -1, -1):
         want[packs[p]] += want[off[p]:off[p] + counts[p]]
     assert sum(counts) > 0
-    thin = any(len(np.intersect1d(packs[p], packs[p + 1])) for p in (0, 2, 4))
-    assert thin == (nc * A_W < 2 * cut)
-    err = np.abs(got.astype(np.float64) - want[:n].astype(np.float64)).max()
-    print("thin", thin, "error", err)
-    if thin:
-        assert err <= (1e-4 if prec == emd.EMD_MIXED else 1e-13)
-    else:
-        assert np.array_equal(got, want[:n])
+    thin = [len(np.intersect1d(packs[p], packs[p + 1])) > 0 for p in (0, 2, 4)]
+    assert thin == [edge < 2 * cut for edge in (nc * A_W, wide * nc * A_W, nc * A_W)]
+    print("thin", thin, "differ", int((got != want[:n]).sum()))
+    assert np.array_equal(got, want[:n])
