@@ -456,22 +456,25 @@ __global__ void k_binit(double *__restrict__ x, double *__restrict__ v,
 
 // per replica sum m v^2 (Temperature/KinE summand,
 // property_temperature.h:54-56) and the shifted pair energy
-// (force_lj_neigh_impl.h:256-300), both compensated: BT_SLICES blocks per
-// replica, BT_K lanes per atom (lane sub takes row entries sub, sub + BT_K,
-// ...), each block's double-double sums to part[(replica * BT_SLICES + slice)
-// * 4 + {0,1} kinetic, {2,3} potential}.  Bound: latency of the row and
-// gather loads; 281 us for both sums of 256 replicas (661 284 atoms), where
-// one block per replica with a thread per row took 611 us for each.
+// (force_lj_neigh_impl.h:256-300), both compensated: SLICES blocks per
+// replica, K lanes per atom (lane sub takes row entries sub, sub + K,
+// ...), each block's double-double sums to part[(replica * SLICES + slice)
+// * 4 + {0,1} kinetic, {2,3} potential}.  With the energy, BT_K lanes and
+// BT_SLICES blocks: bound by the latency of the row and gather loads, 281 us for
+// both sums of 256 replicas (661 284 atoms), where one block per replica with
+// a thread per row took 611 us.  The kinetic sum alone reads no row: one block
+// per replica, a thread per atom (a call 32 us; 299 with the rows walked too).
 constexpr int BT_THREADS = 256, BT_K = 16, BT_SLICES = 16;
+template <int K, int SLICES, bool PE>
 __global__ void __launch_bounds__(BT_THREADS)
 k_bthermo(const double *__restrict__ x, const double *__restrict__ v,
           const rep_info *__restrict__ info, const int *__restrict__ num,
           const unsigned *__restrict__ entries, int cap, const double *__restrict__ mass,
           double lj1, double lj2, double cutsq, double *__restrict__ part) {
 #pragma clang fp contract(off)
-  const int rep = blockIdx.x / BT_SLICES, slice = blockIdx.x % BT_SLICES;
+  const int rep = blockIdx.x / SLICES, slice = blockIdx.x % SLICES;
   const rep_info R = info[rep];
-  const int sub = threadIdx.x % BT_K;
+  const int sub = threadIdx.x % K;
   const double r2invc = 1.0 / cutsq;
   const double r6invc = r2invc * r2invc * r2invc;
   const double eshift = 0.5 * r6invc * (0.5 * lj1 * r6invc - lj2) / 6.0;
@@ -482,16 +485,17 @@ k_bthermo(const double *__restrict__ x, const double *__restrict__ v,
     hi = s;
     lo += e;
   };
-  constexpr int ATOMS = BT_THREADS / BT_K;
-  for (int k = slice * ATOMS + (int)threadIdx.x / BT_K; k < R.n; k += BT_SLICES * ATOMS) {
+  constexpr int ATOMS = BT_THREADS / K;
+  for (int k = slice * ATOMS + (int)threadIdx.x / K; k < R.n; k += SLICES * ATOMS) {
     const int i = R.start + k;
     const size_t o = 3 * (size_t)i;
-    const double x_i = x[o], y_i = x[o + 1], z_i = x[o + 2];
     if (sub == 0)
       add(khi, klo,
           (v[o] * v[o] + v[o + 1] * v[o + 1] + v[o + 2] * v[o + 2]) * mass[rep]);
+    if constexpr (!PE) continue;
+    const double x_i = x[o], y_i = x[o + 1], z_i = x[o + 2];
     const int cnt = num[i];
-    for (int jj = sub; jj < cnt; jj += BT_K) {
+    for (int jj = sub; jj < cnt; jj += K) {
       const unsigned e = entries[(size_t)i * cap + jj];
       const size_t j = e & B_JMASK;
       const unsigned c = e >> B_CODE_SHIFT;
@@ -508,8 +512,10 @@ k_bthermo(const double *__restrict__ x, const double *__restrict__ v,
     }
   }
   block_dd_sum(khi, klo, part, 4);
-  __syncthreads();
-  block_dd_sum(phi, plo, part + 2, 4);
+  if constexpr (PE) {
+    __syncthreads();
+    block_dd_sum(phi, plo, part + 2, 4);
+  }
 }
 
 // -------------------------------------------------------------- host side
@@ -901,11 +907,18 @@ extern "C" emd_status emd_batch_thermo(emd_ctx *ctx, emd_batch *b, double *ke, d
   if (!ctx || !b) return EMD_ERR_ARG;
   if (!b->ready) return emd_set_error(ctx, EMD_ERR_STATE, "emd_batch_thermo before setup");
   if (!ke && !pe) return EMD_OK;
-  const size_t count = 4 * (size_t)b->nrep * BT_SLICES;
+  const int slices = pe ? BT_SLICES : 1;
+  const size_t count = 4 * (size_t)b->nrep * slices;
+  const double *mass = b->part + 4 * (size_t)b->nrep * BT_SLICES;
   std::vector<double> h(count);
-  EMD_LAUNCH(ctx, "batch_thermo", k_bthermo, BT_SLICES * b->nrep, BT_THREADS, 0,
-             b->x[b->cur], b->v, b->info, b->num, b->entries, b->cap, b->part + count, b->lj1,
-             b->lj2, b->cutsq, b->part);
+  if (pe)
+    EMD_LAUNCH(ctx, "batch_thermo", (k_bthermo<BT_K, BT_SLICES, true>), slices * b->nrep,
+               BT_THREADS, 0, b->x[b->cur], b->v, b->info, b->num, b->entries, b->cap, mass,
+               b->lj1, b->lj2, b->cutsq, b->part);
+  else
+    EMD_LAUNCH(ctx, "batch_thermo", (k_bthermo<1, 1, false>), slices * b->nrep, BT_THREADS, 0,
+               b->x[b->cur], b->v, b->info, b->num, b->entries, b->cap, mass, b->lj1, b->lj2,
+               b->cutsq, b->part);
   EMD_HIP(ctx, hipMemcpyAsync(h.data(), b->part, count * sizeof(double), hipMemcpyDeviceToHost,
                               ctx->stream));
   EMD_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -915,9 +928,9 @@ extern "C" emd_status emd_batch_thermo(emd_ctx *ctx, emd_batch *b, double *ke, d
       if (!out) continue;
       // the slices' (hi, lo) pairs, compensated (Neumaier)
       double sum = 0.0, c = 0.0;
-      for (int k = 0; k < BT_SLICES; k++)
+      for (int k = 0; k < slices; k++)
         for (int w = 0; w < 2; w++) {
-          const double v = h[4 * ((size_t)r * BT_SLICES + k) + 2 * what + w], t = sum + v;
+          const double v = h[4 * ((size_t)r * slices + k) + 2 * what + w], t = sum + v;
           c += fabs(sum) >= fabs(v) ? (sum - t) + v : (v - t) + sum;
           sum = t;
         }

@@ -251,3 +251,35 @@ def test_batch_row_overflow_grows_and_rebuilds():
                        for c in ((code >> 2 * a) & 3 for a in range(3)))
             got.add((int(e) & batch.JMASK, sh))
         assert got == want and len(row) == len(want), i
+
+
+def test_batch_thermo_of_one_kind():
+    """emd_batch_thermo asked for one sum gives what it gives with both (the
+    kinetic sums over other slices: compensated, 1e-15), and the kinetic sums
+    alone, which need no neighbour row, take less than half of both's time"""
+    import ctypes as C
+    import time
+    print("case: batch thermo, one sum at a time", flush=True)
+    sh = batch.ensemble(nrep=256, seed=4, nmin=256, nmax=8192)
+    b = batch.Batch(sh["natoms"], sh["box"], precision=EMD_MIXED)
+    b.upload(sh["x"], np.random.default_rng(1).normal(size=sh["x"].shape))
+    b.setup()
+
+    def take(ke, pe):
+        d = lambda a: None if a is None else a.ctypes.data_as(C.POINTER(C.c_double))
+        best = np.inf
+        for _ in range(20):
+            t = time.perf_counter()
+            b.chk(b.L.emd_batch_thermo(b.ctx.h, b.h, d(ke), d(pe)), "thermo")
+            best = min(best, time.perf_counter() - t)
+        return best
+
+    n = len(sh["natoms"])
+    ke, pe, k1, p1 = (np.zeros(n) for _ in range(4))
+    both, kinetic, potential = take(ke, pe), take(k1, None), take(None, p1)
+    b.close()
+    print("us: both %.1f kinetic %.1f potential %.1f" % (both * 1e6, kinetic * 1e6,
+                                                       potential * 1e6))
+    assert np.array_equal(p1, pe) and ke.min() > 0
+    assert np.abs(k1 - ke).max() <= 1e-15 * ke.max()
+    assert kinetic < 0.5 * both
