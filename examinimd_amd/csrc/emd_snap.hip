@@ -1155,50 +1155,56 @@ static double host_cg(int j1, int j2, int j, int k1, int k2) {
   return sum * delta * norm;
 }
 
-// the beta-independent part of the flat Y stream (see k_snap_yflat)
-// LDS byte offsets of the two U_tot reads of every slot of the Y stream
-// (code = offset1 | offset2 << 16, 8-byte words): for each step, each
-// wavefront, each of the two reads and each lane group served in one LDS
-// cycle, the group's distinct U entries are matched to distinct bank
-// residues (u + shift(c)) mod MOD, each entry choosing one copy c
-// (augmenting paths); an entry left unmatched takes the least loaded
+// Copies of U_tot for one read of a lane group served in one LDS cycle: the
+// group's distinct U entries are matched to distinct bank residues (u + shift(c))
+// mod MOD, each entry choosing one copy c (augmenting paths, a free residue
+// taken before any is freed); an entry left unmatched takes the least loaded
 // residue among its copies.  Lanes reading the same entry read the same copy.
+// Bit sets, as this is most of emd_snap_create: 55 of its 113 ms at twojmax 12
+// with arrays of flags (one core of an EPYC host).
 template <class L>
 struct yf_matching {
-  int na = 0;
+  static_assert(L::MOD == 32, "residues in a 32-bit set");
   int addr[L::GROUP], copy_of[L::GROUP], owner[L::MOD];
-  bool seen[L::MOD];
+  uint32_t open, seen;  // residues without an owner; visited by the path
+  bool take(int a, int c, int b) {
+    open &= ~(1u << b);
+    owner[b] = a;
+    copy_of[a] = c;
+    return true;
+  }
   bool augment(int a) {
     for (int c = 0; c < L::NCOPY; c++) {
       const int b = (addr[a] + L::shift(c)) % L::MOD;
-      if (seen[b]) continue;
-      seen[b] = true;
-      if (owner[b] < 0 || augment(owner[b])) {
-        owner[b] = a;
-        copy_of[a] = c;
-        return true;
-      }
+      if (open >> b & 1) return take(a, c, b);
+    }
+    for (int c = 0; c < L::NCOPY; c++) {
+      const int b = (addr[a] + L::shift(c)) % L::MOD;
+      if (seen >> b & 1) continue;
+      seen |= 1u << b;
+      if (augment(owner[b])) return take(a, c, b);
     }
     return false;
   }
   // copies of the group's entries u[0 .. GROUP)
   void assign(const int *u, int *cp, std::vector<int> &index) {
-    na = 0;
+    int na = 0;
     for (int l = 0; l < L::GROUP; l++)
       if (index[u[l]] < 0) {
         index[u[l]] = na;
         addr[na++] = u[l];
       }
-    std::fill(owner, owner + L::MOD, -1);
-    std::fill(copy_of, copy_of + na, -1);
-    int load[L::MOD] = {0};
+    open = ~0u;
+    bool all = true;
     for (int a = 0; a < na; a++) {
-      std::fill(seen, seen + L::MOD, false);
-      augment(a);
+      seen = 0;
+      copy_of[a] = -1;
+      all &= augment(a);
     }
-    for (int a = 0; a < na; a++)
+    int load[L::MOD] = {0};
+    for (int a = 0; a < na && !all; a++)
       if (copy_of[a] >= 0) load[(addr[a] + L::shift(copy_of[a])) % L::MOD]++;
-    for (int a = 0; a < na; a++)
+    for (int a = 0; a < na && !all; a++)
       if (copy_of[a] < 0) {
         int best = 0;
         for (int c = 1; c < L::NCOPY; c++)
@@ -1212,6 +1218,7 @@ struct yf_matching {
   }
 };
 
+// LDS byte offsets of one read (of U entry u) of every slot of a stream
 template <class L>
 static std::vector<unsigned short> yf_offsets(const std::vector<int> &u, int nu) {
   std::vector<int> cp(u.size(), 0), index(nu, -1);
@@ -1243,17 +1250,30 @@ struct yf_slot {
 // odd (depth first: a vertex pairs the edges its subtree left to it, and takes
 // the edge to its parent for an odd one).
 struct yf_pairs {
-  const std::vector<yf_term> &t;
-  std::vector<yf_slot> &out;
-  std::vector<std::vector<int>> adj;
+  const yf_term *t = nullptr;
+  std::vector<yf_slot> *out = nullptr;
+  std::vector<int> first, at, adj;  // edges of vertex v: adj[first[v] .. first[v + 1])
   std::vector<char> used, seen;
-  yf_pairs(const std::vector<yf_term> &terms, int nu, std::vector<yf_slot> &slots)
-      : t(terms), out(slots), adj(nu), used(terms.size(), 0), seen(nu, 0) {
-    for (size_t e = 0; e < t.size(); e++) {
-      adj[t[e].i1].push_back((int)e);
-      if (t[e].i2 != t[e].i1) adj[t[e].i2].push_back((int)e);
+  explicit yf_pairs(int nu) : first(nu + 1), at(nu), seen(nu) {}
+  void split(const std::vector<yf_term> &terms, std::vector<yf_slot> &slots) {
+    t = terms.data();
+    out = &slots;
+    std::fill(first.begin(), first.end(), 0);
+    std::fill(seen.begin(), seen.end(), 0);
+    for (const yf_term &q : terms) {
+      first[q.i1 + 1]++;
+      if (q.i2 != q.i1) first[q.i2 + 1]++;
     }
-    for (const yf_term &q : t)
+    for (size_t v = 1; v < first.size(); v++) first[v] += first[v - 1];
+    std::copy(first.begin(), first.end() - 1, at.begin());
+    adj.resize(first.back());
+    for (size_t e = 0; e < terms.size(); e++) {
+      adj[at[t[e].i1]++] = (int)e;
+      if (t[e].i2 != t[e].i1) adj[at[t[e].i2]++] = (int)e;
+    }
+    used.assign(terms.size(), 0);
+    slots.reserve(terms.size() / 2 + 8);
+    for (const yf_term &q : terms)
       if (!seen[q.i1]) visit(q.i1, -1);
   }
   int other(int e, int v) const { return t[e].i1 == v ? t[e].i2 : t[e].i1; }
@@ -1267,13 +1287,14 @@ struct yf_pairs {
       s.y = s.x;  // weight 0
       s.ky = s.kx;
     }
-    out.push_back(s);
+    out->push_back(s);
   }
   // true if v took the edge to its parent
   bool visit(int v, int parent) {
     seen[v] = 1;
     int left = -1;
-    for (int e : adj[v]) {
+    for (int k = first[v]; k < first[v + 1]; k++) {
+      const int e = adj[k];
       if (used[e]) continue;
       used[e] = 1;
       const int w = other(e, v);
@@ -1355,6 +1376,7 @@ static emd_status snap_build_sflat(emd_ctx *ctx, emd_snap *sn,
   return EMD_OK;
 }
 
+// the beta-independent part of the flat Y stream (see k_snap_yflat)
 static emd_status snap_build_yflat(emd_ctx *ctx, emd_snap *sn) {
   const snap_dev_tables &t = sn->t;
   const int nk = (int)sn->idxj.size() / 3;
@@ -1411,8 +1433,9 @@ static emd_status snap_build_yflat(emd_ctx *ctx, emd_snap *sn) {
   // ---- the slot stream of k_snap_yflat
   std::vector<std::vector<yf_slot>> eslots(t.ny);
   std::vector<int> len(t.ny);
+  yf_pairs pairs(t.nu);
   for (int e = 0; e < t.ny; e++) {
-    yf_pairs(eterms[e], t.nu, eslots[e]);
+    pairs.split(eterms[e], eslots[e]);
     len[e] = (int)eslots[e].size();
   }
   const bool small = t.twojmax <= SNAP_MAXJ;
