@@ -1254,12 +1254,16 @@ k_step_boundary_one(double *__restrict__ x, double *__restrict__ v, double *__re
     emd_halo_update_at(g, x, root, image, n, lx, ly, lz);
 }
 
-// locals + ghosts of a one-workgroup step boundary: one CU moves ~0.35 us per
-// hundred atoms, the separate launches take 6.5 us without a fold (5.5 at 3059
-// atoms in one workgroup, 8.0 at 4941) and 10-14 us with one (9.4 / 11.0
-// mixed / FP64 at 4941, 10.8 / 12.9 at 6083); at 26 000 atoms one workgroup
-// takes 37-47 us
-constexpr int STEP_ONE_MAX = 3500, STEP_ONE_MAX_FOLD = 5500;
+// locals + ghosts of a one-workgroup step boundary.  One CU moves ~0.15 us per
+// hundred atoms, so its time grows where that of the separate launches does
+// not, and in a run these overlap with the ends of their neighbours.  Whole
+// steps, us, one workgroup / separate launches: LJ melts without a fold 2167
+// atoms 7.6 / 7.6, 2745 8.5 / 7.9, 3429 9.2 / 8.0; SNAP (fold) FP64 2552 45.9 /
+// 46.6, 3059 49.9 / 50.1, 3324 57.8 / 57.5, 4941 78.7 / 75.9, mixed 2552 36.5 /
+// 37.1, 3059 39.2 / 39.3, 3324 43.3 / 42.9, 4941 55.5 / 53.4.  (The boundary by
+// itself, repeated, crosses at 3900 without and 3900 / 4900 FP64 / mixed with
+// the fold.)
+constexpr int STEP_ONE_MAX = 2200, STEP_ONE_MAX_FOLD = 3000;
 
 extern "C" emd_status emd_nve_step_boundary(emd_ctx *ctx, emd_system *s, const emd_halo *h,
                                             int fold, int update_halo, double dtf, double dtv,

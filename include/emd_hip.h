@@ -309,8 +309,8 @@ emd_status emd_nve_final_initial(emd_ctx *ctx, emd_system *s, double dtf, double
  * comm->update_force() of step s if `fold` (src/examinimd.cpp:243,
  * comm_serial.h:200-213), final_integrate of s and initial_integrate of s+1
  * (src/examinimd.cpp:249 then 196), and comm->update_halo() of s+1 if
- * `update_halo` (src/examinimd.cpp:226, comm_serial.h:184-197).  Up to 3500
- * local atoms and ghosts (5500 with the fold) the three run in one workgroup
+ * `update_halo` (src/examinimd.cpp:226, comm_serial.h:184-197).  Up to 2200
+ * local atoms and ghosts (3000 with the fold) the three run in one workgroup
  * launch separated by barriers; larger systems get the separate launches.
  * Results are bitwise those of emd_comm_update_force, emd_nve_final_initial
  * and emd_comm_update_halo called in turn. */

@@ -141,11 +141,11 @@ def test_snap_kernel_level_disordered(oracle):
 @pytest.mark.parametrize("mixed", [False, True])
 def test_ghost_force_fold_against_numpy(monkeypatch, nc, cut, mixed):
     """CommSerial::update_force on seeded random forces: the one-workgroup
-    six-phase fold (small halos) and the per-phase launches both equal the
+    six-phase fold (small halos) and the separate launches both equal the
     sequential fold f[pack_p] += f[ghosts_p], p = 5..0, done in numpy.
     (Whole SNAP runs cannot be compared bit for bit: the force scatter onto
     neighbours uses atomics.)  BCC 10^3 gives ~3 000 ghosts (single launch),
-    30^3 ~ 22 000 (per-phase launches)."""
+    30^3 ~ 22 000, more than one workgroup folds (launches per dimension)."""
     import ctypes as C
     from examinimd_amd.pipeline import Pipeline, lattice
     print(f"case: ghost force fold, BCC {nc}^3, cut {cut}, mixed={mixed}", flush=True)
@@ -190,18 +190,17 @@ def test_ghost_force_fold_against_numpy(monkeypatch, nc, cut, mixed):
         results.append((ng, got))
         pl.close()
     print("ghosts", results[0][0])
-    assert (results[0][0] <= 16384) == (nc == 10)
+    assert results[0][0] <= 7000 if nc == 10 else results[0][0] > 16000
     assert np.array_equal(results[0][1], results[1][1])
 
 
 @pytest.mark.parametrize("nc,cut", [(10, 5.73442), (6, 5.73442), (8, 20.0)])
 def test_halo_exchange_one_launch_equals_scans(monkeypatch, nc, cut):
     """exchange_halo of a small system in one workgroup launch gives the
-    ghosts of the six per-phase scans: counts, pack lists, positions,
+    ghosts of the count, offset and emit kernels: counts, pack lists, positions,
     velocities, ids, types, charges, roots and image codes, bit for bit (including the first
-    call, which starts with no capacity and grows).  BCC 8^3 with a 20 A
-    halo depth has ~27 000 local + ghost atoms, more than one workgroup
-    handles: that call falls back to the scans mid-way."""
+    call, which starts with no capacity and grows).  BCC 8^3 with a 20 A halo
+    depth gives its 1024 atoms ~26 000 ghosts, every atom in all 26 lists."""
     import ctypes as C
     from examinimd_amd.pipeline import Pipeline, lattice
     print(f"case: exchange_halo one launch vs scans, BCC {nc}^3, depth {cut}", flush=True)

@@ -4,8 +4,10 @@ of s+1; src/examinimd.cpp:243, 249, 196, 226) as one workgroup launch for
 small systems.  From the same device state (seeded forces on locals and
 ghosts, seeded velocities) it must give the bits of emd_comm_update_force,
 emd_nve_final_initial and emd_comm_update_halo called in turn: positions of
-locals and ghosts, velocities and forces.  BCC 10^3 W with a 5.73 A halo has
-~3 000 ghosts (one launch); 30^3 has ~22 000 (the separate launches)."""
+locals and ghosts, velocities and forces.  Boxes of BCC W with a 5.73 A halo
+on both sides of the one launch's limits, 2200 locals and ghosts without a
+fold and 3000 with it: 6^3 has 1 729, 7^3 2 331 (one launch with the fold only),
+8^3 3 059, 10^3 4 941."""
 import ctypes as C
 
 import numpy as np
@@ -34,7 +36,7 @@ def _put(pl, ptr, a):
                                a.nbytes), "h2d")
 
 
-@pytest.mark.parametrize("nc", [10, 30])
+@pytest.mark.parametrize("nc", [6, 7, 8, 10, 30])
 @pytest.mark.parametrize("precision", [emd.EMD_FP64, emd.EMD_MIXED])
 @pytest.mark.parametrize("fold,halo", [(1, 1), (1, 0), (0, 1)])
 def test_step_boundary_equals_separate_launches(nc, precision, fold, halo):
@@ -56,6 +58,8 @@ def test_step_boundary_equals_separate_launches(nc, precision, fold, halo):
         x0 = _get(pl, pl.s.x, 3 * (n + ng), np.float64)
         v0 = _get(pl, pl.s.v, 3 * n, np.float64)
         out = []
+        pl.chk(L.emd_profile_enable(c, 1), "profile")
+        pl.chk(L.emd_profile_select(c, b"step_boundary"), "profile")
         for fused in (False, True):
             _put(pl, pl.s.x, x0)
             _put(pl, pl.s.v, v0)
@@ -72,10 +76,13 @@ def test_step_boundary_equals_separate_launches(nc, precision, fold, halo):
             out.append({"x": _get(pl, pl.s.x, 3 * (n + ng), np.float64),
                         "v": _get(pl, pl.s.v, 3 * n, np.float64),
                         "f": _get(pl, fptr, 3 * (n + ng), fdt)})
+        ms, one = C.c_double(), C.c_long()
+        pl.chk(L.emd_profile_get(c, b"step_boundary", C.byref(ms), C.byref(one)), "profile")
     finally:
         pl.close()
     print("locals", n, "ghosts", ng)
-    assert (ng <= 16384) == (nc == 10)
+    assert one.value == (n + ng <= (3000 if fold else 2200))
+    assert one.value == (nc <= 6 or (nc == 7 and fold))
     for k in ("x", "v", "f"):
         assert np.array_equal(out[0][k], out[1][k]), k
     # the step moved every atom and (with halo) every ghost
