@@ -80,6 +80,54 @@ def test_residuals_and_energies(n, cuts, prec):
     pl.close()
 
 
+@pytest.mark.parametrize("prec", [emd.EMD_FP64, emd.EMD_MIXED])
+@pytest.mark.parametrize("layout", [emd.EMD_NEIGH_CSR, emd.EMD_NEIGH_2D])
+@pytest.mark.parametrize("ntypes,table,lanes", [(1, True, 0), (2, False, 0), (2, True, 0),
+                                                (20, True, 0), (2, False, 1), (1, False, 8),
+                                                (2, False, 16)])
+def test_forces_and_energies_of_several_types(ntypes, table, lanes, layout, prec):
+    """emd_lj_force_energy_store with per-pair coefficients and cutoffs (the
+    fixed arrays, a table, more types than the arrays hold) and with other lane
+    counts: the bits of emd_lj_force_store and emd_lj_energy_atoms"""
+    print(f"case: force and energy, {ntypes} types, table {table}, lanes {lanes}, layout {layout}, "
+          f"precision {prec}", flush=True)
+    rng = np.random.default_rng(ntypes)
+    n = 1371
+    x = (lattice("fcc", 7, 1.68) + rng.normal(0, 0.04, (1372, 3)))[:n]
+    types = rng.integers(0, ntypes, n)
+    types[0] = ntypes - 1
+    sig = rng.uniform(0.9, 1.05, (ntypes, ntypes))
+    eps, rc = rng.uniform(0.5, 1.5, (ntypes, ntypes)), rng.uniform(1.5, 2.5, (ntypes, ntypes))
+    coeff = np.array([48.0 * eps * sig ** 12, 24.0 * eps * sig ** 6, rc * rc])
+    coeff = np.ascontiguousarray(0.5 * (coeff + coeff.transpose(0, 2, 1)))
+    p = EmdLJParams()
+    p.ntypes = ntypes
+    if table:
+        p.table = coeff.ctypes.data_as(C.POINTER(C.c_double))
+    else:
+        for a in range(ntypes):
+            for b in range(ntypes):
+                p.lj1[a][b], p.lj2[a][b], p.cutsq[a][b] = (float(k) for k in coeff[:, a, b])
+    pl = Pipeline()
+    pl.load(x, (7 * 1.68,) * 3, types=types)
+    pl.build(2.5, layout=layout)
+    L, c, s, nl = pl.L, pl.ctx.h, C.byref(pl.s), C.byref(pl.nl)
+    if lanes:
+        pl.chk(L.emd_lj_set_lanes(c, prec, lanes), "lanes")
+    d = lambda q: C.cast(q, C.POINTER(C.c_double))
+    e1, e2 = _put(pl, np.zeros(n)), _put(pl, np.ones(n))
+    pl.chk(L.emd_lj_force_store(c, s, nl, C.byref(p), prec), "force")
+    pl.chk(L.emd_lj_energy_atoms(c, s, nl, C.byref(p), 0, d(e1)), "energy")
+    want = pl.forces(prec)
+    pl.chk(L.emd_force_zero(c, s, prec), "zero")
+    pl.chk(L.emd_lj_force_energy_store(c, s, nl, C.byref(p), prec, d(e2)), "both")
+    got, eat, both = pl.forces(prec), _get(pl, e1, n), _get(pl, e2, n)
+    pl.close()
+    assert np.abs(want).max() > 1.0 and np.abs(eat).max() > 1.0
+    assert np.array_equal(got, want)
+    assert np.array_equal(both, eat)
+
+
 def test_targets_can_be_replaced():
     """the merged sets keep their targets on the device: assigning other ones
     changes the loss as the definition says"""
