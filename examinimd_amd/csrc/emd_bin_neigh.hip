@@ -9,10 +9,11 @@
 //
 // Neighbour build: one 256-thread block per interior bin.  The block stages
 // the 27 stencil bins' candidates (index + FP64 position) in LDS in stencil
-// order; each wavefront takes atoms of the centre bin and tests 64
-// candidates per step, compacting hits with ballot + popcount so every row
-// comes out in stencil-then-permutation order.  Two passes (count, fill)
-// with an exclusive scan between them, as NeighborCSR does.
+// order; each wavefront takes atoms of the centre bin and tests 128
+// candidates per step, compacting hits with ballot + mbcnt so every row
+// comes out in stencil-then-permutation order.  The first CSR build counts,
+// scans and fills, as NeighborCSR does; later ones, and 2D lists, fill rows
+// padded to a known capacity in one pass (emd_neigh_build).
 #include "emd_internal.hpp"
 
 #include <algorithm>

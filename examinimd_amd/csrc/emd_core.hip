@@ -66,7 +66,6 @@ extern "C" emd_status emd_create(int device, emd_ctx **out) {
     return EMD_ERR_HIP;
   }
   bool ok = hipMalloc(&ctx->d_small, 64 * sizeof(int)) == hipSuccess &&
-            hipMalloc(&ctx->d_dsmall, 64 * sizeof(double)) == hipSuccess &&
             hipHostMalloc(&ctx->h_small, 64 * sizeof(int), hipHostMallocDefault) == hipSuccess &&
             hipHostMalloc(&ctx->h_dsmall, 64 * sizeof(double), hipHostMallocDefault) == hipSuccess &&
             hipHostMalloc(&ctx->h_mail, 2 * EMD_MAIL_INTS * sizeof(int),
@@ -119,7 +118,6 @@ extern "C" emd_status emd_destroy(emd_ctx *ctx) {
   for (auto &r : ctx->prof_pending) { hipEventDestroy(r.start); hipEventDestroy(r.stop); }
   for (auto e : ctx->prof_pool) hipEventDestroy(e);
   if (ctx->d_small) hipFree(ctx->d_small);
-  if (ctx->d_dsmall) hipFree(ctx->d_dsmall);
   if (ctx->h_small) hipHostFree(ctx->h_small);
   if (ctx->h_dsmall) hipHostFree(ctx->h_dsmall);
   if (ctx->h_mail) hipHostFree(ctx->h_mail);

@@ -34,7 +34,6 @@ struct emd_ctx {
 
   // small device + pinned host scratch for scalar results
   int *d_small = nullptr;      // 64 ints
-  double *d_dsmall = nullptr;  // 64 doubles
   int *h_small = nullptr;      // pinned, 64 ints
   double *h_dsmall = nullptr;  // pinned, 64 doubles
 
@@ -154,7 +153,10 @@ struct emd_mail {
   int seq;
 };
 constexpr int EMD_MAIL_INTS = EMD_MAIL_DATA + EMD_MAIL_MAX;
-inline emd_mail emd_mail_next(emd_ctx *ctx) { return emd_mail{ctx->h_mail, ++ctx->mail_seq}; }
+inline int emd_mail_seq(emd_ctx *ctx) {  // (wraps)
+  return ctx->mail_seq = (int)((unsigned)ctx->mail_seq + 1u);
+}
+inline emd_mail emd_mail_next(emd_ctx *ctx) { return emd_mail{ctx->h_mail, emd_mail_seq(ctx)}; }
 // the payload of message m (valid until the next message is posted)
 emd_status emd_mail_wait(emd_ctx *ctx, const emd_mail &m, const int **payload);
 // the same at the end of a call whose arrays go with the count: they are
@@ -182,8 +184,6 @@ emd_status emd_grow_keep_int(emd_ctx *ctx, int **p, int *cap, long count, long k
 
 // -------------------------------------------------------- wave primitives
 #define EMD_WAVE 64
-
-__device__ __forceinline__ int emd_lane() { return __lane_id(); }
 
 __device__ __forceinline__ unsigned long long emd_lanemask_lt() {
   const int l = __lane_id();
@@ -610,32 +610,6 @@ inline neigh_geom emd_neigh_geom(const emd_bins *b) {
   g.nix = b->nbinx - 2 * b->nhalo; g.niy = b->nbiny - 2 * b->nhalo;
   g.niz = b->nbinz - 2 * b->nhalo;
   return g;
-}
-
-// the interior bin of block lr and its 27 stencil bins' offsets and
-// exclusive count prefix (s_pre[27] = candidates of the bin); call with
-// all threads of the block, blockDim.x >= 27
-__device__ __forceinline__ int emd_stencil_setup(const neigh_geom &g, int lr,
-                                                 const int *__restrict__ bincount,
-                                                 const int *__restrict__ binoffsets, int *s_off,
-                                                 int *s_pre) {
-  const int bx = lr / (g.niy * g.niz) + g.nhalo;
-  const int by = (lr / g.niz) % g.niy + g.nhalo;
-  const int bz = lr % g.niz + g.nhalo;
-  const int tid = threadIdx.x;
-  if (tid < 27) {
-    const int ddx = tid / 9 - 1, ddy = (tid / 3) % 3 - 1, ddz = tid % 3 - 1;
-    const int b = ((bx + ddx) * g.nby + (by + ddy)) * g.nbz + (bz + ddz);
-    s_off[tid] = binoffsets[b];
-    s_pre[tid + 1] = bincount[b];
-  }
-  __syncthreads();
-  if (tid == 0) {
-    s_pre[0] = 0;
-    for (int k = 1; k <= 27; k++) s_pre[k] += s_pre[k - 1];
-  }
-  __syncthreads();
-  return (bx * g.nby + by) * g.nbz + bz;
 }
 
 // stencil slot k of candidate c: s_pre[k] <= c < s_pre[k+1] (binary search)

@@ -1011,7 +1011,7 @@ extern "C" emd_status emd_fit_residual(emd_ctx *ctx, const emd_system *s, int pr
       EMD_LAUNCH(ctx, "fit_residual", k_fit_residual<double>, nb, FIT_THREADS, 0, s->f, f_target,
                  n3, g, nbf, start, eatom, e_target, w, econf, part);
   }
-  const emd_mail mail{ctx->h_mail + EMD_MAIL_INTS, ++ctx->mail_seq};
+  const emd_mail mail{ctx->h_mail + EMD_MAIL_INTS, emd_mail_seq(ctx)};
   EMD_LAUNCH(ctx, "fit_residual", k_fit_total, 1, 256, 0, part, nb, mail);
   ctx->fit_pending = true;
   ctx->fit_seq = mail.seq;

@@ -93,10 +93,6 @@ struct stab_entry {
   int a, b, cgoff, tid;
 };
 
-__device__ __forceinline__ int u_idx(const snap_dev_tables &t, int j, int ma, int mb) {
-  return t.ustart[j] + ma * (j + 1) + mb;
-}
-
 template <class T>
 struct cplx {
   T r, i;
@@ -191,10 +187,9 @@ __device__ __forceinline__ double snap_fdivr(double dx, double dy, double dz) {
 // With a force array given (f64 or f32), block i also zeroes its rows
 // i, i + n, i + 2n, ... below ntot (deep_copy(f, 0), src/examinimd.cpp:232,
 // done here instead of in a launch of its own: the force kernels that add
-// into f come after this one).  With p32 or p64 given, the slot's neighbour
-// parameters (snap_par, FP32 or FP64) and the repulsion F/r (fdv) are
-// written as well.
-// (the body of k_snap_neigh for atom i and one wavefront; returns the count)
+// into f come after this one).  The slot's neighbour parameters (par, in T) and
+// the repulsion F/r (fdv) are written as well.
+// (for atom i by one wavefront, in k_snap_neigh_ui; returns the count)
 template <class T>
 __device__ __forceinline__ int snap_compact(const snap_dev_tables &t, int i, const double *__restrict__ x,
                                             const int *__restrict__ row, const int *__restrict__ num,
@@ -252,18 +247,16 @@ __device__ __forceinline__ int snap_compact(const snap_dev_tables &t, int i, con
   return run < maxn ? run : maxn;
 }
 
-// the neighbour parameters of one precision (and the repulsion F/r) from the
-// compacted neighbours, for a U kernel of another precision than the one the
-// compaction wrote
-template <class T>
+// the neighbour parameters in FP64 (and the repulsion F/r) from the compacted
+// neighbours, for FP64 U_tot after a compaction that wrote FP32
 __global__ void __launch_bounds__(64)
 k_snap_par(snap_dev_tables t, const int *__restrict__ nin, const double *__restrict__ nr,
-           int maxn, int n, snap_par<T> *__restrict__ par, double *__restrict__ fdv) {
+           int maxn, int n, snap_par<double> *__restrict__ par, double *__restrict__ fdv) {
   const int i = blockIdx.x;
   if (i >= n) return;
   for (int k = threadIdx.x; k < nin[i]; k += 64) {
     const size_t o = (size_t)i * maxn + k;
-    snap_par_of<T>(t, nr[3 * o], nr[3 * o + 1], nr[3 * o + 2], par[o]);
+    snap_par_of<double>(t, nr[3 * o], nr[3 * o + 1], nr[3 * o + 2], par[o]);
     fdv[o] = snap_fdivr(nr[3 * o], nr[3 * o + 1], nr[3 * o + 2]);
   }
 }
@@ -1739,18 +1732,6 @@ static emd_status snap_scratch(emd_ctx *ctx, emd_snap *sn, int n, int maxn) {
   return EMD_OK;
 }
 
-// the neighbour parameters in T's precision (written by the compaction, or
-// here when it wrote the other precision)
-template <class T>
-static emd_status snap_par_ready(emd_ctx *ctx, emd_snap *sn, int n) {
-  const int prec = std::is_same<T, float>::value ? EMD_MIXED : EMD_FP64;
-  if (sn->par_prec == prec) return EMD_OK;
-  EMD_LAUNCH(ctx, "snap_neigh", k_snap_par<T>, n, 64, 0, sn->t, sn->nin, sn->nr, sn->cap_maxn, n,
-             (snap_par<T> *)sn->par, sn->fdv);
-  sn->par_prec = prec;
-  return EMD_OK;
-}
-
 // The compaction with the neighbour parameters in precision prec and U_tot of
 // every atom, in one launch.  zero_prec: EMD_FP64 or EMD_MIXED to zero that
 // precision's force array (all n_local + n_ghost rows) in the same launch, or -1.
@@ -1786,8 +1767,11 @@ static emd_status snap_neigh_ui(emd_ctx *ctx, const emd_system *s, const emd_nei
 
 // U_tot of every atom in FP64 from the last compaction
 static emd_status launch_ui(emd_ctx *ctx, emd_snap *sn, int n) {
-  EMD_TRY(snap_par_ready<double>(ctx, sn, n));
-  const snap_par<double> *par = (const snap_par<double> *)sn->par;
+  snap_par<double> *par = (snap_par<double> *)sn->par;
+  if (sn->par_prec != EMD_FP64)
+    EMD_LAUNCH(ctx, "snap_neigh", k_snap_par, n, 64, 0, sn->t, sn->nin, sn->nr, sn->cap_maxn, n,
+               par, sn->fdv);
+  sn->par_prec = EMD_FP64;
   if (sn->t.twojmax <= SNAP_MAXJ)
     EMD_LAUNCH(ctx, "snap_ui", (k_snap_ui_rg<double, SNAP_MAXJ>), n, 64, 0, sn->t, sn->rg_map_d,
                sn->nin, par, sn->cap_maxn, n, (double *)sn->u_r, (double *)sn->u_i);
@@ -1804,12 +1788,15 @@ static emd_status snap_y(emd_ctx *ctx, emd_snap *sn, int n) {
                                                     : (const cpair<T> *)sn->yf_w64;
   // Atoms per block: more of them share each code and weight load, but take
   // LDS from other blocks, and leave CUs without a block in small systems.
-  // us at twojmax 8 with 1 / 2 / 3 atoms: FP64 250 atoms 10.7 / 12.4 / 14.8,
-  // 432: 15.9 / 13.5 / 15.7, 16 000: 348 / 223 / 272; mixed 128 atoms 8.0 / 9.2 /
-  // 10.5, 1024: 20.3 / 14.5 / 15.3, 2000: 34 / 22.6 / 20.6, 16 000: 214 / 128 /
-  // 107: one while every atom can have a CU, in FP32 three once there are
-  // six per CU.  Twojmax 12 mixed, 2 (512 threads) / 4: 54 atoms 37 / 54, 1024:
-  // 79 / 71; FP64 with 512 / 1024 threads, two atoms, 1024: 162 / 151.
+  // us at twojmax 8 with 1 / 2 / 3 atoms per block: FP64 250 atoms 11.4 / 12.5 /
+  // 15.2, 300: 15.1 / 12.7 / 15.2, 2000: 51 / 34 / 39, 16 000: 348 / 223 / 272;
+  // mixed 250 atoms 9.4 / 9.5 / 11.1, 300: 11.8 / 9.6 / 11.1, 1024: 18.4 / 13.8 /
+  // 15.2, 1620: 27.4 / 20.6 / 20.6, 1800: 30.1 / 20.8 / 20.1, 16 000: 214 / 128 / 107:
+  // one while every atom can have a CU (256 of them), in FP32 three from six
+  // atoms per CU on.  Twojmax 12, where a block fills a CU's LDS, with 1 / 2 / 4:
+  // FP64 250 atoms 54 / 58, 300: 95 / 59, 1024: 204 / 139; mixed 250 atoms 34 / 32 /
+  // 54, 300: 54 / 33 / 54, 504: 62 / 42 / 57, 588: 81 / 63 / 58, 1024: 116 / 78 / 69:
+  // in FP32 four once blocks of two no longer have a CU each.
   auto launch = [&](auto jc, auto ac) -> emd_status {
     constexpr int J = jc, AT = ac;
     EMD_LAUNCH(ctx, "snap_y", (k_snap_yflat<T, J, AT>), (n + AT - 1) / AT, yf_threads<J>(), 0,
@@ -1822,13 +1809,14 @@ static emd_status snap_y(emd_ctx *ctx, emd_snap *sn, int n) {
   using A1 = std::integral_constant<int, 1>;
   using A2 = std::integral_constant<int, 2>;
   constexpr bool f32 = std::is_same<T, float>::value;
+  const int cus = ctx->num_cu;
   if (sn->t.twojmax > SNAP_MAXJ) {
-    if (n <= 256) return launch(J12{}, A1{});
-    if (f32 && n > 512) return launch(J12{}, std::integral_constant<int, f32 ? 4 : 2>{});
+    if (n <= cus) return launch(J12{}, A1{});
+    if (f32 && n > 2 * cus) return launch(J12{}, std::integral_constant<int, f32 ? 4 : 2>{});
     return launch(J12{}, A2{});
   }
-  if (n <= 256) return launch(J8{}, A1{});
-  if (f32 && n > 1536) return launch(J8{}, std::integral_constant<int, f32 ? 3 : 2>{});
+  if (n <= cus) return launch(J8{}, A1{});
+  if (f32 && n > 6 * cus) return launch(J8{}, std::integral_constant<int, f32 ? 3 : 2>{});
   return launch(J8{}, A2{});
 }
 
@@ -1836,7 +1824,6 @@ static emd_status snap_y(emd_ctx *ctx, emd_snap *sn, int n) {
 template <class T, class TF>
 static emd_status launch_fij(emd_ctx *ctx, emd_snap *sn, int n, const T *yr, const T *yi,
                              TF *f) {
-  EMD_TRY(snap_par_ready<T>(ctx, sn, n));
   const snap_par<T> *par = (const snap_par<T> *)sn->par;
   const int nb = RG_WAVES * (sn->t.twojmax <= SNAP_MAXJ ? rg<SNAP_MAXJ>::NB : rg<SNAP_JBIG>::NB);
   const dim3 grid(n, (sn->cap_maxn + nb - 1) / nb);
@@ -2234,8 +2221,7 @@ template <class T>
 static emd_status snap_adjoint_impl(emd_ctx *ctx, const emd_system *s, const emd_halo *h,
                                     emd_snap *sn, const double *g, double *S) {
   const int n = s->n_local;
-  // U_tot came with the compaction
-  EMD_TRY(snap_par_ready<T>(ctx, sn, n));
+  // the neighbour parameters (in T) and U_tot came with the compaction
   const snap_par<T> *par = (const snap_par<T> *)sn->par;
   if (sn->t.twojmax <= SNAP_MAXJ)
     EMD_LAUNCH(ctx, "snap_adjoint_w", (k_snap_w_rg<T, T, SNAP_MAXJ>), n, 64, 0, sn->t, sn->rg_map_d,
