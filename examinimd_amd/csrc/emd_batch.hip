@@ -64,6 +64,7 @@ struct emd_batch {
   int cap = 0;
   int *flags = nullptr;    // [0] largest row seen
   double *part = nullptr;  // thermo sums (4 * BT_SLICES per replica), then the masses
+  std::vector<float> f_host;  // mixed forces on their way to the caller's doubles
   double *save = nullptr;  // autotune snapshot: x, v, f (FP64 or FP32 bits)
   long step = 0;
   bool ready = false;
@@ -812,15 +813,6 @@ extern "C" emd_status emd_batch_upload(emd_ctx *ctx, emd_batch *b, const double 
   return EMD_OK;
 }
 
-// FP32 forces widened for the download, bound by HBM at 12 bytes a value: 0.3 ms
-// less for 661 000 atoms than on the host (a staging vector, its page faults and
-// one thread's loop), although twice the bytes are copied.
-__global__ void __launch_bounds__(256)
-k_bwiden(const float *__restrict__ f32, double *__restrict__ f, size_t n) {
-  const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) f[k] = (double)f32[k];
-}
-
 extern "C" emd_status emd_batch_download(emd_ctx *ctx, emd_batch *b, double *x, double *v,
                                          double *f) {
   if (!ctx || !b) return EMD_ERR_ARG;
@@ -831,18 +823,25 @@ extern "C" emd_status emd_batch_download(emd_ctx *ctx, emd_batch *b, double *x, 
   if (v)
     EMD_HIP(ctx, hipMemcpyAsync(v, b->v, n3 * sizeof(double), hipMemcpyDeviceToHost,
                                 ctx->stream));
+  // FP32 forces are copied as they are and widened here, through an array that
+  // the ensemble keeps: one made for each call costs its page faults (256
+  // replicas, 661 284 atoms: ~0.4 ms of a sampled run), widening on the device
+  // twice the bytes over PCIe (740 -> 870-920 us for the forces alone, 49 -> 82
+  // for 49 404 atoms)
+  std::vector<float> &f32 = b->f_host;
   if (f) {
-    const double *src = b->f;
     if (b->precision == EMD_MIXED) {
-      // into the position buffer that the next step overwrites
-      double *wide = b->x[1 - b->cur];
-      EMD_LAUNCH(ctx, "batch_download", k_bwiden, emd_blocks((long)n3, 256), 256, 0, b->f32, wide,
-                 n3);
-      src = wide;
+      f32.resize(n3);
+      EMD_HIP(ctx, hipMemcpyAsync(f32.data(), b->f32, n3 * sizeof(float), hipMemcpyDeviceToHost,
+                                  ctx->stream));
+    } else {
+      EMD_HIP(ctx, hipMemcpyAsync(f, b->f, n3 * sizeof(double), hipMemcpyDeviceToHost,
+                                  ctx->stream));
     }
-    EMD_HIP(ctx, hipMemcpyAsync(f, src, n3 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
   }
   EMD_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  if (f && b->precision == EMD_MIXED)
+    for (size_t k = 0; k < n3; k++) f[k] = (double)f32[k];
   return EMD_OK;
 }
 

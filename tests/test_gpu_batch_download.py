@@ -1,7 +1,7 @@
-"""emd_batch_download widens FP32 forces on the device, in the position buffer
-that the next step overwrites: the forces are FP32 values, a second download
-gives the same, and a run continued after a download (anywhere in a rebuild period, with
-and without graph replay) equals one that never downloaded, bit for bit."""
+"""emd_batch_download leaves the ensemble alone: the mixed forces are FP32
+values, a second download gives the same, and a run continued after a download
+(anywhere in a rebuild period, with and without graph replay) equals one that
+never downloaded, bit for bit."""
 import numpy as np
 import pytest
 
