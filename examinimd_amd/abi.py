@@ -73,7 +73,7 @@ class EmdBatchDesc(C.Structure):
 
 HIP_PROTOS = {
     "emd_create": (C.c_int, [C.c_int, P(vp)]),
-    "emd_set_early_counts": (C.c_int, [vp, C.c_int]),
+    "emd_set_early_counts": (C.c_int, [vp, C.c_int, iptr]),
     "emd_destroy": (C.c_int, [vp]),
     "emd_last_error": (C.c_char_p, [vp]),
     "emd_synchronize": (C.c_int, [vp]),

@@ -163,8 +163,9 @@ emd_status emd_mail_wait(emd_ctx *ctx, const emd_mail &m, const int **payload) {
   return EMD_OK;
 }
 
-extern "C" emd_status emd_set_early_counts(emd_ctx *ctx, int on) {
+extern "C" emd_status emd_set_early_counts(emd_ctx *ctx, int on, int *was) {
   if (!ctx) return EMD_ERR_ARG;
+  if (was) *was = ctx->early_counts;
   ctx->early_counts = on != 0;
   return EMD_OK;
 }

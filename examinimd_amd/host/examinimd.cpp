@@ -163,7 +163,8 @@ void ExaMiniMD::run(int nsteps) {
   // position update as one device step boundary (same operations, same order)
   bool deferred_final = false, deferred_fold = false;
   // every module here works on the context's stream
-  EMD_CALL(ctx, emd_set_early_counts(ctx, 1));
+  int early = 0;
+  EMD_CALL(ctx, emd_set_early_counts(ctx, 1, &early));
   for (int step = 1; step <= nsteps; step++) {
     const bool rebuild = step % input->comm_exchange_rate == 0 && step > 0;
     bool halo_updated = false;
@@ -286,7 +287,7 @@ void ExaMiniMD::run(int nsteps) {
     fence();
     other_time += other_timer.seconds();
   }
-  EMD_CALL(ctx, emd_set_early_counts(ctx, 0));
+  EMD_CALL(ctx, emd_set_early_counts(ctx, early, nullptr));
   EMD_CALL(ctx, emd_synchronize(ctx));
   double time = timer.seconds();
   time_total += time;

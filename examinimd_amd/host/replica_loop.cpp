@@ -81,6 +81,8 @@ extern "C" int emd_replica_loop_run(emd_ctx *ctx, const emd_batch_desc *d, const
     if (!st) st = force(ctx, r, p, d->precision);
     off += r.n;
   }
+  int early = 0;  // all of it is on the context's stream
+  if (!st) st = emd_set_early_counts(ctx, 1, &early);
   if (!st) st = emd_synchronize(ctx);
   const auto t0 = std::chrono::steady_clock::now();
   for (int step = 1; step <= nsteps && !st; step++) {
@@ -93,6 +95,7 @@ extern "C" int emd_replica_loop_run(emd_ctx *ctx, const emd_batch_desc *d, const
       if ((st = emd_nve_final(ctx, &r.s, dtf, d->precision))) break;
     }
   }
+  emd_set_early_counts(ctx, early, nullptr);
   if (!st) st = emd_synchronize(ctx);
   const auto t1 = std::chrono::steady_clock::now();
   if (seconds) *seconds = std::chrono::duration<double>(t1 - t0).count();

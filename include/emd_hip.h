@@ -63,9 +63,9 @@ void       *emd_get_stream(emd_ctx *ctx);   /* the hipStream_t all work runs on 
  * emd_comm_exchange_halo and emd_neigh_build return as soon as their counts
  * are known, while kernels that fill their arrays may still run.  For callers
  * that use those arrays only through this library or on the context's stream.
- * Default: off (emd_app_run turns it on for its context while it runs, and
- * off). */
-emd_status  emd_set_early_counts(emd_ctx *ctx, int on);
+ * Default: off; *was (or NULL) receives the setting so far (emd_app_run and
+ * emd_replica_loop_run turn it on for their context while they run). */
+emd_status  emd_set_early_counts(emd_ctx *ctx, int on, int *was);
 const char *emd_version(void);
 
 /* device memory for callers (fixtures, tests, host modules) */

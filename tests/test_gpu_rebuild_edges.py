@@ -80,7 +80,9 @@ def test_arrays_are_complete_with_their_counts(n):
     got = []
     for early in (0, 1):
         if early:
-            pl.chk(L.emd_set_early_counts(c, 1), "early counts")
+            was = C.c_int(-1)
+            pl.chk(L.emd_set_early_counts(c, 1, C.byref(was)), "early counts")
+            assert was.value == 0
         idle, out = [], []
 
         def took(*arrays):
