@@ -325,8 +325,8 @@ __device__ __forceinline__ void y_entry(const snap_dev_tables &t, int e, int &J,
 // each entry adds its runs in thread order (fixed order: deterministic).
 // With AT atoms per block (U_tot of each in LDS) every code and weight load
 // serves AT atoms.
-// Arithmetic (47 % of its issue rate at 16 000 atoms in FP64), LDS reads (40
-// %) and the stream from L2 (54 % of the address units, 14 TB/s) bound it
+// Arithmetic (54 % of its issue rate at 16 000 atoms in FP64), LDS reads (65
+// %) and the stream from L2 (76 % of the address units, 18 TB/s) bound it
 // about equally, so all three had to shrink: one product at a time with the
 // middle columns in full took 303 us for 16 000 atoms (FP64, twojmax 8), 24.4
 // for 2000 (mixed), 222 / 109 for 1024 atoms at twojmax 12 (FP64 / mixed); this
@@ -574,8 +574,8 @@ __global__ void k_yf_weights(int nslots, const unsigned short *__restrict__ key,
 // not exist (ma > j): the borders need no test, and what the lane shifts
 // carry over a group's edge meets only such zeros.  The norm is applied once
 // per atom, to the sums over the neighbours or to Y.
-// FP64 (FP32) arithmetic bounds all three kernels (70 % of its issue rate in
-// the force kernel).  Against U with its factors, FP64, 16 000 atoms of 26
+// FP64 (FP32) arithmetic bounds all three kernels (75 % of its issue rate in
+// the force kernel and W, 70 % in U_tot).  Against U with its factors, FP64, 16 000 atoms of 26
 // neighbours, twojmax 8: U_tot 174 -> 82 us, force 232 -> 144 us; W of 64 BCC
 // configurations of 128 to 1024 atoms 820 -> 262 us; mixed, 2000 atoms:
 // 24.4 -> 15.9 and 28.6 -> 14.9 us.  Twojmax 12,
