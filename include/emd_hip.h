@@ -406,7 +406,9 @@ emd_status emd_lj_adjoint_atoms(emd_ctx *ctx, const emd_system *s, const emd_nei
  * eatom and e_target DEVICE; nconf = 0 leaves the energies out (start,
  * eatom, e_target and w may then be NULL).  econf (DEVICE double[nconf],
  * not e_target, or NULL) receives the E_c.  Does not wait: emd_fit_loss
- * returns the loss of the last call (EMD_ERR_STATE without one). */
+ * returns the loss of the last call (EMD_ERR_STATE without one).  Not for
+ * capture into a graph: the loss is told from earlier ones by a number that
+ * every call takes. */
 emd_status emd_fit_residual(emd_ctx *ctx, const emd_system *s, int precision,
                             const double *f_target, double *g, int nconf, const int *start,
                             const double *eatom, const double *e_target, double *w,
