@@ -131,7 +131,7 @@ k_bin_order(const int *__restrict__ count, const int *__restrict__ offset, int n
 // (mostly broadcasts) where one thread per bin sorting its slice by insertion
 // made a chain of ~170 dependent LDS reads and writes.  Bound: LDS latency
 // and the launch.  A call for the locals and ghosts of an LJ melt, host wait
-// included: 72 -> 13 us at 864 atoms (32 per bin), 75 -> 14 us at 2048; the
+// included, early counts: 72 -> 13 us at 864 atoms (32 per bin), 75 -> 14 us at 2048; the
 // counting sort takes 16 us from 4000 atoms (8000 with ghosts) on.
 constexpr int BIN_ONE_THREADS = 1024;
 constexpr int BIN_ONE_MAX_BINS = 4096;

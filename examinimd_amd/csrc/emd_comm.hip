@@ -198,7 +198,7 @@ __device__ __forceinline__ int halo_bases(const halo_args &a, int tot, int *s_ph
 constexpr int HALO_ONE_THREADS = 1024;
 // local atoms in one workgroup: a whole call takes 14 / 20 / 30 us there with
 // 864 / 2048 / 4000 atoms of an LJ melt and 20 / 20 / 19 us with the three
-// kernels (host wait included; 60 / 68 / 76 us with one pass per phase, and
+// kernels (host wait included, early counts; 60 / 68 / 76 us with one pass per phase, and
 // 194 us from 16 384 atoms on where the three kernels take 19-22)
 constexpr int HALO_ONE_MAX = 2048;
 constexpr int HALO_ONE_WAVES = HALO_ONE_THREADS / EMD_WAVE;
